@@ -30,19 +30,49 @@ static bool pretranspose_pays(int64_t M, int64_t N, int64_t K, int64_t other, in
            (M / 256) * (N / 256) >= 128 && K >= 1024 && other >= 4096 && ld == rows && aligned16(p);
 }
 
+template <typename T>
+static DenseArgs<T> dense_args(bool a_kmajor, bool b_kmajor, int64_t M, int64_t N, int64_t K, const T* A, int64_t lda, const T* B,
+                               int64_t ldb, const T* bias, T* C, int64_t ldc, T* pre, int act) {
+    DenseArgs<T> a;
+    a.A.p = A;
+    a.A.sr = a_kmajor ? lda : 1;
+    a.A.sk = a_kmajor ? 1 : lda;
+    a.A.rows = (int)M;
+    a.A.vec_ok = aligned16(A) && (lda * sizeof(T)) % 16 == 0;
+    a.B.p = B;
+    a.B.sr = b_kmajor ? ldb : 1;
+    a.B.sk = b_kmajor ? 1 : ldb;
+    a.B.rows = (int)N;
+    a.B.vec_ok = aligned16(B) && (ldb * sizeof(T)) % 16 == 0;
+    a.M = (int)M; a.N = (int)N; a.K = (int)K;
+    a.C = C; a.ldc = ldc; a.bias = bias; a.pre = pre; a.act = act;
+    a.c_vec = (reinterpret_cast<uintptr_t>(C) & 7u) == 0 && (reinterpret_cast<uintptr_t>(pre) & 7u) == 0 && ldc % 4 == 0;
+    return a;
+}
+
+// dW (M x K) = dz (M x N) * x' and dx (K x N) = W' * dz in one launch; false if they are not small enough for it
+template <typename T>
+static bool gradient_pair(hipStream_t s, int64_t M, int64_t K, int64_t N, const T* dz, const T* W, int64_t ldw, const T* x, int64_t ldx,
+                          T* dW, T* dx, int* rc) {
+    if (gemm_tile_override() != 0 || M < 1 || N < 1 || K < 1 || ldw < M || ldx < K) return false;
+    DenseArgs<T> a = dense_args<T>(false, false, M, K, N, dz, M, x, ldx, nullptr, dW, M, nullptr, LUXHIP_ACT_IDENTITY);
+    DenseArgs<T> b = dense_args<T>(true, true, K, N, M, W, ldw, dz, M, nullptr, dx, K, nullptr, LUXHIP_ACT_IDENTITY);
+    return launch_split_pair<T>(s, a, b, rc);
+}
+
 // ws_front: bytes at the start of the stream's workspace that the caller is using (operand copies go behind them)
 template <typename T>
 static int gemm_impl(hipStream_t s, int transA, int transB, int64_t M, int64_t N, int64_t K, const T* A, int64_t lda,
                      const T* B, int64_t ldb, const T* bias, T* C, int64_t ldc, T* pre, int act, size_t ws_front = 0) {
-    DenseArgs<T> a;
-    bool a_kmajor = transA != 0, b_kmajor = transB == 0;
+    bool a_kmajor = transA != 0, b_kmajor = transB == 0, copied = false;
     if constexpr (sizeof(T) == 2) {
         bool ta = !a_kmajor && pretranspose_pays<T>(M, N, K, N, lda, M, A);
         bool tb = !b_kmajor && pretranspose_pays<T>(M, N, K, M, ldb, N, B);
         // only the kernel with both operands K-major is faster (a mixed pair is not), and two copies
         // need a longer K to pay than one (measured: 4096 x 4096 x 1024 loses, x 4096 wins)
         if (!((a_kmajor || ta) && (b_kmajor || tb)) || (ta && tb && K < 2048)) ta = tb = false;
-        if (ta || tb) {
+        copied = ta || tb;
+        if (copied) {
             const size_t ab = ta ? (((size_t)M * K * sizeof(T) + 255) & ~size_t(255)) : 0;
             const size_t bb = tb ? (size_t)N * K * sizeof(T) : 0;
             Workspace ws;
@@ -61,19 +91,11 @@ static int gemm_impl(hipStream_t s, int transA, int transB, int64_t M, int64_t N
             }
         }
     }
-    a.A.p = A;
-    a.A.sr = a_kmajor ? lda : 1;
-    a.A.sk = a_kmajor ? 1 : lda;
-    a.A.rows = (int)M;
-    a.A.vec_ok = aligned16(A) && (lda * sizeof(T)) % 16 == 0;
-    a.B.p = B;
-    a.B.sr = b_kmajor ? ldb : 1;
-    a.B.sk = b_kmajor ? 1 : ldb;
-    a.B.rows = (int)N;
-    a.B.vec_ok = aligned16(B) && (ldb * sizeof(T)) % 16 == 0;
-    a.M = (int)M; a.N = (int)N; a.K = (int)K;
-    a.C = C; a.ldc = ldc; a.bias = bias; a.pre = pre; a.act = act;
-    a.c_vec = (reinterpret_cast<uintptr_t>(C) & 7u) == 0 && (reinterpret_cast<uintptr_t>(pre) & 7u) == 0 && ldc % 4 == 0;
+    DenseArgs<T> a = dense_args<T>(a_kmajor, b_kmajor, M, N, K, A, lda, B, ldb, bias, C, ldc, pre, act);
+    if (gemm_tile_override() == 0 && !copied) {       // (operand copies occupy the workspace that it would use)
+        int rc = LUXHIP_OK;
+        if (launch_split<T>(s, a, a_kmajor, b_kmajor, ws_front, &rc)) return rc;
+    }
     if (a_kmajor && b_kmajor) return launch_layout<T, true, true>(s, a);
     if (a_kmajor) return launch_layout<T, true, false>(s, a);
     if (b_kmajor) return launch_layout<T, false, true>(s, a);
@@ -424,6 +446,12 @@ int luxhip_fused_dense_bwd(luxhip_stream_t s, int dtype, int act, int64_t M, int
         rc = bias_act_bwd_dispatch((hipStream_t)s, dtype, act, 1, M, N, delta, y, pre, dz_out, dbias);
         if (rc != LUXHIP_OK) return rc;
         if (dz_out) dzp = dz_out;
+    }
+    if (dW != nullptr && dx != nullptr && W != nullptr && x != nullptr) {
+        const bool done = dtype == LUXHIP_F32
+            ? gradient_pair<float>((hipStream_t)s, M, K, N, (const float*)dzp, (const float*)W, ldw, (const float*)x, ldx, (float*)dW, (float*)dx, &rc)
+            : gradient_pair<bf16_t>((hipStream_t)s, M, K, N, (const bf16_t*)dzp, (const bf16_t*)W, ldw, (const bf16_t*)x, ldx, (bf16_t*)dW, (bf16_t*)dx, &rc);
+        if (done) return rc;
     }
     if (dW != nullptr) {   // dW (M x K) = dz (M x N) * x' (N x K);  x is stored K x N
         rc = gemm_dispatch((hipStream_t)s, dtype, 0, 1, M, K, N, dzp, std::max<int64_t>(M, 1), x, ldx, nullptr, dW,

@@ -1,0 +1,67 @@
+"""Products with few tiles or ragged operands (gemm_split.h) against the fp64 oracle: every
+layout at the edges of tiles, stages and slices, and the fused layer whose two gradient products share a launch."""
+import numpy as np
+import pytest
+
+from oracle import luxlib_oracle as O
+from tests.util import assert_close, dev, f64, host_inputs, rms, stable_seed
+
+pytestmark = pytest.mark.gpu
+
+# below / at / above a tile of 64 and of 128, rows of fewer than two vectors, K of one stage, of a stage and a bit, of
+# several slices with a ragged last one
+SHAPES = [(8, 9, 32), (64, 64, 33), (65, 63, 64), (9, 130, 95), (129, 64, 4099), (130, 131, 1023), (517, 301, 70), (640, 1030, 45)]
+
+
+@pytest.mark.parametrize("dtype", ["f32", "bf16"])
+@pytest.mark.parametrize("transA", [False, True])
+@pytest.mark.parametrize("transB", [False, True])
+def test_ragged_products(gpu, dtype, transA, transB):
+    rng = np.random.default_rng(stable_seed("ragged", dtype, transA, transB))
+    for (M, N, K) in SHAPES:
+        A = rng.normal(size=(K, M) if transA else (M, K))
+        B = rng.normal(size=(N, K) if transB else (K, N))
+        A, B, bias = host_inputs(dtype, A, B, rng.normal(size=M))
+        want = (f64(A).T if transA else f64(A)) @ (f64(B).T if transB else f64(B)) + f64(bias)[:, None]
+        got = gpu.matmul(dev(gpu, A, dtype), dev(gpu, B, dtype), dev(gpu, bias, dtype), transA, transB).to_numpy()
+        again = gpu.matmul(dev(gpu, A, dtype), dev(gpu, B, dtype), dev(gpu, bias, dtype), transA, transB).to_numpy()
+        assert_close(got, want, dtype, f"{dtype} ragged matmul {M}x{N}x{K} tA={transA} tB={transB}")
+        np.testing.assert_array_equal(got, again)          # slices are added in a fixed order
+
+
+@pytest.mark.parametrize("dtype", ["f32", "bf16"])
+def test_zeroed_overlap_is_not_multiplied(gpu, dtype):
+    """The last stage repeats k that are done: they count as zero in both operands, so an infinity there must not turn
+    into a NaN and must count once."""
+    M, N, K = 70, 66, 45
+    A, B = np.ones((M, K)), np.ones((K, N))
+    A[3, 20] = np.inf                                       # k = 20 lies in the part of the last stage that is repeated
+    for transA in (False, True):
+        got = gpu.matmul(dev(gpu, A.T if transA else A, dtype), dev(gpu, B, dtype), None, transA, False).to_numpy()
+        want = np.full((M, N), float(K))
+        want[3] = np.inf
+        np.testing.assert_array_equal(got, want)
+
+
+@pytest.mark.parametrize("dtype", ["f32", "bf16"])
+@pytest.mark.parametrize("act", ["identity", "tanh", "gelu"])
+def test_fused_layer_with_gradients_in_one_launch(gpu, dtype, act):
+    rng = np.random.default_rng(stable_seed("pair", dtype, act))
+    for (M, K, N) in [(64, 32, 32), (65, 47, 33), (200, 300, 70), (130, 64, 515)]:
+        W, x, b, delta = host_inputs(dtype, rng.normal(size=(M, K)) / np.sqrt(K), rng.normal(size=(K, N)), 0.1 * rng.normal(size=M),
+                                     rng.normal(size=(M, N)))
+        y, back = gpu.pullback(gpu.fused_dense_bias_activation, act, *(dev(gpu, a, dtype) for a in (W, x, b)))
+        gW, gx, gb = back(dev(gpu, delta, dtype))
+        wy, wdW, wdx, wdb = O.fused_dense_pullback(act, f64(W), f64(x), f64(b), f64(delta))
+        dz = O.grad_activation(f64(delta), wy, act, O.matmuladd(f64(W), f64(x), f64(b)))
+        if dtype == "bf16":                                 # y, the pre-activation and dz are stored in bf16 in between
+            pre = f64(O.round_to_bf16(O.matmuladd(f64(W), f64(x), f64(b)).astype(np.float32)))
+            dz = O.grad_activation(f64(delta), f64(O.round_to_bf16(wy.astype(np.float32))), act, pre)
+            wdb = dz.sum(axis=1)
+            dz = f64(O.round_to_bf16(dz.astype(np.float32)))
+            wdW, wdx = dz @ f64(x).T, f64(W).T @ dz
+        tag = f"{dtype} {act} {M}x{K}x{N}"
+        assert_close(y.to_numpy(), wy, dtype, tag + " y")
+        assert_close(gW.to_numpy(), wdW, dtype, tag + " dW", scale=np.sqrt(N) * rms(dz) * rms(x))
+        assert_close(gx.to_numpy(), wdx, dtype, tag + " dx", scale=np.sqrt(M) * rms(dz) * rms(W))
+        assert_close(gb.to_numpy(), wdb, dtype, tag + " db")
