@@ -42,6 +42,9 @@ int launch_layout(hipStream_t s, DenseArgs<T>& a);
 template <typename T, bool A_KMAJOR, bool B_KMAJOR>
 int launch_batched_layout(hipStream_t s, DenseArgs<T>& a);
 
+// gemm_skinny.hip: at most 16 columns, A contiguous along m, B along k; false if the problem is another one
+template <typename T>
+bool launch_skinny(hipStream_t s, DenseArgs<T>& a, bool a_kmajor, bool b_kmajor, size_t ws_front, int* rc);
 // gemm_split_*.hip: products with few tiles or ragged operands; false if the problem is not theirs
 template <typename T>
 bool launch_split(hipStream_t s, DenseArgs<T>& a, bool a_kmajor, bool b_kmajor, size_t ws_front, int* rc);

@@ -1,0 +1,208 @@
+// y (M x N) = act.(W (M x K) * x (K x N) .+ bias) for a few columns (N <= 16): serving a handful of tokens.
+//
+// Bound by reading W once (rows of W contiguous along m).  A wave covers 128 (bf16) or 64 (fp32) consecutive m with its
+// sixteen lanes of a quarter, 16 bytes each, and takes 32 (16) k at a time, 8 (4) rows per quarter: eight (four) loads of
+// 1 KiB, all of them cache lines that are used whole.  The matrix instructions take any assignment of rows to lanes as
+// long as both operands agree, so the loaded registers are A fragments as they come in fp32, and after an in-lane 8 x 8
+// transpose of 16-bit values (one v_perm_b32 per dword) in bf16: no LDS, no barrier in the loop.  The sixteen columns of
+// the instruction hold the N columns of x (the others repeat the last one and are not stored).  The next 32 k are
+// requested before the current ones are used.
+//
+// Eight waves of a workgroup split its k range and add up in LDS; `slices` workgroups share a block of m, hand their sums
+// over through device memory, and the last one to arrive adds them in slice order.
+#include <algorithm>
+
+#include "common.h"
+#include "gemm_core.h"
+#include "gemm_dense_decl.h"
+
+namespace luxhip {
+namespace skinny {
+
+constexpr int WAVES = 8, THREADS = WAVES * 64, NMAX = 16;
+typedef float f32x4_v __attribute__((ext_vector_type(4)));
+template <typename T>
+struct Elem;
+template <>
+struct Elem<float> {
+    static constexpr int V = 4;                 // elements per 16 bytes: m per lane, and k per quarter and step
+    typedef uint32_t vec __attribute__((ext_vector_type(4), aligned(4)));
+};
+template <>
+struct Elem<bf16_t> {
+    static constexpr int V = 8;
+    typedef uint32_t vec __attribute__((ext_vector_type(4), aligned(2)));
+};
+
+template <typename T>
+struct Args {
+    const T *W, *x, *bias;
+    T *y, *pre;
+    int64_t ldw, ldx, ldy;
+    int M, N, K, act, slices, kwave;            // kwave: k per wave, a multiple of 4 V
+    float* partial;                             // [block of m][slice][N][16 V]
+    uint32_t* counters;
+};
+
+template <typename T>
+__global__ __launch_bounds__(THREADS) void skinny_gemm_kernel(Args<T> a) {
+    constexpr int V = Elem<T>::V, MT = 16 * V, KSTEP = 4 * V;
+    using vec = typename Elem<T>::vec;
+    __shared__ float sums[WAVES][NMAX * MT];
+    __shared__ uint32_t flag;
+    const int block = blockIdx.x / a.slices, slice = blockIdx.x - block * a.slices;
+    const int m0 = min(block * MT, a.M - MT);
+    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), l = threadIdx.x & 63, lm = l & 15, lq = l >> 4;
+    const int kbeg = (slice * WAVES + w) * a.kwave, kend = min(kbeg + a.kwave, a.K);
+    f32x4_v acc[V];
+#pragma unroll
+    for (int i = 0; i < V; ++i) acc[i] = f32x4_v{0.0f, 0.0f, 0.0f, 0.0f};
+    const T* wp = a.W + m0 + lm * V;
+    const T* xp = a.x + (int64_t)min(lm, a.N - 1) * a.ldx;
+    u32x4_v rw[2][V], rx[2];
+    auto fetch_step = [&](int k, u32x4_v (&dw)[V], u32x4_v& dx) {
+        const int kl = k + lq * V;
+        if (k + KSTEP <= a.K) {                                 // uniform
+#pragma unroll
+            for (int j = 0; j < V; ++j) dw[j] = *reinterpret_cast<const vec*>(wp + (int64_t)(kl + j) * a.ldw);
+            dx = *reinterpret_cast<const vec*>(xp + kl);
+        } else {                                                // past the end of K both operands are zero
+            T e[V];
+#pragma unroll
+            for (int j = 0; j < V; ++j) {
+                dw[j] = u32x4_v{0u, 0u, 0u, 0u};
+                e[j] = T(0);
+                if (kl + j < a.K) {
+                    dw[j] = *reinterpret_cast<const vec*>(wp + (int64_t)(kl + j) * a.ldw);
+                    e[j] = xp[kl + j];
+                }
+            }
+            dx = *reinterpret_cast<const u32x4_v*>(e);
+        }
+    };
+    auto multiply = [&](const u32x4_v (&dw)[V], const u32x4_v& dx) {
+        if constexpr (sizeof(T) == 4) {
+#pragma unroll
+            for (int j = 0; j < V; ++j)
+#pragma unroll
+                for (int i = 0; i < V; ++i)
+                    acc[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(__uint_as_float(dw[j][i]), __uint_as_float(dx[j]), acc[i], 0, 0, 0);
+        } else {
+            const bf16x8_v b = __builtin_bit_cast(bf16x8_v, dx);
+#pragma unroll
+            for (int i = 0; i < V; ++i) {                       // row i of the lane's eight: element i of each of the eight loads
+                u32x4_v f;
+#pragma unroll
+                for (int p = 0; p < 4; ++p)
+                    f[p] = __builtin_amdgcn_perm(dw[2 * p + 1][i / 2], dw[2 * p][i / 2], (i & 1) ? 0x07060302u : 0x05040100u);
+                acc[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_v, f), b, acc[i], 0, 0, 0);
+            }
+        }
+    };
+    if (kbeg < kend) {
+        fetch_step(kbeg, rw[0], rx[0]);
+        int k = kbeg;
+        for (; k + 2 * KSTEP <= kend; k += 2 * KSTEP) {
+            fetch_step(k + KSTEP, rw[1], rx[1]);
+            multiply(rw[0], rx[0]);
+            if (k + 2 * KSTEP < kend) fetch_step(k + 2 * KSTEP, rw[0], rx[0]);
+            multiply(rw[1], rx[1]);
+        }
+        if (k < kend) {
+            const bool more = k + KSTEP < kend;
+            if (more) fetch_step(k + KSTEP, rw[1], rx[1]);
+            multiply(rw[0], rx[0]);
+            if (more) multiply(rw[1], rx[1]);
+        }
+    }
+    // acc[i][r] of lane l: m = m0 + (4 (l / 16) + r) V + i, n = l % 16
+    if (lm < a.N) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+#pragma unroll
+            for (int i = 0; i < V; ++i) sums[w][lm * MT + (4 * lq + r) * V + i] = acc[i][r];
+    }
+    __syncthreads();
+    const int total = a.N * MT;
+    float v[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+        const int e = threadIdx.x + u * THREADS;
+        v[u] = 0.0f;
+        if (e < total)
+#pragma unroll
+            for (int q = 0; q < WAVES; ++q) v[u] += sums[q][e];
+    }
+    if (a.slices > 1) {
+        float* mine = a.partial + ((size_t)block * a.slices + slice) * (NMAX * MT);
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const int e = threadIdx.x + u * THREADS;
+            if (e < total) publish(mine + e, v[u]);
+        }
+        publish_done();
+        if (!arrive_last(a.counters + block, (uint32_t)a.slices, &flag)) return;
+        const float* all = a.partial + (size_t)block * a.slices * (NMAX * MT);
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const int e = threadIdx.x + u * THREADS;
+            v[u] = 0.0f;
+            if (e < total)
+#pragma unroll 4
+                for (int q = 0; q < a.slices; ++q) v[u] += fetch(all + (size_t)q * (NMAX * MT) + e);
+        }
+    }
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+        const int e = threadIdx.x + u * THREADS;
+        if (e < total) {
+            const int n = e / MT, m = m0 + e % MT;
+            const int64_t off = (int64_t)n * a.ldy + m;
+            float o[1] = {v[u] + (a.bias ? ld(a.bias + m) : 0.0f)};
+            if (a.pre) st(a.pre + off, o[0]);
+            act_vec(a.act, o);
+            st(a.y + off, o[0]);
+        }
+    }
+}
+
+template <typename T>
+int launch(hipStream_t s, const DenseArgs<T>& d, size_t ws_front) {
+    constexpr int V = Elem<T>::V, MT = 16 * V, KSTEP = 4 * V;
+    Args<T> a;
+    a.W = d.A.p; a.x = d.B.p; a.bias = d.bias; a.y = d.C; a.pre = d.pre;
+    a.ldw = d.A.sk; a.ldx = d.B.sr; a.ldy = d.ldc;
+    a.M = d.M; a.N = d.N; a.K = d.K; a.act = d.act;
+    const int64_t cus = num_cus() > 0 ? num_cus() : 256, blocks = ceil_div(d.M, MT);
+    // at most one workgroup (eight waves with sixteen loads in flight each) per compute unit: a second one gains nothing
+    // (11008 x 4096: 18.6 us against 20.4 with two in bf16, 29.7 against 38.2 in fp32); at least two steps of k per wave
+    int64_t slices = std::max<int64_t>(1, std::min<int64_t>(cus / blocks, d.K / (2 * KSTEP * WAVES)));
+    if (blocks > (int64_t)kWorkspaceCounters) slices = 1;
+    a.kwave = (int)(ceil_div(ceil_div(d.K, slices * WAVES), KSTEP) * KSTEP);
+    a.slices = (int)ceil_div(d.K, (int64_t)a.kwave * WAVES);
+    a.partial = nullptr; a.counters = nullptr;
+    if (a.slices > 1) {
+        Workspace ws;
+        const int rc = get_workspace(s, ws_front + (size_t)blocks * a.slices * NMAX * MT * sizeof(float), &ws);
+        if (rc != LUXHIP_OK) return rc;
+        a.partial = reinterpret_cast<float*>(ws.data + ws_front);
+        a.counters = ws.counters;
+    }
+    ProfScope ps(sizeof(T) == 2 ? "skinny_gemm_kernel<bf16>" : "skinny_gemm_kernel<f32>", s);
+    skinny_gemm_kernel<T><<<dim3((unsigned)(blocks * a.slices)), dim3(THREADS), 0, s>>>(a);
+    LUX_CHECK_LAUNCH();
+    return LUXHIP_OK;
+}
+
+}  // namespace skinny
+
+template <typename T>
+bool launch_skinny(hipStream_t s, DenseArgs<T>& d, bool ak, bool bk, size_t ws_front, int* rc) {
+    if (ak || !bk || d.N > skinny::NMAX || d.N < 1 || d.M < 16 * skinny::Elem<T>::V || d.K < 1) return false;
+    *rc = skinny::launch<T>(s, d, ws_front);
+    return true;
+}
+template bool launch_skinny<float>(hipStream_t, DenseArgs<float>&, bool, bool, size_t, int*);
+template bool launch_skinny<bf16_t>(hipStream_t, DenseArgs<bf16_t>&, bool, bool, size_t, int*);
+
+}  // namespace luxhip

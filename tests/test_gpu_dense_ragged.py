@@ -1,5 +1,6 @@
-"""Products with few tiles or ragged operands (gemm_split.h) against the fp64 oracle: every
-layout at the edges of tiles, stages and slices, and the fused layer whose two gradient products share a launch."""
+"""Products with few tiles, ragged operands or few columns (gemm_split.h, gemm_skinny.hip) against the fp64 oracle: every
+layout at the edges of tiles, stages and slices, the fused layer whose two gradient products share a launch, and the layer
+that a handful of tokens pass through."""
 import numpy as np
 import pytest
 
@@ -65,3 +66,16 @@ def test_fused_layer_with_gradients_in_one_launch(gpu, dtype, act):
         assert_close(gW.to_numpy(), wdW, dtype, tag + " dW", scale=np.sqrt(N) * rms(dz) * rms(x))
         assert_close(gx.to_numpy(), wdx, dtype, tag + " dx", scale=np.sqrt(M) * rms(dz) * rms(W))
         assert_close(gb.to_numpy(), wdb, dtype, tag + " db")
+
+
+@pytest.mark.parametrize("dtype", ["f32", "bf16"])
+@pytest.mark.parametrize("act", ["identity", "gelu"])
+def test_few_columns(gpu, dtype, act):
+    rng = np.random.default_rng(stable_seed("skinny", dtype, act))
+    for (M, N, K) in [(128, 1, 1), (131, 16, 31), (256, 2, 32), (300, 5, 1000), (2055, 3, 4097), (64, 15, 517)]:
+        W, x, b = host_inputs(dtype, rng.normal(size=(M, K)) / np.sqrt(K), rng.normal(size=(K, N)), rng.normal(size=M))
+        args = tuple(dev(gpu, a, dtype) for a in (W, x, b))
+        want = O.fused_dense_pullback(act, f64(W), f64(x), f64(b), np.zeros((M, N)))[0]
+        got = gpu.fused_dense_bias_activation(act, *args).to_numpy()
+        assert_close(got, want, dtype, f"{dtype} {act} {M}x{N}x{K}")
+        np.testing.assert_array_equal(got, gpu.pullback(gpu.fused_dense_bias_activation, act, *args)[0].to_numpy())
