@@ -1,12 +1,14 @@
 // Convolution entry points: layout transforms, filter repacking, launch logic of the
 // implicit-GEMM kernels (conv_kernels.h) and the split-K reduction of the filter gradient.
 #include <algorithm>
+#include <vector>
 
 #include "common.h"
 #include "act_vec.h"
 #include "conv_kernels.h"
 #include "conv_patch.h"
 #include "conv_wgrad_patch.h"
+#include "conv_any.h"
 
 namespace luxhip {
 
@@ -127,6 +129,116 @@ __global__ __launch_bounds__(256) void whcn_to_cwhn_pack_kernel(const T* __restr
     }
 }
 
+// Channel-contiguous copy with the channels of every group padded with zeros to Cp, for any number of positions and
+// channels: out (groups * Cp, P, N) from in (P, groups * Cg, N), 16-byte stores.  Tiles of 64 positions x 64 padded channels
+// go through LDS; the reads are one element per lane (64 consecutive positions of a channel per wave), since the rows of a
+// ragged plane start at any address.  `zeros` positions of zeros follow the last image.  Blocks behind the transform's
+// repack the filter.
+struct PackSub {
+    int rw, rh, s0w, stw, s0h, sth;      // residue and tap shifts (shift s of residue r is tap (s stride + r) / dilation)
+    int TW, K, Kpad, merged_w;           // merged_w > 0: the residue comes from the column, merged_w residues along w
+    int64_t wm, first;                   // element offset in the packed filter; first element of this part
+};
+struct PackSubs {
+    PackSub sub[cany::MAX_SUBS];
+    int n, dgrad, Cp, Ncols, Cch, grp;
+    int64_t total;
+};
+template <typename T>
+__device__ __forceinline__ void pack_sub_element(const T* __restrict__ w, T* __restrict__ out, const ConvGeom& g, const PackSubs& ps, int64_t idx) {
+    if (idx >= ps.total) return;
+    PackSub q = ps.sub[0];
+#pragma unroll
+    for (int i = 1; i < cany::MAX_SUBS; ++i)
+        if (i < ps.n && idx >= ps.sub[i].first) q = ps.sub[i];
+    const int e = (int)(idx - q.first);
+    const int col = e / q.Kpad, k = e - col * q.Kpad;
+    T v = T(0);
+    const int t = k / ps.Cp, c = k - t * ps.Cp;
+    const int th = t / q.TW, tw = t - th * q.TW;
+    if (k < q.K && c < (ps.dgrad ? g.Cout_g : g.Cin_g)) {
+        int ci = c, co = ps.grp * g.Cout_g + col, ka = tw, kb = th;
+        bool tap = true;
+        if (ps.dgrad) {
+            const int res = q.merged_w > 0 ? col / ps.Cch : 0;
+            ci = col - res * ps.Cch;
+            co = ps.grp * g.Cout_g + c;
+            const int rh = q.merged_w > 0 ? res / q.merged_w : q.rh, rw = q.merged_w > 0 ? res % q.merged_w : q.rw;
+            const int nw = (q.s0w + tw * q.stw) * g.sw + rw, nh = (q.s0h + th * q.sth) * g.sh + rh;
+            ka = nw / g.dw;
+            kb = nh / g.dh;
+            tap = nw >= 0 && nh >= 0 && ka * g.dw == nw && kb * g.dh == nh && ka < g.kW && kb < g.kH;
+        }
+        if (tap) {
+            const int a = g.flip ? ka : g.kW - 1 - ka, b = g.flip ? kb : g.kH - 1 - kb;
+            v = w[a + g.kW * (b + g.kH * (ci + g.Cin_g * co))];
+        }
+    }
+    out[q.wm + e] = v;
+}
+template <typename T>
+__global__ __launch_bounds__(256) void pad_to_cwhn_pack_kernel(const T* __restrict__ in, T* __restrict__ out, int P, int Cg, int Cp, int groups,
+                                                               int N, int zeros, int tiles_p, int tiles_c, int blocks, const T* __restrict__ w,
+                                                               T* __restrict__ wout, ConvGeom g, PackSubs ps) {
+    constexpr int V = 16 / (int)sizeof(T), PITCH = 64 + 4 / (int)sizeof(T);
+    __shared__ __align__(16) T tile[64 * PITCH];
+    if ((int)blockIdx.x >= blocks) {
+        pack_sub_element<T>(w, wout, g, ps, (int64_t)((int)blockIdx.x - blocks) * 256 + threadIdx.x);
+        return;
+    }
+    const int Ct = groups * Cp;
+    if (Ct == V) {                                   // a chunk per position: no transpose
+        const int64_t pos = (int64_t)blockIdx.x * 256 + threadIdx.x;
+        if (pos >= (int64_t)P * N + zeros) return;
+        T e[V];
+#pragma unroll
+        for (int c = 0; c < V; ++c) e[c] = T(0);
+        if (pos < (int64_t)P * N) {
+            const int n = (int)(pos / P);
+            const T* src = in + (int64_t)n * P * groups * Cg + (pos - (int64_t)n * P);
+#pragma unroll
+            for (int c = 0; c < V; ++c)
+                if (c < Cg) e[c] = src[(int64_t)c * P];     // one group: Cp == V
+        }
+        *reinterpret_cast<raw16_t*>(out + pos * V) = *reinterpret_cast<const raw16_t*>(e);
+        return;
+    }
+    const int n = blockIdx.x / (tiles_p * tiles_c), rest = blockIdx.x - n * (tiles_p * tiles_c);
+    const int c0 = (rest / tiles_p) * 64, p0 = (rest % tiles_p) * 64;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    if (n < N) {
+        const T* src = in + (int64_t)n * P * groups * Cg;
+        T v[16];
+#pragma unroll
+        for (int j = 0; j < 16; ++j) {
+            const int cp = c0 + wave + 4 * j, grp = cp / Cp, c = cp - grp * Cp;
+            const bool ok = cp < Ct && c < Cg && p0 + lane < P;
+            v[j] = src[ok ? (int64_t)(grp * Cg + c) * P + p0 + lane : 0];
+            if (!ok) v[j] = T(0);
+        }
+#pragma unroll
+        for (int j = 0; j < 16; ++j) tile[(wave + 4 * j) * PITCH + lane] = v[j];
+    } else {
+#pragma unroll
+        for (int j = 0; j < 16; ++j) tile[(wave + 4 * j) * PITCH + lane] = T(0);
+    }
+    __syncthreads();
+    constexpr int VC = 64 / V;
+    const int Pn = n < N ? P : zeros;
+    T* dst = out + (int64_t)n * P * Ct;
+#pragma unroll
+    for (int it = 0; it < 64 * VC / 256; ++it) {
+        const int idx = threadIdx.x + it * 256, pp = idx / VC, cv = idx % VC;
+        if (p0 + pp < Pn && c0 + cv * V < Ct) {
+            raw16_t r;
+            T* e = reinterpret_cast<T*>(&r);
+#pragma unroll
+            for (int k = 0; k < V; ++k) e[k] = tile[(cv * V + k) * PITCH + pp];
+            *reinterpret_cast<raw16_t*>(dst + (int64_t)(p0 + pp) * Ct + c0 + cv * V) = r;
+        }
+    }
+}
+
 // First pass of the fused pullback (bf16; P and C multiples of 8, 16-byte aligned pointers): one pass over delta
 // writes dz = delta .* act'(y, pre) as it lies (p contiguous: what the window and the direct filter-gradient kernels
 // read), its channel-contiguous copy dzT (what the input-gradient kernels read) and the bias gradient's partial sums,
@@ -234,40 +346,42 @@ __global__ __launch_bounds__(256) void conv_dbias_finalize_kernel(const float* _
 // added in order.
 template <typename T>
 __global__ __launch_bounds__(256) void wgrad_reduce_kernel(const float* __restrict__ partial, T* __restrict__ dw, ConvGeom g,
-                                                           int grp, int slices, int reduce_blocks, BiasPartials bp) {
+                                                           int grp, int slices, int reduce_blocks, int Cp, int64_t slice_stride,
+                                                           BiasPartials bp) {
     if ((int)blockIdx.x >= reduce_blocks) {       // workgroups behind the reduction: one channel of the bias gradient each
         conv_dbias_finalize_channel(bp.partial, bp.dbias, bp.C, bp.slices, (int)blockIdx.x - reduce_blocks);
         return;
     }
-    const int Mrows = g.kW * g.kH * g.Cin_g;
+    const int Mrows = g.kW * g.kH * Cp;                // Cp: channels per tap in the partial sums (padded)
     const int total = Mrows * g.Cout_g;
     const int idx = (blockIdx.x * blockDim.x + threadIdx.x) * 4;
     if (idx >= total) return;
     float acc[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-    const bool vec = (total & 3) == 0;                 // then idx + 3 < total and every slice row is 16-byte aligned
+    const bool vec = (total & 3) == 0 && (slice_stride & 3) == 0;   // then idx + 3 < total and every slice row is 16-byte aligned
     if (vec) {
         int sl = 0;
         for (; sl + 8 <= slices; sl += 8) {
             float4 v[8];
 #pragma unroll
-            for (int u = 0; u < 8; ++u) v[u] = *reinterpret_cast<const float4*>(partial + (size_t)(sl + u) * total + idx);
+            for (int u = 0; u < 8; ++u) v[u] = *reinterpret_cast<const float4*>(partial + (size_t)(sl + u) * slice_stride + idx);
 #pragma unroll
             for (int u = 0; u < 8; ++u) { acc[0] += v[u].x; acc[1] += v[u].y; acc[2] += v[u].z; acc[3] += v[u].w; }
         }
         for (; sl < slices; ++sl) {
-            const float4 v = *reinterpret_cast<const float4*>(partial + (size_t)sl * total + idx);
+            const float4 v = *reinterpret_cast<const float4*>(partial + (size_t)sl * slice_stride + idx);
             acc[0] += v.x; acc[1] += v.y; acc[2] += v.z; acc[3] += v.w;
         }
     } else {
         for (int sl = 0; sl < slices; ++sl)
             for (int e = 0; e < 4; ++e)
-                if (idx + e < total) acc[e] += partial[(size_t)sl * total + idx + e];
+                if (idx + e < total) acc[e] += partial[(size_t)sl * slice_stride + idx + e];
     }
     for (int e = 0; e < 4; ++e) {
         const int id = idx + e;
         if (id >= total) break;
         const int m = id % Mrows, col = id / Mrows;
-        const int t = m / g.Cin_g, ci = m - t * g.Cin_g;
+        const int t = m / Cp, ci = m - t * Cp;
+        if (ci >= g.Cin_g) continue;
         const int ka = t % g.kW, kb = t / g.kW;
         const int a = g.flip ? ka : g.kW - 1 - ka, b = g.flip ? kb : g.kH - 1 - kb;
         st(dw + a + g.kW * (b + g.kH * (ci + g.Cin_g * (grp * g.Cout_g + col))), acc[e]);
@@ -330,6 +444,9 @@ static int pack_filter(hipStream_t s, const T* w, T* out, const ConvGeom& g, int
     return LUXHIP_OK;
 }
 
+template <typename T>
+static int to_cwhn_padded(hipStream_t s, const T* in, T* out, int P, int Cg, int groups, int N, int zeros, const ConvGeom& g);
+
 // transpose_to_cwhn(in -> out) and pack_filter(w -> wout) in one launch where the 16-byte transform applies
 template <typename T>
 static int transpose_and_pack(hipStream_t s, const T* in, T* out, int P, int C, int N, const T* w, T* wout, const ConvGeom& g, int for_dgrad) {
@@ -339,7 +456,7 @@ static int transpose_and_pack(hipStream_t s, const T* in, T* out, int P, int C, 
     const int64_t pack_blocks = ceil_div((int64_t)g.kW * g.kH * g.Cin_g * g.Cout, 256);
     const int64_t gz = N + ceil_div(pack_blocks, gx * gy);
     if (!vec || N < 1 || gy > 65535 || gz > 65535) {
-        int rc = transpose_to_cwhn<T>(s, in, out, P, C, N);
+        int rc = to_cwhn_padded<T>(s, in, out, P, C / g.groups, g.groups, N, 0, g);
         if (rc != LUXHIP_OK) return rc;
         return pack_filter<T>(s, w, wout, g, for_dgrad);
     }
@@ -394,34 +511,201 @@ static int conv_dz_cwhn_pack(hipStream_t s, int act, const ConvGeom& g, const bf
     return LUXHIP_OK;
 }
 
+// ----------------------------------------------------------------------------- any channel count, any stride (conv_any.h)
+// Channels of a group padded to whole 16-byte chunks
 template <typename T>
-static void fill_gather(GatherK<T>& q, const ConvGeom& g, bool dgrad) {
+static int padded(int c) {
     constexpr int V = GemmTraits<T>::VEC;
-    q.kW = g.kW; q.sw = g.sw; q.sh = g.sh; q.pw = g.pw; q.ph = g.ph; q.dw = g.dw; q.dh = g.dh;
-    q.dgrad = dgrad;
-    if (!dgrad) {            // rows: output positions; source: xT
-        q.Ctot = g.Cin; q.Cg = g.Cin_g; q.P = g.OW; q.PQ = g.OW * g.OH; q.SP = g.W; q.SQ = g.H;
-    } else {                 // rows: input positions; source: dyT
-        q.Ctot = g.Cout; q.Cg = g.Cout_g; q.P = g.W; q.PQ = g.W * g.H; q.SP = g.OW; q.SQ = g.OH;
-    }
-    q.M = q.PQ * g.N;
-    q.divP = FastDiv((uint32_t)q.P); q.divPQ = FastDiv((uint32_t)q.PQ); q.divCg = FastDiv((uint32_t)q.Cg);
-    q.divkW = FastDiv((uint32_t)g.kW); q.divsw = FastDiv((uint32_t)g.sw); q.divsh = FastDiv((uint32_t)g.sh);
-    q.vec_ok = (q.Cg % V == 0) && (q.Ctot % V == 0);
+    return (c + V - 1) / V * V;
+}
+// The 3 x 3 window kernel of conv_patch.h takes the problem (pointer alignment is checked again at the launch)
+template <typename T>
+static bool window_shape(const ConvGeom& g, bool dgrad) {
+    if (sizeof(T) != 2 || g.sw != 1 || g.sh != 1 || g.dw != 1 || g.dh != 1 || g.OW != g.W || g.OH != g.H) return false;
+    cpatch::Problem p{};
+    p.Ctot = dgrad ? g.Cout : g.Cin; p.Cg = dgrad ? g.Cout_g : g.Cin_g; p.P = g.W; p.Q = g.H; p.N = g.N; p.kW = g.kW; p.kH = g.kH;
+    p.Ncols = dgrad ? g.Cin_g : g.Cout_g;
+    return cpatch::applicable(p);
+}
+// The whole-tap kernels: channels per group in whole stages, for the input gradient a unit stride, and enough work to fill
+// the chip with their large tiles.  Below that the kernels of conv_any.h are ahead: bf16 5 x 5, 192 -> 16 channels on 25 x 25
+// x 18 107 us against 33, fp32 5 x 5, 208 -> 40 on 66 x 66 x 4 417 against 162; with the chip full they are not: bf16 3 x 3,
+// 128 channels on 56 x 56 x 64 63 us (window kernel) against 132, fp32 541 against 550.
+template <typename T>
+static bool tap_shape(const ConvGeom& g, bool dgrad) {
+    const int Cg = dgrad ? g.Cout_g : g.Cin_g, Ncols = dgrad ? g.Cin_g : g.Cout_g;
+    const int64_t src = dgrad ? (int64_t)g.OW * g.OH * g.Cout * g.N : (int64_t)g.W * g.H * g.Cin * g.N;
+    if (Cg % GemmTraits<T>::BK != 0 || (dgrad && (g.sw != 1 || g.sh != 1)) || src >= (int64_t(1) << 30)) return false;
+    if (option_conv_tile() != 0) return true;
+    const int64_t rows = dgrad ? (int64_t)g.W * g.H * g.N : (int64_t)g.OW * g.OH * g.N, cus = num_cus() > 0 ? num_cus() : 256;
+    const int64_t tiles_n = ceil_div(Ncols, 128);
+    if (window_shape<T>(g, dgrad)) return ceil_div(rows, 256) * ceil_div(Ncols, 64) >= cus;
+    return ceil_div(rows, sizeof(T) == 2 ? 512 : 128) * tiles_n >= cus && Ncols * 4 >= tiles_n * 128 * 3;
 }
 
-// fprop (dgrad == false): out = y; dgrad: out = dx.  src is the channel-contiguous activation,
+struct Residue { int count, q0, s0, sstep, taps, k0; };     // rows, first q, first shift and step, taps
+// Residue r of one dimension of the input gradient: input positions i = stride q + r - pad in [0, L)
+static Residue residue(int r, int L, int pad, int stride, int dil, int taps) {
+    auto floor_div = [](int a, int b) { return a >= 0 ? a / b : -((-a + b - 1) / b); };
+    Residue z{0, 0, 0, 1, 0, 0};
+    z.q0 = -floor_div(r - pad, stride);                      // ceil((pad - r) / stride)
+    z.count = std::max(0, floor_div(L - 1 + pad - r, stride) - z.q0 + 1);
+    int gq = stride, t = dil;
+    while (t) { const int u = gq % t; gq = t; t = u; }
+    z.sstep = dil / gq;
+    if (r % gq == 0)
+        for (int k = 0; k < std::min(taps, stride / gq); ++k)
+            if (((int64_t)k * dil - r) % stride == 0) { z.k0 = k; z.taps = (taps - 1 - k) / (stride / gq) + 1; z.s0 = (k * dil - r) / stride; break; }
+    return z;
+}
+
+// The sub-problems of one convolution, in groups of one launch each.
+template <typename T>
+struct AnyPlan {
+    struct Launch { cany::Sub sub[cany::MAX_SUBS]; PackSub pack[cany::MAX_SUBS]; int n; };
+    std::vector<Launch> launches;
+    int Ncols = 0, Cch = 0, res_w = 0, merged = 0, Cp = 0;
+    int64_t wm_elems = 0;                                    // packed filter of one group
+    void add(const Residue& rw, int RA, const Residue& rh, int RB, int N, int w0, int wstep, int TW, int h0, int hstep, int TH, int ow0, int oh0,
+             int r_w, int r_h) {
+        if (RA <= 0 || RB <= 0) return;
+        if (launches.empty() || launches.back().n == cany::MAX_SUBS) { launches.emplace_back(); launches.back().n = 0; }
+        Launch& l = launches.back();
+        cany::Sub& q = l.sub[l.n];
+        q.RA = RA; q.RAB = RA * RB; q.M = RA * RB * N;
+        q.w0 = w0; q.wstep = wstep; q.h0 = h0; q.hstep = hstep; q.TW = std::max(TW, 1); q.TH = TH;
+        q.K = TW * TH * Cp;
+        q.Kpad = (q.K + GemmTraits<T>::BK - 1) / GemmTraits<T>::BK * GemmTraits<T>::BK;
+        q.ow0 = ow0; q.oh0 = oh0; q.wm = wm_elems;
+        q.divRA = FastDiv((uint32_t)RA); q.divRAB = FastDiv((uint32_t)(RA * RB)); q.divTW = FastDiv((uint32_t)q.TW);
+        PackSub& k = l.pack[l.n];
+        k = PackSub{r_w, r_h, rw.s0, rw.sstep, rh.s0, rh.sstep, q.TW, q.K, q.Kpad, res_w, wm_elems, 0};
+        wm_elems += (int64_t)Ncols * q.Kpad;
+        ++l.n;
+    }
+    AnyPlan(const ConvGeom& g, bool dgrad) {
+        Cp = padded<T>(dgrad ? g.Cout_g : g.Cin_g);
+        Ncols = Cch = dgrad ? g.Cin_g : g.Cout_g;
+        const Residue none{0, 0, 0, 1, 0, 0};
+        if (!dgrad) {
+            add(none, g.OW, none, g.OH, g.N, -g.pw, g.dw, g.kW, -g.ph, g.dh, g.kH, 0, 0, 0, 0);
+            return;
+        }
+        std::vector<Residue> rw(g.sw), rh(g.sh);
+        for (int r = 0; r < g.sw; ++r) rw[r] = residue(r, g.W, g.pw, g.sw, g.dw, g.kW);
+        for (int r = 0; r < g.sh; ++r) rh[r] = residue(r, g.H, g.ph, g.sh, g.dh, g.kH);
+        // one problem per residue, or all residues as columns of one: whichever is less work in 32-column tiles
+        const int R = g.sw * g.sh;
+        auto cols = [](int n) { return (double)((n + 31) / 32 * 32); };
+        double apart = 0.0, together = 1e30;
+        for (const Residue& a : rw)
+            for (const Residue& b : rh) apart += (double)a.count * b.count * a.taps * b.taps * cols(g.Cin_g);
+        auto unite = [](const std::vector<Residue>& v, Residue& u) {
+            u = Residue{0, 1 << 30, 1 << 30, 1, 0, 0};
+            int q1 = -(1 << 30), s1 = -(1 << 30);
+            for (const Residue& z : v) {
+                if (z.count > 0) { u.q0 = std::min(u.q0, z.q0); q1 = std::max(q1, z.q0 + z.count - 1); }
+                if (z.taps > 0) { u.s0 = std::min(u.s0, z.s0); s1 = std::max(s1, z.s0 + (z.taps - 1) * z.sstep); }
+            }
+            u.count = q1 - u.q0 + 1;
+            u.taps = s1 - u.s0 + 1;
+        };
+        Residue uw, uh;
+        if (R > 1 && g.dw == 1 && g.dh == 1) {
+            unite(rw, uw);
+            unite(rh, uh);
+            together = (double)uw.count * uh.count * uw.taps * uh.taps * cols(R * g.Cin_g);
+        }
+        if (together < apart) {
+            merged = 1;
+            res_w = g.sw;
+            Ncols = R * g.Cin_g;
+            add(uw, uw.count, uh, uh.count, g.N, uw.q0 - uw.s0, -1, uw.taps, uh.q0 - uh.s0, -1, uh.taps, g.sw * uw.q0 - g.pw, g.sh * uh.q0 - g.ph, 0, 0);
+            return;
+        }
+        for (int b = 0; b < g.sh; ++b)
+            for (int a = 0; a < g.sw; ++a)
+                add(rw[a], rw[a].count, rh[b], rh[b].count, g.N, rw[a].q0 - rw[a].s0, -rw[a].sstep, rw[a].taps, rh[b].q0 - rh[b].s0, -rh[b].sstep,
+                    rh[b].taps, g.sw * rw[a].q0 + a - g.pw, g.sh * rh[b].q0 + b - g.ph, a, b);
+    }
+    PackSubs pack(const ConvGeom& g, bool dgrad, int grp, size_t launch) const {
+        PackSubs p;
+        p.n = launches[launch].n; p.dgrad = dgrad; p.Cp = Cp; p.Ncols = Ncols; p.Cch = Cch; p.grp = grp; p.total = 0;
+        for (int i = 0; i < p.n; ++i) {
+            p.sub[i] = launches[launch].pack[i];
+            p.sub[i].first = p.total;
+            p.total += (int64_t)Ncols * p.sub[i].Kpad;
+        }
+        return p;
+    }
+};
+
+// Padded channel-contiguous copy of `in` (if out != NULL) and the packed filter of group 0, launch 0 (if wout != NULL), in one
+// launch
+template <typename T>
+static int pad_and_pack(hipStream_t s, const T* in, T* out, int P, int Cg, int groups, int N, int zeros, const T* w, T* wout, const ConvGeom& g,
+                        const PackSubs* ps) {
+    constexpr int V = GemmTraits<T>::VEC;
+    const int Cp = padded<T>(Cg), Ct = groups * Cp;
+    PackSubs none;
+    none.n = 0; none.total = 0;
+    int64_t blocks = 0;
+    const int tiles_p = (int)ceil_div(std::max(P, zeros), 64), tiles_c = (int)ceil_div(Ct, 64);
+    if (out != nullptr) blocks = Ct == V ? ceil_div((int64_t)P * N + zeros, 256) : (int64_t)tiles_p * tiles_c * (N + (zeros > 0));
+    const int64_t pack = wout != nullptr ? ceil_div(ps->total, 256) : 0;
+    LUX_UNSUPPORTED_IF(blocks + pack >= (int64_t(1) << 31), "conv: tensor too large for the layout transform");
+    if (blocks + pack == 0) return LUXHIP_OK;
+    ProfScope prof("whcn_to_cwhn_kernel", s);
+    pad_to_cwhn_pack_kernel<T><<<(unsigned)(blocks + pack), 256, 0, s>>>(in, out, P, Cg, Cp, groups, N, zeros, tiles_p, tiles_c, (int)blocks, w, wout, g,
+                                                                         wout != nullptr ? *ps : none);
+    LUX_CHECK_LAUNCH();
+    return LUXHIP_OK;
+}
+
+// Channel-contiguous copy of a tensor in the padded layout (the plain layout where no padding is needed)
+template <typename T>
+static int to_cwhn_padded(hipStream_t s, const T* in, T* out, int P, int Cg, int groups, int N, int zeros, const ConvGeom& g) {
+    if (padded<T>(Cg) == Cg && zeros == 0 && P % GemmTraits<T>::VEC == 0 && aligned16(in)) return transpose_to_cwhn<T>(s, in, out, P, Cg * groups, N);
+    return pad_and_pack<T>(s, in, out, P, Cg, groups, N, zeros, nullptr, nullptr, g, nullptr);
+}
+
+// fprop / dgrad of one problem through conv_any.h.  src: padded channel-contiguous activations; wm: workspace for the packed
+// filter of one group; packed: group 0, launch 0 of the filter is already there.  ws_front: bytes of the workspace in use.
+template <typename T>
+static int run_conv_any(hipStream_t s, const ConvGeom& g, bool dgrad, const AnyPlan<T>& plan, const T* src, const T* w, T* wm, bool packed, const T* bias,
+                        T* out, T* pre, int act, size_t ws_front) {
+    for (int grp = 0; grp < g.groups; ++grp)
+        for (size_t li = 0; li < plan.launches.size(); ++li) {
+            const typename AnyPlan<T>::Launch& l = plan.launches[li];
+            if (!packed || grp > 0 || li > 0) {
+                const PackSubs ps = plan.pack(g, dgrad, grp, li);
+                const int rc = pad_and_pack<T>(s, nullptr, nullptr, 0, 1, 1, 0, 0, w, wm, g, &ps);
+                if (rc != LUXHIP_OK) return rc;
+            }
+            cany::Args<T> a;
+            a.src = src + (size_t)grp * plan.Cp;
+            a.wm = wm; a.bias = bias; a.out = out; a.pre = pre;
+            a.Ctot = g.groups * plan.Cp; a.Cp = plan.Cp;
+            if (!dgrad) { a.SP = g.W; a.SQ = g.H; a.ss_w = g.sw; a.ss_h = g.sh; a.P = g.OW; a.Q = g.OH; a.os_w = a.os_h = 1; a.Ctot_out = g.Cout; }
+            else { a.SP = g.OW; a.SQ = g.OH; a.ss_w = a.ss_h = 1; a.P = g.W; a.Q = g.H; a.os_w = g.sw; a.os_h = g.sh; a.Ctot_out = g.Cin; }
+            a.PQ = a.P * a.Q;
+            a.Ncols = plan.Ncols; a.Cch = plan.Cch; a.res_w = std::max(plan.res_w, 1); a.merged = plan.merged;
+            a.col_off = grp * plan.Cch; a.act = act; a.subs = l.n;
+            a.divCp = FastDiv((uint32_t)plan.Cp); a.divCch = FastDiv((uint32_t)plan.Cch);
+            for (int i = 0; i < l.n; ++i) a.sub[i] = l.sub[i];
+            const int rc = cany::launch_any<T>(s, a, ws_front, dgrad);
+            if (rc != LUXHIP_OK) return rc;
+        }
+    return LUXHIP_OK;
+}
+
+// fprop (dgrad == false): out = y; dgrad: out = dx, for problems of tap_shape().  src is the channel-contiguous activation,
 // wm the packed filter (all groups), zeros a few zero bytes in device memory.
 template <typename T>
 static int run_conv_gemm(hipStream_t s, const ConvGeom& g, bool dgrad, const T* src, const T* wm, const T* bias, T* out,
                          T* pre, int act, const void* zeros) {
     const int Tt = g.kW * g.kH;
     const int Cg = dgrad ? g.Cout_g : g.Cin_g;
-    const int64_t src_elems = dgrad ? (int64_t)g.OW * g.OH * g.Cout * g.N : (int64_t)g.W * g.H * g.Cin * g.N;
-    // whole-tap stages: a K stage never straddles a filter tap; the transposed-convolution index
-    // map of dgrad is only that simple for unit stride
-    const bool tap_path = Cg % GemmTraits<T>::BK == 0 && (!dgrad || (g.sw == 1 && g.sh == 1)) && aligned16(src) &&
-                          aligned16(wm) && src_elems < (int64_t(1) << 30);
     for (int grp = 0; grp < g.groups; ++grp) {
         const int Ncols = dgrad ? g.Cin_g : g.Cout_g;
         const int K = Tt * Cg;
@@ -447,60 +731,49 @@ static int run_conv_gemm(hipStream_t s, const ConvGeom& g, bool dgrad, const T* 
                 }
             }
         }
-        if (tap_path) {
-            ConvTapArgs<T> a;
-            TapGeom<T>& q = a.tap;
-            q.kW = g.kW; q.sw = g.sw; q.sh = g.sh; q.pw = g.pw; q.ph = g.ph; q.dw = g.dw; q.dh = g.dh;
-            q.dgrad = dgrad;
-            q.Cg = Cg;
-            if (!dgrad) { q.Ctot = g.Cin; q.P = g.OW; q.PQ = g.OW * g.OH; q.SP = g.W; q.SQ = g.H; }
-            else { q.Ctot = g.Cout; q.P = g.W; q.PQ = g.W * g.H; q.SP = g.OW; q.SQ = g.OH; }
-            q.M = q.PQ * g.N;
-            q.divP = FastDiv((uint32_t)q.P); q.divPQ = FastDiv((uint32_t)q.PQ); q.divCg = FastDiv((uint32_t)q.Cg);
-            q.divkW = FastDiv((uint32_t)g.kW);
-            q.src = src + (size_t)grp * Cg;
-            q.zero = zeros;
-            a.Wm = Wm; a.K = K; a.Ncols = Ncols;
-            a.out = out; a.pre = pre; a.bias = bias;
-            a.Ctot_out = dgrad ? g.Cin : g.Cout;
-            a.col_off = grp * Ncols;
-            a.act = act;
-            a.m_begin = 0;
-            rc = launch_conv_tap_any<T>(s, a);
-        } else {
-            ConvGemmArgs<T> a;
-            fill_gather(a.gather, g, dgrad);
-            a.gather.src = src;
-            a.gather.c_off = grp * a.gather.Cg;
-            a.gather.vec_ok = a.gather.vec_ok && aligned16(src);
-            a.K = K; a.Ncols = Ncols; a.Wm = Wm;
-            a.out = out; a.pre = pre; a.bias = bias;
-            a.Ctot_out = dgrad ? g.Cin : g.Cout;
-            a.col_off = grp * a.Ncols;
-            a.act = act;
-            rc = launch_conv_gemm_any<T>(s, a);
-        }
+        ConvTapArgs<T> a;
+        TapGeom<T>& q = a.tap;
+        q.kW = g.kW; q.sw = g.sw; q.sh = g.sh; q.pw = g.pw; q.ph = g.ph; q.dw = g.dw; q.dh = g.dh;
+        q.dgrad = dgrad;
+        q.Cg = Cg;
+        if (!dgrad) { q.Ctot = g.Cin; q.P = g.OW; q.PQ = g.OW * g.OH; q.SP = g.W; q.SQ = g.H; }
+        else { q.Ctot = g.Cout; q.P = g.W; q.PQ = g.W * g.H; q.SP = g.OW; q.SQ = g.OH; }
+        q.M = q.PQ * g.N;
+        q.divP = FastDiv((uint32_t)q.P); q.divPQ = FastDiv((uint32_t)q.PQ); q.divCg = FastDiv((uint32_t)q.Cg);
+        q.divkW = FastDiv((uint32_t)g.kW);
+        q.src = src + (size_t)grp * Cg;
+        q.zero = zeros;
+        a.Wm = Wm; a.K = K; a.Ncols = Ncols;
+        a.out = out; a.pre = pre; a.bias = bias;
+        a.Ctot_out = dgrad ? g.Cin : g.Cout;
+        a.col_off = grp * Ncols;
+        a.act = act;
+        a.m_begin = 0;
+        rc = launch_conv_tap_any<T>(s, a);
         if (rc != LUXHIP_OK) return rc;
     }
     return LUXHIP_OK;
 }
 
+// Rows (taps x padded channels), columns and slices of the filter gradient's partial sums
+struct WgradPlan { int Mrows, Ncols, slices, kslice; bool narrow; };
 template <typename T>
-static int wgrad_plan(const ConvGeom& g, int* slices, int* kslice, bool* small) {
+static int wgrad_plan(const ConvGeom& g, bool any, WgradPlan* p) {
     constexpr int BK = GemmTraits<T>::BK;
-    const int Mrows = g.kW * g.kH * g.Cin_g;
-    *small = Mrows <= 64 || g.Cout_g <= 64;
-    const int tile = *small ? 64 : 128;
-    const int64_t tiles = ceil_div(Mrows, tile) * ceil_div(g.Cout_g, tile);
+    p->Mrows = g.kW * g.kH * (any ? padded<T>(g.Cin_g) : g.Cin_g);
+    p->Ncols = any ? padded<T>(g.Cout_g) : g.Cout_g;
+    p->narrow = p->Mrows <= 64 || p->Ncols <= 64;
+    const int tile = p->narrow ? 64 : 128;
+    const int64_t tiles = ceil_div(p->Mrows, tile) * ceil_div(p->Ncols, tile);
     const int64_t Ktotal = (int64_t)g.OW * g.OH * g.N;
     // as many slices as keep every workgroup resident at once (two per compute unit): one more
     // would add a whole round for a single straggler
     int64_t want = std::max<int64_t>(1, 2 * (int64_t)std::max(1, num_cus()) / (tiles * g.groups));
     int64_t ks = ceil_div(ceil_div(Ktotal, want), BK) * BK;
     ks = std::max<int64_t>(ks, 4 * BK);
-    *kslice = (int)ks;
-    *slices = (int)ceil_div(Ktotal, ks);
-    LUX_UNSUPPORTED_IF(*slices > 65535, "conv wgrad: too many k slices");
+    p->kslice = (int)ks;
+    p->slices = (int)ceil_div(Ktotal, ks);
+    LUX_UNSUPPORTED_IF(p->slices > 65535, "conv wgrad: too many k slices");
     return LUXHIP_OK;
 }
 
@@ -516,16 +789,6 @@ static bool wgrad_window_shape(const ConvGeom& g) {
     return wpatch::applicable(p, num_cus() > 0 ? num_cus() : 256);
 }
 
-template <typename T>
-static size_t wgrad_partial_bytes(const ConvGeom& g) {
-    int slices = 1, kslice = 0;
-    bool small = false;
-    if (wgrad_plan<T>(g, &slices, &kslice, &small) != LUXHIP_OK) return 0;
-    if (wgrad_window_shape<T>(g))
-        slices = std::max(slices, wpatch::image_lanes(g.N, (g.Cin_g / 64) * ((g.Cout_g + 63) / 64), num_cus() > 0 ? num_cus() : 256));
-    return align256((size_t)slices * g.kW * g.kH * g.Cin_g * g.Cout_g * sizeof(float));
-}
-
 // bf16 fast path of the filter gradient: conditions under which conv_wgrad_direct_kernel applies
 template <typename T>
 static bool wgrad_direct_ok(const ConvGeom& g, const void* xT, const void* dy) {
@@ -535,20 +798,33 @@ static bool wgrad_direct_ok(const ConvGeom& g, const void* xT, const void* dy) {
            (int64_t)g.W * g.H * g.Cin * g.N < (int64_t(1) << 30) && PQ * g.Cout * g.N < (int64_t(1) << 30);
 }
 
-// dy: WHCN cotangent (used by the direct bf16 kernel); dyT: its channel-contiguous copy (used by
-// the general kernel; may be NULL when wgrad_direct_ok).
+template <typename T>
+static size_t wgrad_partial_bytes(const ConvGeom& g) {
+    size_t bytes = 0;
+    for (int any = 0; any < 2; ++any) {
+        WgradPlan p;
+        if (wgrad_plan<T>(g, any != 0, &p) != LUXHIP_OK) return 0;
+        if (wgrad_window_shape<T>(g))
+            p.slices = std::max(p.slices, wpatch::image_lanes(g.N, (g.Cin_g / 64) * ((g.Cout_g + 63) / 64), num_cus() > 0 ? num_cus() : 256));
+        bytes = std::max(bytes, (size_t)p.slices * p.Mrows * p.Ncols * sizeof(float));
+    }
+    return align256(bytes);
+}
+
+// dy: WHCN cotangent (used by the window and the direct bf16 kernels); dyT: its channel-contiguous copy with padded channels,
+// followed by BK positions of zeros where there are fewer than BK positions in all (used by the general kernel).
 template <typename T>
 static int run_wgrad(hipStream_t s, const ConvGeom& g, const T* xT, const T* dy, const T* dyT, float* partial, T* dw,
                      const void* zeros, const BiasPartials* bias = nullptr) {
-    constexpr int V = GemmTraits<T>::VEC;
-    int slices, kslice;
-    bool small;
-    int rc = wgrad_plan<T>(g, &slices, &kslice, &small);
-    if (rc != LUXHIP_OK) return rc;
     const bool direct = wgrad_direct_ok<T>(g, xT, dy);
     const bool window = wgrad_window_shape<T>(g) && aligned16(xT) && aligned16(dy) && aligned16(partial);
+    WgradPlan plan;
+    int rc = wgrad_plan<T>(g, !direct && !window, &plan);
+    if (rc != LUXHIP_OK) return rc;
+    int slices = plan.slices;
+    const int kslice = plan.kslice;
     for (int grp = 0; grp < g.groups; ++grp) {
-        const int Mrows = g.kW * g.kH * g.Cin_g;
+        const int Mrows = plan.Mrows;
         if (window) {
             if constexpr (sizeof(T) == 2) {
                 wpatch::Problem p;
@@ -580,18 +856,18 @@ static int run_wgrad(hipStream_t s, const ConvGeom& g, const T* xT, const T* dy,
                 rc = launch_conv_wgrad_direct(s, a, slices);
             }
         } else {
-            ConvWgradArgs<T> a;
-            GatherMN<T>& q = a.gather;
-            q.src = xT; q.Ctot = g.Cin; q.c_off = grp * g.Cin_g; q.Cg = g.Cin_g; q.Mrows = Mrows;
-            q.OW = g.OW; q.OWOH = g.OW * g.OH; q.SP = g.W; q.SQ = g.H; q.kW = g.kW; q.sw = g.sw; q.sh = g.sh; q.pw = g.pw;
-            q.ph = g.ph; q.dw = g.dw; q.dh = g.dh;
-            q.vec_ok = (g.Cin_g % V == 0) && (g.Cin % V == 0) && aligned16(xT);
-            q.divOW = FastDiv((uint32_t)q.OW); q.divOWOH = FastDiv((uint32_t)q.OWOH); q.divCg = FastDiv((uint32_t)q.Cg);
-            q.divkW = FastDiv((uint32_t)g.kW);
-            a.dyT = dyT; a.Cout = g.Cout; a.co_off = grp * g.Cout_g; a.Cout_g = g.Cout_g;
-            a.Ktotal = g.OW * g.OH * g.N; a.kslice = kslice; a.partial = partial;
-            a.dy_vec_ok = (g.Cout % V == 0) && (g.Cout_g % V == 0) && aligned16(dyT);
-            rc = launch_conv_wgrad_any<T>(s, a, slices, small);
+            cany::WgradArgs<T> a;
+            const int Cp = padded<T>(g.Cin_g);
+            a.src = xT + (size_t)grp * Cp; a.Ctot = g.groups * Cp; a.Cp = Cp; a.Mrows = Mrows;
+            a.dyT = dyT + (size_t)grp * plan.Ncols; a.Ytot = g.groups * plan.Ncols; a.Ncols = plan.Ncols;
+            a.zero = zeros;
+            a.OW = g.OW; a.OWOH = g.OW * g.OH; a.SP = g.W; a.SQ = g.H;
+            a.kW = g.kW; a.sw = g.sw; a.sh = g.sh; a.pw = g.pw; a.ph = g.ph; a.dw = g.dw; a.dh = g.dh;
+            a.divOW = FastDiv((uint32_t)a.OW); a.divOWOH = FastDiv((uint32_t)a.OWOH); a.divCp = FastDiv((uint32_t)Cp); a.divkW = FastDiv((uint32_t)g.kW);
+            a.positions = g.OW * g.OH * g.N;
+            a.Ktotal = std::max(a.positions, GemmTraits<T>::BK);
+            a.kslice = kslice; a.partial = partial;
+            rc = cany::launch_any_wgrad<T>(s, a, slices, plan.narrow);
         }
         if (rc != LUXHIP_OK) return rc;
         ProfScope ps("wgrad_reduce_kernel", s);
@@ -599,55 +875,117 @@ static int run_wgrad(hipStream_t s, const ConvGeom& g, const T* xT, const T* dy,
         const int reduce_blocks = (int)ceil_div(total, 1024);
         BiasPartials bp;
         if (bias != nullptr && grp == g.groups - 1) bp = *bias;       // the bias gradient's channels ride on the last group's launch
-        wgrad_reduce_kernel<T><<<(unsigned)(reduce_blocks + bp.C), 256, 0, s>>>(partial, dw, g, grp, slices, reduce_blocks, bp);
+        wgrad_reduce_kernel<T><<<(unsigned)(reduce_blocks + bp.C), 256, 0, s>>>(partial, dw, g, grp, slices, reduce_blocks, Mrows / (g.kW * g.kH),
+                                                                           (int64_t)Mrows * plan.Ncols, bp);
         LUX_CHECK_LAUNCH();
     }
     return LUXHIP_OK;
 }
 
 // ----------------------------------------------------------------------------- typed entry points
+// Positions of zeros that follow the channel-contiguous cotangent: the filter gradient contracts at least one stage
+template <typename T>
+static int dy_zeros(const ConvGeom& g) {
+    const int64_t pos = (int64_t)g.OW * g.OH * g.N;
+    return pos < GemmTraits<T>::BK ? GemmTraits<T>::BK : 0;
+}
+// Bytes of the padded channel-contiguous copies and of the packed filter (either form)
+template <typename T>
+static size_t xt_bytes(const ConvGeom& g) { return align256((size_t)g.W * g.H * g.N * g.groups * padded<T>(g.Cin_g) * sizeof(T)); }
+template <typename T>
+static size_t dyt_bytes(const ConvGeom& g) {
+    return align256(((size_t)g.OW * g.OH * g.N + dy_zeros<T>(g)) * g.groups * padded<T>(g.Cout_g) * sizeof(T));
+}
+template <typename T>
+static size_t filter_bytes(const ConvGeom& g, bool any, const AnyPlan<T>& plan) {
+    return align256(any ? (size_t)plan.wm_elems * sizeof(T) : (size_t)g.kW * g.kH * g.Cin_g * g.Cout * sizeof(T));
+}
+// A caller's channel-contiguous copy of x serves the kernels as it is
+template <typename T>
+static bool kept_usable(const ConvGeom& g, const T* kept) { return kept != nullptr && padded<T>(g.Cin_g) == g.Cin_g && aligned16(kept); }
+
+// (C, P) -> (Cp, P) per group with zeros in the new channels: a caller's unpadded copy of x, when x itself is not given
+template <typename T>
+__global__ __launch_bounds__(256) void repad_cwhn_kernel(const T* __restrict__ in, T* __restrict__ out, int64_t total, int Cg, int Cp) {
+    for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < total; i += (int64_t)gridDim.x * 256) {
+        const int64_t row = i / Cp;
+        const int c = (int)(i - row * Cp);
+        out[i] = c < Cg ? in[row * Cg + c] : T(0);
+    }
+}
+
 template <typename T>
 static int conv_fwd_t(hipStream_t s, int act, const ConvGeom& g, const T* x, const T* w, const T* bias, T* y, T* pre,
                       T* xt_keep) {
+    const bool any = !tap_shape<T>(g, false);
+    const AnyPlan<T> plan(g, false);
     // xt_keep: caller's buffer of x's size that keeps the channel-contiguous copy of x for the pullback
-    const size_t xb = xt_keep ? 0 : align256((size_t)g.W * g.H * g.Cin * g.N * sizeof(T));
-    const size_t wb = align256((size_t)g.kW * g.kH * g.Cin_g * g.Cout * sizeof(T));
+    const bool keep = kept_usable<T>(g, xt_keep);
+    const size_t xb = keep ? 0 : xt_bytes<T>(g), wb = filter_bytes<T>(g, any, plan);
     Workspace ws;
-    int rc = get_workspace(s, xb + wb, &ws);
+    // the slices of conv_any.h take memory behind these; reserve it here, where no pointer into the workspace is live yet
+    int rc = get_workspace(s, xb + wb + (any ? cany::most_partial_bytes() : 0), &ws);
     if (rc != LUXHIP_OK) return rc;
-    T* xT = xt_keep ? xt_keep : reinterpret_cast<T*>(ws.data);
+    T* xT = keep ? xt_keep : reinterpret_cast<T*>(ws.data);
     T* wF = reinterpret_cast<T*>(ws.data + xb);
-    if ((rc = transpose_and_pack<T>(s, x, xT, g.W * g.H, g.Cin, g.N, w, wF, g, 0)) != LUXHIP_OK) return rc;
-    return run_conv_gemm<T>(s, g, false, xT, wF, bias, y, pre, act, ws.zeros);
+    if (xt_keep != nullptr && !keep) {
+        if ((rc = transpose_to_cwhn<T>(s, x, xt_keep, g.W * g.H, g.Cin, g.N)) != LUXHIP_OK) return rc;
+    }
+    if (!any) {
+        if ((rc = transpose_and_pack<T>(s, x, xT, g.W * g.H, g.Cin, g.N, w, wF, g, 0)) != LUXHIP_OK) return rc;
+        return run_conv_gemm<T>(s, g, false, xT, wF, bias, y, pre, act, ws.zeros);
+    }
+    const PackSubs ps = plan.pack(g, false, 0, 0);
+    if ((rc = pad_and_pack<T>(s, x, xT, g.W * g.H, g.Cin_g, g.groups, g.N, 0, w, wF, g, &ps)) != LUXHIP_OK) return rc;
+    return run_conv_any<T>(s, g, false, plan, xT, w, wF, true, bias, y, pre, act, xb + wb);
+}
+
+// dx from the channel-contiguous cotangent; packed: the filter of the first launch is in wD
+template <typename T>
+static int run_dgrad(hipStream_t s, const ConvGeom& g, bool any, const AnyPlan<T>& plan, const T* dyT, const T* w, T* wD, bool packed, T* dx,
+                     size_t ws_front, const void* zeros) {
+    if (any) return run_conv_any<T>(s, g, true, plan, dyT, w, wD, packed, nullptr, dx, nullptr, LUXHIP_ACT_IDENTITY, ws_front);
+    return run_conv_gemm<T>(s, g, true, dyT, wD, nullptr, dx, nullptr, LUXHIP_ACT_IDENTITY, zeros);
+}
+// dyT (padded) and the filter packed for the input gradient, in one launch
+template <typename T>
+static int dy_transpose_and_pack(hipStream_t s, const ConvGeom& g, bool any, const AnyPlan<T>& plan, const T* dy, T* dyT, const T* w, T* wD) {
+    if (!any && dy_zeros<T>(g) > 0) {
+        const int rc = to_cwhn_padded<T>(s, dy, dyT, g.OW * g.OH, g.Cout_g, g.groups, g.N, dy_zeros<T>(g), g);
+        return rc != LUXHIP_OK ? rc : pack_filter<T>(s, w, wD, g, 1);
+    }
+    if (!any) return transpose_and_pack<T>(s, dy, dyT, g.OW * g.OH, g.Cout, g.N, w, wD, g, 1);
+    if (plan.launches.empty()) return to_cwhn_padded<T>(s, dy, dyT, g.OW * g.OH, g.Cout_g, g.groups, g.N, dy_zeros<T>(g), g);
+    const PackSubs ps = plan.pack(g, true, 0, 0);
+    return pad_and_pack<T>(s, dy, dyT, g.OW * g.OH, g.Cout_g, g.groups, g.N, dy_zeros<T>(g), w, wD, g, &ps);
 }
 
 template <typename T>
 static int conv_bwd_data_t(hipStream_t s, const ConvGeom& g, const T* dy, const T* w, T* dx) {
-    const size_t yb = align256((size_t)g.OW * g.OH * g.Cout * g.N * sizeof(T));
-    const size_t wb = align256((size_t)g.kW * g.kH * g.Cin_g * g.Cout * sizeof(T));
+    const bool any = !tap_shape<T>(g, true);
+    const AnyPlan<T> plan(g, true);
+    const size_t yb = dyt_bytes<T>(g), wb = filter_bytes<T>(g, any, plan);
     Workspace ws;
-    int rc = get_workspace(s, yb + wb, &ws);
+    int rc = get_workspace(s, yb + wb + (any ? cany::most_partial_bytes() : 0), &ws);
     if (rc != LUXHIP_OK) return rc;
     T* dyT = reinterpret_cast<T*>(ws.data);
     T* wD = reinterpret_cast<T*>(ws.data + yb);
-    if ((rc = transpose_and_pack<T>(s, dy, dyT, g.OW * g.OH, g.Cout, g.N, w, wD, g, 1)) != LUXHIP_OK) return rc;
-    return run_conv_gemm<T>(s, g, true, dyT, wD, nullptr, dx, nullptr, LUXHIP_ACT_IDENTITY, ws.zeros);
+    if ((rc = dy_transpose_and_pack<T>(s, g, any, plan, dy, dyT, w, wD)) != LUXHIP_OK) return rc;
+    return run_dgrad<T>(s, g, any, plan, dyT, w, wD, true, dx, yb + wb, ws.zeros);
 }
 
 template <typename T>
 static int conv_bwd_filter_t(hipStream_t s, const ConvGeom& g, const T* x, const T* dy, T* dw) {
-    const size_t xb = align256((size_t)g.W * g.H * g.Cin * g.N * sizeof(T));
-    const size_t yb = align256((size_t)g.OW * g.OH * g.Cout * g.N * sizeof(T));
-    const size_t pb = wgrad_partial_bytes<T>(g);
+    const size_t xb = xt_bytes<T>(g), yb = dyt_bytes<T>(g), pb = wgrad_partial_bytes<T>(g);
     Workspace ws;
     int rc = get_workspace(s, xb + yb + pb, &ws);
     if (rc != LUXHIP_OK) return rc;
     T* xT = reinterpret_cast<T*>(ws.data);
     T* dyT = reinterpret_cast<T*>(ws.data + xb);
     float* partial = reinterpret_cast<float*>(ws.data + xb + yb);
-    if ((rc = transpose_to_cwhn<T>(s, x, xT, g.W * g.H, g.Cin, g.N)) != LUXHIP_OK) return rc;
+    if ((rc = to_cwhn_padded<T>(s, x, xT, g.W * g.H, g.Cin_g, g.groups, g.N, 0, g)) != LUXHIP_OK) return rc;
     if (!wgrad_direct_ok<T>(g, xT, dy)) {   // the direct kernel reads dy as it is
-        if ((rc = transpose_to_cwhn<T>(s, dy, dyT, g.OW * g.OH, g.Cout, g.N)) != LUXHIP_OK) return rc;
+        if ((rc = to_cwhn_padded<T>(s, dy, dyT, g.OW * g.OH, g.Cout_g, g.groups, g.N, dy_zeros<T>(g), g)) != LUXHIP_OK) return rc;
     }
     return run_wgrad<T>(s, g, xT, dy, dyT, partial, dw, ws.zeros);
 }
@@ -655,35 +993,36 @@ static int conv_bwd_filter_t(hipStream_t s, const ConvGeom& g, const T* x, const
 template <typename T>
 static int fused_conv_bwd_t(hipStream_t s, int dtype, int act, const ConvGeom& g, const T* delta, const T* y,
                             const T* pre, const T* x, const T* w, T* dz, T* dw, T* dx, T* dbias, const T* xt_kept) {
-    const size_t xb = xt_kept ? 0 : align256((size_t)g.W * g.H * g.Cin * g.N * sizeof(T));
-    const size_t yb = align256((size_t)g.OW * g.OH * g.Cout * g.N * sizeof(T));
-    const size_t wb = align256((size_t)g.kW * g.kH * g.Cin_g * g.Cout * sizeof(T));
-    const size_t pb = wgrad_partial_bytes<T>(g);
+    const bool any = !tap_shape<T>(g, true), kept = kept_usable<T>(g, xt_kept);
+    const AnyPlan<T> plan(g, true);
+    const size_t xb = kept ? 0 : xt_bytes<T>(g), yb = dyt_bytes<T>(g), wb = filter_bytes<T>(g, any, plan), pb = wgrad_partial_bytes<T>(g);
     // bf16: dz, its channel-contiguous copy and the bias gradient in one pass, when both a pass over delta and a
     // transposing copy would run
     bool one_pass = false;
     if constexpr (sizeof(T) == 2)
-        one_pass = (act != LUXHIP_ACT_IDENTITY || dbias != nullptr) && (dw != nullptr || dx != nullptr) &&
-                   dz_cwhn_ok(g.OW * g.OH, g.Cout, g.N, delta, y, pre, dz, nullptr);
+        one_pass = (act != LUXHIP_ACT_IDENTITY || dbias != nullptr) && (dw != nullptr || dx != nullptr) && padded<T>(g.Cout_g) == g.Cout_g &&
+                   dy_zeros<T>(g) == 0 && dz_cwhn_ok(g.OW * g.OH, g.Cout, g.N, delta, y, pre, dz, nullptr);
     const size_t bb = one_pass && dbias != nullptr ? dz_cwhn_partial_bytes(g.OW * g.OH, g.Cout, g.N) : 0;
     // reserve everything up front: the bias-gradient pass below uses the start of the same
     // workspace, and the buffer must not be reallocated while pointers into it are live
     Workspace ws;
-    int rc = get_workspace(s, xb + yb + wb + pb + bb, &ws);
+    int rc = get_workspace(s, xb + yb + wb + pb + bb + (any ? cany::most_partial_bytes() : 0), &ws);
     if (rc != LUXHIP_OK) return rc;
-    const T* xT = xt_kept ? xt_kept : reinterpret_cast<const T*>(ws.data);
+    const T* xT = kept ? xt_kept : reinterpret_cast<const T*>(ws.data);
     T* dzT = reinterpret_cast<T*>(ws.data + xb);
     T* wD = reinterpret_cast<T*>(ws.data + xb + yb);
     float* partial = reinterpret_cast<float*>(ws.data + xb + yb + wb);
     const T* dzp = delta;
+    bool packed = dx != nullptr;          // the filter is in wD when the input gradient starts
     BiasPartials bias_later;              // set by the single pass when the filter gradient's reduction will finish the bias gradient
     if (one_pass) {
         if constexpr (sizeof(T) == 2) {
             bf16_t* dz_out = act == LUXHIP_ACT_IDENTITY ? nullptr : reinterpret_cast<bf16_t*>(dz);
+            packed = packed && !any;
             rc = conv_dz_cwhn_pack(s, act, g, reinterpret_cast<const bf16_t*>(delta), reinterpret_cast<const bf16_t*>(y),
                                    reinterpret_cast<const bf16_t*>(pre), dz_out, reinterpret_cast<bf16_t*>(dzT),
                                    reinterpret_cast<float*>(ws.data + xb + yb + wb + pb), reinterpret_cast<bf16_t*>(dbias),
-                                   reinterpret_cast<const bf16_t*>(w), dx != nullptr ? reinterpret_cast<bf16_t*>(wD) : nullptr,
+                                   reinterpret_cast<const bf16_t*>(w), packed ? reinterpret_cast<bf16_t*>(wD) : nullptr,
                                    dw != nullptr ? &bias_later : nullptr);
             if (rc != LUXHIP_OK) return rc;
             if (dz_out) dzp = dz;
@@ -696,16 +1035,24 @@ static int fused_conv_bwd_t(hipStream_t s, int dtype, int act, const ConvGeom& g
             if (dz_out) dzp = dz_out;
         }
         if (dw == nullptr && dx == nullptr) return LUXHIP_OK;
-        if (dx != nullptr) rc = transpose_and_pack<T>(s, dzp, dzT, g.OW * g.OH, g.Cout, g.N, w, wD, g, 1);
-        else rc = transpose_to_cwhn<T>(s, dzp, dzT, g.OW * g.OH, g.Cout, g.N);
+        if (dx != nullptr) rc = dy_transpose_and_pack<T>(s, g, any, plan, dzp, dzT, w, wD);
+        else rc = to_cwhn_padded<T>(s, dzp, dzT, g.OW * g.OH, g.Cout_g, g.groups, g.N, dy_zeros<T>(g), g);
         if (rc != LUXHIP_OK) return rc;
     }
     if (dx != nullptr) {
-        if ((rc = run_conv_gemm<T>(s, g, true, dzT, wD, nullptr, dx, nullptr, LUXHIP_ACT_IDENTITY, ws.zeros)) != LUXHIP_OK) return rc;
+        if ((rc = run_dgrad<T>(s, g, any, plan, dzT, w, wD, packed, dx, xb + yb + wb + pb + bb, ws.zeros)) != LUXHIP_OK) return rc;
     }
     if (dw != nullptr) {
-        if (!xt_kept && (rc = transpose_to_cwhn<T>(s, x, reinterpret_cast<T*>(ws.data), g.W * g.H, g.Cin, g.N)) != LUXHIP_OK)
-            return rc;
+        if (!kept) {
+            T* xw = reinterpret_cast<T*>(ws.data);
+            if (x != nullptr) {
+                if ((rc = to_cwhn_padded<T>(s, x, xw, g.W * g.H, g.Cin_g, g.groups, g.N, 0, g)) != LUXHIP_OK) return rc;
+            } else {
+                const int64_t total = (int64_t)g.W * g.H * g.N * g.groups * padded<T>(g.Cin_g);
+                repad_cwhn_kernel<T><<<(unsigned)std::min<int64_t>(ceil_div(total, 256), 65536), 256, 0, s>>>(xt_kept, xw, total, g.Cin_g, padded<T>(g.Cin_g));
+                LUX_CHECK_LAUNCH();
+            }
+        }
         if ((rc = run_wgrad<T>(s, g, xT, dzp, dzT, partial, dw, ws.zeros, bias_later.dbias != nullptr ? &bias_later : nullptr)) != LUXHIP_OK)
             return rc;
     }

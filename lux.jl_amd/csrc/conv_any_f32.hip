@@ -1,0 +1,8 @@
+// Kernels of conv_any.h, storage f32.
+#include "conv_any_launch.h"
+namespace luxhip {
+namespace cany {
+template int launch_any<float>(hipStream_t, Args<float>&, size_t, bool);
+template int launch_any_wgrad<float>(hipStream_t, WgradArgs<float>&, int, bool);
+}
+}

@@ -1,14 +1,7 @@
 // fprop / dgrad implicit-GEMM kernels, storage type f32: tile selection + instantiation.
 #include "conv_kernels.h"
 namespace luxhip {
-template <>
-int launch_conv_gemm_any<float>(hipStream_t s, ConvGemmArgs<float>& a) {
-    const int64_t cus = num_cus() > 0 ? num_cus() : 256;
-    if (a.Ncols > 64 && ceil_div(a.gather.M, 256) * ceil_div(a.Ncols, 128) >= cus) return launch_conv_gemm<float, 4, 2>(s, a);
-    if (a.Ncols > 64 && a.gather.M > 64) return launch_conv_gemm<float, 2, 2>(s, a);
-    return launch_conv_gemm<float, 1, 1>(s, a);
-}
-// whole-tap stages through registers: 128 x 128 tiles (two workgroups per compute unit).  The
+// Whole-tap stages through registers: 128 x 128 tiles (two workgroups per compute unit).  The
 // tiles run in rounds of `resident` workgroups; a last round with only a few tiles (at most 10 %
 // of all) would cost a whole tile time for little work, so those rows go to 64 x 64 tiles.
 template <>

@@ -1,11 +1,6 @@
 // wgrad implicit-GEMM kernels, storage type bf16: tile selection + instantiation.
 #include "conv_kernels.h"
 namespace luxhip {
-template <>
-int launch_conv_wgrad_any<bf16_t>(hipStream_t s, ConvWgradArgs<bf16_t>& a, int slices, bool small) {
-    if (small) return launch_conv_wgrad<bf16_t, 1, 1>(s, a, slices);
-    return launch_conv_wgrad<bf16_t, 2, 2>(s, a, slices);
-}
 // 128 x 128 tiles on 4 waves, 4 LDS stages (two workgroups per compute unit)
 int launch_conv_wgrad_direct(hipStream_t s, ConvWgradDirectArgs& a, int slices) {
     using ML = GemmMainloop<bf16_t, 2, 2, false, true, true, 2, 4, 2>;

@@ -30,103 +30,6 @@ struct ConvGeom {
     int flip;
 };
 
-// Rows m = (p, q, n) of the implicit im2col matrix, gathered from a channel-contiguous source.
-template <typename T>
-struct GatherK {
-    const T* src;
-    int Ctot, c_off, Cg;       // source channel count, first channel of the group, channels per group
-    int P, PQ, M;              // row space: p in [0,P), q, n;  PQ = P*Q
-    int SP, SQ;                // source spatial extent
-    int kW, sw, sh, pw, ph, dw, dh;
-    int dgrad, vec_ok;
-    FastDiv divP, divPQ, divCg, divkW, divsw, divsh;
-
-    __device__ __forceinline__ bool locate(int m, int k, int64_t& off) const {
-        const int n = (int)divPQ.div((uint32_t)m);
-        const int rem = m - n * PQ;
-        const int q = (int)divP.div((uint32_t)rem);
-        const int p = rem - q * P;
-        const int t = (int)divCg.div((uint32_t)k);
-        const int c = k - t * Cg;
-        const int kb = (int)divkW.div((uint32_t)t);
-        const int ka = t - kb * kW;
-        int sp, sq;
-        if (!dgrad) {
-            sp = p * sw + ka * dw - pw;
-            sq = q * sh + kb * dh - ph;
-        } else {
-            const int tp = p + pw - ka * dw, tq = q + ph - kb * dh;
-            if (tp < 0 || tq < 0) return false;
-            sp = (int)divsw.div((uint32_t)tp);
-            sq = (int)divsh.div((uint32_t)tq);
-            if (sp * sw != tp || sq * sh != tq) return false;
-        }
-        if (sp < 0 || sp >= SP || sq < 0 || sq >= SQ) return false;
-        off = (((int64_t)n * SQ + sq) * SP + sp) * Ctot + c_off + c;
-        return true;
-    }
-};
-
-template <typename T, int ROWS>
-struct ConvGatherLoaderK {
-    using Tr = GemmTraits<T>;
-    static constexpr bool KMAJOR = true;
-    static constexpr int CHUNKS = ROWS * Tr::BK / Tr::VEC;
-    static constexpr int PER_THREAD = CHUNKS / kGemmThreads;
-    u32x4_v reg[PER_THREAD];
-    const GatherK<T>& g;
-    int m0, K;
-    __device__ __forceinline__ ConvGatherLoaderK(const GatherK<T>& gg, int row0, int k_total) : g(gg), m0(row0), K(k_total) {}
-
-    __device__ __forceinline__ void load(int k0) {
-#pragma unroll
-        for (int i = 0; i < PER_THREAD; ++i) {
-            const int id = threadIdx.x + i * kGemmThreads;
-            const int r = id / (Tr::BK / Tr::VEC);
-            const int k = k0 + (id % (Tr::BK / Tr::VEC)) * Tr::VEC;
-            const int m = m0 + r;
-            u32x4_v v = {0u, 0u, 0u, 0u};
-            if (m < g.M && k < K) {
-                if (g.vec_ok) {          // K % VEC == 0 and chunks never straddle a tap
-                    int64_t off;
-                    if (g.locate(m, k, off)) v = *reinterpret_cast<const u32x4_v*>(g.src + off);
-                } else {
-                    T tmp[Tr::VEC];
-#pragma unroll
-                    for (int e = 0; e < Tr::VEC; ++e) {
-                        int64_t off;
-                        tmp[e] = (k + e < K && g.locate(m, k + e, off)) ? g.src[off] : T(0);
-                    }
-                    v = *reinterpret_cast<const u32x4_v*>(tmp);
-                }
-            }
-            reg[i] = v;
-        }
-    }
-
-    __device__ __forceinline__ void store(T* lds) const {
-#pragma unroll
-        for (int i = 0; i < PER_THREAD; ++i) {
-            const int id = threadIdx.x + i * kGemmThreads;
-            const int r = id / (Tr::BK / Tr::VEC), k = (id % (Tr::BK / Tr::VEC)) * Tr::VEC;
-            *reinterpret_cast<u32x4_v*>(lds + lds_chunk_offset<T, true, ROWS>(r, k)) = reg[i];
-        }
-    }
-};
-
-template <typename T>
-struct ConvGemmArgs {
-    GatherK<T> gather;
-    Operand<T> Wm;                     // filter matrix, K-major, rows = output columns of this group
-    int K, Ncols;                      // contraction length, number of output columns (channels of the group)
-    // epilogue: element (m=(p,q,n), col) -> out[(m - n*PQ) + PQ*(col_off + col + Ctot_out*n)]
-    T* out;
-    T* pre;
-    const T* bias;                     // per output column (global channel index), may be null
-    int Ctot_out, col_off, act;
-    int tiles_m, tiles_n;
-};
-
 // Epilogue of fprop / dgrad: element (m = (p, q, n), col) -> out[(m - n*PQ) + PQ*(col_off + col +
 // Ctot_out*n)], with bias per output channel and the activation.  The image index of a row is
 // decoded once per row, the channel terms once per column.  CHECK (tiles that stick out of the
@@ -188,48 +91,6 @@ __device__ __forceinline__ void conv_epilogue(const f32x16_v (&acc)[WM][WN], int
         LUX_CONV_EPI(false, 2, false);
     }
 #undef LUX_CONV_EPI
-}
-
-// fprop and dgrad share this kernel (the gather loader's `dgrad` flag picks the index map).
-// Persistent: workgroup b handles tiles b, b + gridDim.x, ...
-template <typename T, int WM, int WN>
-__global__ __launch_bounds__(kGemmThreads) void conv_gemm_kernel(ConvGemmArgs<T> a) {
-    using ML = GemmMainloop<T, WM, WN, true, true>;
-    extern __shared__ __align__(16) unsigned char lds_raw[];
-    T* lds = reinterpret_cast<T*>(lds_raw);
-    const GatherK<T>& g = a.gather;
-    const int total = a.tiles_m * a.tiles_n;
-    for (int t = blockIdx.x; t < total; t += gridDim.x) {
-        int tm, tn;
-        tile_coords(t, a.tiles_m, a.tiles_n, tm, tn);
-        const int m0 = tm * ML::TILE_M, n0 = tn * ML::TILE_N;
-        ConvGatherLoaderK<T, ML::TILE_M> la(g, m0, a.K);
-        typename ML::PlainLoaderB lb(a.Wm, n0, a.K);
-        f32x16_v acc[WM][WN];
-        ML::run(la, lb, a.K, lds, acc);
-        conv_epilogue<ML, T, WM, WN>(acc, m0, n0, g.M, g.PQ, g.divPQ, a.Ncols, a.col_off, a.Ctot_out, a.bias, a.out, a.pre, a.act);
-        __syncthreads();   // every wave is done with the LDS stages before the next tile refills them
-    }
-}
-
-template <typename T, int WM, int WN>
-int launch_conv_gemm(hipStream_t s, ConvGemmArgs<T>& a) {
-    using ML = GemmMainloop<T, WM, WN, true, true>;
-    a.tiles_m = (int)ceil_div(a.gather.M, ML::TILE_M);
-    a.tiles_n = (int)ceil_div(a.Ncols, ML::TILE_N);
-    auto kernel = conv_gemm_kernel<T, WM, WN>;
-    static ResidentOnce ro;    // workgroups that fit the device at once
-    const int resident = ro.get([&](hipError_t& err) {
-        err = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)ML::LDS_BYTES);
-        return err == hipSuccess ? persistent_grid(kernel, kGemmThreads, ML::LDS_BYTES, int64_t(1) << 40) : 0;
-    });
-    LUX_CHECK_HIP(ro.error);
-    const int grid = (int)std::min<int64_t>((int64_t)a.tiles_m * a.tiles_n, resident);
-    ProfScope ps(a.gather.dgrad ? (sizeof(T) == 2 ? "conv_dgrad_kernel<bf16>" : "conv_dgrad_kernel<f32>")
-                                : (sizeof(T) == 2 ? "conv_fprop_kernel<bf16>" : "conv_fprop_kernel<f32>"), s);
-    kernel<<<dim3((unsigned)grid), dim3(kGemmThreads), ML::LDS_BYTES, s>>>(a);
-    LUX_CHECK_LAUNCH();
-    return LUXHIP_OK;
 }
 
 // ----------------------------------------------------------------------------- whole-tap stages
@@ -461,138 +322,6 @@ int launch_conv_tap(hipStream_t s, ConvTapArgs<T>& a) {
 template <typename T>
 int launch_conv_tap_any(hipStream_t s, ConvTapArgs<T>& a);   // picks the tile; conv_inst_*.hip
 
-template <typename T>
-int launch_conv_gemm_any(hipStream_t s, ConvGemmArgs<T>& a);   // picks the tile; conv_inst_*.hip
-
-// ----------------------------------------------------------------------------- wgrad
-// A(m'=(tap,ci), k'=(ow,oh,n)): MN-major gather from xT (runs of ci at one input position).
-template <typename T>
-struct GatherMN {
-    const T* src;              // xT
-    int Ctot, c_off, Cg;       // Cin, g*Cin_g, Cin_g
-    int Mrows;                 // taps * Cin_g
-    int OW, OWOH;              // k' decoding
-    int SP, SQ;                // W, H
-    int kW, sw, sh, pw, ph, dw, dh;
-    int vec_ok;
-    FastDiv divOW, divOWOH, divCg, divkW;
-
-    __device__ __forceinline__ bool locate(int mrow, int kp, int64_t& off) const {
-        const int t = (int)divCg.div((uint32_t)mrow);
-        const int c = mrow - t * Cg;
-        const int kb = (int)divkW.div((uint32_t)t);
-        const int ka = t - kb * kW;
-        const int n = (int)divOWOH.div((uint32_t)kp);
-        const int rem = kp - n * OWOH;
-        const int oh = (int)divOW.div((uint32_t)rem);
-        const int ow = rem - oh * OW;
-        const int sp = ow * sw + ka * dw - pw, sq = oh * sh + kb * dh - ph;
-        if (sp < 0 || sp >= SP || sq < 0 || sq >= SQ) return false;
-        off = (((int64_t)n * SQ + sq) * SP + sp) * Ctot + c_off + c;
-        return true;
-    }
-};
-
-template <typename T, int ROWS>
-struct ConvGatherLoaderMN {
-    using Tr = GemmTraits<T>;
-    static constexpr bool KMAJOR = false;
-    static constexpr int CHUNKS = ROWS * Tr::BK / Tr::VEC;
-    static constexpr int PER_THREAD = CHUNKS / kGemmThreads;
-    u32x4_v reg[PER_THREAD];
-    const GatherMN<T>& g;
-    int m0, kbase, Kend;       // Kend = one past the last k' of this slice
-    __device__ __forceinline__ ConvGatherLoaderMN(const GatherMN<T>& gg, int row0, int kb, int ke)
-        : g(gg), m0(row0), kbase(kb), Kend(ke) {}
-
-    __device__ __forceinline__ void load(int k0) {
-#pragma unroll
-        for (int i = 0; i < PER_THREAD; ++i) {
-            const int id = threadIdx.x + i * kGemmThreads;
-            const int kp = kbase + k0 + id / (ROWS / Tr::VEC);
-            const int mrow = m0 + (id % (ROWS / Tr::VEC)) * Tr::VEC;
-            u32x4_v v = {0u, 0u, 0u, 0u};
-            if (kp < Kend && mrow < g.Mrows) {
-                if (g.vec_ok) {
-                    int64_t off;
-                    if (g.locate(mrow, kp, off)) v = *reinterpret_cast<const u32x4_v*>(g.src + off);
-                } else {
-                    T tmp[Tr::VEC];
-#pragma unroll
-                    for (int e = 0; e < Tr::VEC; ++e) {
-                        int64_t off;
-                        tmp[e] = (mrow + e < g.Mrows && g.locate(mrow + e, kp, off)) ? g.src[off] : T(0);
-                    }
-                    v = *reinterpret_cast<const u32x4_v*>(tmp);
-                }
-            }
-            reg[i] = v;
-        }
-    }
-
-    __device__ __forceinline__ void store(T* lds) const {
-#pragma unroll
-        for (int i = 0; i < PER_THREAD; ++i) {
-            const int id = threadIdx.x + i * kGemmThreads;
-            const int k = id / (ROWS / Tr::VEC), r = (id % (ROWS / Tr::VEC)) * Tr::VEC;
-            *reinterpret_cast<u32x4_v*>(lds + lds_chunk_offset<T, false, ROWS>(r, k)) = reg[i];
-        }
-    }
-};
-
-template <typename T>
-struct ConvWgradArgs {
-    GatherMN<T> gather;
-    const T* dyT;           // [k'][Cout] channel-contiguous
-    int Cout, co_off, Cout_g;
-    int Ktotal, kslice;     // OW*OH*N and the k' extent of one slice
-    float* partial;         // [slice][Mrows][Cout_g]
-    int dy_vec_ok;
-    int tiles_m, tiles_n;
-};
-
-template <typename T, int WM, int WN>
-__global__ __launch_bounds__(kGemmThreads) void conv_wgrad_kernel(ConvWgradArgs<T> a) {
-    using ML = GemmMainloop<T, WM, WN, false, false>;
-    extern __shared__ __align__(16) unsigned char lds_raw[];
-    T* lds = reinterpret_cast<T*>(lds_raw);
-    const int tile = blockIdx.x, slice = blockIdx.y;
-    const int tm = tile % a.tiles_m, tn = tile / a.tiles_m;
-    const int m0 = tm * ML::TILE_M, n0 = tn * ML::TILE_N;
-    const int kbeg = slice * a.kslice, kend = min(kbeg + a.kslice, a.Ktotal);
-    const GatherMN<T>& g = a.gather;
-    ConvGatherLoaderMN<T, ML::TILE_M> la(g, m0, kbeg, kend);
-    Operand<T> B;
-    B.p = a.dyT + (int64_t)kbeg * a.Cout + a.co_off;
-    B.sr = 1; B.sk = a.Cout; B.rows = a.Cout_g; B.vec_ok = a.dy_vec_ok;
-    typename ML::PlainLoaderB lb(B, n0, kend - kbeg);
-    f32x16_v acc[WM][WN];
-    ML::run(la, lb, kend - kbeg, lds, acc);
-    float* out = a.partial + (size_t)slice * g.Mrows * a.Cout_g;
-    const int Mrows = g.Mrows, Ncols = a.Cout_g;
-    ML::for_each(acc, m0, n0, [&](int m, int col, float v) {
-        if (m < Mrows && col < Ncols) out[(size_t)m + (size_t)col * Mrows] = v;
-    });
-}
-
-template <typename T, int WM, int WN>
-int launch_conv_wgrad(hipStream_t s, ConvWgradArgs<T>& a, int slices) {
-    using ML = GemmMainloop<T, WM, WN, false, false>;
-    a.tiles_m = (int)ceil_div(a.gather.Mrows, ML::TILE_M);
-    a.tiles_n = (int)ceil_div(a.Cout_g, ML::TILE_N);
-    auto kernel = conv_wgrad_kernel<T, WM, WN>;
-    static ResidentOnce ro;   // here only the one-time raise of the dynamic LDS limit
-    ro.get([&](hipError_t& err) {
-        err = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)ML::LDS_BYTES);
-        return 1;
-    });
-    LUX_CHECK_HIP(ro.error);
-    ProfScope ps(sizeof(T) == 2 ? "conv_wgrad_kernel<bf16>" : "conv_wgrad_kernel<f32>", s);
-    kernel<<<dim3((unsigned)(a.tiles_m * a.tiles_n), (unsigned)slices), dim3(kGemmThreads), ML::LDS_BYTES, s>>>(a);
-    LUX_CHECK_LAUNCH();
-    return LUXHIP_OK;
-}
-
 // ----------------------------------------------------------------------------- wgrad, bf16 straight into LDS
 // A(m' = (tap, ci), k' = (ow, oh, n)) gathered from the channel-contiguous xT into the MN-major
 // LDS layout: a thread's 16-byte chunk always covers the same 8 channels of the same tap, so
@@ -766,8 +495,5 @@ __global__ __launch_bounds__(NWM * NWN * 64) void conv_wgrad_direct_kernel(ConvW
 }
 
 int launch_conv_wgrad_direct(hipStream_t s, ConvWgradDirectArgs& a, int slices);   // conv_inst_wgrad_bf16.hip
-
-template <typename T>
-int launch_conv_wgrad_any(hipStream_t s, ConvWgradArgs<T>& a, int slices, bool small);   // conv_inst_*.hip
 
 }  // namespace luxhip

@@ -35,20 +35,21 @@ struct UnalignedVec<bf16_t> { typedef uint32_t type __attribute__((ext_vector_ty
 
 // One stage (BK of k) of an operand tile of ROWS rows in registers, rows r0 .. r0 + ROWS - 1 (r0 + ROWS <= rows, or
 // r0 = 0 and rows < ROWS: `bounded`).
-template <typename T, bool KMAJOR, int ROWS>
+template <typename T, bool KMAJOR_, int ROWS>
 struct Loader {
+    static constexpr bool KMAJOR = KMAJOR_;
     using Tr = GemmTraits<T>;
-    static constexpr int PER = ROWS * Tr::BK / Tr::VEC / THREADS;
-    static_assert(PER >= 1 && ROWS * Tr::BK / Tr::VEC % THREADS == 0, "a stage splits evenly over the workgroup");
+    static constexpr int CHUNKS = ROWS * Tr::BK / Tr::VEC;
+    static constexpr int PER = CHUNKS > THREADS ? CHUNKS / THREADS : 1;
+    static_assert(CHUNKS % THREADS == 0 || THREADS % CHUNKS == 0, "a stage splits evenly over the workgroup");
     static constexpr int CPR = KMAJOR ? Tr::BK / Tr::VEC : ROWS / Tr::VEC;      // chunks per LDS row
-    static constexpr int STEP = THREADS / CPR;
     const char* base;          // uniform: element (r0, k = 0)
     int64_t k_bytes;           // uniform
     uint32_t voff[PER];        // per thread
     int sh[PER];               // MN-major, bounded: elements that the chunk at the end of the rows is moved by
     bool bounded;              // uniform
     __device__ __forceinline__ static void coords(int i, int& r, int& k) {
-        const int id = threadIdx.x + i * THREADS;
+        const int id = CHUNKS < THREADS ? (int)threadIdx.x % CHUNKS : (int)threadIdx.x + i * THREADS;   // fewer chunks than threads: doubly
         if constexpr (KMAJOR) { r = id / CPR; k = (id % CPR) * Tr::VEC; }
         else { k = id / CPR; r = (id % CPR) * Tr::VEC; }
     }
@@ -116,55 +117,54 @@ struct Plan {
     uint32_t* counters;        // one per tile
 };
 
-template <typename T, int W, bool AK, bool BKM>
-struct Body {
-    static constexpr int U = W == 1 ? 4 : 2;
-    using ML = GemmMainloop<T, W, W, AK, BKM>;
+// The main loop over loaders of the two operands: a workgroup of NWM x NWN waves, each with WM x WN accumulators.
+template <typename T, int WM, int WN, int NWM, int NWN, class LA, class LB>
+struct Core {
+    static constexpr bool AK = LA::KMAJOR, BKM = LB::KMAJOR;
+    using ML = GemmMainloop<T, WM, WN, AK, BKM, false, NWN, 0, NWM>;
     using Tr = GemmTraits<T>;
-    using LA = Loader<T, AK, ML::TILE_M>;
-    using LB = Loader<T, BKM, ML::TILE_N>;
+    static constexpr int U = LA::PER + LB::PER <= 2 ? 4 : 2;
     static constexpr size_t LDS_BYTES = (size_t)U * ML::STAGE_ELEMS * sizeof(T);
+    static_assert(NWM * NWN * 64 == THREADS, "four waves");
 
-    __device__ __forceinline__ static void compute(const T* As, const T* Bs, int wave_m, int wave_n, f32x16_v (&acc)[W][W]) {
+    __device__ __forceinline__ static void compute(const T* As, const T* Bs, int wave_m, int wave_n, f32x16_v (&acc)[WM][WN]) {
         if constexpr (sizeof(T) == 2) {
 #pragma unroll
             for (int kk = 0; kk < Tr::BK / 16; ++kk) {
-                bf16x8_v fa[W], fb[W];
+                bf16x8_v fa[WM], fb[WN];
 #pragma unroll
-                for (int i = 0; i < W; ++i) fa[i] = load_frag_bf16<AK, ML::TILE_M>(As, wave_m + i * 32, kk);
+                for (int i = 0; i < WM; ++i) fa[i] = load_frag_bf16<AK, ML::TILE_M>(As, wave_m + i * 32, kk);
 #pragma unroll
-                for (int j = 0; j < W; ++j) fb[j] = load_frag_bf16<BKM, ML::TILE_N>(Bs, wave_n + j * 32, kk);
+                for (int j = 0; j < WN; ++j) fb[j] = load_frag_bf16<BKM, ML::TILE_N>(Bs, wave_n + j * 32, kk);
 #pragma unroll
-                for (int i = 0; i < W; ++i)
+                for (int i = 0; i < WM; ++i)
 #pragma unroll
-                    for (int j = 0; j < W; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fb[j], fa[i], acc[i][j], 0, 0, 0);
+                    for (int j = 0; j < WN; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fb[j], fa[i], acc[i][j], 0, 0, 0);
             }
         } else {
 #pragma unroll
             for (int kw = 0; kw < Tr::BK / 8; ++kw) {
-                float fa[W][4], fb[W][4];
+                float fa[WM][4], fb[WN][4];
 #pragma unroll
-                for (int i = 0; i < W; ++i) load_frag_f32<AK, ML::TILE_M>(As, wave_m + i * 32, kw, fa[i]);
+                for (int i = 0; i < WM; ++i) load_frag_f32<AK, ML::TILE_M>(As, wave_m + i * 32, kw, fa[i]);
 #pragma unroll
-                for (int j = 0; j < W; ++j) load_frag_f32<BKM, ML::TILE_N>(Bs, wave_n + j * 32, kw, fb[j]);
+                for (int j = 0; j < WN; ++j) load_frag_f32<BKM, ML::TILE_N>(Bs, wave_n + j * 32, kw, fb[j]);
 #pragma unroll
                 for (int s = 0; s < 4; ++s)
 #pragma unroll
-                    for (int i = 0; i < W; ++i)
+                    for (int i = 0; i < WM; ++i)
 #pragma unroll
-                        for (int j = 0; j < W; ++j)
+                        for (int j = 0; j < WN; ++j)
                             acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(fb[j][s], fa[i][s], acc[i][j], 0, 0, 0);
             }
         }
     }
 
-    // k range [kbeg, kend) of the tile at (m0, n0)
-    __device__ __forceinline__ static void run(const DenseArgs<T>& a, int kbeg, int kend, int m0, int n0, T* lds, f32x16_v (&acc)[W][W]) {
+    // k range [kbeg, kend)
+    __device__ __forceinline__ static void run(const LA& la, const LB& lb, int kbeg, int kend, T* lds, f32x16_v (&acc)[WM][WN]) {
         const int w = threadIdx.x >> 6;
-        const int wave_m = (w & 1) * (W * 32), wave_n = (w >> 1) * (W * 32);
+        const int wave_m = (w % NWM) * (WM * 32), wave_n = (w / NWM) * (WN * 32);
         ML::zero(acc);
-        const LA la(a.A, m0);
-        const LB lb(a.B, n0);
         u32x4_v ra[U][LA::PER], rb[U][LB::PER];
         int skip[U];
         auto fetch_stages = [&](int k0) {
@@ -197,20 +197,20 @@ struct Body {
     }
 
     // hand-off of a slice's accumulators; true in the workgroup that holds the sum and runs the epilogue
-    __device__ __forceinline__ static bool combine(const Plan& p, int tile, int slice, f32x16_v (&acc)[W][W]) {
+    __device__ __forceinline__ static bool combine(const Plan& p, int tile, int slice, f32x16_v (&acc)[WM][WN]) {
         __shared__ uint32_t flag;
-        constexpr int PAIRS = W * W * 8;
+        constexpr int PAIRS = WM * WN * 8;
         uint64_t* mine = reinterpret_cast<uint64_t*>(p.partial) + ((size_t)tile * p.slices + slice) * (PAIRS * THREADS) + threadIdx.x;
         static_for<PAIRS>([&](auto Q) {
             constexpr int q = decltype(Q)::value, ij = q / 8, r = (q % 8) * 2;
-            const uint64_t v = ((uint64_t)__float_as_uint(acc[ij / W][ij % W][r + 1]) << 32) | __float_as_uint(acc[ij / W][ij % W][r]);
+            const uint64_t v = ((uint64_t)__float_as_uint(acc[ij / WN][ij % WN][r + 1]) << 32) | __float_as_uint(acc[ij / WN][ij % WN][r]);
             __hip_atomic_store(mine + q * THREADS, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         });
         publish_done();
         if (!arrive_last(p.counters + tile, (uint32_t)p.slices, &flag)) return false;
         ML::zero(acc);
         const uint64_t* all = reinterpret_cast<const uint64_t*>(p.partial) + (size_t)tile * p.slices * (PAIRS * THREADS) + threadIdx.x;
-#pragma unroll (W == 1 ? 4 : 1)
+#pragma unroll (WM * WN == 1 ? 4 : 1)
         for (int s = 0; s < p.slices; ++s) {
             uint64_t v[PAIRS];
             static_for<PAIRS>([&](auto Q) {
@@ -219,13 +219,16 @@ struct Body {
             });
             static_for<PAIRS>([&](auto Q) {
                 constexpr int q = decltype(Q)::value, ij = q / 8, r = (q % 8) * 2;
-                acc[ij / W][ij % W][r] += __uint_as_float((uint32_t)v[q]);
-                acc[ij / W][ij % W][r + 1] += __uint_as_float((uint32_t)(v[q] >> 32));
+                acc[ij / WN][ij % WN][r] += __uint_as_float((uint32_t)v[q]);
+                acc[ij / WN][ij % WN][r + 1] += __uint_as_float((uint32_t)(v[q] >> 32));
             });
         }
         return true;
     }
 };
+
+template <typename T, int W, bool AK, bool BKM>
+using Body = Core<T, W, W, 2, 2, Loader<T, AK, 64 * W>, Loader<T, BKM, 64 * W>>;
 
 // One (tile, slice) of a product; `id` counts the slices of a tile together.
 template <typename T, int W, bool AK, bool BKM, bool PLAIN = false>
@@ -238,7 +241,9 @@ __device__ __forceinline__ void tile_slice(const DenseArgs<T>& a, const Plan& p,
     const int m0 = max(min(tm * ML::TILE_M, a.M - ML::TILE_M), 0), n0 = max(min(tn * ML::TILE_N, a.N - ML::TILE_N), 0);
     const int kbeg = slice * p.kslice, kend = min(kbeg + p.kslice, a.K);
     f32x16_v acc[W][W];
-    B::run(a, kbeg, kend, m0, n0, lds, acc);
+    const Loader<T, AK, 64 * W> la(a.A, m0);
+    const Loader<T, BKM, 64 * W> lb(a.B, n0);
+    B::run(la, lb, kbeg, kend, lds, acc);
     if (p.slices > 1 && !B::combine(p, tile, slice, acc)) return;
     if constexpr (PLAIN) dense_epilogue_as<ML, T, W, W, true, 0, false>(acc, a, m0, n0);      // no bias, no activation
     else if (a.M >= ML::TILE_M && a.N >= ML::TILE_N) dense_epilogue<ML, T, W, W, true>(acc, a, m0, n0);

@@ -1269,9 +1269,11 @@ def rrule_fused_conv_bias_activation(act: str, weight, x, b, cdims: DenseConvDim
         return _from_inner_output(cdims, y2), back3
     y = DeviceArray(cdims.y_shape, dt)
     pre = DeviceArray(cdims.y_shape, dt) if aid in _NEEDS_PRE else None
-    xt = DeviceArray(x.shape, dt)      # the channel-contiguous copy of x, kept for the filter gradient
+    # the channel-contiguous copy of x, kept for the filter gradient; where the kernels pad the channels of a group to whole
+    # 16-byte chunks their copy is not of x's shape, and making it again costs less than a second, unpadded one
+    xt = DeviceArray(x.shape, dt) if (cdims._c.Cin // cdims.groups) * x.itemsize % 16 == 0 else None
     _lib.call("luxhip_conv_fwd", current_stream(), y.code, aid, C.byref(cdims._c), x.ptr, weight.ptr, _p(b), y.ptr, _p(pre),
-              xt.ptr)
+              _p(xt))
 
     def back(delta):
         dw = DeviceArray(weight.shape, dt)
@@ -1279,7 +1281,7 @@ def rrule_fused_conv_bias_activation(act: str, weight, x, b, cdims: DenseConvDim
         db = None if b is None else DeviceArray(b.shape, dt)
         dz = None if aid == 0 else DeviceArray(cdims.y_shape, dt)
         _lib.call("luxhip_fused_conv_bwd", current_stream(), y.code, aid, C.byref(cdims._c), delta.ptr, y.ptr, _p(pre),
-                  x.ptr, weight.ptr, _p(dz), dw.ptr, dx.ptr, _p(db), xt.ptr)
+                  x.ptr, weight.ptr, _p(dz), dw.ptr, dx.ptr, _p(db), _p(xt))
         return dw, dx, db
 
     return y, back

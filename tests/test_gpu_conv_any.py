@@ -1,0 +1,86 @@
+"""Convolutions of any channel count and stride (conv_any.h) against the fp64 oracle: padded channels, the residues of a
+strided input gradient apart and merged, taps that some residues do not have, contractions shorter than a stage and cut into
+slices, and the kept copy of x whose channels the kernels would pad."""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+from oracle import luxlib_oracle as O
+from tests.util import assert_close, dev, f64, host_inputs, stable_seed
+
+pytestmark = pytest.mark.gpu
+
+CASES = [
+    # x shape, w shape, stride, pad, dilation, groups, flip
+    ((17, 15, 3, 3), (7, 7, 3, 20), 2, 3, 1, 1, False),              # residues merged into columns: 2 x 2 of 3 channels
+    ((9, 11, 6, 2), (5, 4, 2, 9), 3, (2, 1, 0, 2), 1, 3, True),      # 9 residues, groups of 2 -> 3 channels
+    ((13, 11, 5, 3), (2, 4, 5, 7), (2, 3), (1, 0, 3, 3), (3, 2), 1, False),   # stride and dilation share no factor
+    ((14, 10, 6, 2), (3, 3, 6, 5), 2, 2, 2, 1, False),               # ... share a factor: residues without taps
+    ((19, 17, 72, 2), (3, 3, 72, 40), 2, 1, 1, 1, False),            # one problem per residue
+    ((16, 9, 24, 3), (1, 1, 24, 33), 2, 0, 1, 1, False),             # three of four residues are zero
+    ((4, 4, 3, 1), (3, 3, 3, 4), 2, 1, 1, 1, False),                 # 4 output positions: less than a stage
+    ((6, 6, 200, 1), (5, 5, 200, 24), 1, 2, 1, 1, False),            # few rows, 5000 k: slices
+    ((23, 9, 61, 2), (3, 3, 61, 130), 1, (0, 1, 1, 0), 1, 1, True),  # more than 128 columns, ragged in everything
+    ((5, 3, 8, 2), (3, 3, 8, 8), 4, 2, 1, 1, False),                 # stride beyond the filter
+]
+
+
+@pytest.mark.parametrize("dtype", ["f32", "bf16"])
+@pytest.mark.parametrize("case", range(len(CASES)))
+def test_conv_any(gpu, dtype, case):
+    xs, ws, stride, pad, dil, groups, flip = CASES[case]
+    rng = np.random.default_rng(stable_seed("conv_any", case))
+    kw = dict(stride=stride, padding=pad, dilation=dil, groups=groups, flipkernel=flip)
+    gd, od = gpu.DenseConvDims(xs, ws, **kw), O.ConvDims(xs, ws, **kw)
+    x, w, b, dy = host_inputs(dtype, rng.normal(size=xs), rng.normal(size=ws) / np.sqrt(ws[0] * ws[1] * ws[2]), rng.normal(size=ws[3]),
+                              rng.normal(size=od.y_shape()))
+    dx_, dw_, db_, ddy = (dev(gpu, a, dtype) for a in (x, w, b, dy))
+    wy, wdw, wdx = O.conv(f64(x), f64(w), od), O.conv_filter_grad(f64(x), f64(dy), od), O.conv_data_grad(f64(dy), f64(w), od)
+    tag = f"{dtype} conv_any {case}"
+    y = gpu.fused_conv_bias_activation("relu", dw_, dx_, db_, gd)
+    assert_close(y.to_numpy(), np.maximum(wy + f64(b)[None, None, :, None], 0.0), dtype, tag + " y")
+    gx, gw = gpu.conv_data_grad(ddy, dw_, gd), gpu.conv_filter_grad(dx_, ddy, gd)
+    assert_close(gx.to_numpy(), wdx, dtype, tag + " dx")
+    assert_close(gw.to_numpy(), wdw, dtype, tag + " dw")
+    # the fused pullback (identity: dz is the cotangent) makes the same gradients
+    _, back = gpu.pullback(gpu.fused_conv_bias_activation, "identity", dw_, dx_, db_, gd)
+    fw, fx, fb = back(ddy)
+    np.testing.assert_array_equal(fx.to_numpy(), gx.to_numpy())
+    np.testing.assert_array_equal(fw.to_numpy(), gw.to_numpy())
+    assert_close(fb.to_numpy(), f64(dy).sum(axis=(0, 1, 3)), dtype, tag + " db")
+
+
+@pytest.mark.parametrize("dtype", ["f32", "bf16"])
+@pytest.mark.parametrize("xs,ws", [((9, 7, 5, 3), (3, 3, 5, 12)), ((8, 8, 16, 2), (3, 3, 16, 12))])
+def test_kept_copy_alone(gpu, dtype, xs, ws):
+    """xt_keep is the unpadded channel-contiguous copy whatever the channel count, and the pullback takes it in place of x."""
+    rng = np.random.default_rng(stable_seed("kept", xs))
+    gd, od = gpu.DenseConvDims(xs, ws, padding=1), O.ConvDims(xs, ws, padding=1)
+    x, w, dy = host_inputs(dtype, rng.normal(size=xs), rng.normal(size=ws), rng.normal(size=od.y_shape()))
+    dx_, dw_, ddy = (dev(gpu, a, dtype) for a in (x, w, dy))
+    y, kept, gw = gpu.DeviceArray(gd.y_shape, dtype), gpu.DeviceArray(xs, dtype), gpu.DeviceArray(ws, dtype)
+    s = gpu.current_stream()
+    gpu._lib.call("luxhip_conv_fwd", s, y.code, 0, C.byref(gd._c), dx_.ptr, dw_.ptr, None, y.ptr, None, kept.ptr)
+    np.testing.assert_array_equal(kept.to_numpy().ravel(order="F").reshape((xs[2], xs[0], xs[1], xs[3]), order="F"),
+                                  np.transpose(dx_.to_numpy(), (2, 0, 1, 3)))
+    gpu._lib.call("luxhip_fused_conv_bwd", s, y.code, 0, C.byref(gd._c), ddy.ptr, y.ptr, None, None, dw_.ptr, None, gw.ptr, None, None, kept.ptr)
+    assert_close(gw.to_numpy(), O.conv_filter_grad(f64(x), f64(dy), od), dtype, f"{dtype} dw from the kept copy")
+
+
+@pytest.mark.parametrize("dtype", ["f32", "bf16"])
+def test_whole_tap_kernels_at_small_sizes(gpu, dtype):
+    """conv_tile 42 takes the whole-tap kernels where the automatic choice prefers conv_any.h."""
+    gpu.set_option("conv_tile", 42)
+    try:
+        for xs, ws, stride, pad, dil, groups, flip in [((13, 11, 64, 3), (3, 2, 32, 64), (2, 1), (1, 0, 2, 1), (1, 2), 2, True),
+                                                       ((8, 8, 32, 5), (3, 3, 32, 320), 1, 1, 1, 1, False)]:
+            rng = np.random.default_rng(stable_seed("tap", xs))
+            kw = dict(stride=stride, padding=pad, dilation=dil, groups=groups, flipkernel=flip)
+            gd, od = gpu.DenseConvDims(xs, ws, **kw), O.ConvDims(xs, ws, **kw)
+            x, w, dy = host_inputs(dtype, rng.normal(size=xs), rng.normal(size=ws), rng.normal(size=od.y_shape()))
+            assert_close(gpu.conv(dev(gpu, x, dtype), dev(gpu, w, dtype), gd).to_numpy(), O.conv(f64(x), f64(w), od), dtype, "tap y")
+            assert_close(gpu.conv_data_grad(dev(gpu, dy, dtype), dev(gpu, w, dtype), gd).to_numpy(), O.conv_data_grad(f64(dy), f64(w), od),
+                         dtype, "tap dx")
+    finally:
+        gpu.set_option("conv_tile", 0)
