@@ -26,13 +26,6 @@ namespace split {
 
 constexpr int THREADS = 256;
 
-template <typename T>
-struct UnalignedVec;
-template <>
-struct UnalignedVec<float> { typedef uint32_t type __attribute__((ext_vector_type(4), aligned(4))); };
-template <>
-struct UnalignedVec<bf16_t> { typedef uint32_t type __attribute__((ext_vector_type(4), aligned(2))); };
-
 // One stage (BK of k) of an operand tile of ROWS rows in registers, rows r0 .. r0 + ROWS - 1 (r0 + ROWS <= rows, or
 // r0 = 0 and rows < ROWS: `bounded`).
 template <typename T, bool KMAJOR_, int ROWS>

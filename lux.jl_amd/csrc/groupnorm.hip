@@ -23,22 +23,12 @@ constexpr int kGnCache = 8;  // vectors per thread kept in registers
 
 struct GnGeom {
     uint32_t I, Cg, G, C;
-    uint32_t nvec;         // vectors per slice = I*Cg / VEC
+    uint32_t nvec, vpr;    // vectors per slice (Cg vpr) and per row of I elements
+    uint32_t m;            // elements per slice
     uint32_t parts, pvec;  // workgroups per slice (cached kernels; 1 otherwise) and vectors per part = nvec / parts
-    FastDiv chdiv;         // vector index -> channel within group: / (I / VEC)   (VEC == 1: / I)
+    FastDiv chdiv;         // vector index -> channel within group: / vpr
     float inv_m;           // 1 / (I*Cg)
 };
-
-template <typename T, int VEC>
-__device__ __forceinline__ void gn_load(const T* p, size_t off, float (&v)[VEC]) {
-    if constexpr (VEC == 1) v[0] = ld(p + off);
-    else Vec<T>::load(p + off, v);
-}
-template <typename T, int VEC>
-__device__ __forceinline__ void gn_store(T* p, size_t off, const float (&v)[VEC]) {
-    if constexpr (VEC == 1) st(p + off, v[0]);
-    else Vec<T>::store(p + off, v);
-}
 
 // ------------------------------------------------------------------------------- forward
 // Exchange area of the split kernels: `epoch`-tagged words, K per part, parts of a slice adjacent.
@@ -63,38 +53,41 @@ struct InRunning {
     float momentum, corrected;     // corrected = momentum * I / (I - 1)
 };
 
-template <typename T, int ACT, int VEC, bool CACHED>
+template <typename T, int ACT, int VEC, bool CACHED, bool RAGGED>
 __global__ void gn_fwd_kernel(const T* __restrict__ x, const T* __restrict__ gamma, const T* __restrict__ beta, T* y,
                               float* save_mean, float* save_invstd, GnGeom g, float eps, InRunning<T> rs) {
     __shared__ float sm[16];
     __shared__ uint32_t last_flag;
     const uint32_t slice = blockIdx.x;              // = n*G + k
     const uint32_t k = slice % g.G;
-    const size_t base = (size_t)slice * g.nvec * VEC;
+    const size_t base = (size_t)slice * g.m;
+    using R = RowVec<VEC, RAGGED>;
+    auto row_vec = [&](uint32_t q) { return R(q, g.I, g.vpr, g.chdiv); };
     const uint32_t T_ = blockDim.x;
     using K = Kept<T, VEC>;
     typename K::type kv[CACHED ? kGnCache : 1];   // cached: the slice as it lies in memory; loads past its end re-read the last vector
     float v[1][VEC];
+    auto counts = [&](uint32_t q, int e) { return !RAGGED || (uint32_t)e >= row_vec(q).skip; };
 
     // pass 1: mean
     float sum = 0.0f;
     if constexpr (CACHED) {
 #pragma unroll
-        for (int u = 0; u < kGnCache; ++u) kv[u] = K::load(x, base + (size_t)min(u * T_ + threadIdx.x, g.nvec - 1) * VEC);
+        for (int u = 0; u < kGnCache; ++u) kv[u] = kept_load<T, VEC, RAGGED>(x, base + row_vec(min(u * T_ + threadIdx.x, g.nvec - 1)).off);
 #pragma unroll
         for (int u = 0; u < kGnCache; ++u) {
             const uint32_t q = u * T_ + threadIdx.x;
             if (q < g.nvec) {
                 K::get(kv[u], v[0]);
 #pragma unroll
-                for (int e = 0; e < VEC; ++e) sum += v[0][e];
+                for (int e = 0; e < VEC; ++e) sum += counts(q, e) ? v[0][e] : 0.0f;
             }
         }
     } else {
         for (uint32_t q = threadIdx.x; q < g.nvec; q += T_) {
-            gn_load<T, VEC>(x, base + (size_t)q * VEC, v[0]);
+            row_load<T, VEC, RAGGED>(x, base + row_vec(q).off, v[0]);
 #pragma unroll
-            for (int e = 0; e < VEC; ++e) sum += v[0][e];
+            for (int e = 0; e < VEC; ++e) sum += counts(q, e) ? v[0][e] : 0.0f;
         }
     }
     const float mean = block_sum(sum, sm) * g.inv_m;
@@ -107,14 +100,14 @@ __global__ void gn_fwd_kernel(const T* __restrict__ x, const T* __restrict__ gam
             if (q < g.nvec) {
                 K::get(kv[u], v[0]);
 #pragma unroll
-                for (int e = 0; e < VEC; ++e) dev = fmaf(v[0][e] - mean, v[0][e] - mean, dev);
+                for (int e = 0; e < VEC; ++e) dev = counts(q, e) ? fmaf(v[0][e] - mean, v[0][e] - mean, dev) : dev;
             }
         }
     } else {
         for (uint32_t q = threadIdx.x; q < g.nvec; q += T_) {
-            gn_load<T, VEC>(x, base + (size_t)q * VEC, v[0]);
+            row_load<T, VEC, RAGGED>(x, base + row_vec(q).off, v[0]);
 #pragma unroll
-            for (int e = 0; e < VEC; ++e) dev = fmaf(v[0][e] - mean, v[0][e] - mean, dev);
+            for (int e = 0; e < VEC; ++e) dev = counts(q, e) ? fmaf(v[0][e] - mean, v[0][e] - mean, dev) : dev;
         }
     }
     const float var = block_sum(dev, sm) * g.inv_m;
@@ -158,13 +151,14 @@ __global__ void gn_fwd_kernel(const T* __restrict__ x, const T* __restrict__ gam
         __syncthreads();
     }
     auto emit = [&](uint32_t q, const float (&xv)[VEC]) {
-        const uint32_t j = g.chdiv.div(q), c = k * g.Cg + j;
+        const R rv = row_vec(q);
+        const uint32_t j = RAGGED ? rv.row : g.chdiv.div(q), c = k * g.Cg + j;
         const float sc = tabled ? chan[2 * j] : (gamma ? ld(gamma + c) : 1.0f) * invstd;
         const float sh = tabled ? chan[2 * j + 1] : fmaf(-mean, sc, beta ? ld(beta + c) : 0.0f);
         float o[VEC];
 #pragma unroll
         for (int e = 0; e < VEC; ++e) o[e] = Act<ACT>::f(fmaf(xv[e], sc, sh));
-        gn_store<T, VEC>(y, base + (size_t)q * VEC, o);
+        row_store<T, VEC, RAGGED>(y, base + rv.off, o, rv.skip);
     };
     if constexpr (CACHED) {
 #pragma unroll
@@ -177,7 +171,7 @@ __global__ void gn_fwd_kernel(const T* __restrict__ x, const T* __restrict__ gam
         }
     } else {
         for (uint32_t q = threadIdx.x; q < g.nvec; q += T_) {
-            gn_load<T, VEC>(x, base + (size_t)q * VEC, v[0]);
+            row_load<T, VEC, RAGGED>(x, base + row_vec(q).off, v[0]);
             emit(q, v[0]);
         }
     }
@@ -205,7 +199,7 @@ __device__ __forceinline__ void wave_channel_accumulate(float* accg, float* accb
     }
 }
 
-template <typename T, int ACT, int VEC, bool CACHED, bool AFFINE>
+template <typename T, int ACT, int VEC, bool CACHED, bool AFFINE, bool RAGGED>
 __global__ void gn_bwd_kernel(const T* __restrict__ delta, const T* __restrict__ x, const T* __restrict__ gamma,
                               const T* __restrict__ beta, const float* __restrict__ save_mean,
                               const float* __restrict__ save_invstd, T* dx, float* pdg, float* pdb, T* dgamma,
@@ -220,7 +214,9 @@ __global__ void gn_bwd_kernel(const T* __restrict__ delta, const T* __restrict__
     const uint32_t slice = blockIdx.x / parts, part = blockIdx.x - slice * parts;
     const uint32_t k = slice % g.G, n = slice / g.G;
     const uint32_t qbeg = part * g.pvec, qend = CACHED ? qbeg + g.pvec : g.nvec;   // this workgroup's vectors of the slice
-    const size_t base = (size_t)slice * g.nvec * VEC;
+    const size_t base = (size_t)slice * g.m;
+    using R = RowVec<VEC, RAGGED>;
+    auto row_vec = [&](uint32_t q) { return R(q, g.I, g.vpr, g.chdiv); };
     const float mean = save_mean[slice], invstd = save_invstd[slice];
     // the normalised value: with 16-bit storage one fused multiply-add (x carries 8 bits, so the rounding of mean * invstd
     // does not show); fp32 storage subtracts first, which keeps every bit when x is close to the mean
@@ -285,6 +281,7 @@ __global__ void gn_bwd_kernel(const T* __restrict__ delta, const T* __restrict__
     // dy and g = dy * gamma for one vector; also returns the channel's parameters
     auto grad_terms = [&](uint32_t q, const float (&dv)[VEC], const float (&xv)[VEC], float (&gv)[VEC], float& a, float& b) {
         const uint32_t j = g.chdiv.div(q), c = k * g.Cg + j;
+        const uint32_t skip = row_vec(q).skip;
         const float gm = tabled ? chan[3 * j] : (gamma ? ld(gamma + c) : 1.0f);
         const float sc = tabled ? chan[3 * j + 1] : gm * invstd;
         const float sh = tabled ? chan[3 * j + 2] : fmaf(-mean, sc, beta ? ld(beta + c) : 0.0f);
@@ -299,6 +296,7 @@ __global__ void gn_bwd_kernel(const T* __restrict__ delta, const T* __restrict__
             }
             const float xh = xhat(xv[e]);
             gv[e] = dy * gm;
+            if (RAGGED && (uint32_t)e < skip) continue;
             a = fmaf(dy, xh, a);
             b += dy;
         }
@@ -325,9 +323,9 @@ __global__ void gn_bwd_kernel(const T* __restrict__ delta, const T* __restrict__
     if constexpr (CACHED) {
 #pragma unroll
         for (int u = 0; u < kGnCache; ++u) {
-            const size_t off = base + (size_t)min(qbeg + u * T_ + threadIdx.x, qend - 1) * VEC;   // past the end: last vector again
-            kd[u] = K::load(delta, off);
-            kv[u] = K::load(x, off);
+            const size_t off = base + row_vec(min(qbeg + u * T_ + threadIdx.x, qend - 1)).off;   // past the end: last vector again
+            kd[u] = kept_load<T, VEC, RAGGED>(delta, off);
+            kv[u] = kept_load<T, VEC, RAGGED>(x, off);
         }
     }
     if constexpr (CACHED) {
@@ -343,6 +341,7 @@ __global__ void gn_bwd_kernel(const T* __restrict__ delta, const T* __restrict__
                     grad_terms(q, d[0], v[0], gv, a, b);
 #pragma unroll
                     for (int e = 0; e < VEC; ++e) {
+                        if (RAGGED && (uint32_t)e < row_vec(q).skip) continue;
                         const float xh = xhat(v[0][e]);
                         s1 += gv[e];
                         s2 = fmaf(gv[e], xh, s2);
@@ -378,11 +377,12 @@ __global__ void gn_bwd_kernel(const T* __restrict__ delta, const T* __restrict__
             const bool active = q < g.nvec;
             float gv[VEC], a = 0.0f, b = 0.0f;
             if (active) {
-                gn_load<T, VEC>(delta, base + (size_t)q * VEC, d[0]);
-                gn_load<T, VEC>(x, base + (size_t)q * VEC, v[0]);
+                row_load<T, VEC, RAGGED>(delta, base + row_vec(q).off, d[0]);
+                row_load<T, VEC, RAGGED>(x, base + row_vec(q).off, v[0]);
                 grad_terms(q, d[0], v[0], gv, a, b);
 #pragma unroll
                 for (int e = 0; e < VEC; ++e) {
+                    if (RAGGED && (uint32_t)e < row_vec(q).skip) continue;
                     const float xh = xhat(v[0][e]);
                     s1 += gv[e];
                     s2 = fmaf(gv[e], xh, s2);
@@ -407,11 +407,12 @@ __global__ void gn_bwd_kernel(const T* __restrict__ delta, const T* __restrict__
                 float t1 = 0.0f, t2 = 0.0f;
                 for (uint32_t q = i * g.pvec + threadIdx.x; q < (i + 1) * g.pvec; q += T_) {
                     float gv[VEC], a, b;
-                    gn_load<T, VEC>(delta, base + (size_t)q * VEC, d[0]);
-                    gn_load<T, VEC>(x, base + (size_t)q * VEC, v[0]);
+                    row_load<T, VEC, RAGGED>(delta, base + row_vec(q).off, d[0]);
+                    row_load<T, VEC, RAGGED>(x, base + row_vec(q).off, v[0]);
                     grad_terms(q, d[0], v[0], gv, a, b);
 #pragma unroll
                     for (int e = 0; e < VEC; ++e) {
+                        if (RAGGED && (uint32_t)e < row_vec(q).skip) continue;
                         t1 += gv[e];
                         t2 = fmaf(gv[e], xhat(v[0][e]), t2);
                     }
@@ -476,7 +477,7 @@ __global__ void gn_bwd_kernel(const T* __restrict__ delta, const T* __restrict__
             const float xh = xhat(xv[e]);
             o[e] = invstd * (gv[e] - s1 - xh * s2);
         }
-        gn_store<T, VEC>(dx, base + (size_t)q * VEC, o);
+        row_store<T, VEC, RAGGED>(dx, base + row_vec(q).off, o, row_vec(q).skip);
     };
     if constexpr (CACHED) {
 #pragma unroll
@@ -484,8 +485,8 @@ __global__ void gn_bwd_kernel(const T* __restrict__ delta, const T* __restrict__
             const uint32_t q = qbeg + u * T_ + threadIdx.x;
             if (q < qend) {
                 if (refetch) {
-                    gn_load<T, VEC>(delta, base + (size_t)q * VEC, d[0]);
-                    gn_load<T, VEC>(x, base + (size_t)q * VEC, v[0]);
+                    row_load<T, VEC, RAGGED>(delta, base + row_vec(q).off, d[0]);
+                    row_load<T, VEC, RAGGED>(x, base + row_vec(q).off, v[0]);
                     emit(q, d[0], v[0]);
                     continue;
                 }
@@ -501,7 +502,7 @@ __global__ void gn_bwd_kernel(const T* __restrict__ delta, const T* __restrict__
                         const float xh = xhat(v[0][e]);
                         o[e] = fmaf(xh, k2, fmaf(d[0][e], kg, k1));
                     }
-                    gn_store<T, VEC>(dx, base + (size_t)q * VEC, o);
+                    row_store<T, VEC, RAGGED>(dx, base + row_vec(q).off, o, row_vec(q).skip);
                 } else {
                     emit(q, d[0], v[0]);
                 }
@@ -509,8 +510,8 @@ __global__ void gn_bwd_kernel(const T* __restrict__ delta, const T* __restrict__
         }
     } else {
         for (uint32_t q = threadIdx.x; q < g.nvec; q += T_) {
-            gn_load<T, VEC>(delta, base + (size_t)q * VEC, d[0]);
-            gn_load<T, VEC>(x, base + (size_t)q * VEC, v[0]);
+            row_load<T, VEC, RAGGED>(delta, base + row_vec(q).off, d[0]);
+            row_load<T, VEC, RAGGED>(x, base + row_vec(q).off, v[0]);
             emit(q, d[0], v[0]);
         }
     }
@@ -532,7 +533,7 @@ static int gn_check(int dtype, int act, int64_t I, int64_t C, int64_t G, int64_t
 
 struct GnLaunch {
     GnGeom g;
-    bool vec, cached;
+    bool vec, ragged, cached;
     unsigned threads, blocks;
 };
 
@@ -541,11 +542,14 @@ static GnLaunch gn_plan(int64_t I, int64_t C, int64_t G, int64_t N, bool ptr_ok,
     constexpr int V = Vec<T>::N;
     GnLaunch L;
     const int64_t Cg = C / G, m = I * Cg;
-    L.vec = ptr_ok && I % V == 0;
+    L.vec = I >= V;
+    L.ragged = L.vec && !(ptr_ok && I % V == 0);
     const int vv = L.vec ? V : 1;
     L.g.I = (uint32_t)I; L.g.Cg = (uint32_t)Cg; L.g.G = (uint32_t)G; L.g.C = (uint32_t)C;
-    L.g.nvec = (uint32_t)(m / vv);
-    L.g.chdiv = FastDiv((uint32_t)(I / vv));
+    L.g.vpr = (uint32_t)ceil_div(I, vv);
+    L.g.nvec = (uint32_t)Cg * L.g.vpr;
+    L.g.m = (uint32_t)m;
+    L.g.chdiv = FastDiv(L.g.vpr);
     L.g.inv_m = 1.0f / (float)m;
     // A slice that would need a 1024-thread workgroup can be split between two 512-thread
     // workgroups (each owns whole channels): two of them fit a compute unit even with the
@@ -555,7 +559,7 @@ static GnLaunch gn_plan(int64_t I, int64_t C, int64_t G, int64_t N, bool ptr_ok,
     // pullback asks for it.
     L.g.parts = 1;
     if (allow_split && L.vec && (int64_t)L.g.nvec > 512 * kGnCache && (int64_t)L.g.nvec <= 2 * 512 * kGnCache && Cg % 2 == 0 &&
-        (L.g.nvec / 2) % (uint32_t)(I / vv) == 0 && (size_t)(G * N) * 2 * 3 * 2 <= kWorkspaceFlags)
+        (L.g.nvec / 2) % L.g.vpr == 0 && (size_t)(G * N) * 2 * 3 * 2 <= kWorkspaceFlags)
         L.g.parts = 2;
     L.g.pvec = L.g.nvec / L.g.parts;
     int64_t t = 64;
@@ -593,15 +597,19 @@ static int gn_fwd_impl(hipStream_t s, int act, int64_t I, int64_t C, int64_t G, 
         rs.N = (uint32_t)N;
     }
     ProfScope ps("gn_fwd_kernel", s, true);
+#define GN_FWD_V(A, VV, CA, RA) launch_exact(ps, gn_fwd_kernel<T, A, VV, CA, RA>, dim3(L.blocks), dim3(L.threads), 0, s, x, gamma, beta, y, save_mean, save_invstd, L.g, eps, rs)
 #define GN_FWD(A)                                                                                                     \
     do {                                                                                                              \
-        if (L.vec && L.cached) launch_exact(ps, gn_fwd_kernel<T, A, V, true>, dim3(L.blocks), dim3(L.threads), 0, s, x, gamma, beta, y, save_mean, save_invstd, L.g, eps, rs);   \
-        else if (L.vec) launch_exact(ps, gn_fwd_kernel<T, A, V, false>, dim3(L.blocks), dim3(L.threads), 0, s, x, gamma, beta, y, save_mean, save_invstd, L.g, eps, rs);        \
-        else if (L.cached) launch_exact(ps, gn_fwd_kernel<T, A, 1, true>, dim3(L.blocks), dim3(L.threads), 0, s, x, gamma, beta, y, save_mean, save_invstd, L.g, eps, rs);      \
-        else launch_exact(ps, gn_fwd_kernel<T, A, 1, false>, dim3(L.blocks), dim3(L.threads), 0, s, x, gamma, beta, y, save_mean, save_invstd, L.g, eps, rs);                   \
+        if (L.vec && L.cached && !L.ragged) GN_FWD_V(A, V, true, false);                                              \
+        else if (L.vec && L.cached) GN_FWD_V(A, V, true, true);                                                       \
+        else if (L.vec && !L.ragged) GN_FWD_V(A, V, false, false);                                                    \
+        else if (L.vec) GN_FWD_V(A, V, false, true);                                                                  \
+        else if (L.cached) GN_FWD_V(A, 1, true, false);                                                               \
+        else GN_FWD_V(A, 1, false, false);                                                                            \
     } while (0)
     LUX_DISPATCH_ACT(act, GN_FWD);
 #undef GN_FWD
+#undef GN_FWD_V
     LUX_CHECK_LAUNCH();
     return LUXHIP_OK;
 }
@@ -647,17 +655,19 @@ static int gn_bwd_impl(hipStream_t s, int act, int64_t I, int64_t C, int64_t G, 
     }
     {
         ProfScope ps("gn_bwd_kernel", s, true);
-#define GN_BWD_A(A, VV, CA)                                                                                           \
+#define GN_BWD_A(A, VV, CA, RA)                                                                                       \
     do {                                                                                                              \
-        if (affine) launch_exact(ps, gn_bwd_kernel<T, A, VV, CA, true>, dim3(L.blocks), dim3(L.threads), lds_bytes, s, delta, x, gamma, beta, save_mean, save_invstd, dx, pdg, pdb, dgamma, dbeta, counters, cstride, (uint32_t)N, L.g, ex); \
-        else launch_exact(ps, gn_bwd_kernel<T, A, VV, CA, false>, dim3(L.blocks), dim3(L.threads), lds_bytes, s, delta, x, gamma, beta, save_mean, save_invstd, dx, pdg, pdb, dgamma, dbeta, counters, cstride, (uint32_t)N, L.g, ex);       \
+        if (affine) launch_exact(ps, gn_bwd_kernel<T, A, VV, CA, true, RA>, dim3(L.blocks), dim3(L.threads), lds_bytes, s, delta, x, gamma, beta, save_mean, save_invstd, dx, pdg, pdb, dgamma, dbeta, counters, cstride, (uint32_t)N, L.g, ex); \
+        else launch_exact(ps, gn_bwd_kernel<T, A, VV, CA, false, RA>, dim3(L.blocks), dim3(L.threads), lds_bytes, s, delta, x, gamma, beta, save_mean, save_invstd, dx, pdg, pdb, dgamma, dbeta, counters, cstride, (uint32_t)N, L.g, ex);       \
     } while (0)
 #define GN_BWD(A)                                                                                                     \
     do {                                                                                                              \
-        if (L.vec && L.cached) GN_BWD_A(A, V, true);                                                                  \
-        else if (L.vec) GN_BWD_A(A, V, false);                                                                        \
-        else if (L.cached) GN_BWD_A(A, 1, true);                                                                      \
-        else GN_BWD_A(A, 1, false);                                                                                   \
+        if (L.vec && L.cached && !L.ragged) GN_BWD_A(A, V, true, false);                                              \
+        else if (L.vec && L.cached) GN_BWD_A(A, V, true, true);                                                       \
+        else if (L.vec && !L.ragged) GN_BWD_A(A, V, false, false);                                                    \
+        else if (L.vec) GN_BWD_A(A, V, false, true);                                                                  \
+        else if (L.cached) GN_BWD_A(A, 1, true, false);                                                               \
+        else GN_BWD_A(A, 1, false, false);                                                                            \
     } while (0)
         LUX_DISPATCH_ACT(act, GN_BWD);
 #undef GN_BWD

@@ -9,6 +9,8 @@
 //             reduction (threads along l, coalesced; R split into slices, partials combined
 //             in a fixed order by ln_param_finalize_kernel).
 //             ln_bwd_fused_kernel: both in one pass for columns that one wavefront holds.
+// Columns of any length are read and written in 16-byte vectors (RowVec in common.h); fp32 1023 x 6001 (24.6 MB a tensor):
+// forward 13.9 -> 10.6 us, pullback 17.4 + 11.7 + 4.0 (dx, a second read for the parameters, their sum) -> 18.8 + 5.8 us.
 #include <algorithm>
 
 #include "common.h"
@@ -17,15 +19,16 @@ namespace luxhip {
 
 constexpr int kLnCache = 8;   // vectors per thread kept in registers
 
-template <typename T, int VEC>
-__device__ __forceinline__ void ln_load(const T* p, size_t off, float (&v)[VEC]) {
-    if constexpr (VEC == 1) v[0] = ld(p + off);
-    else Vec<T>::load(p + off, v);
+// Vector q of a column of L elements (see RowVec in common.h for columns that are no multiple of a vector)
+template <int VEC, bool RAGGED>
+__device__ __forceinline__ uint32_t ln_off(uint32_t q, uint32_t L) {
+    if constexpr (RAGGED) return min(q * VEC, L - VEC);
+    else return q * VEC;
 }
-template <typename T, int VEC>
-__device__ __forceinline__ void ln_store(T* p, size_t off, const float (&v)[VEC]) {
-    if constexpr (VEC == 1) st(p + off, v[0]);
-    else Vec<T>::store(p + off, v);
+template <int VEC, bool RAGGED>
+__device__ __forceinline__ uint32_t ln_skip(uint32_t q, uint32_t L) {
+    if constexpr (RAGGED) return q * VEC + VEC > L ? q * VEC + VEC - L : 0u;
+    else return 0u;
 }
 
 // Sum over the threads that share a column: the wave (WAVE) or the workgroup.
@@ -36,55 +39,58 @@ __device__ __forceinline__ float col_sum(float v, float* sm) {
 }
 
 // ------------------------------------------------------------------------------- forward
-template <typename T, int ACT, int VEC, bool WAVE, bool CACHED>
+// CACHE: vectors per thread kept in registers; 0: the column is read from memory again
+template <typename T, int ACT, int VEC, bool WAVE, int CACHE, bool RAGGED>
 __global__ __launch_bounds__(WAVE ? 256 : 1024) void ln_fwd_kernel(const T* __restrict__ x, const T* __restrict__ gamma, const T* __restrict__ beta, T* y,
-                              float* save_mean, float* save_invstd, uint32_t nvec, uint32_t R, float inv_L, float eps) {
+                              float* save_mean, float* save_invstd, uint32_t L, uint32_t nvec, uint32_t R, float inv_L, float eps) {
+    constexpr bool CACHED = CACHE > 0;
     __shared__ float sm[16];
     const uint32_t tpc = WAVE ? 64u : blockDim.x;                       // threads per column
     const uint32_t t = WAVE ? (threadIdx.x & 63u) : threadIdx.x;
     const uint32_t r = WAVE ? blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6) : blockIdx.x;
     if (r >= R) return;                                                 // whole waves / workgroups only
-    const size_t base = (size_t)r * nvec * VEC;
+    const size_t base = (size_t)r * L;
     using K = Kept<T, VEC>;
-    typename K::type kv[CACHED ? kLnCache : 1];   // cached: the column; loads past its end re-read the last vector
+    typename K::type kv[CACHED ? CACHE : 1];   // cached: the column; loads past its end re-read the last vector
     float v[1][VEC];
+    auto counts = [&](uint32_t q, int e) { return !RAGGED || (uint32_t)e >= ln_skip<VEC, RAGGED>(q, L); };
     float sum = 0.0f;
     if constexpr (CACHED) {
 #pragma unroll
-        for (int u = 0; u < kLnCache; ++u) kv[u] = K::load(x, base + (size_t)min(u * tpc + t, nvec - 1) * VEC);
+        for (int u = 0; u < CACHE; ++u) kv[u] = kept_load<T, VEC, RAGGED>(x, base + ln_off<VEC, RAGGED>(min(u * tpc + t, nvec - 1), L));
 #pragma unroll
-        for (int u = 0; u < kLnCache; ++u) {
+        for (int u = 0; u < CACHE; ++u) {
             const uint32_t q = u * tpc + t;
             if (q < nvec) {
                 K::get(kv[u], v[0]);
 #pragma unroll
-                for (int e = 0; e < VEC; ++e) sum += v[0][e];
+                for (int e = 0; e < VEC; ++e) sum += counts(q, e) ? v[0][e] : 0.0f;
             }
         }
     } else {
         for (uint32_t q = t; q < nvec; q += tpc) {
-            ln_load<T, VEC>(x, base + (size_t)q * VEC, v[0]);
+            row_load<T, VEC, RAGGED>(x, base + ln_off<VEC, RAGGED>(q, L), v[0]);
 #pragma unroll
-            for (int e = 0; e < VEC; ++e) sum += v[0][e];
+            for (int e = 0; e < VEC; ++e) sum += counts(q, e) ? v[0][e] : 0.0f;
         }
     }
     const float mean = col_sum<WAVE>(sum, sm) * inv_L;
     float dev = 0.0f;
     if constexpr (CACHED) {
 #pragma unroll
-        for (int u = 0; u < kLnCache; ++u) {
+        for (int u = 0; u < CACHE; ++u) {
             const uint32_t q = u * tpc + t;
             if (q < nvec) {
                 K::get(kv[u], v[0]);
 #pragma unroll
-                for (int e = 0; e < VEC; ++e) dev = fmaf(v[0][e] - mean, v[0][e] - mean, dev);
+                for (int e = 0; e < VEC; ++e) dev = counts(q, e) ? fmaf(v[0][e] - mean, v[0][e] - mean, dev) : dev;
             }
         }
     } else {
         for (uint32_t q = t; q < nvec; q += tpc) {
-            ln_load<T, VEC>(x, base + (size_t)q * VEC, v[0]);
+            row_load<T, VEC, RAGGED>(x, base + ln_off<VEC, RAGGED>(q, L), v[0]);
 #pragma unroll
-            for (int e = 0; e < VEC; ++e) dev = fmaf(v[0][e] - mean, v[0][e] - mean, dev);
+            for (int e = 0; e < VEC; ++e) dev = counts(q, e) ? fmaf(v[0][e] - mean, v[0][e] - mean, dev) : dev;
         }
     }
     const float var = col_sum<WAVE>(dev, sm) * inv_L;
@@ -96,8 +102,8 @@ __global__ __launch_bounds__(WAVE ? 256 : 1024) void ln_fwd_kernel(const T* __re
     auto emit = [&](uint32_t q, const float (&xv)[VEC]) {
         float gm[VEC], bt[VEC], o[VEC];
         if (gamma) {
-            ln_load<T, VEC>(gamma, (size_t)q * VEC, gm);
-            ln_load<T, VEC>(beta, (size_t)q * VEC, bt);
+            row_load<T, VEC, RAGGED>(gamma, ln_off<VEC, RAGGED>(q, L), gm);
+            row_load<T, VEC, RAGGED>(beta, ln_off<VEC, RAGGED>(q, L), bt);
         }
 #pragma unroll
         for (int e = 0; e < VEC; ++e) {
@@ -105,11 +111,11 @@ __global__ __launch_bounds__(WAVE ? 256 : 1024) void ln_fwd_kernel(const T* __re
             const float sh = fmaf(-mean, sc, gamma ? bt[e] : 0.0f);
             o[e] = Act<ACT>::f(fmaf(xv[e], sc, sh));
         }
-        ln_store<T, VEC>(y, base + (size_t)q * VEC, o);
+        row_store<T, VEC, RAGGED>(y, base + ln_off<VEC, RAGGED>(q, L), o, ln_skip<VEC, RAGGED>(q, L));
     };
     if constexpr (CACHED) {
 #pragma unroll
-        for (int u = 0; u < kLnCache; ++u) {
+        for (int u = 0; u < CACHE; ++u) {
             const uint32_t q = u * tpc + t;
             if (q < nvec) {
                 K::get(kv[u], v[0]);
@@ -118,7 +124,7 @@ __global__ __launch_bounds__(WAVE ? 256 : 1024) void ln_fwd_kernel(const T* __re
         }
     } else {
         for (uint32_t q = t; q < nvec; q += tpc) {
-            ln_load<T, VEC>(x, base + (size_t)q * VEC, v[0]);
+            row_load<T, VEC, RAGGED>(x, base + ln_off<VEC, RAGGED>(q, L), v[0]);
             emit(q, v[0]);
         }
     }
@@ -126,14 +132,14 @@ __global__ __launch_bounds__(WAVE ? 256 : 1024) void ln_fwd_kernel(const T* __re
 
 // ------------------------------------------------------------------------------- pullback: dx
 // dy for one vector, given the column statistics and the affine parameters at its positions.
-template <typename T, int ACT, int VEC>
-__device__ __forceinline__ void ln_dy(const T* gamma, const T* beta, uint32_t q, float mean, float invstd,
+template <typename T, int ACT, int VEC, bool RAGGED>
+__device__ __forceinline__ void ln_dy(const T* gamma, const T* beta, uint32_t off, float mean, float invstd,
                                       const float (&dv)[VEC], const float (&xv)[VEC], float (&dy)[VEC],
                                       float (&gm)[VEC]) {
     float bt[VEC];
     if (gamma) {
-        ln_load<T, VEC>(gamma, (size_t)q * VEC, gm);
-        if constexpr (ACT != LUXHIP_ACT_IDENTITY) ln_load<T, VEC>(beta, (size_t)q * VEC, bt);
+        row_load<T, VEC, RAGGED>(gamma, off, gm);
+        if constexpr (ACT != LUXHIP_ACT_IDENTITY) row_load<T, VEC, RAGGED>(beta, off, bt);
     } else {
 #pragma unroll
         for (int e = 0; e < VEC; ++e) { gm[e] = 1.0f; bt[e] = 0.0f; }
@@ -164,26 +170,28 @@ __device__ __forceinline__ void ln_dy_regs(const float (&gm)[VEC], const float (
     }
 }
 
-template <typename T, int ACT, int VEC, bool WAVE, bool CACHED>
+template <typename T, int ACT, int VEC, bool WAVE, int CACHE, bool RAGGED>
 __global__ __launch_bounds__(WAVE ? 256 : 1024) void ln_bwd_dx_kernel(const T* __restrict__ delta, const T* __restrict__ x, const T* __restrict__ gamma,
                                  const T* __restrict__ beta, const float* __restrict__ save_mean,
-                                 const float* __restrict__ save_invstd, T* dx, uint32_t nvec, uint32_t R, float inv_L) {
+                                 const float* __restrict__ save_invstd, T* dx, uint32_t L, uint32_t nvec, uint32_t R, float inv_L) {
+    constexpr bool CACHED = CACHE > 0;
     __shared__ float sm[16];
     const uint32_t tpc = WAVE ? 64u : blockDim.x;
     const uint32_t t = WAVE ? (threadIdx.x & 63u) : threadIdx.x;
     const uint32_t r = WAVE ? blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6) : blockIdx.x;
     if (r >= R) return;
-    const size_t base = (size_t)r * nvec * VEC;
+    const size_t base = (size_t)r * L;
     const float mean = save_mean[r], invstd = save_invstd[r];
     using K = Kept<T, VEC>;
-    typename K::type kd[CACHED ? kLnCache : 1], kv[CACHED ? kLnCache : 1];
+    typename K::type kd[CACHED ? CACHE : 1], kv[CACHED ? CACHE : 1];
     float d[1][VEC], v[1][VEC];
     float s1 = 0.0f, s2 = 0.0f;
     auto accumulate = [&](uint32_t q, const float (&dv)[VEC], const float (&xv)[VEC]) {
         float dy[VEC], gm[VEC];
-        ln_dy<T, ACT, VEC>(gamma, beta, q, mean, invstd, dv, xv, dy, gm);
+        ln_dy<T, ACT, VEC, RAGGED>(gamma, beta, ln_off<VEC, RAGGED>(q, L), mean, invstd, dv, xv, dy, gm);
 #pragma unroll
         for (int e = 0; e < VEC; ++e) {
+            if (RAGGED && (uint32_t)e < ln_skip<VEC, RAGGED>(q, L)) continue;
             const float g = gm[e] * dy[e];
             s1 += g;
             s2 = fmaf(g, (xv[e] - mean) * invstd, s2);
@@ -191,13 +199,13 @@ __global__ __launch_bounds__(WAVE ? 256 : 1024) void ln_bwd_dx_kernel(const T* _
     };
     if constexpr (CACHED) {
 #pragma unroll
-        for (int u = 0; u < kLnCache; ++u) {
-            const size_t off = base + (size_t)min(u * tpc + t, nvec - 1) * VEC;   // past the end: re-read the last vector
-            kd[u] = K::load(delta, off);
-            kv[u] = K::load(x, off);
+        for (int u = 0; u < CACHE; ++u) {
+            const size_t off = base + ln_off<VEC, RAGGED>(min(u * tpc + t, nvec - 1), L);   // past the end: re-read the last vector
+            kd[u] = kept_load<T, VEC, RAGGED>(delta, off);
+            kv[u] = kept_load<T, VEC, RAGGED>(x, off);
         }
 #pragma unroll
-        for (int u = 0; u < kLnCache; ++u) {
+        for (int u = 0; u < CACHE; ++u) {
             const uint32_t q = u * tpc + t;
             if (q < nvec) {
                 K::get(kd[u], d[0]);
@@ -207,8 +215,8 @@ __global__ __launch_bounds__(WAVE ? 256 : 1024) void ln_bwd_dx_kernel(const T* _
         }
     } else {
         for (uint32_t q = t; q < nvec; q += tpc) {
-            ln_load<T, VEC>(delta, base + (size_t)q * VEC, d[0]);
-            ln_load<T, VEC>(x, base + (size_t)q * VEC, v[0]);
+            row_load<T, VEC, RAGGED>(delta, base + ln_off<VEC, RAGGED>(q, L), d[0]);
+            row_load<T, VEC, RAGGED>(x, base + ln_off<VEC, RAGGED>(q, L), v[0]);
             accumulate(q, d[0], v[0]);
         }
     }
@@ -216,17 +224,17 @@ __global__ __launch_bounds__(WAVE ? 256 : 1024) void ln_bwd_dx_kernel(const T* _
     s2 = col_sum<WAVE>(s2, sm) * inv_L;
     auto emit = [&](uint32_t q, const float (&dv)[VEC], const float (&xv)[VEC]) {
         float dy[VEC], gm[VEC], o[VEC];
-        ln_dy<T, ACT, VEC>(gamma, beta, q, mean, invstd, dv, xv, dy, gm);
+        ln_dy<T, ACT, VEC, RAGGED>(gamma, beta, ln_off<VEC, RAGGED>(q, L), mean, invstd, dv, xv, dy, gm);
 #pragma unroll
         for (int e = 0; e < VEC; ++e) {
             const float xh = (xv[e] - mean) * invstd;
             o[e] = invstd * (gm[e] * dy[e] - s1 - xh * s2);
         }
-        ln_store<T, VEC>(dx, base + (size_t)q * VEC, o);
+        row_store<T, VEC, RAGGED>(dx, base + ln_off<VEC, RAGGED>(q, L), o, ln_skip<VEC, RAGGED>(q, L));
     };
     if constexpr (CACHED) {
 #pragma unroll
-        for (int u = 0; u < kLnCache; ++u) {
+        for (int u = 0; u < CACHE; ++u) {
             const uint32_t q = u * tpc + t;
             if (q < nvec) {
                 K::get(kd[u], d[0]);
@@ -236,8 +244,8 @@ __global__ __launch_bounds__(WAVE ? 256 : 1024) void ln_bwd_dx_kernel(const T* _
         }
     } else {
         for (uint32_t q = t; q < nvec; q += tpc) {
-            ln_load<T, VEC>(delta, base + (size_t)q * VEC, d[0]);
-            ln_load<T, VEC>(x, base + (size_t)q * VEC, v[0]);
+            row_load<T, VEC, RAGGED>(delta, base + ln_off<VEC, RAGGED>(q, L), d[0]);
+            row_load<T, VEC, RAGGED>(x, base + ln_off<VEC, RAGGED>(q, L), v[0]);
             emit(q, d[0], v[0]);
         }
     }
@@ -252,34 +260,34 @@ __global__ __launch_bounds__(WAVE ? 256 : 1024) void ln_bwd_dx_kernel(const T* _
 // in pair order through LDS; row `blockIdx.x` of pg / pb receives the result and
 // ln_param_finalize_kernel adds the rows in order.  delta and x are read once.
 constexpr int kLnFusedCache = kLnCache / 2;
-template <typename T, int ACT, int VEC>
+template <typename T, int ACT, int VEC, int CACHE, bool RAGGED>
 __global__ __launch_bounds__(256) void ln_bwd_fused_kernel(const T* __restrict__ delta, const T* __restrict__ x,
                                                            const T* __restrict__ gamma, const T* __restrict__ beta,
                                                            const float* __restrict__ save_mean,
                                                            const float* __restrict__ save_invstd, T* dx, float* pg, float* pb,
-                                                           uint32_t nvec, uint32_t R, float inv_L) {
+                                                           uint32_t L, uint32_t nvec, uint32_t R, float inv_L) {
     __shared__ float red[2][2][128 * VEC];
     __shared__ float colsum[2][2][2];                  // [pair][wave of the pair][s1, s2]
     const uint32_t w = threadIdx.x >> 6, pair = w >> 1, half = w & 1u;
     const uint32_t t = half * 64u + (threadIdx.x & 63u);          // 0..127 inside the pair
     const uint32_t pairs = gridDim.x * 2u;
     using K = Kept<T, VEC>;
-    float ag[kLnFusedCache][VEC], ab[kLnFusedCache][VEC];
+    float ag[CACHE][VEC], ab[CACHE][VEC];
 #pragma unroll
-    for (int u = 0; u < kLnFusedCache; ++u)
+    for (int u = 0; u < CACHE; ++u)
 #pragma unroll
         for (int e = 0; e < VEC; ++e) { ag[u][e] = 0.0f; ab[u][e] = 0.0f; }
     // The affine parameters at this thread's positions are the same for every column: read once and kept as they lie
     // in memory.  (Read inside the second pass they would sit between the dx stores, and a wave's memory operations
     // complete in the order of their issue: every such load would wait for the store before it.)
-    typename K::type kgm[kLnFusedCache], kbt[kLnFusedCache];
+    typename K::type kgm[CACHE], kbt[CACHE];
     const bool affine = gamma != nullptr;
     if (affine) {
 #pragma unroll
-        for (int u = 0; u < kLnFusedCache; ++u) {
-            const size_t off = (size_t)min(u * 128u + t, nvec - 1) * VEC;
-            kgm[u] = K::load(gamma, off);
-            if constexpr (ACT != LUXHIP_ACT_IDENTITY) kbt[u] = K::load(beta, off);
+        for (int u = 0; u < CACHE; ++u) {
+            const size_t off = ln_off<VEC, RAGGED>(min(u * 128u + t, nvec - 1), L);
+            kgm[u] = kept_load<T, VEC, RAGGED>(gamma, off);
+            if constexpr (ACT != LUXHIP_ACT_IDENTITY) kbt[u] = kept_load<T, VEC, RAGGED>(beta, off);
         }
     }
     auto params = [&](int u, float (&gm)[VEC], float (&bt)[VEC]) {
@@ -296,18 +304,18 @@ __global__ __launch_bounds__(256) void ln_bwd_fused_kernel(const T* __restrict__
         const uint32_t r = it * pairs + blockIdx.x * 2u + pair;
         const bool live = r < R;                                  // uniform per wavefront
         const uint32_t rc = live ? r : R - 1;
-        const size_t base = (size_t)rc * nvec * VEC;
+        const size_t base = (size_t)rc * L;
         const float mean = save_mean[rc], invstd = save_invstd[rc];
-        typename K::type kd[kLnFusedCache], kv[kLnFusedCache];
+        typename K::type kd[CACHE], kv[CACHE];
 #pragma unroll
-        for (int u = 0; u < kLnFusedCache; ++u) {
-            const size_t off = base + (size_t)min(u * 128u + t, nvec - 1) * VEC;   // past the end: the last vector again
-            kd[u] = K::load(delta, off);
-            kv[u] = K::load(x, off);
+        for (int u = 0; u < CACHE; ++u) {
+            const size_t off = base + ln_off<VEC, RAGGED>(min(u * 128u + t, nvec - 1), L);   // past the end: the last vector again
+            kd[u] = kept_load<T, VEC, RAGGED>(delta, off);
+            kv[u] = kept_load<T, VEC, RAGGED>(x, off);
         }
         float s1 = 0.0f, s2 = 0.0f;
 #pragma unroll
-        for (int u = 0; u < kLnFusedCache; ++u) {
+        for (int u = 0; u < CACHE; ++u) {
             const uint32_t q = u * 128u + t;
             if (q < nvec && live) {
                 float d[VEC], v[VEC], dy[VEC], gm[VEC], bt[VEC];
@@ -317,6 +325,7 @@ __global__ __launch_bounds__(256) void ln_bwd_fused_kernel(const T* __restrict__
                 ln_dy_regs<ACT, VEC>(gm, bt, mean, invstd, d, v, dy);
 #pragma unroll
                 for (int e = 0; e < VEC; ++e) {
+                    if (RAGGED && (uint32_t)e < ln_skip<VEC, RAGGED>(q, L)) continue;
                     const float xh = (v[e] - mean) * invstd;
                     const float g = gm[e] * dy[e];
                     s1 += g;
@@ -334,7 +343,7 @@ __global__ __launch_bounds__(256) void ln_bwd_fused_kernel(const T* __restrict__
         s2 = (colsum[pair][0][1] + colsum[pair][1][1]) * inv_L;
         __syncthreads();                                          // colsum is rewritten in the next round
 #pragma unroll
-        for (int u = 0; u < kLnFusedCache; ++u) {
+        for (int u = 0; u < CACHE; ++u) {
             const uint32_t q = u * 128u + t;
             if (q < nvec && live) {
                 float d[VEC], v[VEC], dy[VEC], gm[VEC], bt[VEC], o[VEC];
@@ -347,14 +356,14 @@ __global__ __launch_bounds__(256) void ln_bwd_fused_kernel(const T* __restrict__
                     const float xh = (v[e] - mean) * invstd;
                     o[e] = invstd * (gm[e] * dy[e] - s1 - xh * s2);
                 }
-                ln_store<T, VEC>(dx, base + (size_t)q * VEC, o);
+                row_store<T, VEC, RAGGED>(dx, base + ln_off<VEC, RAGGED>(q, L), o, ln_skip<VEC, RAGGED>(q, L));
             }
         }
     }
     // sums of the two pairs, in pair order, one cached vector at a time
-    const size_t row = (size_t)blockIdx.x * nvec * VEC;
+    const size_t row = (size_t)blockIdx.x * L;
 #pragma unroll
-    for (int u = 0; u < kLnFusedCache; ++u) {
+    for (int u = 0; u < CACHE; ++u) {
 #pragma unroll
         for (int e = 0; e < VEC; ++e) {
             red[0][pair][t * VEC + e] = ag[u][e];
@@ -362,8 +371,9 @@ __global__ __launch_bounds__(256) void ln_bwd_fused_kernel(const T* __restrict__
         }
         __syncthreads();
         for (uint32_t i = threadIdx.x; i < 128u * VEC; i += 256u) {
-            const uint32_t l = u * 128u * VEC + i;
-            if (l < nvec * VEC) {
+            const uint32_t q = u * 128u + i / VEC, e = i % VEC;
+            const uint32_t l = ln_off<VEC, RAGGED>(q, L) + e;
+            if (q < nvec && e >= ln_skip<VEC, RAGGED>(q, L)) {
                 pg[row + l] = red[0][0][i] + red[0][1][i];
                 pb[row + l] = red[1][0][i] + red[1][1][i];
             }
@@ -375,31 +385,32 @@ __global__ __launch_bounds__(256) void ln_bwd_fused_kernel(const T* __restrict__
 // ------------------------------------------------------------------------------- pullback: dgamma, dbeta
 // grid (ceil(nvec / 64), S): a thread owns one vector of positions l and walks over the
 // columns of slice s; partial sums go to pg/pb[s][l].
-template <typename T, int ACT, int VEC>
+template <typename T, int ACT, int VEC, bool RAGGED>
 __global__ __launch_bounds__(64) void ln_param_grad_kernel(const T* __restrict__ delta, const T* __restrict__ x,
                                                            const T* __restrict__ gamma, const T* __restrict__ beta,
                                                            const float* __restrict__ save_mean,
                                                            const float* __restrict__ save_invstd, float* pg, float* pb,
-                                                           uint32_t nvec, uint32_t R, uint32_t cols_per_slice) {
+                                                           uint32_t L, uint32_t nvec, uint32_t R, uint32_t cols_per_slice) {
     const uint32_t q = blockIdx.x * 64 + threadIdx.x;
     if (q >= nvec) return;
+    const uint32_t l0 = ln_off<VEC, RAGGED>(q, L);
     const uint32_t r0 = blockIdx.y * cols_per_slice, r1 = min(r0 + cols_per_slice, R);
     float gm[VEC], bt[VEC], ag[VEC], ab[VEC];
     if (gamma) {
-        ln_load<T, VEC>(gamma, (size_t)q * VEC, gm);
-        ln_load<T, VEC>(beta, (size_t)q * VEC, bt);
+        row_load<T, VEC, RAGGED>(gamma, l0, gm);
+        row_load<T, VEC, RAGGED>(beta, l0, bt);
     }
 #pragma unroll
     for (int e = 0; e < VEC; ++e) {
         ag[e] = 0.0f; ab[e] = 0.0f;
         if (!gamma) { gm[e] = 1.0f; bt[e] = 0.0f; }
     }
-    const size_t stride = (size_t)nvec * VEC;
+    const size_t stride = L;
 #pragma unroll 4
     for (uint32_t r = r0; r < r1; ++r) {
         float dv[VEC], xv[VEC];
-        ln_load<T, VEC>(delta, r * stride + (size_t)q * VEC, dv);
-        ln_load<T, VEC>(x, r * stride + (size_t)q * VEC, xv);
+        row_load<T, VEC, RAGGED>(delta, r * stride + l0, dv);
+        row_load<T, VEC, RAGGED>(x, r * stride + l0, xv);
         const float mean = save_mean[r], invstd = save_invstd[r];
 #pragma unroll
         for (int e = 0; e < VEC; ++e) {
@@ -413,9 +424,10 @@ __global__ __launch_bounds__(64) void ln_param_grad_kernel(const T* __restrict__
             ab[e] += dy;
         }
     }
-    const size_t o = (size_t)blockIdx.y * stride + (size_t)q * VEC;
+    const size_t o = (size_t)blockIdx.y * stride + l0;
 #pragma unroll
-    for (int e = 0; e < VEC; ++e) { pg[o + e] = ag[e]; pb[o + e] = ab[e]; }
+    for (int e = 0; e < VEC; ++e)
+        if (!RAGGED || (uint32_t)e >= ln_skip<VEC, RAGGED>(q, L)) { pg[o + e] = ag[e]; pb[o + e] = ab[e]; }
 }
 
 // dgamma[l] = sum_s pg[s][l], dbeta likewise.  Workgroup of LW positions x (1024 / LW) slice groups:
@@ -459,7 +471,7 @@ __global__ __launch_bounds__(1024) void ln_param_finalize_kernel(const float* __
 
 // ------------------------------------------------------------------------------- host side
 struct LnPlan {
-    bool vec, wave, cached;
+    bool vec, ragged, wave, cached;
     uint32_t nvec;
     unsigned threads, blocks;
 };
@@ -468,8 +480,9 @@ template <typename T>
 static LnPlan ln_plan(int64_t L, int64_t R, bool ptr_ok) {
     constexpr int V = Vec<T>::N;
     LnPlan p;
-    p.vec = ptr_ok && L % V == 0;
-    p.nvec = (uint32_t)(L / (p.vec ? V : 1));
+    p.vec = L >= V;
+    p.ragged = p.vec && !(ptr_ok && L % V == 0);
+    p.nvec = (uint32_t)ceil_div(L, p.vec ? V : 1);
     p.wave = p.nvec <= 64u * kLnCache;
     if (p.wave) {
         p.cached = true;
@@ -496,14 +509,21 @@ static int ln_check(int dtype, int act, int64_t L, int64_t R) {
     return LUXHIP_OK;
 }
 
+// Columns that a wave holds take the variant with as many registers as the column needs (a wave of 256 vectors that is built
+// for 512 loads its last vector four times over)
+#define LN_ONE(KERNEL, A, VV, WV, CA, RA, ...) launch_exact(ps, KERNEL<T, A, VV, WV, CA, RA>, dim3(p.blocks), dim3(p.threads), 0, s, __VA_ARGS__)
+#define LN_RAGGED(KERNEL, A, WV, CA, ...)                                                               \
+    do {                                                                                                \
+        if (p.ragged) LN_ONE(KERNEL, A, V, WV, CA, true, __VA_ARGS__);                                  \
+        else LN_ONE(KERNEL, A, V, WV, CA, false, __VA_ARGS__);                                          \
+    } while (0)
 #define LN_VARIANTS(KERNEL, A, ...)                                                                     \
     do {                                                                                                \
-        if (p.vec && p.wave) launch_exact(ps, KERNEL<T, A, V, true, true>, dim3(p.blocks), dim3(p.threads), 0, s, __VA_ARGS__);   \
-        else if (p.vec && p.cached) launch_exact(ps, KERNEL<T, A, V, false, true>, dim3(p.blocks), dim3(p.threads), 0, s, __VA_ARGS__);  \
-        else if (p.vec) launch_exact(ps, KERNEL<T, A, V, false, false>, dim3(p.blocks), dim3(p.threads), 0, s, __VA_ARGS__);      \
-        else if (p.wave) launch_exact(ps, KERNEL<T, A, 1, true, true>, dim3(p.blocks), dim3(p.threads), 0, s, __VA_ARGS__);       \
-        else if (p.cached) launch_exact(ps, KERNEL<T, A, 1, false, true>, dim3(p.blocks), dim3(p.threads), 0, s, __VA_ARGS__);    \
-        else launch_exact(ps, KERNEL<T, A, 1, false, false>, dim3(p.blocks), dim3(p.threads), 0, s, __VA_ARGS__);                 \
+        if (p.vec && p.wave && p.nvec <= 64u * 4) LN_RAGGED(KERNEL, A, true, 4, __VA_ARGS__);           \
+        else if (p.vec && p.wave) LN_RAGGED(KERNEL, A, true, kLnCache, __VA_ARGS__);                    \
+        else if (p.vec && p.cached) LN_RAGGED(KERNEL, A, false, kLnCache, __VA_ARGS__);                 \
+        else if (p.vec) LN_RAGGED(KERNEL, A, false, 0, __VA_ARGS__);                                    \
+        else LN_ONE(KERNEL, A, 1, true, kLnCache, false, __VA_ARGS__);       /* fewer elements than a vector */ \
     } while (0)
 
 template <typename T>
@@ -514,7 +534,7 @@ static int ln_fwd_impl(hipStream_t s, int act, int64_t L, int64_t R, const T* x,
     LnPlan p = ln_plan<T>(L, R, ptr_ok);
     const float inv_L = 1.0f / (float)L;
     ProfScope ps("ln_fwd_kernel", s, true);
-#define LN_FWD(A) LN_VARIANTS(ln_fwd_kernel, A, x, gamma, beta, y, save_mean, save_invstd, p.nvec, (uint32_t)R, inv_L, eps)
+#define LN_FWD(A) LN_VARIANTS(ln_fwd_kernel, A, x, gamma, beta, y, save_mean, save_invstd, (uint32_t)L, p.nvec, (uint32_t)R, inv_L, eps)
     LUX_DISPATCH_ACT(act, LN_FWD);
 #undef LN_FWD
     LUX_CHECK_LAUNCH();
@@ -539,9 +559,17 @@ static int ln_bwd_impl(hipStream_t s, int act, int64_t L, int64_t R, const T* de
         float* pb = pg + (size_t)blocks * L;
         {
             ProfScope ps("ln_bwd_fused_kernel", s, true);
-#define LN_FUSED(A) launch_exact(ps, ln_bwd_fused_kernel<T, A, V>, dim3((unsigned)blocks), dim3(256), 0, s, delta, x, gamma, beta, save_mean, save_invstd, dx, pg, pb, p.nvec, (uint32_t)R, inv_L)
+#define LN_FUSED_V(A, CA, RA) launch_exact(ps, ln_bwd_fused_kernel<T, A, V, CA, RA>, dim3((unsigned)blocks), dim3(256), 0, s, delta, x, gamma, beta, save_mean, save_invstd, dx, pg, pb, (uint32_t)L, p.nvec, (uint32_t)R, inv_L)
+#define LN_FUSED(A)                                                                       \
+    do {                                                                                  \
+        if (p.nvec <= 128u * 2 && p.ragged) LN_FUSED_V(A, 2, true);                       \
+        else if (p.nvec <= 128u * 2) LN_FUSED_V(A, 2, false);                             \
+        else if (p.ragged) LN_FUSED_V(A, kLnFusedCache, true);                            \
+        else LN_FUSED_V(A, kLnFusedCache, false);                                         \
+    } while (0)
             LUX_DISPATCH_ACT(act, LN_FUSED);
 #undef LN_FUSED
+#undef LN_FUSED_V
         }
         LUX_CHECK_LAUNCH();
         ProfScope ps2("ln_param_finalize_kernel", s);
@@ -551,7 +579,7 @@ static int ln_bwd_impl(hipStream_t s, int act, int64_t L, int64_t R, const T* de
     }
     {
         ProfScope ps("ln_bwd_dx_kernel", s, true);
-#define LN_BWD(A) LN_VARIANTS(ln_bwd_dx_kernel, A, delta, x, gamma, beta, save_mean, save_invstd, dx, p.nvec, (uint32_t)R, inv_L)
+#define LN_BWD(A) LN_VARIANTS(ln_bwd_dx_kernel, A, delta, x, gamma, beta, save_mean, save_invstd, dx, (uint32_t)L, p.nvec, (uint32_t)R, inv_L)
         LUX_DISPATCH_ACT(act, LN_BWD);
 #undef LN_BWD
     }
@@ -572,8 +600,9 @@ static int ln_bwd_impl(hipStream_t s, int act, int64_t L, int64_t R, const T* de
             ProfScope ps("ln_param_grad_kernel", s);
 #define LN_PG(A)                                                                                                           \
     do {                                                                                                                   \
-        if (p.vec) ln_param_grad_kernel<T, A, V><<<grid, 64, 0, s>>>(delta, x, gamma, beta, save_mean, save_invstd, pg, pb, p.nvec, (uint32_t)R, cols); \
-        else ln_param_grad_kernel<T, A, 1><<<grid, 64, 0, s>>>(delta, x, gamma, beta, save_mean, save_invstd, pg, pb, p.nvec, (uint32_t)R, cols);       \
+        if (p.ragged) ln_param_grad_kernel<T, A, V, true><<<grid, 64, 0, s>>>(delta, x, gamma, beta, save_mean, save_invstd, pg, pb, (uint32_t)L, p.nvec, (uint32_t)R, cols); \
+        else if (p.vec) ln_param_grad_kernel<T, A, V, false><<<grid, 64, 0, s>>>(delta, x, gamma, beta, save_mean, save_invstd, pg, pb, (uint32_t)L, p.nvec, (uint32_t)R, cols); \
+        else ln_param_grad_kernel<T, A, 1, false><<<grid, 64, 0, s>>>(delta, x, gamma, beta, save_mean, save_invstd, pg, pb, (uint32_t)L, p.nvec, (uint32_t)R, cols);       \
     } while (0)
             LUX_DISPATCH_ACT(act, LN_PG);
 #undef LN_PG
