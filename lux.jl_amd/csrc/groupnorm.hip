@@ -205,6 +205,7 @@ __global__ void gn_bwd_kernel(const T* __restrict__ delta, const T* __restrict__
                               const float* __restrict__ save_invstd, T* dx, float* pdg, float* pdb, T* dgamma,
                               T* dbeta, uint32_t* counters, uint32_t cstride, uint32_t N, GnGeom g, GnExchange ex) {
     extern __shared__ float lds[];                  // [16] reduction scratch, then [nw][Cg] x 2
+    __shared__ float rowsum[2][AFFINE ? 1024 : 1];
     float* sm = lds;
     const uint32_t T_ = blockDim.x, nw = T_ >> 6, w = threadIdx.x >> 6;
     float* accg = lds + 16 + (size_t)w * g.Cg;
@@ -454,14 +455,32 @@ __global__ void gn_bwd_kernel(const T* __restrict__ delta, const T* __restrict__
         // partials of the group's channels in sample order
         uint32_t* last_flag = reinterpret_cast<uint32_t*>(lds + 15);   // a word of the reduction scratch that is free now
         if (arrive_last(counters + (size_t)k * cstride, N * parts, last_flag)) {
-            for (uint32_t j = threadIdx.x; j < g.Cg; j += T_) {
+            // the threads form rows of Cg: row r adds samples r, r + rows, ..., then one row adds the rows' sums in order.
+            // (One row alone would make N round trips to memory, one after the other, at the end of the kernel: 35 x 35 x 96 x 24
+            // fp32 22.3 against 16.5 us, 64 x 64 x 256 x 16 bf16 46.2 against 43.3 for forward and pullback.)
+            const uint32_t rows = g.Cg < T_ ? min(T_ / g.Cg, N) : 1u;
+            for (uint32_t j0 = 0; j0 < g.Cg; j0 += T_) {
+                const uint32_t r = threadIdx.x / min(g.Cg, T_), j = j0 + threadIdx.x - r * min(g.Cg, T_);
                 float tg = 0.0f, tb = 0.0f;
-                for (uint32_t nn = 0; nn < N; ++nn) {
-                    tg += fetch(pdg + (size_t)nn * g.C + k * g.Cg + j);
-                    tb += fetch(pdb + (size_t)nn * g.C + k * g.Cg + j);
+                if (r < rows && j < g.Cg) {
+#pragma unroll 4
+                    for (uint32_t nn = r; nn < N; nn += rows) {
+                        tg += fetch(pdg + (size_t)nn * g.C + k * g.Cg + j);
+                        tb += fetch(pdb + (size_t)nn * g.C + k * g.Cg + j);
+                    }
                 }
-                if (dgamma) st(dgamma + k * g.Cg + j, tg);
-                if (dbeta) st(dbeta + k * g.Cg + j, tb);
+                rowsum[0][threadIdx.x] = tg;
+                rowsum[1][threadIdx.x] = tb;
+                __syncthreads();
+                if (r == 0 && j < g.Cg) {
+                    for (uint32_t q = 1; q < rows; ++q) {
+                        tg += rowsum[0][threadIdx.x + q * g.Cg];
+                        tb += rowsum[1][threadIdx.x + q * g.Cg];
+                    }
+                    if (dgamma) st(dgamma + k * g.Cg + j, tg);
+                    if (dbeta) st(dbeta + k * g.Cg + j, tb);
+                }
+                __syncthreads();
             }
         }
     }
