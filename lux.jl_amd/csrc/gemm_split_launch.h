@@ -124,12 +124,16 @@ bool launch_split_pair(hipStream_t s, DenseArgs<T>& a, DenseArgs<T>& b, int* rc)
     Plan pa = make_plan<T, 1>(a, ca.slices, &front), pb = make_plan<T, 1>(b, cb.slices, &front);
     const int64_t na = (int64_t)a.tiles_m * a.tiles_n * pa.slices, nb = (int64_t)b.tiles_m * b.tiles_n * pb.slices;
     if (na > 2 * cus && nb > 2 * cus) return false;               // each fills the chip by itself
+    // one counter for each tile of a product with slices, those of b behind those of a
+    const int64_t counters_a = pa.slices > 1 ? (int64_t)a.tiles_m * a.tiles_n : 0;
+    const int64_t counters_b = pb.slices > 1 ? (int64_t)b.tiles_m * b.tiles_n : 0;
+    if (counters_a + counters_b > (int64_t)kWorkspaceCounters || na + nb >= (int64_t(1) << 31)) return false;
     if (front > 0) {
         Workspace ws;
         *rc = get_workspace(s, front, &ws);
         if (*rc != LUXHIP_OK) return true;
         place(pa, ws, 0);
-        place(pb, ws, a.tiles_m * a.tiles_n);
+        place(pb, ws, (int)counters_a);
     }
     ProfScope ps(sizeof(T) == 2 ? "split_gemm_pair_kernel<bf16>" : "split_gemm_pair_kernel<f32>", s);
     constexpr size_t lds = std::max(Body<T, 1, false, false>::LDS_BYTES, Body<T, 1, true, true>::LDS_BYTES);

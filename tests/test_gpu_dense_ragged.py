@@ -68,6 +68,21 @@ def test_fused_layer_with_gradients_in_one_launch(gpu, dtype, act):
         assert_close(gb.to_numpy(), wdb, dtype, tag + " db")
 
 
+def test_gradients_of_a_layer_with_more_tiles_than_counters(gpu):
+    """dW has 70000 tiles and one slice, dx one tile and sixteen slices: only dx takes arrival counters.  All values are
+    -1, 0 or 1 and every sum stays below M < 2^24, so fp32 holds each partial sum exactly, whatever the order (rounded
+    inputs would need a bound for sums of 4.5 million terms)."""
+    M, K, N = 70000 * 64, 8, 16
+    rng = np.random.default_rng(stable_seed("tall"))
+    W, x, delta = (rng.integers(-1, 2, size=s).astype(np.float32) for s in ((M, K), (K, N), (M, N)))
+    args = tuple(dev(gpu, a, "f32") for a in (W, x, np.zeros(M, np.float32)))
+    _, back = gpu.pullback(gpu.fused_dense_bias_activation, "identity", *args)
+    gW, gx, gb = back(dev(gpu, delta, "f32"))
+    np.testing.assert_array_equal(gW.to_numpy(), f64(delta) @ f64(x).T)
+    np.testing.assert_array_equal(gx.to_numpy(), f64(W).T @ f64(delta))
+    np.testing.assert_array_equal(gb.to_numpy(), f64(delta).sum(axis=1))
+
+
 @pytest.mark.parametrize("dtype", ["f32", "bf16"])
 @pytest.mark.parametrize("act", ["identity", "gelu"])
 def test_few_columns(gpu, dtype, act):
