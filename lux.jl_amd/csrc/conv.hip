@@ -689,7 +689,7 @@ static int run_conv_any(hipStream_t s, const ConvGeom& g, bool dgrad, const AnyP
             if (!dgrad) { a.SP = g.W; a.SQ = g.H; a.ss_w = g.sw; a.ss_h = g.sh; a.P = g.OW; a.Q = g.OH; a.os_w = a.os_h = 1; a.Ctot_out = g.Cout; }
             else { a.SP = g.OW; a.SQ = g.OH; a.ss_w = a.ss_h = 1; a.P = g.W; a.Q = g.H; a.os_w = g.sw; a.os_h = g.sh; a.Ctot_out = g.Cin; }
             a.PQ = a.P * a.Q;
-            a.Ncols = plan.Ncols; a.Cch = plan.Cch; a.res_w = std::max(plan.res_w, 1); a.merged = plan.merged;
+            a.Ncols = plan.Ncols; a.Cch = plan.Cch; a.res_w = std::max(plan.res_w, 1); a.merged = plan.merged; a.kW = g.kW; a.kH = g.kH;
             a.col_off = grp * plan.Cch; a.act = act; a.subs = l.n;
             a.divCp = FastDiv((uint32_t)plan.Cp); a.divCch = FastDiv((uint32_t)plan.Cch);
             for (int i = 0; i < l.n; ++i) a.sub[i] = l.sub[i];

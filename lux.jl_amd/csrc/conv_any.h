@@ -11,8 +11,9 @@
 // sub-problem of one launch.  Where a residue has few channels (the first layer of an image network: 3) all residues
 // become columns of one problem instead, over the union of their taps: 2 x 2 residues of 3 channels share the rows they
 // read, and fill 12 columns of a 32-column tile instead of 3.
-// (A tap that a residue lacks is a zero weight there: a non-finite cotangent makes NaN of up to `stride` positions on either
-// side of those that it reaches.  Residues apart would keep those finite, at three times the gathers: 49 taps against 16.)
+// A tap that a residue lacks is a zero weight there, and zero times a non-finite cotangent is NaN where the residue does not
+// see that cotangent at all.  So a sum that comes out NaN is taken again over the residue's own taps (own_taps_sum below);
+// the others pay one comparison.  (Residues apart would need no such thing, at three times the gathers: 49 taps against 16.)
 //
 // The main loop is the one of gemm_split.h: several stages per trip to memory, K cut into slices where tiles are few.
 //
@@ -55,6 +56,7 @@ struct Args {
     int os_w, os_h;
     int Ncols, Cch;            // columns; channels per residue (merged: Ncols = residues * Cch)
     int res_w;                 // merged: residues along w
+    int kW, kH;                // merged (dilation 1): tap t of residue r is filter tap t * os + r, where there is one
     int col_off, Ctot_out, act;
     int subs, merged;
     char* partial;
@@ -120,6 +122,29 @@ struct Shape {
     using Core = split::Core<T, WM, WN, NWM, NWN, LA, LB>;
 };
 
+// Merged residues: the sum of row (a, b, n) and column col over the taps that the column's residue (rw, rh) has.  A NaN among
+// the terms ends it, so a cotangent that is NaN throughout costs one term per element.
+template <typename T>
+__device__ __forceinline__ float own_taps_sum(const Args<T>& g, const Sub& q, int a, int b, int n, int col, int rw, int rh) {
+    const int nw = (g.kW - rw + g.os_w - 1) / g.os_w, nh = (g.kH - rh + g.os_h - 1) / g.os_h;
+    const T* wcol = g.wm + q.wm + (int64_t)col * q.Kpad;
+    float sum = 0.0f;
+    for (int th = 0; th < nh; ++th) {
+        const int sq = b * g.ss_h + q.h0 + th * q.hstep;
+        if ((unsigned)sq >= (unsigned)g.SQ) continue;
+        for (int tw = 0; tw < nw; ++tw) {
+            const int sp = a * g.ss_w + q.w0 + tw * q.wstep;
+            if ((unsigned)sp >= (unsigned)g.SP) continue;
+            const T* x = g.src + (int64_t)((n * g.SQ + sq) * g.SP + sp) * g.Ctot;
+            const T* w = wcol + (th * q.TW + tw) * g.Cp;
+#pragma unroll 1
+            for (int c = 0; c < g.Cp; ++c) sum = fmaf(ld(x + c), ld(w + c), sum);
+            if (sum != sum) return sum;
+        }
+    }
+    return sum;
+}
+
 template <typename T, int WM, int WN, int NWM, int NWN>
 __global__ __launch_bounds__(split::THREADS) void conv_any_kernel(Args<T> g) {
     using S = Shape<T, WM, WN, NWM, NWN>;
@@ -135,6 +160,7 @@ __global__ __launch_bounds__(split::THREADS) void conv_any_kernel(Args<T> g) {
     int tm, tn;
     tile_coords(tile, q.tiles_m, q.tiles_n, tm, tn);
     const int m0 = tm * S::TILE_M, n0 = tn * S::TILE_N;
+    static_assert(WM <= 2 && WN <= 2, "32 accumulator bits per i below");
     f32x16_v acc[WM][WN];
     {
         const typename S::LA la(g, q, m0);
@@ -165,6 +191,7 @@ __global__ __launch_bounds__(split::THREADS) void conv_any_kernel(Args<T> g) {
         ih[i] = b * g.os_h + q.oh0;
         row[i] = (int64_t)n * g.Ctot_out * g.PQ + (int64_t)ih[i] * g.P + iw[i];
     }
+    bool nan = false;                  // merged: among this lane's sums
     static_for<WN * 16>([&](auto JR) {
         constexpr int j = decltype(JR)::value / 16, r = decltype(JR)::value % 16;
         const int col = nb + j * 32 + ((r >> 2) << 3) + (r & 3);
@@ -184,7 +211,10 @@ __global__ __launch_bounds__(split::THREADS) void conv_any_kernel(Args<T> g) {
             for (int i = 0; i < WM; ++i) {
                 v[i] = acc[i][j][r] + bv;
                 st_ok[i] = ok[i];
-                if (g.merged) st_ok[i] = ok[i] && (unsigned)(iw[i] + rw) < (unsigned)g.P && (unsigned)(ih[i] + rh) < (unsigned)g.Q;
+                if (g.merged) {
+                    st_ok[i] = ok[i] && (unsigned)(iw[i] + rw) < (unsigned)g.P && (unsigned)(ih[i] + rh) < (unsigned)g.Q;
+                    nan = nan || v[i] != v[i];
+                }
             }
             if (g.pre != nullptr) {
 #pragma unroll
@@ -198,6 +228,25 @@ __global__ __launch_bounds__(split::THREADS) void conv_any_kernel(Args<T> g) {
                 if (st_ok[i]) st(g.out + coff + row[i], v[i]);
         }
     });
+    if (!nan) return;
+    uint64_t nans = 0;                 // bit 32 i + 16 j + r
+    static_for<WM * WN * 16>([&](auto E) {
+        constexpr int i = decltype(E)::value / (WN * 16), jr = decltype(E)::value % (WN * 16);
+        const float v = acc[i][jr / 16][jr % 16];
+        if (v != v) nans |= uint64_t(1) << (32 * i + jr);
+    });
+    while (nans != 0) {                // an input gradient: no bias, no activation
+        const int e = __builtin_ctzll(nans), r = e & 15;
+        nans &= nans - 1;
+        const int m = mb + (e & 32), col = nb + 2 * (e & 16) + ((r >> 2) << 3) + (r & 3);
+        if (m >= q.M || col >= g.Ncols) continue;
+        const int n = (int)q.divRAB.div((uint32_t)m), rem = m - n * q.RAB;
+        const int b = (int)q.divRA.div((uint32_t)rem), a = rem - b * q.RA;
+        const int res = (int)g.divCch.div((uint32_t)col), ch = col - res * g.Cch, rh = res / g.res_w, rw = res - rh * g.res_w;
+        const int ow = a * g.os_w + q.ow0 + rw, oh = b * g.os_h + q.oh0 + rh;
+        if ((unsigned)ow < (unsigned)g.P && (unsigned)oh < (unsigned)g.Q)
+            st(g.out + (int64_t)(n * g.Ctot_out + g.col_off + ch) * g.PQ + (int64_t)oh * g.P + ow, own_taps_sum<T>(g, q, a, b, n, col, rw, rh));
+    }
 }
 
 // ----------------------------------------------------------------------------- filter gradient

@@ -84,3 +84,28 @@ def test_whole_tap_kernels_at_small_sizes(gpu, dtype):
                          dtype, "tap dx")
     finally:
         gpu.set_option("conv_tile", 0)
+
+
+@pytest.mark.parametrize("dtype", ["f32", "bf16"])
+@pytest.mark.parametrize("xs,ws,stride,pad,groups", [
+    ((37, 29, 3, 2), (7, 7, 3, 20), 2, 3, 1),                # one residue column block
+    ((9, 11, 6, 2), (5, 4, 2, 9), 3, (2, 1, 0, 2), 3),       # nine residues, groups
+    ((9, 8, 3, 1), (5, 5, 3, 640), 2, 2, 1),                 # contraction cut into slices
+    ((21, 20, 12, 2), (7, 7, 12, 16), 2, 3, 1),              # residues over more than one column tile
+])
+def test_nonfinite_cotangent_reaches_its_window_only(gpu, dtype, xs, ws, stride, pad, groups):
+    """An infinite and a NaN cotangent: the input gradient is non-finite exactly where the filter's window sees them."""
+    rng = np.random.default_rng(stable_seed("nonfinite", xs))
+    kw = dict(stride=stride, padding=pad, groups=groups)
+    gd, od = gpu.DenseConvDims(xs, ws, **kw), O.ConvDims(xs, ws, **kw)
+    w, dy = host_inputs(dtype, rng.normal(size=ws) / np.sqrt(ws[0] * ws[1] * ws[3]), rng.normal(size=od.y_shape()))
+    bad = {(1, 2, 0, 0): np.inf, (od.y_shape()[0] - 1, 1, ws[3] - 1, xs[3] - 1): np.nan}
+    dy, reach = dy.copy(), np.zeros(od.y_shape())
+    for at in bad:
+        dy[at], reach[at] = 0, 1
+    want, seen = O.conv_data_grad(f64(dy), f64(w), od), O.conv_data_grad(reach, np.ones(ws), od) > 0
+    for at, value in bad.items():
+        dy[at] = value
+    got = f64(gpu.conv_data_grad(dev(gpu, dy, dtype), dev(gpu, w, dtype), gd).to_numpy())
+    np.testing.assert_array_equal(np.isfinite(got), ~seen)
+    assert_close(np.where(seen, 0.0, got), np.where(seen, 0.0, want), dtype, f"{dtype} finite part of dx")
