@@ -90,8 +90,11 @@ int launch_layouts(hipStream_t s, DenseArgs<T>& a, bool ak, bool bk, int slices,
 }  // namespace split
 
 // The kernels of gemm_split.h take the problem, and are faster on it than the big-tile kernels: those keep whole aligned
-// 128 x 128 tiles that fill the chip once (bf16 4096 x 1024 x 2048: 26 us against 35, 2048 x 4096 x 2048: 50 against 50;
-// fp32 4096 x 2048 x 1024: 137 against 144), but not fewer (1024^3: bf16 13.3 against 9.2, fp32 71 against 28).
+// 128 x 128 tiles that nearly fill the chip.  With 160 and more of the 256 compute units in use they are ahead in bf16
+// (us, big tiles against these: 1920 x 2048 x 2048 27.4 / 36.3, 1280 x 2048 x 4096 46.9 / 62.0), with 128 they are not
+// (1024 x 2048 x 4096 45.5 / 41.9; 1024^3 13.3 / 9.2), nor where K is short (1536 x 2048 x 128 5.6 / 5.3 up to 192 tiles,
+// 1920 x 2048 x 128 6.0 / 6.6).  In fp32 the line lies between 192 tiles (1536 x 2048 x 1024 80.4 / 73.0) and 208
+// (1664 x 2048 x 1024 81.3 / 88.1).
 template <typename T>
 bool split_takes(const DenseArgs<T>& a) {
     using Tr = GemmTraits<T>;
@@ -99,7 +102,8 @@ bool split_takes(const DenseArgs<T>& a) {
     const int64_t lim = (int64_t(1) << 31) / (256 * (int64_t)sizeof(T));
     if (std::max(a.A.sr, a.A.sk) >= lim || std::max(a.B.sr, a.B.sk) >= lim) return false;
     const int64_t cus = num_cus() > 0 ? num_cus() : 256;
-    return !(whole_tiles<T, 128, 128>(a) && (int64_t)(a.M / 128) * (a.N / 128) >= cus);
+    const int64_t busy = sizeof(T) == 2 && a.K >= 512 ? cus / 2 : cus * 3 / 4;
+    return !(whole_tiles<T, 128, 128>(a) && (int64_t)(a.M / 128) * (a.N / 128) > busy);
 }
 
 template <typename T>

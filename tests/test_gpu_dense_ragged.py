@@ -94,3 +94,33 @@ def test_few_columns(gpu, dtype, act):
         got = gpu.fused_dense_bias_activation(act, *args).to_numpy()
         assert_close(got, want, dtype, f"{dtype} {act} {M}x{N}x{K}")
         np.testing.assert_array_equal(got, gpu.pullback(gpu.fused_dense_bias_activation, act, *args)[0].to_numpy())
+
+
+def kernels_of(gpu, f):
+    """Names of the kernels that f launches."""
+    import ctypes
+    import json
+    buf = ctypes.create_string_buffer(1 << 16)
+    gpu._lib.call("luxhip_profile_enable", 1)
+    try:
+        f()
+        gpu._lib.call("luxhip_profile_report", buf, len(buf))
+    finally:
+        gpu._lib.call("luxhip_profile_enable", 0)
+    return {k["kernel"] for k in json.loads(buf.value.decode())}
+
+
+@pytest.mark.parametrize("dtype,M,N,K,split", [
+    ("bf16", 1280, 2048, 512, False), ("bf16", 1024, 2048, 512, True), ("bf16", 1536, 2048, 128, True), ("bf16", 1664, 2048, 128, False),
+    ("f32", 1664, 2048, 128, False), ("f32", 1536, 2048, 128, True),
+])
+def test_whole_tiles_that_nearly_fill_the_chip(gpu, dtype, M, N, K, split):
+    """Either side of the line between the big-tile kernels and those of gemm_split.h (small whole numbers: exact in fp32)."""
+    rng = np.random.default_rng(stable_seed("whole", M, K))
+    A, B = rng.integers(-2, 3, size=(M, K)).astype(np.float32), rng.integers(-2, 3, size=(K, N)).astype(np.float32)
+    dA, dB = dev(gpu, A, dtype), dev(gpu, B, dtype)
+    out = []
+    names = kernels_of(gpu, lambda: out.append(gpu.matmul(dA, dB, None, False, False)))
+    assert any("split" in n for n in names) == split, names
+    want = A @ B
+    np.testing.assert_array_equal(out[0].to_numpy(), want if dtype == "f32" else O.round_to_bf16(want))
