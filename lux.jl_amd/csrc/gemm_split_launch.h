@@ -94,7 +94,9 @@ int launch_layouts(hipStream_t s, DenseArgs<T>& a, bool ak, bool bk, int slices,
 // (us, big tiles against these: 1920 x 2048 x 2048 27.4 / 36.3, 1280 x 2048 x 4096 46.9 / 62.0), with 128 they are not
 // (1024 x 2048 x 4096 45.5 / 41.9; 1024^3 13.3 / 9.2), nor where K is short (1536 x 2048 x 128 5.6 / 5.3 up to 192 tiles,
 // 1920 x 2048 x 128 6.0 / 6.6).  In fp32 the line lies between 192 tiles (1536 x 2048 x 1024 80.4 / 73.0) and 208
-// (1664 x 2048 x 1024 81.3 / 88.1).
+// (1664 x 2048 x 1024 81.3 / 88.1).  Aligned operands of less than a tile in one dimension and many tiles in the other are
+// streamed by the big-tile kernels as well while K is short (fp32 1000000 x 9 x 100 178.9 / 193.1, bf16 300000 x 9 x 32
+// 14.2 / 15.8; but 24 x 200000 x 512 38.7 / 33.8).
 template <typename T>
 bool split_takes(const DenseArgs<T>& a) {
     using Tr = GemmTraits<T>;
@@ -102,6 +104,7 @@ bool split_takes(const DenseArgs<T>& a) {
     const int64_t lim = (int64_t(1) << 31) / (256 * (int64_t)sizeof(T));
     if (std::max(a.A.sr, a.A.sk) >= lim || std::max(a.B.sr, a.B.sk) >= lim) return false;
     const int64_t cus = num_cus() > 0 ? num_cus() : 256;
+    if (a.A.vec_ok && a.B.vec_ok && a.K <= 128 && std::min(a.M, a.N) < 64 && ceil_div(std::max(a.M, a.N), 64) > 4 * cus) return false;
     const int64_t busy = sizeof(T) == 2 && a.K >= 512 ? cus / 2 : cus * 3 / 4;
     return !(whole_tiles<T, 128, 128>(a) && (int64_t)(a.M / 128) * (a.N / 128) > busy);
 }
