@@ -196,9 +196,24 @@ int launch(hipStream_t s, const DenseArgs<T>& d, size_t ws_front) {
 
 }  // namespace skinny
 
+// Rows enough for several workgroups per compute unit fill the chip in tiles of 64 columns too, and what those pad costs less
+// than the sums over eight waves do here: bf16 keeps to one workgroup per compute unit (one column, tiles against this
+// kernel, us: 300000 x 128 18.8 / 24.1, 100000 x 1024 34.4 / 39.6, 30000 x 2048 26.0 / 25.4; 16 columns: 1000000 x 32
+// 48.7 / 118.9), fp32, whose matrix rate is a sixteenth, to two where the k of its waves is mostly padding (one column:
+// 100000 x 100 18.8 / 25.1, x 128 20.9 / 18.9; 30000 x 256 14.0 / 8.5; nine columns: 300000 x 512 186.2 / 147.0).
+// With less than a step of k fp32 keeps to one as well (30000 x 8 4.0 / 5.8, 10000 x 8 4.2 / 3.6).
+template <typename T>
+static bool skinny_pays(int64_t M, int64_t K) {
+    constexpr int V = skinny::Elem<T>::V, MT = 16 * V, KSTEP = 4 * V;
+    const int64_t cus = num_cus() > 0 ? num_cus() : 256, blocks = ceil_div(M, MT);
+    if (blocks <= (sizeof(T) == 2 || K < KSTEP ? cus : 2 * cus)) return true;
+    const int64_t kpad = ceil_div(ceil_div(K, skinny::WAVES), KSTEP) * KSTEP * skinny::WAVES;
+    return sizeof(T) == 4 && 7 * K > 4 * kpad + 380;
+}
+
 template <typename T>
 bool launch_skinny(hipStream_t s, DenseArgs<T>& d, bool ak, bool bk, size_t ws_front, int* rc) {
-    if (ak || !bk || d.N > skinny::NMAX || d.N < 1 || d.M < 16 * skinny::Elem<T>::V || d.K < 1) return false;
+    if (ak || !bk || d.N > skinny::NMAX || d.N < 1 || d.M < 16 * skinny::Elem<T>::V || d.K < 1 || !skinny_pays<T>(d.M, d.K)) return false;
     *rc = skinny::launch<T>(s, d, ws_front);
     return true;
 }

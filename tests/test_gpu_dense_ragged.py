@@ -124,3 +124,18 @@ def test_whole_tiles_that_nearly_fill_the_chip(gpu, dtype, M, N, K, split):
     assert any("split" in n for n in names) == split, names
     want = A @ B
     np.testing.assert_array_equal(out[0].to_numpy(), want if dtype == "f32" else O.round_to_bf16(want))
+
+
+@pytest.mark.parametrize("dtype,M,K,skinny", [
+    ("bf16", 32768, 64, True), ("bf16", 32769, 64, False), ("f32", 32768, 100, True), ("f32", 32769, 100, False),
+    ("f32", 32769, 256, True), ("f32", 32769, 260, False), ("f32", 16384, 15, True), ("f32", 16385, 15, False),
+])
+def test_few_columns_and_many_rows(gpu, dtype, M, K, skinny):
+    """Rows for more workgroups than the chip takes at once go to the tiled kernels unless K is long (exact whole numbers)."""
+    rng = np.random.default_rng(stable_seed("tall layer", M, K))
+    W, x = rng.integers(-2, 3, size=(M, K)).astype(np.float32), rng.integers(-2, 3, size=(K, 3)).astype(np.float32)
+    dW, dx, out = dev(gpu, W, dtype), dev(gpu, x, dtype), []
+    names = kernels_of(gpu, lambda: out.append(gpu.matmul(dW, dx, None, False, False)))
+    assert any("skinny" in n for n in names) == skinny, names
+    want = W @ x
+    np.testing.assert_array_equal(out[0].to_numpy(), want if dtype == "f32" else O.round_to_bf16(want))
