@@ -204,8 +204,7 @@ __global__ void gn_bwd_kernel(const T* __restrict__ delta, const T* __restrict__
                               const T* __restrict__ beta, const float* __restrict__ save_mean,
                               const float* __restrict__ save_invstd, T* dx, float* pdg, float* pdb, T* dgamma,
                               T* dbeta, uint32_t* counters, uint32_t cstride, uint32_t N, GnGeom g, GnExchange ex) {
-    extern __shared__ float lds[];                  // [16] reduction scratch, then [nw][Cg] x 2
-    __shared__ float rowsum[2][AFFINE ? 1024 : 1];
+    extern __shared__ float lds[];                  // [16] reduction scratch, then [nw][Cg] x 2, later [T_] x 2
     float* sm = lds;
     const uint32_t T_ = blockDim.x, nw = T_ >> 6, w = threadIdx.x >> 6;
     float* accg = lds + 16 + (size_t)w * g.Cg;
@@ -459,6 +458,7 @@ __global__ void gn_bwd_kernel(const T* __restrict__ delta, const T* __restrict__
             // (One row alone would make N round trips to memory, one after the other, at the end of the kernel: 35 x 35 x 96 x 24
             // fp32 22.3 against 16.5 us, 64 x 64 x 256 x 16 bf16 46.2 against 43.3 for forward and pullback.)
             const uint32_t rows = g.Cg < T_ ? min(T_ / g.Cg, N) : 1u;
+            float* const rowsum = lds + 16;              // the waves' accumulators were read before publish_done
             for (uint32_t j0 = 0; j0 < g.Cg; j0 += T_) {
                 const uint32_t r = threadIdx.x / min(g.Cg, T_), j = j0 + threadIdx.x - r * min(g.Cg, T_);
                 float tg = 0.0f, tb = 0.0f;
@@ -469,13 +469,13 @@ __global__ void gn_bwd_kernel(const T* __restrict__ delta, const T* __restrict__
                         tb += fetch(pdb + (size_t)nn * g.C + k * g.Cg + j);
                     }
                 }
-                rowsum[0][threadIdx.x] = tg;
-                rowsum[1][threadIdx.x] = tb;
+                rowsum[threadIdx.x] = tg;
+                rowsum[T_ + threadIdx.x] = tb;
                 __syncthreads();
                 if (r == 0 && j < g.Cg) {
                     for (uint32_t q = 1; q < rows; ++q) {
-                        tg += rowsum[0][threadIdx.x + q * g.Cg];
-                        tb += rowsum[1][threadIdx.x + q * g.Cg];
+                        tg += rowsum[threadIdx.x + q * g.Cg];
+                        tb += rowsum[T_ + threadIdx.x + q * g.Cg];
                     }
                     if (dgamma) st(dgamma + k * g.Cg + j, tg);
                     if (dbeta) st(dbeta + k * g.Cg + j, tb);
@@ -640,7 +640,8 @@ static int gn_bwd_impl(hipStream_t s, int act, int64_t I, int64_t C, int64_t G, 
     constexpr int V = Vec<T>::N;
     GnLaunch L = gn_plan<T>(I, C, G, N, aligned16(x) && aligned16(delta) && aligned16(dx), !stream_capturing(s));
     const bool affine = gamma != nullptr && (dgamma != nullptr || dbeta != nullptr);
-    // LDS: 16 floats of reduction scratch + 2 * nw * Cg accumulators
+    // LDS: 16 floats of reduction scratch + 2 * nw * Cg accumulators, in whose place the last workgroup puts two sums per
+    // thread.  Together with the kernel's static arrays (under 1 KiB) that stays below the 64 KiB of an ordinary launch.
     size_t lds_bytes = 64;
     if (affine) {
         while (L.threads > 64 && (16 + 2 * (size_t)(L.threads / 64) * L.g.Cg) * 4 > 60 * 1024) {
@@ -652,7 +653,7 @@ static int gn_bwd_impl(hipStream_t s, int act, int64_t I, int64_t C, int64_t G, 
             L.g.pvec = L.g.nvec;
             L.blocks = (unsigned)(G * N);
         }
-        lds_bytes = (16 + 2 * (size_t)(L.threads / 64) * L.g.Cg) * 4;
+        lds_bytes = (16 + 2 * std::max<size_t>((size_t)(L.threads / 64) * L.g.Cg, L.threads)) * 4;
         LUX_UNSUPPORTED_IF(lds_bytes > 60 * 1024, "groupnorm_bwd: %u channels per group exceed the LDS accumulators", L.g.Cg);
     }
     float *pdg = nullptr, *pdb = nullptr;

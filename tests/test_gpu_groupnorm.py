@@ -13,7 +13,10 @@ CASES = [((6, 2), 2), ((4, 4, 6, 2), 3), ((2, 2, 6, 2), 2), ((5, 12, 3), 4), ((1
          # slices that two workgroups share (fp32: 19200 elements per slice, bf16: 65536)
          ((40, 40, 24, 2), 2), ((64, 64, 32, 2), 2),
          # 72 channels per group: more than the kernels' LDS tables of channel parameters hold
-         ((4, 4, 144, 2), 2)]
+         ((4, 4, 144, 2), 2),
+         # as many accumulators as the pullback's LDS takes: an odd number of channels, so one workgroup of 1024 threads
+         # (fp32, then bf16) or 512
+         ((6, 6, 942, 2), 2), ((9, 8, 471, 2), 1), ((4, 3, 941, 2), 1)]
 
 
 @pytest.fixture(params=["wait", "no_wait"])
