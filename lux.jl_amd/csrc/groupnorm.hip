@@ -583,6 +583,16 @@ static GnLaunch gn_plan(int64_t I, int64_t C, int64_t G, int64_t N, bool ptr_ok,
     L.g.pvec = L.g.nvec / L.g.parts;
     int64_t t = 64;
     while (t < 1024 && t * kGnCache < L.g.pvec) t <<= 1;
+    if (L.ragged) {
+        // Ragged rows in vectors take a quarter or an eighth of the trips that single elements took, but not of the threads
+        // while the chip has room for them: a slice on one wave is one chain of trips, and the last wave's sums wait for it
+        // (bf16 7 x 7 x 256 x 16 in 4 groups, forward and pullback: 18.4 us element by
+        // element, 36.1 on 64 threads per slice; with 4096 slices 64 threads are ahead, bf16 21 x 21 x 64 x 128: 21.7 against 28.4)
+        const int64_t cus = num_cus() > 0 ? num_cus() : 256;
+        int64_t single = 64;
+        while (single < 512 && single * kGnCache < m) single <<= 1;
+        while (t < single && G * N * t < 1024 * cus) t <<= 1;
+    }
     L.threads = (unsigned)t;
     L.cached = (int64_t)L.g.pvec <= t * kGnCache;
     if (!L.cached) { L.g.parts = 1; L.g.pvec = L.g.nvec; }
