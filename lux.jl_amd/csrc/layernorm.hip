@@ -476,12 +476,31 @@ struct LnPlan {
     unsigned threads, blocks;
 };
 
+// Ragged columns (RowVec in common.h) go element by element where vectors would leave most of a wave idle.  Measured, us,
+// elements against vectors, 2^24 elements: one pass forward (bf16 also pays for rows at odd addresses) fp32 99 42 / 47, 198
+// 28 / 26, 295 24 / 24 (gelu 26 / 29), 390 24 / 22; bf16 98 44 / 73, 258 25 / 24 (gelu 28 / 31), 390 21 / 18, 511 18 / 20.
 template <typename T>
-static LnPlan ln_plan(int64_t L, int64_t R, bool ptr_ok) {
+static bool ln_ragged_vectors(int64_t L, int64_t nvec) {
+    return L > 64 * kLnCache || (nvec * 20 >= 13 * 64 * ceil_div(nvec, 64) && (L * (int64_t)sizeof(T)) % 4 == 0);
+}
+// The pullback that makes all gradients in one pass has two waves per column: fp32 99 93 / 160, 198 76 / 87, 258 75 / 65;
+// bf16 198 65 / 84 (gelu 85 / 135), 390 55 / 49 (72 / 76), 450 54 / 43.  Up to 2048 columns it takes what the two kernels
+// and the launch between them do (bf16 257 x 512 8.3 / 7.1, x 2048 9.2 / 11.9), except that long bf16 columns which are too
+// many for one each and too few for several lose to the sum of the partial gradients (2293 x 2048 with gelu 24.9 / 32.7,
+// x 512 11.6 / 14.6, x 4096 41.9 / 39.1).
+template <typename T>
+static bool ln_ragged_fused(int64_t L, int64_t R, int64_t nvec) {
+    if (sizeof(T) == 2 && L > 2048 && R >= 1024 && R < 3072) return false;
+    return R <= 2048 || nvec >= (sizeof(T) == 2 ? 52 : 60);
+}
+
+// elements: ragged columns one element at a time
+template <typename T>
+static LnPlan ln_plan(int64_t L, int64_t R, bool ragged, bool elements) {
     constexpr int V = Vec<T>::N;
     LnPlan p;
-    p.vec = L >= V;
-    p.ragged = p.vec && !(ptr_ok && L % V == 0);
+    p.vec = L >= V && !(ragged && elements);
+    p.ragged = p.vec && ragged;
     p.nvec = (uint32_t)ceil_div(L, p.vec ? V : 1);
     p.wave = p.nvec <= 64u * kLnCache;
     if (p.wave) {
@@ -523,7 +542,7 @@ static int ln_check(int dtype, int act, int64_t L, int64_t R) {
         else if (p.vec && p.wave) LN_RAGGED(KERNEL, A, true, kLnCache, __VA_ARGS__);                    \
         else if (p.vec && p.cached) LN_RAGGED(KERNEL, A, false, kLnCache, __VA_ARGS__);                 \
         else if (p.vec) LN_RAGGED(KERNEL, A, false, 0, __VA_ARGS__);                                    \
-        else LN_ONE(KERNEL, A, 1, true, kLnCache, false, __VA_ARGS__);       /* fewer elements than a vector */ \
+        else LN_ONE(KERNEL, A, 1, true, kLnCache, false, __VA_ARGS__);       /* element by element */    \
     } while (0)
 
 template <typename T>
@@ -531,7 +550,8 @@ static int ln_fwd_impl(hipStream_t s, int act, int64_t L, int64_t R, const T* x,
                        T* y, float* save_mean, float* save_invstd) {
     constexpr int V = Vec<T>::N;
     const bool ptr_ok = aligned16(x) && aligned16(y) && (gamma == nullptr || (aligned16(gamma) && aligned16(beta)));
-    LnPlan p = ln_plan<T>(L, R, ptr_ok);
+    const bool ragged = !(ptr_ok && L % V == 0);
+    LnPlan p = ln_plan<T>(L, R, ragged, !ln_ragged_vectors<T>(L, ceil_div(L, V)));
     const float inv_L = 1.0f / (float)L;
     ProfScope ps("ln_fwd_kernel", s, true);
 #define LN_FWD(A) LN_VARIANTS(ln_fwd_kernel, A, x, gamma, beta, y, save_mean, save_invstd, (uint32_t)L, p.nvec, (uint32_t)R, inv_L, eps)
@@ -547,9 +567,12 @@ static int ln_bwd_impl(hipStream_t s, int act, int64_t L, int64_t R, const T* de
     constexpr int V = Vec<T>::N;
     const bool ptr_ok = aligned16(x) && aligned16(delta) && aligned16(dx) &&
                         (gamma == nullptr || (aligned16(gamma) && aligned16(beta)));
-    LnPlan p = ln_plan<T>(L, R, ptr_ok);
+    const bool ragged = !(ptr_ok && L % V == 0), params = gamma != nullptr && (dgamma != nullptr || dbeta != nullptr);
+    const int64_t nvec = ceil_div(L, V);
+    const bool one_pass = L >= V && nvec <= 64 * kLnCache && params && R >= 64 && (!ragged || ln_ragged_fused<T>(L, R, nvec));
+    LnPlan p = ln_plan<T>(L, R, ragged, !one_pass && (params && R >= 64 ? nvec <= 64 * kLnCache : !ln_ragged_vectors<T>(L, nvec)));
     const float inv_L = 1.0f / (float)L;
-    if (p.vec && p.wave && gamma != nullptr && (dgamma != nullptr || dbeta != nullptr) && R >= 64) {
+    if (one_pass) {
         // one pass over delta and x: dx and the per-position sums of every workgroup
         const int64_t blocks = std::min<int64_t>(ceil_div(R, 2), 3 * (int64_t)(num_cus() > 0 ? num_cus() : 256));
         Workspace ws;
@@ -579,7 +602,11 @@ static int ln_bwd_impl(hipStream_t s, int act, int64_t L, int64_t R, const T* de
     }
     {
         ProfScope ps("ln_bwd_dx_kernel", s, true);
-#define LN_BWD(A) LN_VARIANTS(ln_bwd_dx_kernel, A, delta, x, gamma, beta, save_mean, save_invstd, dx, (uint32_t)L, p.nvec, (uint32_t)R, inv_L)
+#define LN_BWD(A)                                                                                                         \
+    do {                                                                                                                  \
+        if (!p.vec && !p.wave) LN_ONE(ln_bwd_dx_kernel, A, 1, false, kLnCache, false, delta, x, gamma, beta, save_mean, save_invstd, dx, (uint32_t)L, p.nvec, (uint32_t)R, inv_L); \
+        else LN_VARIANTS(ln_bwd_dx_kernel, A, delta, x, gamma, beta, save_mean, save_invstd, dx, (uint32_t)L, p.nvec, (uint32_t)R, inv_L);                       \
+    } while (0)
         LUX_DISPATCH_ACT(act, LN_BWD);
 #undef LN_BWD
     }

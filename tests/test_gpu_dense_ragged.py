@@ -5,7 +5,7 @@ import numpy as np
 import pytest
 
 from oracle import luxlib_oracle as O
-from tests.util import assert_close, dev, f64, host_inputs, rms, stable_seed
+from tests.util import assert_close, dev, f64, host_inputs, kernels_of, rms, stable_seed
 
 pytestmark = pytest.mark.gpu
 
@@ -94,20 +94,6 @@ def test_few_columns(gpu, dtype, act):
         got = gpu.fused_dense_bias_activation(act, *args).to_numpy()
         assert_close(got, want, dtype, f"{dtype} {act} {M}x{N}x{K}")
         np.testing.assert_array_equal(got, gpu.pullback(gpu.fused_dense_bias_activation, act, *args)[0].to_numpy())
-
-
-def kernels_of(gpu, f):
-    """Names of the kernels that f launches."""
-    import ctypes
-    import json
-    buf = ctypes.create_string_buffer(1 << 16)
-    gpu._lib.call("luxhip_profile_enable", 1)
-    try:
-        f()
-        gpu._lib.call("luxhip_profile_report", buf, len(buf))
-    finally:
-        gpu._lib.call("luxhip_profile_enable", 0)
-    return {k["kernel"] for k in json.loads(buf.value.decode())}
 
 
 @pytest.mark.parametrize("dtype,M,N,K,split", [

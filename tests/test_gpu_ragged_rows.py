@@ -5,7 +5,7 @@ import numpy as np
 import pytest
 
 from oracle import luxlib_oracle as O
-from tests.util import assert_close, dev, f64, host_inputs, rms, stable_seed
+from tests.util import assert_close, dev, f64, host_inputs, kernels_of, rms, stable_seed
 
 pytestmark = pytest.mark.gpu
 
@@ -45,3 +45,20 @@ def test_layernorm(gpu, dtype, act):
         sd = np.sqrt(f64(x).var(axis=0).min() + eps)
         for name, a, w in zip(("dx", "dgamma", "dbeta"), got, want):
             assert_close(a.to_numpy(), w, dtype, f"{tag} {name}", scale=rms(delta) * (1.5 / sd if name == "dx" else np.sqrt(R)))
+
+
+@pytest.mark.parametrize("dtype,L,R,fused", [
+    ("f32", 67, 2048, True), ("f32", 67, 2049, False), ("f32", 237, 2049, True), ("bf16", 406, 2049, False), ("bf16", 409, 2049, True),
+    ("bf16", 2293, 1023, True), ("bf16", 2293, 1024, False),
+])
+def test_layernorm_on_either_side_of_the_one_pass_pullback(gpu, dtype, L, R, fused):
+    rng = np.random.default_rng(stable_seed("ln route", L, R))
+    x, g, b, delta = host_inputs(dtype, rng.normal(size=(L, R)) + 0.5, rng.uniform(0.5, 1.5, (L, 1)), 0.1 * rng.normal(size=(L, 1)), rng.normal(size=(L, R)))
+    _, back = gpu.pullback(gpu.layernorm, dev(gpu, x, dtype), dev(gpu, g, dtype), dev(gpu, b, dtype), "tanh", (1,), 1e-3)
+    got, d = [], dev(gpu, delta, dtype)
+    names = kernels_of(gpu, lambda: got.extend(back(d)))
+    assert ("ln_bwd_fused_kernel" in names) == fused, names
+    want = O.layernorm_pullback(f64(x), f64(g), f64(b), "tanh", (0,), 1e-3, f64(delta))
+    sd = np.sqrt(f64(x).var(axis=0).min() + 1e-3)
+    for name, a, w in zip(("dx", "dgamma", "dbeta"), got, want):
+        assert_close(a.to_numpy(), w, dtype, f"{dtype} {L}x{R} {name}", scale=rms(delta) * (1.5 / sd if name == "dx" else np.sqrt(R)))

@@ -78,3 +78,17 @@ def stable_seed(*parts):
     """Seed that does not depend on Python's per-process string hashing."""
     import zlib
     return zlib.crc32(repr(parts).encode()) & 0x7FFFFFFF
+
+
+def kernels_of(gpu, f):
+    """Names of the kernels that f launches."""
+    import ctypes
+    import json
+    buf = ctypes.create_string_buffer(1 << 16)
+    gpu._lib.call("luxhip_profile_enable", 1)
+    try:
+        f()
+        gpu._lib.call("luxhip_profile_report", buf, len(buf))
+    finally:
+        gpu._lib.call("luxhip_profile_enable", 0)
+    return {k["kernel"] for k in json.loads(buf.value.decode())}
