@@ -1,6 +1,8 @@
 // Convolution entry points: layout transforms, filter repacking, launch logic of the
 // implicit-GEMM kernels (conv_kernels.h) and the split-K reduction of the filter gradient.
 #include <algorithm>
+#include <cmath>
+#include <utility>
 #include <vector>
 
 #include "common.h"
@@ -543,19 +545,33 @@ static bool tap_shape(const ConvGeom& g, bool dgrad) {
     return ceil_div(rows, sizeof(T) == 2 ? 512 : 128) * tiles_n >= cus && Ncols * 4 >= tiles_n * 128 * 3;
 }
 
-struct Residue { int count, q0, s0, sstep, taps, k0; };     // rows, first q, first shift and step, taps
-// Residue r of one dimension of the input gradient: input positions i = stride q + r - pad in [0, L)
-static Residue residue(int r, int L, int pad, int stride, int dil, int taps) {
-    auto floor_div = [](int a, int b) { return a >= 0 ? a / b : -((-a + b - 1) / b); };
-    Residue z{0, 0, 0, 1, 0, 0};
-    z.q0 = -floor_div(r - pad, stride);                      // ceil((pad - r) / stride)
-    z.count = std::max(0, floor_div(L - 1 + pad - r, stride) - z.q0 + 1);
+struct Residue { int r, count, q0, s0, sstep, taps; };      // residue, rows, first q, first shift and step, taps
+// Residue r of one dimension of the input gradient: input positions i = stride q + r - pad in [0, L); k0 is its first tap (taps
+// if it has none)
+static Residue residue(int r, int k0, int L, int pad, int stride, int dil, int taps) {
+    auto floor_div = [](int64_t a, int64_t b) { return a >= 0 ? a / b : -((-a + b - 1) / b); };
+    Residue z{r, 0, 0, 0, 1, 0};
+    z.q0 = (int)-floor_div((int64_t)r - pad, stride);        // ceil((pad - r) / stride)
+    z.count = (int)std::max<int64_t>(0, floor_div((int64_t)L - 1 + pad - r, stride) - z.q0 + 1);
     int gq = stride, t = dil;
     while (t) { const int u = gq % t; gq = t; t = u; }
     z.sstep = dil / gq;
-    if (r % gq == 0)
-        for (int k = 0; k < std::min(taps, stride / gq); ++k)
-            if (((int64_t)k * dil - r) % stride == 0) { z.k0 = k; z.taps = (taps - 1 - k) / (stride / gq) + 1; z.s0 = (k * dil - r) / stride; break; }
+    if (k0 < taps) { z.taps = (taps - 1 - k0) / (stride / gq) + 1; z.s0 = (int)(((int64_t)k0 * dil - r) / stride); }
+    return z;
+}
+// The residues that have taps (no more than there are taps), by number, and with `all` also those without; a position of a
+// residue without taps has a gradient of zero
+static std::vector<Residue> residues(bool all, int L, int pad, int stride, int dil, int taps) {
+    std::vector<Residue> z;
+    std::vector<std::pair<int, int>> first;                  // (residue, its first tap)
+    int gq = stride, t = dil;
+    while (t) { const int u = gq % t; gq = t; t = u; }
+    for (int k = 0; k < std::min(taps, stride / gq); ++k) first.emplace_back((int)((int64_t)k * dil % stride), k);
+    if (all)
+        for (int r = 0; r < stride; ++r)
+            if (std::none_of(first.begin(), first.end(), [&](const std::pair<int, int>& f) { return f.first == r; })) first.emplace_back(r, taps);
+    std::sort(first.begin(), first.end());
+    for (const auto& f : first) z.push_back(residue(f.first, f.second, L, pad, stride, dil, taps));
     return z;
 }
 
@@ -565,9 +581,9 @@ struct AnyPlan {
     struct Launch { cany::Sub sub[cany::MAX_SUBS]; PackSub pack[cany::MAX_SUBS]; int n; };
     std::vector<Launch> launches;
     int Ncols = 0, Cch = 0, res_w = 0, merged = 0, Cp = 0;
+    bool zero_first = false;                                 // some positions of dx belong to no sub-problem: clear it before
     int64_t wm_elems = 0;                                    // packed filter of one group
-    void add(const Residue& rw, int RA, const Residue& rh, int RB, int N, int w0, int wstep, int TW, int h0, int hstep, int TH, int ow0, int oh0,
-             int r_w, int r_h) {
+    void add(const Residue& rw, int RA, const Residue& rh, int RB, int N, int w0, int wstep, int TW, int h0, int hstep, int TH, int ow0, int oh0) {
         if (RA <= 0 || RB <= 0) return;
         if (launches.empty() || launches.back().n == cany::MAX_SUBS) { launches.emplace_back(); launches.back().n = 0; }
         Launch& l = launches.back();
@@ -579,54 +595,55 @@ struct AnyPlan {
         q.ow0 = ow0; q.oh0 = oh0; q.wm = wm_elems;
         q.divRA = FastDiv((uint32_t)RA); q.divRAB = FastDiv((uint32_t)(RA * RB)); q.divTW = FastDiv((uint32_t)q.TW);
         PackSub& k = l.pack[l.n];
-        k = PackSub{r_w, r_h, rw.s0, rw.sstep, rh.s0, rh.sstep, q.TW, q.K, q.Kpad, res_w, wm_elems, 0};
+        k = PackSub{rw.r, rh.r, rw.s0, rw.sstep, rh.s0, rh.sstep, q.TW, q.K, q.Kpad, res_w, wm_elems, 0};
         wm_elems += (int64_t)Ncols * q.Kpad;
         ++l.n;
     }
     AnyPlan(const ConvGeom& g, bool dgrad) {
         Cp = padded<T>(dgrad ? g.Cout_g : g.Cin_g);
         Ncols = Cch = dgrad ? g.Cin_g : g.Cout_g;
-        const Residue none{0, 0, 0, 1, 0, 0};
+        const Residue none{0, 0, 0, 0, 1, 0};
         if (!dgrad) {
-            add(none, g.OW, none, g.OH, g.N, -g.pw, g.dw, g.kW, -g.ph, g.dh, g.kH, 0, 0, 0, 0);
+            add(none, g.OW, none, g.OH, g.N, -g.pw, g.dw, g.kW, -g.ph, g.dh, g.kH, 0, 0);
             return;
         }
-        std::vector<Residue> rw(g.sw), rh(g.sh);
-        for (int r = 0; r < g.sw; ++r) rw[r] = residue(r, g.W, g.pw, g.sw, g.dw, g.kW);
-        for (int r = 0; r < g.sh; ++r) rh[r] = residue(r, g.H, g.ph, g.sh, g.dh, g.kH);
-        // one problem per residue, or all residues as columns of one: whichever is less work in 32-column tiles
-        const int R = g.sw * g.sh;
-        auto cols = [](int n) { return (double)((n + 31) / 32 * 32); };
-        double apart = 0.0, together = 1e30;
+        // Where all residues fit one launch, those without taps write their zeros in it; of more (a stride of 32 has 1024)
+        // only those with taps are problems, and dx is cleared first if there are others (64 x 64 x 32 x 16, 1 x 1, stride 32:
+        // 43 us, against 2022 with 256 launches)
+        const int64_t R = (int64_t)g.sw * g.sh;
+        const bool all = R <= cany::MAX_SUBS;
+        const std::vector<Residue> rw = residues(all, g.W, g.pw, g.sw, g.dw, g.kW), rh = residues(all, g.H, g.ph, g.sh, g.dh, g.kH);
+        // One problem per residue, or all residues as columns of one: whichever is less work in 32-column tiles.  A launch
+        // and the repacking of its filters (10 us, at the rates that such problems reach) count as work.  (64 -> 256 channels,
+        // 16 x 16, stride 16 on 64 x 64 x 16, forward and pullback in bf16: 849 us with 64 launches, 148 with one.)
+        auto cols = [](double n) { return std::ceil(n / 32.0) * 32.0; };
+        const double per_launch = (sizeof(T) == 2 ? 1.5e9 : 3e8) / ((double)g.N * Cp);
+        double apart = std::ceil((double)rw.size() * rh.size() / cany::MAX_SUBS - 1.0) * per_launch, together = 1e30, rows = 0.0;
         for (const Residue& a : rw)
-            for (const Residue& b : rh) apart += (double)a.count * b.count * a.taps * b.taps * cols(g.Cin_g);
-        auto unite = [](const std::vector<Residue>& v, Residue& u) {
-            u = Residue{0, 1 << 30, 1 << 30, 1, 0, 0};
-            int q1 = -(1 << 30), s1 = -(1 << 30);
-            for (const Residue& z : v) {
-                if (z.count > 0) { u.q0 = std::min(u.q0, z.q0); q1 = std::max(q1, z.q0 + z.count - 1); }
-                if (z.taps > 0) { u.s0 = std::min(u.s0, z.s0); s1 = std::max(s1, z.s0 + (z.taps - 1) * z.sstep); }
-            }
-            u.count = q1 - u.q0 + 1;
-            u.taps = s1 - u.s0 + 1;
+            for (const Residue& b : rh) { apart += (double)a.count * b.count * a.taps * b.taps * cols(g.Cin_g); rows += (double)a.count * b.count; }
+        auto unite = [](int L, int pad, int stride, const std::vector<Residue>& v) {      // dilation 1: every residue starts at shift 0
+            Residue u{0, (L - 1 + pad) / stride - pad / stride + 1, pad / stride, 0, 1, 0};
+            for (const Residue& z : v) u.taps = std::max(u.taps, z.taps);
+            return u;
         };
-        Residue uw, uh;
-        if (R > 1 && g.dw == 1 && g.dh == 1) {
-            unite(rw, uw);
-            unite(rh, uh);
-            together = (double)uw.count * uh.count * uw.taps * uh.taps * cols(R * g.Cin_g);
+        Residue uw{}, uh{};
+        if (R > 1 && R * g.Cin_g <= 65536 && g.dw == 1 && g.dh == 1) {
+            uw = unite(g.W, g.pw, g.sw, rw);
+            uh = unite(g.H, g.ph, g.sh, rh);
+            together = (double)uw.count * uh.count * uw.taps * uh.taps * cols((double)R * g.Cin_g);
         }
         if (together < apart) {
             merged = 1;
             res_w = g.sw;
-            Ncols = R * g.Cin_g;
-            add(uw, uw.count, uh, uh.count, g.N, uw.q0 - uw.s0, -1, uw.taps, uh.q0 - uh.s0, -1, uh.taps, g.sw * uw.q0 - g.pw, g.sh * uh.q0 - g.ph, 0, 0);
+            Ncols = (int)R * g.Cin_g;
+            add(uw, uw.count, uh, uh.count, g.N, uw.q0, -1, uw.taps, uh.q0, -1, uh.taps, g.sw * uw.q0 - g.pw, g.sh * uh.q0 - g.ph);
             return;
         }
-        for (int b = 0; b < g.sh; ++b)
-            for (int a = 0; a < g.sw; ++a)
-                add(rw[a], rw[a].count, rh[b], rh[b].count, g.N, rw[a].q0 - rw[a].s0, -rw[a].sstep, rw[a].taps, rh[b].q0 - rh[b].s0, -rh[b].sstep,
-                    rh[b].taps, g.sw * rw[a].q0 + a - g.pw, g.sh * rh[b].q0 + b - g.ph, a, b);
+        zero_first = rows < (double)g.W * g.H;
+        for (const Residue& b : rh)
+            for (const Residue& a : rw)
+                add(a, a.count, b, b.count, g.N, a.q0 - a.s0, -a.sstep, a.taps, b.q0 - b.s0, -b.sstep, b.taps, g.sw * a.q0 + a.r - g.pw,
+                    g.sh * b.q0 + b.r - g.ph);
     }
     PackSubs pack(const ConvGeom& g, bool dgrad, int grp, size_t launch) const {
         PackSubs p;
@@ -669,11 +686,27 @@ static int to_cwhn_padded(hipStream_t s, const T* in, T* out, int P, int Cg, int
     return pad_and_pack<T>(s, in, out, P, Cg, groups, N, zeros, nullptr, nullptr, g, nullptr);
 }
 
+template <typename T>
+__global__ __launch_bounds__(256) void clear_kernel(T* out, int64_t n) {
+    for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (int64_t)gridDim.x * 256) out[i] = T(0);
+}
+template <typename T>
+static int clear_elements(hipStream_t s, T* out, int64_t n) {
+    if ((reinterpret_cast<uintptr_t>(out) & 3u) == 0) return luxhip_fill_zero(out, (size_t)n * sizeof(T), s);
+    clear_kernel<T><<<(unsigned)std::min<int64_t>(ceil_div(n, 256), 4096), 256, 0, s>>>(out, n);
+    LUX_CHECK_LAUNCH();
+    return LUXHIP_OK;
+}
+
 // fprop / dgrad of one problem through conv_any.h.  src: padded channel-contiguous activations; wm: workspace for the packed
 // filter of one group; packed: group 0, launch 0 of the filter is already there.  ws_front: bytes of the workspace in use.
 template <typename T>
 static int run_conv_any(hipStream_t s, const ConvGeom& g, bool dgrad, const AnyPlan<T>& plan, const T* src, const T* w, T* wm, bool packed, const T* bias,
                         T* out, T* pre, int act, size_t ws_front) {
+    if (plan.zero_first) {
+        const int rc = clear_elements<T>(s, out, (int64_t)g.W * g.H * g.Cin * g.N);
+        if (rc != LUXHIP_OK) return rc;
+    }
     for (int grp = 0; grp < g.groups; ++grp)
         for (size_t li = 0; li < plan.launches.size(); ++li) {
             const typename AnyPlan<T>::Launch& l = plan.launches[li];

@@ -7,7 +7,7 @@ import numpy as np
 import pytest
 
 from oracle import luxlib_oracle as O
-from tests.util import assert_close, dev, f64, host_inputs, stable_seed
+from tests.util import assert_close, dev, f64, host_inputs, kernels_of, stable_seed
 
 pytestmark = pytest.mark.gpu
 
@@ -23,6 +23,10 @@ CASES = [
     ((6, 6, 200, 1), (5, 5, 200, 24), 1, 2, 1, 1, False),            # few rows, 5000 k: slices
     ((23, 9, 61, 2), (3, 3, 61, 130), 1, (0, 1, 1, 0), 1, 1, True),  # more than 128 columns, ragged in everything
     ((5, 3, 8, 2), (3, 3, 8, 8), 4, 2, 1, 1, False),                 # stride beyond the filter
+    ((16, 15, 32, 2), (4, 5, 32, 24), (4, 5), 0, 1, 1, False),       # as many taps as residues, whole column tiles: one problem
+    ((33, 34, 32, 2), (1, 1, 32, 24), 9, 0, 1, 1, False),            # one residue of 81 has taps
+    ((20, 19, 33, 1), (3, 2, 33, 8), (7, 6), (2, 0, 1, 3), (2, 3), 1, True),   # 6 of 42, dilated; an odd number of bf16 elements
+    ((6, 5, 4, 2), (2, 2, 2, 6), 1000, 0, 1, 2, False),              # stride far beyond the input
 ]
 
 
@@ -49,6 +53,20 @@ def test_conv_any(gpu, dtype, case):
     np.testing.assert_array_equal(fx.to_numpy(), gx.to_numpy())
     np.testing.assert_array_equal(fw.to_numpy(), gw.to_numpy())
     assert_close(fb.to_numpy(), f64(dy).sum(axis=(0, 1, 3)), dtype, tag + " db")
+
+
+@pytest.mark.parametrize("xs,ws,stride,dil,launches", [
+    ((64, 64, 32, 1), (8, 8, 32, 16), 8, 1, 1),              # residues as columns
+    ((64, 64, 32, 1), (1, 1, 32, 16), 32, 1, 1),             # one residue has taps, the rest is cleared
+    ((64, 64, 8, 1), (3, 3, 8, 8), 4, 2, 1),                 # four residues of sixteen have taps
+    ((40, 40, 8, 1), (3, 3, 8, 8), 5, 2, 3),                 # nine of twenty-five
+])
+def test_input_gradient_of_a_large_stride_takes_few_launches(gpu, xs, ws, stride, dil, launches):
+    gd = gpu.DenseConvDims(xs, ws, stride=stride, dilation=dil)
+    rng = np.random.default_rng(stable_seed("launches", xs, ws))
+    dy, w = (dev(gpu, rng.normal(size=s).astype(np.float32), "f32") for s in (gd.y_shape, ws))
+    count = kernels_of(gpu, lambda: gpu.conv_data_grad(dy, w, gd))
+    assert count["conv_dgrad_kernel<f32>"] == launches, count
 
 
 @pytest.mark.parametrize("dtype", ["f32", "bf16"])

@@ -81,7 +81,7 @@ def stable_seed(*parts):
 
 
 def kernels_of(gpu, f):
-    """Names of the kernels that f launches."""
+    """The kernels that f launches, with their number."""
     import ctypes
     import json
     buf = ctypes.create_string_buffer(1 << 16)
@@ -91,4 +91,4 @@ def kernels_of(gpu, f):
         gpu._lib.call("luxhip_profile_report", buf, len(buf))
     finally:
         gpu._lib.call("luxhip_profile_enable", 0)
-    return {k["kernel"] for k in json.loads(buf.value.decode())}
+    return {k["kernel"]: k["count"] for k in json.loads(buf.value.decode())}
