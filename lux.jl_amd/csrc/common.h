@@ -49,6 +49,9 @@ struct Workspace {
 };
 constexpr size_t kWorkspaceZeroBytes = 256;
 int get_workspace(hipStream_t s, size_t bytes, Workspace* out);
+// False where get_workspace would refuse: `s` records a graph and its workspace is smaller.  A kernel that only gains from
+// scratch memory (the slices of a contraction) goes without it then.
+bool workspace_holds(hipStream_t s, size_t bytes);
 // True while `s` records into a HIP graph.  Kernels whose arguments carry the workspace epoch (the
 // resident batchnorm kernels, the split groupnorm pullback) would find their own tagged words again
 // on every replay of the graph, so the operators take their other code paths while a stream captures.

@@ -583,6 +583,15 @@ struct AnyPlan {
     int Ncols = 0, Cch = 0, res_w = 0, merged = 0, Cp = 0;
     bool zero_first = false;                                 // some positions of dx belong to no sub-problem: clear it before
     int64_t wm_elems = 0;                                    // packed filter of one group
+    bool slices = true;                                      // contractions may be cut (workspace for the partial sums)
+    // Memory for the slices of any launch: what a call reserves behind its `front` bytes, unless the stream is recording and
+    // its workspace has no room for them (then the contractions stay whole)
+    size_t reserve(hipStream_t s, size_t front) {
+        size_t most = 0;
+        for (Launch& l : launches) most = std::max(most, cany::choose_any<T>(l.sub, l.n, Ncols, true).bytes);
+        slices = workspace_holds(s, front + most);
+        return front + (slices ? most : 0);
+    }
     void add(const Residue& rw, int RA, const Residue& rh, int RB, int N, int w0, int wstep, int TW, int h0, int hstep, int TH, int ow0, int oh0) {
         if (RA <= 0 || RB <= 0) return;
         if (launches.empty() || launches.back().n == cany::MAX_SUBS) { launches.emplace_back(); launches.back().n = 0; }
@@ -726,7 +735,7 @@ static int run_conv_any(hipStream_t s, const ConvGeom& g, bool dgrad, const AnyP
             a.col_off = grp * plan.Cch; a.act = act; a.subs = l.n;
             a.divCp = FastDiv((uint32_t)plan.Cp); a.divCch = FastDiv((uint32_t)plan.Cch);
             for (int i = 0; i < l.n; ++i) a.sub[i] = l.sub[i];
-            const int rc = cany::launch_any<T>(s, a, ws_front, dgrad);
+            const int rc = cany::launch_any<T>(s, a, ws_front, dgrad, plan.slices);
             if (rc != LUXHIP_OK) return rc;
         }
     return LUXHIP_OK;
@@ -951,13 +960,13 @@ template <typename T>
 static int conv_fwd_t(hipStream_t s, int act, const ConvGeom& g, const T* x, const T* w, const T* bias, T* y, T* pre,
                       T* xt_keep) {
     const bool any = !tap_shape<T>(g, false);
-    const AnyPlan<T> plan(g, false);
+    AnyPlan<T> plan(g, false);
     // xt_keep: caller's buffer of x's size that keeps the channel-contiguous copy of x for the pullback
     const bool keep = kept_usable<T>(g, xt_keep);
     const size_t xb = keep ? 0 : xt_bytes<T>(g), wb = filter_bytes<T>(g, any, plan);
     Workspace ws;
     // the slices of conv_any.h take memory behind these; reserve it here, where no pointer into the workspace is live yet
-    int rc = get_workspace(s, xb + wb + (any ? cany::most_partial_bytes() : 0), &ws);
+    int rc = get_workspace(s, any ? plan.reserve(s, xb + wb) : xb + wb, &ws);
     if (rc != LUXHIP_OK) return rc;
     T* xT = keep ? xt_keep : reinterpret_cast<T*>(ws.data);
     T* wF = reinterpret_cast<T*>(ws.data + xb);
@@ -996,10 +1005,10 @@ static int dy_transpose_and_pack(hipStream_t s, const ConvGeom& g, bool any, con
 template <typename T>
 static int conv_bwd_data_t(hipStream_t s, const ConvGeom& g, const T* dy, const T* w, T* dx) {
     const bool any = !tap_shape<T>(g, true);
-    const AnyPlan<T> plan(g, true);
+    AnyPlan<T> plan(g, true);
     const size_t yb = dyt_bytes<T>(g), wb = filter_bytes<T>(g, any, plan);
     Workspace ws;
-    int rc = get_workspace(s, yb + wb + (any ? cany::most_partial_bytes() : 0), &ws);
+    int rc = get_workspace(s, any ? plan.reserve(s, yb + wb) : yb + wb, &ws);
     if (rc != LUXHIP_OK) return rc;
     T* dyT = reinterpret_cast<T*>(ws.data);
     T* wD = reinterpret_cast<T*>(ws.data + yb);
@@ -1027,7 +1036,7 @@ template <typename T>
 static int fused_conv_bwd_t(hipStream_t s, int dtype, int act, const ConvGeom& g, const T* delta, const T* y,
                             const T* pre, const T* x, const T* w, T* dz, T* dw, T* dx, T* dbias, const T* xt_kept) {
     const bool any = !tap_shape<T>(g, true), kept = kept_usable<T>(g, xt_kept);
-    const AnyPlan<T> plan(g, true);
+    AnyPlan<T> plan(g, true);
     const size_t xb = kept ? 0 : xt_bytes<T>(g), yb = dyt_bytes<T>(g), wb = filter_bytes<T>(g, any, plan), pb = wgrad_partial_bytes<T>(g);
     // bf16: dz, its channel-contiguous copy and the bias gradient in one pass, when both a pass over delta and a
     // transposing copy would run
@@ -1039,7 +1048,7 @@ static int fused_conv_bwd_t(hipStream_t s, int dtype, int act, const ConvGeom& g
     // reserve everything up front: the bias-gradient pass below uses the start of the same
     // workspace, and the buffer must not be reallocated while pointers into it are live
     Workspace ws;
-    int rc = get_workspace(s, xb + yb + wb + pb + bb + (any ? cany::most_partial_bytes() : 0), &ws);
+    int rc = get_workspace(s, any && dx != nullptr ? plan.reserve(s, xb + yb + wb + pb + bb) : xb + yb + wb + pb + bb, &ws);
     if (rc != LUXHIP_OK) return rc;
     const T* xT = kept ? xt_kept : reinterpret_cast<const T*>(ws.data);
     T* dzT = reinterpret_cast<T*>(ws.data + xb);

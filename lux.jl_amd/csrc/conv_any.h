@@ -336,10 +336,12 @@ __global__ __launch_bounds__(split::THREADS) void conv_any_wgrad_kernel(WgradArg
     });
 }
 
-// Most memory that the slices of a launch take (launch_any keeps to it)
-constexpr size_t most_partial_bytes() { return size_t(32) << 20; }
+// Tile and slices of a launch, and the bytes that its slices take (32 MiB at most)
+struct Choice { int tile, slices; size_t bytes; };
 template <typename T>
-int launch_any(hipStream_t s, Args<T>& a, size_t ws_front, bool dgrad);          // conv_any_*.hip
+Choice choose_any(Sub* sub, int subs, int Ncols, bool may_slice);                // conv_any_*.hip; fills in the tiling of sub[]
+template <typename T>
+int launch_any(hipStream_t s, Args<T>& a, size_t ws_front, bool dgrad, bool may_slice);
 template <typename T>
 int launch_any_wgrad(hipStream_t s, WgradArgs<T>& a, int slices, bool narrow);
 

@@ -28,55 +28,65 @@ int launch_shape(hipStream_t s, Args<T>& a, int blocks, bool dgrad) {
 }
 
 template <typename T>
-int launch_any(hipStream_t s, Args<T>& a, size_t ws_front, bool dgrad) {
+Choice choose_any(Sub* sub, int subs, int Ncols, bool may_slice) {
     constexpr int BK = GemmTraits<T>::BK;
+    constexpr size_t most_bytes = size_t(32) << 20;
     const int64_t cus = num_cus() > 0 ? num_cus() : 256;
     const Tile* tl = tiles<T>();
-    int best = 0, best_s = 1;
+    Choice best{0, 1, 0};
     double t_best = 1e30;
     int kmax = 0;
-    for (int i = 0; i < a.subs; ++i) kmax = std::max(kmax, a.sub[i].Kpad);
+    for (int i = 0; i < subs; ++i) kmax = std::max(kmax, sub[i].Kpad);
     for (int c = 0; c < 5; ++c) {
         int64_t nt = 0;
         double work = 0.0;                                           // tiles x k
-        for (int i = 0; i < a.subs; ++i) {
-            const int64_t t = ceil_div(a.sub[i].M, tl[c].m) * ceil_div(a.Ncols, tl[c].n);
+        for (int i = 0; i < subs; ++i) {
+            const int64_t t = ceil_div(sub[i].M, tl[c].m) * ceil_div(Ncols, tl[c].n);
             nt += t;
-            work += (double)t * (a.sub[i].Kpad + 100);
+            work += (double)t * (sub[i].Kpad + 100);
         }
         for (int sl = 1; sl <= 8; ++sl) {
-            if (sl > 1 && (kmax / sl < 2 * BK || nt > 16384 || (size_t)(nt * sl) * tl[c].m * tl[c].n * sizeof(float) > most_partial_bytes())) break;
+            if (sl > 1 && (!may_slice || kmax / sl < 2 * BK || nt > 16384 || (size_t)(nt * sl) * tl[c].m * tl[c].n * sizeof(float) > most_bytes)) break;
             const double k = (double)kmax / sl + 100;
             const double per_cu = nt * sl <= 4 * cus ? (double)ceil_div(nt * sl, cus) * k : work / cus;
             double t = std::max(tl[c].alone * k, tl[c].shared * per_cu);
             if (sl > 1) t += 1.5 + 0.5 * (tl[c].m * tl[c].n / 4096.0) * sl + (double)nt * sl * tl[c].m * tl[c].n * 8.0 / 5e6;
-            if (t < t_best) { t_best = t; best = c; best_s = sl; }
+            if (t < t_best) { t_best = t; best.tile = c; best.slices = sl; }
         }
     }
-    size_t bytes = 0;
+    for (int i = 0; i < subs; ++i) {
+        Sub& q = sub[i];
+        q.tiles_m = (int)ceil_div(q.M, tl[best.tile].m);
+        q.tiles_n = (int)ceil_div(Ncols, tl[best.tile].n);
+        q.kslice = (int)(ceil_div(ceil_div(q.Kpad, best.slices), BK) * BK);
+        q.slices = q.kslice > 0 ? (int)ceil_div(q.Kpad, q.kslice) : 1;
+        q.partial = (int64_t)best.bytes;
+        if (q.slices > 1) best.bytes += (size_t)q.tiles_m * q.tiles_n * q.slices * tl[best.tile].m * tl[best.tile].n * sizeof(float);
+    }
+    return best;
+}
+
+template <typename T>
+int launch_any(hipStream_t s, Args<T>& a, size_t ws_front, bool dgrad, bool may_slice) {
+    const Choice c = choose_any<T>(a.sub, a.subs, a.Ncols, may_slice);
     int blocks = 0, nt = 0;
     for (int i = 0; i < a.subs; ++i) {
         Sub& q = a.sub[i];
-        q.tiles_m = (int)ceil_div(q.M, tl[best].m);
-        q.tiles_n = (int)ceil_div(a.Ncols, tl[best].n);
-        q.kslice = (int)(ceil_div(ceil_div(q.Kpad, best_s), BK) * BK);
-        q.slices = q.kslice > 0 ? (int)ceil_div(q.Kpad, q.kslice) : 1;
         q.first_block = blocks;
         q.first_tile = nt;
-        q.partial = (int64_t)bytes;
         const int64_t t = (int64_t)q.tiles_m * q.tiles_n;
         LUX_UNSUPPORTED_IF(blocks + t * q.slices >= (int64_t(1) << 31), "conv: too many tiles");
         blocks += (int)(t * q.slices);
-        if (q.slices > 1) { bytes += (size_t)t * q.slices * tl[best].m * tl[best].n * sizeof(float); nt += (int)t; }
+        if (q.slices > 1) nt += (int)t;
     }
     if (blocks == 0) return LUXHIP_OK;
     Workspace ws;
-    const int rc = get_workspace(s, ws_front + bytes, &ws);
+    const int rc = get_workspace(s, ws_front + c.bytes, &ws);
     if (rc != LUXHIP_OK) return rc;
     a.partial = ws.data + ws_front;
     a.counters = ws.counters;
     a.zero = ws.zeros;
-    switch (best) {
+    switch (c.tile) {
         case 0: return launch_shape<T, 1, 1, 2, 2>(s, a, blocks, dgrad);
         case 1: return launch_shape<T, 2, 1, 2, 2>(s, a, blocks, dgrad);
         case 2: return launch_shape<T, 2, 2, 2, 2>(s, a, blocks, dgrad);

@@ -178,6 +178,7 @@ int launch(hipStream_t s, const DenseArgs<T>& d, size_t ws_front) {
     // (11008 x 4096: 18.6 us against 20.4 with two in bf16, 29.7 against 38.2 in fp32); at least two steps of k per wave
     int64_t slices = std::max<int64_t>(1, std::min<int64_t>(cus / blocks, d.K / (2 * KSTEP * WAVES)));
     if (blocks > (int64_t)kWorkspaceCounters) slices = 1;
+    if (slices > 1 && !workspace_holds(s, ws_front + (size_t)blocks * slices * NMAX * MT * sizeof(float))) slices = 1;
     a.kwave = (int)(ceil_div(ceil_div(d.K, slices * WAVES), KSTEP) * KSTEP);
     a.slices = (int)ceil_div(d.K, (int64_t)a.kwave * WAVES);
     a.partial = nullptr; a.counters = nullptr;

@@ -66,10 +66,12 @@ inline void place(Plan& p, const Workspace& ws, int first_counter) {
 template <typename T, int W, bool AK, bool BKM>
 int launch_cfg(hipStream_t s, DenseArgs<T>& a, int slices, size_t ws_front) {
     using B = Body<T, W, AK, BKM>;
-    Plan p = make_plan<T, W>(a, slices, &ws_front);
+    size_t bytes = ws_front;
+    Plan p = make_plan<T, W>(a, slices, &bytes);
+    if (p.slices > 1 && !workspace_holds(s, bytes)) p = make_plan<T, W>(a, 1, &bytes);
     if (p.slices > 1) {
         Workspace ws;
-        const int rc = get_workspace(s, ws_front, &ws);
+        const int rc = get_workspace(s, bytes, &ws);
         if (rc != LUXHIP_OK) return rc;
         place(p, ws, 0);
     }
@@ -129,6 +131,11 @@ bool launch_split_pair(hipStream_t s, DenseArgs<T>& a, DenseArgs<T>& b, int* rc)
     if (ca.w != 1 || cb.w != 1) return false;
     size_t front = 0;
     Plan pa = make_plan<T, 1>(a, ca.slices, &front), pb = make_plan<T, 1>(b, cb.slices, &front);
+    if (front > 0 && !workspace_holds(s, front)) {
+        front = 0;
+        pa = make_plan<T, 1>(a, 1, &front);
+        pb = make_plan<T, 1>(b, 1, &front);
+    }
     const int64_t na = (int64_t)a.tiles_m * a.tiles_n * pa.slices, nb = (int64_t)b.tiles_m * b.tiles_n * pb.slices;
     if (na > 2 * cus && nb > 2 * cus) return false;               // each fills the chip by itself
     // one counter for each tile of a product with slices, those of b behind those of a

@@ -240,6 +240,13 @@ int get_workspace(hipStream_t s, size_t bytes, Workspace* out) {
     return LUXHIP_OK;
 }
 
+bool workspace_holds(hipStream_t s, size_t bytes) {
+    if (!stream_capturing(s)) return true;
+    std::lock_guard<std::mutex> lk(g_mu);
+    const auto it = g_ws.find(s);
+    return it != g_ws.end() && it->second.base != nullptr && it->second.counters != nullptr && it->second.data_bytes >= bytes;
+}
+
 __global__ void fill_zero_kernel(uint32_t* p, size_t nwords) {
     size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
     const size_t stride = (size_t)gridDim.x * blockDim.x;

@@ -121,3 +121,67 @@ def test_a_training_step_replays_from_a_graph(gpu):
     finally:
         hip.hipGraphExecDestroy(graph_exec)
         hip.hipGraphDestroy(graph)
+
+
+@pytest.mark.parametrize("reserve", [0, 1])
+def test_products_on_a_stream_without_room_for_slices(gpu, reserve):
+    """Products that cut their contraction into slices keep it whole where the stream records and its workspace is too small
+    for the partial sums: dense products on a stream that has no workspace at all, a convolution on one that has the smallest
+    (8 MiB).  Small whole numbers, so every order of the sums gives the same bits."""
+    hip = _hip()
+    rng = np.random.default_rng(5)
+    ints = lambda *s: np.asfortranarray(rng.integers(-2, 3, size=s).astype(np.float32))
+    d = lambda a: gpu.DeviceArray.from_numpy(a)
+    stream = C.c_void_p()
+    gpu._lib.call("luxhip_stream_create", C.byref(stream))
+    if reserve:
+        gpu._lib.call("luxhip_reserve", stream, 1)
+    M, N, K = 130, 131, 2046
+    W, x, few, dz = ints(M, K), ints(K, N), ints(K, 3), ints(M, N)
+    cd = gpu.DenseConvDims((64, 64, 128, 1), (3, 3, 128, 128), padding=1)
+    cx, cw = ints(64, 64, 128, 1), ints(3, 3, 128, 128)
+    dW, dx_, dfew, ddz, dcx, dcw = map(d, (W, x, few, dz, cx, cw))
+    outs = {"tiled": (M, N), "few": (M, 3), "dw": (M, K), "dx": (K, N)}
+    if reserve:
+        outs.update(conv=cd.y_shape)
+
+    def run(s):
+        o = {k: gpu.DeviceArray(v, "f32") for k, v in outs.items()}
+        gpu._lib.call("luxhip_matmul", s, 0, 0, 0, M, N, K, dW.ptr, M, dx_.ptr, K, None, o["tiled"].ptr, M)
+        gpu._lib.call("luxhip_matmul", s, 0, 0, 0, M, 3, K, dW.ptr, M, dfew.ptr, K, None, o["few"].ptr, M)
+        gpu._lib.call("luxhip_fused_dense_bwd", s, 0, 0, M, K, N, ddz.ptr, None, None, dW.ptr, M, dx_.ptr, K, None, o["dw"].ptr,
+                      o["dx"].ptr, None)
+        if reserve:
+            gpu._lib.call("luxhip_conv_fwd", s, 0, 0, C.byref(cd._c), dcx.ptr, dcw.ptr, None, o["conv"].ptr, None, None)
+        return o
+
+    want = run(gpu.current_stream())                  # this stream has, or gets, the room
+    pool = run(gpu.current_stream())                  # ... and the pool the blocks that the recording takes
+    gpu.synchronize()
+    del pool
+    assert hip.hipStreamBeginCapture(stream, THREAD_LOCAL) == 0
+    graph = C.c_void_p()
+    try:
+        got = run(stream)
+    finally:
+        rc = hip.hipStreamEndCapture(stream, C.byref(graph))
+    assert rc == 0 and graph.value
+    graph_exec = C.c_void_p()
+    assert hip.hipGraphInstantiate(C.byref(graph_exec), graph, None, None, 0) == 0
+    try:
+        for _ in range(3):
+            for a in got.values():
+                gpu._lib.call("luxhip_fill_zero", a.ptr, a.size * 4, gpu.current_stream())
+            gpu.synchronize()
+            assert hip.hipGraphLaunch(graph_exec, stream) == 0
+            gpu._lib.call("luxhip_stream_synchronize", stream)
+            for k in outs:
+                np.testing.assert_array_equal(got[k].to_numpy(), want[k].to_numpy(), err_msg=k)
+    finally:
+        hip.hipGraphExecDestroy(graph_exec)
+        hip.hipGraphDestroy(graph)
+        gpu._lib.call("luxhip_stream_destroy", stream)
+    np.testing.assert_array_equal(want["tiled"].to_numpy(), W @ x)
+    np.testing.assert_array_equal(want["few"].to_numpy(), W @ few)
+    np.testing.assert_array_equal(want["dw"].to_numpy(), dz @ x.T)
+    np.testing.assert_array_equal(want["dx"].to_numpy(), W.T @ dz)
