@@ -132,7 +132,7 @@ __global__ __launch_bounds__(256) void whcn_to_cwhn_pack_kernel(const T* __restr
 }
 
 // Channel-contiguous copy with the channels of every group padded with zeros to Cp, for any number of positions and
-// channels: out (groups * Cp, P, N) from in (P, groups * Cg, N), 16-byte stores.  Tiles of 64 positions x 64 padded channels
+// channels: out (groups * Cp, P, N) from the first groups * Cg channels of in (P, Cin, N), 16-byte stores.  Tiles of 64 positions x 64 padded channels
 // go through LDS; the reads are one element per lane (64 consecutive positions of a channel per wave), since the rows of a
 // ragged plane start at any address.  `zeros` positions of zeros follow the last image.  Blocks behind the transform's
 // repack the filter.
@@ -143,28 +143,30 @@ struct PackSub {
 };
 struct PackSubs {
     PackSub sub[cany::MAX_SUBS];
-    int n, dgrad, Cp, Ncols, Cch, grp;
-    int64_t total;
+    int n, dgrad, Cp, Ncols, Cch;
+    int64_t per_group, wm_group, total;  // elements of a group in this launch and in all launches; in this launch over all groups
 };
 template <typename T>
 __device__ __forceinline__ void pack_sub_element(const T* __restrict__ w, T* __restrict__ out, const ConvGeom& g, const PackSubs& ps, int64_t idx) {
     if (idx >= ps.total) return;
+    const int grp = (int)(idx / ps.per_group);
+    idx -= grp * ps.per_group;
     PackSub q = ps.sub[0];
 #pragma unroll
     for (int i = 1; i < cany::MAX_SUBS; ++i)
         if (i < ps.n && idx >= ps.sub[i].first) q = ps.sub[i];
-    const int e = (int)(idx - q.first);
-    const int col = e / q.Kpad, k = e - col * q.Kpad;
+    const int64_t e = idx - q.first;
+    const int col = (int)(e / q.Kpad), k = (int)(e - (int64_t)col * q.Kpad);
     T v = T(0);
     const int t = k / ps.Cp, c = k - t * ps.Cp;
     const int th = t / q.TW, tw = t - th * q.TW;
     if (k < q.K && c < (ps.dgrad ? g.Cout_g : g.Cin_g)) {
-        int ci = c, co = ps.grp * g.Cout_g + col, ka = tw, kb = th;
+        int ci = c, co = grp * g.Cout_g + col, ka = tw, kb = th;
         bool tap = true;
         if (ps.dgrad) {
             const int res = q.merged_w > 0 ? col / ps.Cch : 0;
             ci = col - res * ps.Cch;
-            co = ps.grp * g.Cout_g + c;
+            co = grp * g.Cout_g + c;
             const int rh = q.merged_w > 0 ? res / q.merged_w : q.rh, rw = q.merged_w > 0 ? res % q.merged_w : q.rw;
             const int nw = (q.s0w + tw * q.stw) * g.sw + rw, nh = (q.s0h + th * q.sth) * g.sh + rh;
             ka = nw / g.dw;
@@ -176,10 +178,10 @@ __device__ __forceinline__ void pack_sub_element(const T* __restrict__ w, T* __r
             v = w[a + g.kW * (b + g.kH * (ci + g.Cin_g * co))];
         }
     }
-    out[q.wm + e] = v;
+    out[grp * ps.wm_group + q.wm + e] = v;
 }
 template <typename T>
-__global__ __launch_bounds__(256) void pad_to_cwhn_pack_kernel(const T* __restrict__ in, T* __restrict__ out, int P, int Cg, int Cp, int groups,
+__global__ __launch_bounds__(256) void pad_to_cwhn_pack_kernel(const T* __restrict__ in, T* __restrict__ out, int P, int Cin, int Cg, int Cp, int groups,
                                                                int N, int zeros, int tiles_p, int tiles_c, int blocks, const T* __restrict__ w,
                                                                T* __restrict__ wout, ConvGeom g, PackSubs ps) {
     constexpr int V = 16 / (int)sizeof(T), PITCH = 64 + 4 / (int)sizeof(T);
@@ -197,7 +199,7 @@ __global__ __launch_bounds__(256) void pad_to_cwhn_pack_kernel(const T* __restri
         for (int c = 0; c < V; ++c) e[c] = T(0);
         if (pos < (int64_t)P * N) {
             const int n = (int)(pos / P);
-            const T* src = in + (int64_t)n * P * groups * Cg + (pos - (int64_t)n * P);
+            const T* src = in + (int64_t)n * P * Cin + (pos - (int64_t)n * P);
 #pragma unroll
             for (int c = 0; c < V; ++c)
                 if (c < Cg) e[c] = src[(int64_t)c * P];     // one group: Cp == V
@@ -209,7 +211,7 @@ __global__ __launch_bounds__(256) void pad_to_cwhn_pack_kernel(const T* __restri
     const int c0 = (rest / tiles_p) * 64, p0 = (rest % tiles_p) * 64;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     if (n < N) {
-        const T* src = in + (int64_t)n * P * groups * Cg;
+        const T* src = in + (int64_t)n * P * Cin;
         T v[16];
 #pragma unroll
         for (int j = 0; j < 16; ++j) {
@@ -447,7 +449,7 @@ static int pack_filter(hipStream_t s, const T* w, T* out, const ConvGeom& g, int
 }
 
 template <typename T>
-static int to_cwhn_padded(hipStream_t s, const T* in, T* out, int P, int Cg, int groups, int N, int zeros, const ConvGeom& g);
+static int to_cwhn_padded(hipStream_t s, const T* in, T* out, int P, int Cin, int Cg, int groups, int N, int zeros, const ConvGeom& g);
 
 // transpose_to_cwhn(in -> out) and pack_filter(w -> wout) in one launch where the 16-byte transform applies
 template <typename T>
@@ -458,7 +460,7 @@ static int transpose_and_pack(hipStream_t s, const T* in, T* out, int P, int C, 
     const int64_t pack_blocks = ceil_div((int64_t)g.kW * g.kH * g.Cin_g * g.Cout, 256);
     const int64_t gz = N + ceil_div(pack_blocks, gx * gy);
     if (!vec || N < 1 || gy > 65535 || gz > 65535) {
-        int rc = to_cwhn_padded<T>(s, in, out, P, C / g.groups, g.groups, N, 0, g);
+        int rc = to_cwhn_padded<T>(s, in, out, P, C, C / g.groups, g.groups, N, 0, g);
         if (rc != LUXHIP_OK) return rc;
         return pack_filter<T>(s, w, wout, g, for_dgrad);
     }
@@ -586,9 +588,11 @@ struct AnyPlan {
     bool slices = true;                                      // contractions may be cut (workspace for the partial sums)
     // Memory for the slices of any launch: what a call reserves behind its `front` bytes, unless the stream is recording and
     // its workspace has no room for them (then the contractions stay whole)
-    size_t reserve(hipStream_t s, size_t front) {
+    size_t reserve(hipStream_t s, size_t front, int at_a_time, int groups) {
         size_t most = 0;
-        for (Launch& l : launches) most = std::max(most, cany::choose_any<T>(l.sub, l.n, Ncols, true).bytes);
+        for (Launch& l : launches)
+            for (int n : {at_a_time, groups % at_a_time})    // the last of them may be fewer
+                if (n > 0) most = std::max(most, cany::choose_any<T>(l.sub, l.n, Ncols, n, true).bytes * n);
         slices = workspace_holds(s, front + most);
         return front + (slices ? most : 0);
     }
@@ -654,22 +658,23 @@ struct AnyPlan {
                 add(a, a.count, b, b.count, g.N, a.q0 - a.s0, -a.sstep, a.taps, b.q0 - b.s0, -b.sstep, b.taps, g.sw * a.q0 + a.r - g.pw,
                     g.sh * b.q0 + b.r - g.ph);
     }
-    PackSubs pack(const ConvGeom& g, bool dgrad, int grp, size_t launch) const {
+    PackSubs pack(const ConvGeom& g, bool dgrad, size_t launch) const {
         PackSubs p;
-        p.n = launches[launch].n; p.dgrad = dgrad; p.Cp = Cp; p.Ncols = Ncols; p.Cch = Cch; p.grp = grp; p.total = 0;
+        p.n = launches[launch].n; p.dgrad = dgrad; p.Cp = Cp; p.Ncols = Ncols; p.Cch = Cch; p.wm_group = wm_elems; p.per_group = 0;
         for (int i = 0; i < p.n; ++i) {
             p.sub[i] = launches[launch].pack[i];
-            p.sub[i].first = p.total;
-            p.total += (int64_t)Ncols * p.sub[i].Kpad;
+            p.sub[i].first = p.per_group;
+            p.per_group += (int64_t)Ncols * p.sub[i].Kpad;
         }
+        p.total = p.per_group * g.groups;
         return p;
     }
 };
 
-// Padded channel-contiguous copy of `in` (if out != NULL) and the packed filter of group 0, launch 0 (if wout != NULL), in one
-// launch
+// Padded channel-contiguous copy of the first `groups` groups of `in`, which has Cin channels (if out != NULL), and the packed
+// filter of all groups of a launch (if wout != NULL), in one launch
 template <typename T>
-static int pad_and_pack(hipStream_t s, const T* in, T* out, int P, int Cg, int groups, int N, int zeros, const T* w, T* wout, const ConvGeom& g,
+static int pad_and_pack(hipStream_t s, const T* in, T* out, int P, int Cin, int Cg, int groups, int N, int zeros, const T* w, T* wout, const ConvGeom& g,
                         const PackSubs* ps) {
     constexpr int V = GemmTraits<T>::VEC;
     const int Cp = padded<T>(Cg), Ct = groups * Cp;
@@ -679,20 +684,37 @@ static int pad_and_pack(hipStream_t s, const T* in, T* out, int P, int Cg, int g
     const int tiles_p = (int)ceil_div(std::max(P, zeros), 64), tiles_c = (int)ceil_div(Ct, 64);
     if (out != nullptr) blocks = Ct == V ? ceil_div((int64_t)P * N + zeros, 256) : (int64_t)tiles_p * tiles_c * (N + (zeros > 0));
     const int64_t pack = wout != nullptr ? ceil_div(ps->total, 256) : 0;
-    LUX_UNSUPPORTED_IF(blocks + pack >= (int64_t(1) << 31), "conv: tensor too large for the layout transform");
+    LUX_UNSUPPORTED_IF(blocks + pack >= (int64_t(1) << 24), "conv: tensor too large for the layout transform");
     if (blocks + pack == 0) return LUXHIP_OK;
     ProfScope prof("whcn_to_cwhn_kernel", s);
-    pad_to_cwhn_pack_kernel<T><<<(unsigned)(blocks + pack), 256, 0, s>>>(in, out, P, Cg, Cp, groups, N, zeros, tiles_p, tiles_c, (int)blocks, w, wout, g,
-                                                                         wout != nullptr ? *ps : none);
+    pad_to_cwhn_pack_kernel<T><<<(unsigned)(blocks + pack), 256, 0, s>>>(in, out, P, Cin, Cg, Cp, groups, N, zeros, tiles_p, tiles_c, (int)blocks, w, wout,
+                                                                         g, wout != nullptr ? *ps : none);
     LUX_CHECK_LAUNCH();
     return LUXHIP_OK;
 }
 
 // Channel-contiguous copy of a tensor in the padded layout (the plain layout where no padding is needed)
 template <typename T>
-static int to_cwhn_padded(hipStream_t s, const T* in, T* out, int P, int Cg, int groups, int N, int zeros, const ConvGeom& g) {
-    if (padded<T>(Cg) == Cg && zeros == 0 && P % GemmTraits<T>::VEC == 0 && aligned16(in)) return transpose_to_cwhn<T>(s, in, out, P, Cg * groups, N);
-    return pad_and_pack<T>(s, in, out, P, Cg, groups, N, zeros, nullptr, nullptr, g, nullptr);
+static int to_cwhn_padded(hipStream_t s, const T* in, T* out, int P, int Cin, int Cg, int groups, int N, int zeros, const ConvGeom& g) {
+    if (padded<T>(Cg) == Cg && Cin == Cg * groups && zeros == 0 && P % GemmTraits<T>::VEC == 0 && aligned16(in))
+        return transpose_to_cwhn<T>(s, in, out, P, Cin, N);
+    return pad_and_pack<T>(s, in, out, P, Cin, Cg, groups, N, zeros, nullptr, nullptr, g, nullptr);
+}
+
+// Groups [first, first + n) of a convolution.  Where channels are padded, the copies hold as many groups at a time as take no
+// more memory than the tensor itself or 64 MiB: a depthwise bf16 layer would need eight times the tensor for all of them.
+struct Groups { int first, n; };
+template <typename T>
+static int groups_at_a_time(const ConvGeom& g, bool x, bool y) {
+    int64_t n = g.groups;
+    auto fit = [&](int64_t positions, int Cg) {
+        if (padded<T>(Cg) == Cg) return;
+        const int64_t room = std::max<int64_t>(int64_t(64) << 20, positions * Cg * g.groups * (int64_t)sizeof(T));
+        n = std::min(n, std::max<int64_t>(1, room / (positions * padded<T>(Cg) * (int64_t)sizeof(T))));
+    };
+    if (x) fit((int64_t)g.W * g.H * g.N, g.Cin_g);
+    if (y) fit((int64_t)g.OW * g.OH * g.N, g.Cout_g);
+    return (int)std::min<int64_t>(n, 32768);                 // (a dimension of the grid)
 }
 
 template <typename T>
@@ -707,37 +729,38 @@ static int clear_elements(hipStream_t s, T* out, int64_t n) {
     return LUXHIP_OK;
 }
 
-// fprop / dgrad of one problem through conv_any.h.  src: padded channel-contiguous activations; wm: workspace for the packed
-// filter of one group; packed: group 0, launch 0 of the filter is already there.  ws_front: bytes of the workspace in use.
+// fprop / dgrad of the groups `gr` through conv_any.h.  src: padded channel-contiguous activations, of these groups alone
+// where channels are padded, else of all; wm: workspace for the packed filter of all groups; packed: launch 0 of the filter is
+// already there.  ws_front: bytes of the workspace in use.
 template <typename T>
-static int run_conv_any(hipStream_t s, const ConvGeom& g, bool dgrad, const AnyPlan<T>& plan, const T* src, const T* w, T* wm, bool packed, const T* bias,
-                        T* out, T* pre, int act, size_t ws_front) {
-    if (plan.zero_first) {
+static int run_conv_any(hipStream_t s, const ConvGeom& g, bool dgrad, const AnyPlan<T>& plan, Groups gr, const T* src, const T* w, T* wm, bool packed,
+                        const T* bias, T* out, T* pre, int act, size_t ws_front) {
+    const bool alone = plan.Cp != (dgrad ? g.Cout_g : g.Cin_g);
+    if (plan.zero_first && gr.first == 0) {
         const int rc = clear_elements<T>(s, out, (int64_t)g.W * g.H * g.Cin * g.N);
         if (rc != LUXHIP_OK) return rc;
     }
-    for (int grp = 0; grp < g.groups; ++grp)
-        for (size_t li = 0; li < plan.launches.size(); ++li) {
-            const typename AnyPlan<T>::Launch& l = plan.launches[li];
-            if (!packed || grp > 0 || li > 0) {
-                const PackSubs ps = plan.pack(g, dgrad, grp, li);
-                const int rc = pad_and_pack<T>(s, nullptr, nullptr, 0, 1, 1, 0, 0, w, wm, g, &ps);
-                if (rc != LUXHIP_OK) return rc;
-            }
-            cany::Args<T> a;
-            a.src = src + (size_t)grp * plan.Cp;
-            a.wm = wm; a.bias = bias; a.out = out; a.pre = pre;
-            a.Ctot = g.groups * plan.Cp; a.Cp = plan.Cp;
-            if (!dgrad) { a.SP = g.W; a.SQ = g.H; a.ss_w = g.sw; a.ss_h = g.sh; a.P = g.OW; a.Q = g.OH; a.os_w = a.os_h = 1; a.Ctot_out = g.Cout; }
-            else { a.SP = g.OW; a.SQ = g.OH; a.ss_w = a.ss_h = 1; a.P = g.W; a.Q = g.H; a.os_w = g.sw; a.os_h = g.sh; a.Ctot_out = g.Cin; }
-            a.PQ = a.P * a.Q;
-            a.Ncols = plan.Ncols; a.Cch = plan.Cch; a.res_w = std::max(plan.res_w, 1); a.merged = plan.merged; a.kW = g.kW; a.kH = g.kH;
-            a.col_off = grp * plan.Cch; a.act = act; a.subs = l.n;
-            a.divCp = FastDiv((uint32_t)plan.Cp); a.divCch = FastDiv((uint32_t)plan.Cch);
-            for (int i = 0; i < l.n; ++i) a.sub[i] = l.sub[i];
-            const int rc = cany::launch_any<T>(s, a, ws_front, dgrad, plan.slices);
+    for (size_t li = 0; li < plan.launches.size(); ++li) {
+        const typename AnyPlan<T>::Launch& l = plan.launches[li];
+        if (gr.first == 0 && !(packed && li == 0)) {
+            const PackSubs ps = plan.pack(g, dgrad, li);
+            const int rc = pad_and_pack<T>(s, nullptr, nullptr, 0, 1, 1, 1, 0, 0, w, wm, g, &ps);
             if (rc != LUXHIP_OK) return rc;
         }
+        cany::Args<T> a;
+        a.src = src + (alone ? 0 : (size_t)gr.first * plan.Cp);
+        a.wm = wm + gr.first * plan.wm_elems; a.wm_group = plan.wm_elems; a.bias = bias; a.out = out; a.pre = pre;
+        a.Ctot = (alone ? gr.n : g.groups) * plan.Cp; a.Cp = plan.Cp;
+        if (!dgrad) { a.SP = g.W; a.SQ = g.H; a.ss_w = g.sw; a.ss_h = g.sh; a.P = g.OW; a.Q = g.OH; a.os_w = a.os_h = 1; a.Ctot_out = g.Cout; }
+        else { a.SP = g.OW; a.SQ = g.OH; a.ss_w = a.ss_h = 1; a.P = g.W; a.Q = g.H; a.os_w = g.sw; a.os_h = g.sh; a.Ctot_out = g.Cin; }
+        a.PQ = a.P * a.Q;
+        a.Ncols = plan.Ncols; a.Cch = plan.Cch; a.res_w = std::max(plan.res_w, 1); a.merged = plan.merged; a.kW = g.kW; a.kH = g.kH;
+        a.col_off = gr.first * plan.Cch; a.act = act; a.subs = l.n;
+        a.divCp = FastDiv((uint32_t)plan.Cp); a.divCch = FastDiv((uint32_t)plan.Cch);
+        for (int i = 0; i < l.n; ++i) a.sub[i] = l.sub[i];
+        const int rc = cany::launch_any<T>(s, a, gr.n, ws_front, dgrad, plan.slices);
+        if (rc != LUXHIP_OK) return rc;
+    }
     return LUXHIP_OK;
 }
 
@@ -854,9 +877,10 @@ static size_t wgrad_partial_bytes(const ConvGeom& g) {
 }
 
 // dy: WHCN cotangent (used by the window and the direct bf16 kernels); dyT: its channel-contiguous copy with padded channels,
-// followed by BK positions of zeros where there are fewer than BK positions in all (used by the general kernel).
+// followed by BK positions of zeros where there are fewer than BK positions in all (used by the general kernel).  Where
+// channels are padded, xT / dyT hold the groups `gr` alone, else all of them.
 template <typename T>
-static int run_wgrad(hipStream_t s, const ConvGeom& g, const T* xT, const T* dy, const T* dyT, float* partial, T* dw,
+static int run_wgrad(hipStream_t s, const ConvGeom& g, Groups gr, const T* xT, const T* dy, const T* dyT, float* partial, T* dw,
                      const void* zeros, const BiasPartials* bias = nullptr) {
     const bool direct = wgrad_direct_ok<T>(g, xT, dy);
     const bool window = wgrad_window_shape<T>(g) && aligned16(xT) && aligned16(dy) && aligned16(partial);
@@ -865,7 +889,7 @@ static int run_wgrad(hipStream_t s, const ConvGeom& g, const T* xT, const T* dy,
     if (rc != LUXHIP_OK) return rc;
     int slices = plan.slices;
     const int kslice = plan.kslice;
-    for (int grp = 0; grp < g.groups; ++grp) {
+    for (int grp = gr.first; grp < gr.first + gr.n; ++grp) {
         const int Mrows = plan.Mrows;
         if (window) {
             if constexpr (sizeof(T) == 2) {
@@ -900,8 +924,9 @@ static int run_wgrad(hipStream_t s, const ConvGeom& g, const T* xT, const T* dy,
         } else {
             cany::WgradArgs<T> a;
             const int Cp = padded<T>(g.Cin_g);
-            a.src = xT + (size_t)grp * Cp; a.Ctot = g.groups * Cp; a.Cp = Cp; a.Mrows = Mrows;
-            a.dyT = dyT + (size_t)grp * plan.Ncols; a.Ytot = g.groups * plan.Ncols; a.Ncols = plan.Ncols;
+            const bool x_alone = Cp != g.Cin_g, y_alone = plan.Ncols != g.Cout_g;
+            a.src = xT + (size_t)(x_alone ? grp - gr.first : grp) * Cp; a.Ctot = (x_alone ? gr.n : g.groups) * Cp; a.Cp = Cp; a.Mrows = Mrows;
+            a.dyT = dyT + (size_t)(y_alone ? grp - gr.first : grp) * plan.Ncols; a.Ytot = (y_alone ? gr.n : g.groups) * plan.Ncols; a.Ncols = plan.Ncols;
             a.zero = zeros;
             a.OW = g.OW; a.OWOH = g.OW * g.OH; a.SP = g.W; a.SQ = g.H;
             a.kW = g.kW; a.sw = g.sw; a.sh = g.sh; a.pw = g.pw; a.ph = g.ph; a.dw = g.dw; a.dh = g.dh;
@@ -933,26 +958,31 @@ static int dy_zeros(const ConvGeom& g) {
 }
 // Bytes of the padded channel-contiguous copies and of the packed filter (either form)
 template <typename T>
-static size_t xt_bytes(const ConvGeom& g) { return align256((size_t)g.W * g.H * g.N * g.groups * padded<T>(g.Cin_g) * sizeof(T)); }
+static size_t xt_bytes(const ConvGeom& g, int n) {       // n: groups at a time, where padded
+    const int Cp = padded<T>(g.Cin_g);
+    return align256((size_t)g.W * g.H * g.N * (Cp != g.Cin_g ? n : g.groups) * Cp * sizeof(T));
+}
 template <typename T>
-static size_t dyt_bytes(const ConvGeom& g) {
-    return align256(((size_t)g.OW * g.OH * g.N + dy_zeros<T>(g)) * g.groups * padded<T>(g.Cout_g) * sizeof(T));
+static size_t dyt_bytes(const ConvGeom& g, int n) {
+    const int Cp = padded<T>(g.Cout_g);
+    return align256(((size_t)g.OW * g.OH * g.N + dy_zeros<T>(g)) * (Cp != g.Cout_g ? n : g.groups) * Cp * sizeof(T));
 }
 template <typename T>
 static size_t filter_bytes(const ConvGeom& g, bool any, const AnyPlan<T>& plan) {
-    return align256(any ? (size_t)plan.wm_elems * sizeof(T) : (size_t)g.kW * g.kH * g.Cin_g * g.Cout * sizeof(T));
+    return align256(any ? (size_t)plan.wm_elems * g.groups * sizeof(T) : (size_t)g.kW * g.kH * g.Cin_g * g.Cout * sizeof(T));
 }
 // A caller's channel-contiguous copy of x serves the kernels as it is
 template <typename T>
 static bool kept_usable(const ConvGeom& g, const T* kept) { return kept != nullptr && padded<T>(g.Cin_g) == g.Cin_g && aligned16(kept); }
 
-// (C, P) -> (Cp, P) per group with zeros in the new channels: a caller's unpadded copy of x, when x itself is not given
+// (C, P) -> (Cp, P) per group with zeros in the new channels, for the groups whose first channel is at `in` (Cin channels in a
+// row): a caller's unpadded copy of x, when x itself is not given
 template <typename T>
-__global__ __launch_bounds__(256) void repad_cwhn_kernel(const T* __restrict__ in, T* __restrict__ out, int64_t total, int Cg, int Cp) {
+__global__ __launch_bounds__(256) void repad_cwhn_kernel(const T* __restrict__ in, T* __restrict__ out, int64_t total, int Cin, int Cg, int groups, int Cp) {
     for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < total; i += (int64_t)gridDim.x * 256) {
-        const int64_t row = i / Cp;
-        const int c = (int)(i - row * Cp);
-        out[i] = c < Cg ? in[row * Cg + c] : T(0);
+        const int64_t row = i / Cp, pos = row / groups;
+        const int c = (int)(i - row * Cp), grp = (int)(row - pos * groups);
+        out[i] = c < Cg ? in[pos * Cin + grp * Cg + c] : T(0);
     }
 }
 
@@ -963,10 +993,11 @@ static int conv_fwd_t(hipStream_t s, int act, const ConvGeom& g, const T* x, con
     AnyPlan<T> plan(g, false);
     // xt_keep: caller's buffer of x's size that keeps the channel-contiguous copy of x for the pullback
     const bool keep = kept_usable<T>(g, xt_keep);
-    const size_t xb = keep ? 0 : xt_bytes<T>(g), wb = filter_bytes<T>(g, any, plan);
+    const int n = keep ? std::min(g.groups, 32768) : groups_at_a_time<T>(g, true, false);
+    const size_t xb = keep ? 0 : xt_bytes<T>(g, n), wb = filter_bytes<T>(g, any, plan);
     Workspace ws;
     // the slices of conv_any.h take memory behind these; reserve it here, where no pointer into the workspace is live yet
-    int rc = get_workspace(s, any ? plan.reserve(s, xb + wb) : xb + wb, &ws);
+    int rc = get_workspace(s, any ? plan.reserve(s, xb + wb, n, g.groups) : xb + wb, &ws);
     if (rc != LUXHIP_OK) return rc;
     T* xT = keep ? xt_keep : reinterpret_cast<T*>(ws.data);
     T* wF = reinterpret_cast<T*>(ws.data + xb);
@@ -977,59 +1008,101 @@ static int conv_fwd_t(hipStream_t s, int act, const ConvGeom& g, const T* x, con
         if ((rc = transpose_and_pack<T>(s, x, xT, g.W * g.H, g.Cin, g.N, w, wF, g, 0)) != LUXHIP_OK) return rc;
         return run_conv_gemm<T>(s, g, false, xT, wF, bias, y, pre, act, ws.zeros);
     }
-    const PackSubs ps = plan.pack(g, false, 0, 0);
-    if ((rc = pad_and_pack<T>(s, x, xT, g.W * g.H, g.Cin_g, g.groups, g.N, 0, w, wF, g, &ps)) != LUXHIP_OK) return rc;
-    return run_conv_any<T>(s, g, false, plan, xT, w, wF, true, bias, y, pre, act, xb + wb);
+    const PackSubs ps = plan.pack(g, false, 0);
+    for (Groups gr{0, 0}; gr.first < g.groups; gr.first += gr.n) {
+        gr.n = std::min(n, g.groups - gr.first);
+        const bool first = gr.first == 0;
+        if (plan.Cp != g.Cin_g || first) {
+            const int copied = plan.Cp != g.Cin_g ? gr.n : g.groups;
+            rc = pad_and_pack<T>(s, x + (size_t)gr.first * g.Cin_g * g.W * g.H, xT, g.W * g.H, g.Cin, g.Cin_g, copied, g.N, 0, w, first ? wF : nullptr, g, &ps);
+            if (rc != LUXHIP_OK) return rc;
+        }
+        if ((rc = run_conv_any<T>(s, g, false, plan, gr, xT, w, wF, true, bias, y, pre, act, xb + wb)) != LUXHIP_OK) return rc;
+    }
+    return LUXHIP_OK;
 }
 
-// dx from the channel-contiguous cotangent; packed: the filter of the first launch is in wD
+// dx of the groups `gr` from the channel-contiguous cotangent; packed: the filter of the first launch is in wD.  The whole-tap
+// kernels (no padding: one call for all groups) know no part of the groups.
 template <typename T>
-static int run_dgrad(hipStream_t s, const ConvGeom& g, bool any, const AnyPlan<T>& plan, const T* dyT, const T* w, T* wD, bool packed, T* dx,
+static int run_dgrad(hipStream_t s, const ConvGeom& g, bool any, const AnyPlan<T>& plan, Groups gr, const T* dyT, const T* w, T* wD, bool packed, T* dx,
                      size_t ws_front, const void* zeros) {
-    if (any) return run_conv_any<T>(s, g, true, plan, dyT, w, wD, packed, nullptr, dx, nullptr, LUXHIP_ACT_IDENTITY, ws_front);
-    return run_conv_gemm<T>(s, g, true, dyT, wD, nullptr, dx, nullptr, LUXHIP_ACT_IDENTITY, zeros);
+    if (any) return run_conv_any<T>(s, g, true, plan, gr, dyT, w, wD, packed, nullptr, dx, nullptr, LUXHIP_ACT_IDENTITY, ws_front);
+    return gr.first == 0 ? run_conv_gemm<T>(s, g, true, dyT, wD, nullptr, dx, nullptr, LUXHIP_ACT_IDENTITY, zeros) : LUXHIP_OK;
 }
-// dyT (padded) and the filter packed for the input gradient, in one launch
+// dyT of the groups `gr` (of all groups with the first ones, where nothing is padded)
 template <typename T>
-static int dy_transpose_and_pack(hipStream_t s, const ConvGeom& g, bool any, const AnyPlan<T>& plan, const T* dy, T* dyT, const T* w, T* wD) {
+static int dy_copy(hipStream_t s, const ConvGeom& g, Groups gr, const T* dy, T* dyT) {
+    const bool alone = padded<T>(g.Cout_g) != g.Cout_g;
+    if (!alone && gr.first > 0) return LUXHIP_OK;
+    return to_cwhn_padded<T>(s, dy + (size_t)gr.first * g.Cout_g * g.OW * g.OH, dyT, g.OW * g.OH, g.Cout, g.Cout_g, alone ? gr.n : g.groups, g.N,
+                             dy_zeros<T>(g), g);
+}
+// The same, and with the first groups the filter packed for the input gradient, in one launch
+template <typename T>
+static int dy_copy_and_pack(hipStream_t s, const ConvGeom& g, bool any, const AnyPlan<T>& plan, Groups gr, const T* dy, T* dyT, const T* w, T* wD) {
+    if (gr.first > 0 || plan.launches.empty()) return dy_copy<T>(s, g, gr, dy, dyT);
     if (!any && dy_zeros<T>(g) > 0) {
-        const int rc = to_cwhn_padded<T>(s, dy, dyT, g.OW * g.OH, g.Cout_g, g.groups, g.N, dy_zeros<T>(g), g);
+        const int rc = dy_copy<T>(s, g, gr, dy, dyT);
         return rc != LUXHIP_OK ? rc : pack_filter<T>(s, w, wD, g, 1);
     }
     if (!any) return transpose_and_pack<T>(s, dy, dyT, g.OW * g.OH, g.Cout, g.N, w, wD, g, 1);
-    if (plan.launches.empty()) return to_cwhn_padded<T>(s, dy, dyT, g.OW * g.OH, g.Cout_g, g.groups, g.N, dy_zeros<T>(g), g);
-    const PackSubs ps = plan.pack(g, true, 0, 0);
-    return pad_and_pack<T>(s, dy, dyT, g.OW * g.OH, g.Cout_g, g.groups, g.N, dy_zeros<T>(g), w, wD, g, &ps);
+    const PackSubs ps = plan.pack(g, true, 0);
+    return pad_and_pack<T>(s, dy, dyT, g.OW * g.OH, g.Cout, g.Cout_g, plan.Cp != g.Cout_g ? gr.n : g.groups, g.N, dy_zeros<T>(g), w, wD, g, &ps);
+}
+// xT of the groups `gr`, likewise; from the caller's unpadded copy where x is not given
+template <typename T>
+static int x_copy(hipStream_t s, const ConvGeom& g, Groups gr, const T* x, const T* unpadded, T* xT) {
+    const int Cp = padded<T>(g.Cin_g);
+    const bool alone = Cp != g.Cin_g;
+    if (!alone && gr.first > 0) return LUXHIP_OK;
+    const int n = alone ? gr.n : g.groups;
+    if (x != nullptr)
+        return to_cwhn_padded<T>(s, x + (size_t)gr.first * g.Cin_g * g.W * g.H, xT, g.W * g.H, g.Cin, g.Cin_g, n, g.N, 0, g);
+    const int64_t total = (int64_t)g.W * g.H * g.N * n * Cp;
+    repad_cwhn_kernel<T><<<(unsigned)std::min<int64_t>(ceil_div(total, 256), 65536), 256, 0, s>>>(unpadded + (size_t)gr.first * g.Cin_g, xT, total, g.Cin,
+                                                                                               g.Cin_g, n, Cp);
+    LUX_CHECK_LAUNCH();
+    return LUXHIP_OK;
 }
 
 template <typename T>
 static int conv_bwd_data_t(hipStream_t s, const ConvGeom& g, const T* dy, const T* w, T* dx) {
     const bool any = !tap_shape<T>(g, true);
     AnyPlan<T> plan(g, true);
-    const size_t yb = dyt_bytes<T>(g), wb = filter_bytes<T>(g, any, plan);
+    const int n = groups_at_a_time<T>(g, false, true);
+    const size_t yb = dyt_bytes<T>(g, n), wb = filter_bytes<T>(g, any, plan);
     Workspace ws;
-    int rc = get_workspace(s, any ? plan.reserve(s, yb + wb) : yb + wb, &ws);
+    int rc = get_workspace(s, any ? plan.reserve(s, yb + wb, n, g.groups) : yb + wb, &ws);
     if (rc != LUXHIP_OK) return rc;
     T* dyT = reinterpret_cast<T*>(ws.data);
     T* wD = reinterpret_cast<T*>(ws.data + yb);
-    if ((rc = dy_transpose_and_pack<T>(s, g, any, plan, dy, dyT, w, wD)) != LUXHIP_OK) return rc;
-    return run_dgrad<T>(s, g, any, plan, dyT, w, wD, true, dx, yb + wb, ws.zeros);
+    for (Groups gr{0, 0}; gr.first < g.groups; gr.first += gr.n) {
+        gr.n = std::min(n, g.groups - gr.first);
+        if ((rc = dy_copy_and_pack<T>(s, g, any, plan, gr, dy, dyT, w, wD)) != LUXHIP_OK) return rc;
+        if ((rc = run_dgrad<T>(s, g, any, plan, gr, dyT, w, wD, true, dx, yb + wb, ws.zeros)) != LUXHIP_OK) return rc;
+    }
+    return LUXHIP_OK;
 }
 
 template <typename T>
 static int conv_bwd_filter_t(hipStream_t s, const ConvGeom& g, const T* x, const T* dy, T* dw) {
-    const size_t xb = xt_bytes<T>(g), yb = dyt_bytes<T>(g), pb = wgrad_partial_bytes<T>(g);
+    const int n = groups_at_a_time<T>(g, true, true);
+    const size_t xb = xt_bytes<T>(g, n), yb = dyt_bytes<T>(g, n), pb = wgrad_partial_bytes<T>(g);
     Workspace ws;
     int rc = get_workspace(s, xb + yb + pb, &ws);
     if (rc != LUXHIP_OK) return rc;
     T* xT = reinterpret_cast<T*>(ws.data);
     T* dyT = reinterpret_cast<T*>(ws.data + xb);
     float* partial = reinterpret_cast<float*>(ws.data + xb + yb);
-    if ((rc = to_cwhn_padded<T>(s, x, xT, g.W * g.H, g.Cin_g, g.groups, g.N, 0, g)) != LUXHIP_OK) return rc;
-    if (!wgrad_direct_ok<T>(g, xT, dy)) {   // the direct kernel reads dy as it is
-        if ((rc = to_cwhn_padded<T>(s, dy, dyT, g.OW * g.OH, g.Cout_g, g.groups, g.N, dy_zeros<T>(g), g)) != LUXHIP_OK) return rc;
+    for (Groups gr{0, 0}; gr.first < g.groups; gr.first += gr.n) {
+        gr.n = std::min(n, g.groups - gr.first);
+        if ((rc = x_copy<T>(s, g, gr, x, nullptr, xT)) != LUXHIP_OK) return rc;
+        // the direct kernel reads dy as it is
+        if (!wgrad_direct_ok<T>(g, xT, dy) && (rc = dy_copy<T>(s, g, gr, dy, dyT)) != LUXHIP_OK) return rc;
+        if ((rc = run_wgrad<T>(s, g, gr, xT, dy, dyT, partial, dw, ws.zeros)) != LUXHIP_OK) return rc;
     }
-    return run_wgrad<T>(s, g, xT, dy, dyT, partial, dw, ws.zeros);
+    return LUXHIP_OK;
 }
 
 template <typename T>
@@ -1037,7 +1110,8 @@ static int fused_conv_bwd_t(hipStream_t s, int dtype, int act, const ConvGeom& g
                             const T* pre, const T* x, const T* w, T* dz, T* dw, T* dx, T* dbias, const T* xt_kept) {
     const bool any = !tap_shape<T>(g, true), kept = kept_usable<T>(g, xt_kept);
     AnyPlan<T> plan(g, true);
-    const size_t xb = kept ? 0 : xt_bytes<T>(g), yb = dyt_bytes<T>(g), wb = filter_bytes<T>(g, any, plan), pb = wgrad_partial_bytes<T>(g);
+    const int n = groups_at_a_time<T>(g, dw != nullptr && !kept, true);
+    const size_t xb = kept ? 0 : xt_bytes<T>(g, n), yb = dyt_bytes<T>(g, n), wb = filter_bytes<T>(g, any, plan), pb = wgrad_partial_bytes<T>(g);
     // bf16: dz, its channel-contiguous copy and the bias gradient in one pass, when both a pass over delta and a
     // transposing copy would run
     bool one_pass = false;
@@ -1048,7 +1122,7 @@ static int fused_conv_bwd_t(hipStream_t s, int dtype, int act, const ConvGeom& g
     // reserve everything up front: the bias-gradient pass below uses the start of the same
     // workspace, and the buffer must not be reallocated while pointers into it are live
     Workspace ws;
-    int rc = get_workspace(s, any && dx != nullptr ? plan.reserve(s, xb + yb + wb + pb + bb) : xb + yb + wb + pb + bb, &ws);
+    int rc = get_workspace(s, any && dx != nullptr ? plan.reserve(s, xb + yb + wb + pb + bb, n, g.groups) : xb + yb + wb + pb + bb, &ws);
     if (rc != LUXHIP_OK) return rc;
     const T* xT = kept ? xt_kept : reinterpret_cast<const T*>(ws.data);
     T* dzT = reinterpret_cast<T*>(ws.data + xb);
@@ -1077,26 +1151,21 @@ static int fused_conv_bwd_t(hipStream_t s, int dtype, int act, const ConvGeom& g
             if (dz_out) dzp = dz_out;
         }
         if (dw == nullptr && dx == nullptr) return LUXHIP_OK;
-        if (dx != nullptr) rc = dy_transpose_and_pack<T>(s, g, any, plan, dzp, dzT, w, wD);
-        else rc = to_cwhn_padded<T>(s, dzp, dzT, g.OW * g.OH, g.Cout_g, g.groups, g.N, dy_zeros<T>(g), g);
-        if (rc != LUXHIP_OK) return rc;
     }
-    if (dx != nullptr) {
-        if ((rc = run_dgrad<T>(s, g, any, plan, dzT, w, wD, packed, dx, xb + yb + wb + pb + bb, ws.zeros)) != LUXHIP_OK) return rc;
-    }
-    if (dw != nullptr) {
-        if (!kept) {
-            T* xw = reinterpret_cast<T*>(ws.data);
-            if (x != nullptr) {
-                if ((rc = to_cwhn_padded<T>(s, x, xw, g.W * g.H, g.Cin_g, g.groups, g.N, 0, g)) != LUXHIP_OK) return rc;
-            } else {
-                const int64_t total = (int64_t)g.W * g.H * g.N * g.groups * padded<T>(g.Cin_g);
-                repad_cwhn_kernel<T><<<(unsigned)std::min<int64_t>(ceil_div(total, 256), 65536), 256, 0, s>>>(xt_kept, xw, total, g.Cin_g, padded<T>(g.Cin_g));
-                LUX_CHECK_LAUNCH();
-            }
+    for (Groups gr{0, 0}; gr.first < g.groups; gr.first += gr.n) {
+        gr.n = std::min(n, g.groups - gr.first);
+        if (!one_pass) {
+            rc = dx != nullptr ? dy_copy_and_pack<T>(s, g, any, plan, gr, dzp, dzT, w, wD) : dy_copy<T>(s, g, gr, dzp, dzT);
+            if (rc != LUXHIP_OK) return rc;
         }
-        if ((rc = run_wgrad<T>(s, g, xT, dzp, dzT, partial, dw, ws.zeros, bias_later.dbias != nullptr ? &bias_later : nullptr)) != LUXHIP_OK)
-            return rc;
+        if (dx != nullptr) {
+            if ((rc = run_dgrad<T>(s, g, any, plan, gr, dzT, w, wD, packed, dx, xb + yb + wb + pb + bb, ws.zeros)) != LUXHIP_OK) return rc;
+        }
+        if (dw != nullptr) {
+            if (!kept && (rc = x_copy<T>(s, g, gr, x, xt_kept, reinterpret_cast<T*>(ws.data))) != LUXHIP_OK) return rc;
+            rc = run_wgrad<T>(s, g, gr, xT, dzp, dzT, partial, dw, ws.zeros, bias_later.dbias != nullptr ? &bias_later : nullptr);
+            if (rc != LUXHIP_OK) return rc;
+        }
     }
     return LUXHIP_OK;
 }

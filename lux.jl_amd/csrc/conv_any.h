@@ -46,8 +46,8 @@ constexpr int MAX_SUBS = 4;       // a stride of 2; larger strides take more lau
 
 template <typename T>
 struct Args {
-    const T* src;              // channel-contiguous, first channel of the group
-    const T* wm;
+    const T* src;              // channel-contiguous, first channel of the first group of the launch (one blockIdx.y each)
+    const T* wm;               // its packed filter
     const void* zero;
     const T* bias;
     T *out, *pre;
@@ -59,6 +59,8 @@ struct Args {
     int kW, kH;                // merged (dilation 1): tap t of residue r is filter tap t * os + r, where there is one
     int col_off, Ctot_out, act;
     int subs, merged;
+    int64_t wm_group, partial_group;   // packed filter elements and bytes of partial sums per group
+    int sliced_tiles;          // counters per group
     char* partial;
     uint32_t* counters;
     FastDiv divCp, divCch;
@@ -74,9 +76,10 @@ struct RowLoader {
     static_assert(PER >= 1, "at least one chunk per thread");
     const Args<T>& g;
     const Sub& q;
+    const T* src;
     int pos[PER], ps[PER], qs[PER];
     int chunk;
-    __device__ __forceinline__ RowLoader(const Args<T>& gg, const Sub& s, int m0) : g(gg), q(s) {
+    __device__ __forceinline__ RowLoader(const Args<T>& gg, const Sub& s, const T* x, int m0) : g(gg), q(s), src(x) {
         chunk = (threadIdx.x % CPR) * Tr::VEC;
 #pragma unroll
         for (int i = 0; i < PER; ++i) {
@@ -103,7 +106,7 @@ struct RowLoader {
         for (int i = 0; i < PER; ++i) {
             const int sp = ps[i] + dp, sq = qs[i] + dq;
             const bool valid = tap && (unsigned)sp < (unsigned)g.SP && (unsigned)sq < (unsigned)g.SQ;
-            const T* p = g.src + ((int64_t)((pos[i] + sq) * g.SP + sp) * g.Ctot + c);
+            const T* p = src + ((int64_t)((pos[i] + sq) * g.SP + sp) * g.Ctot + c);
             reg[i] = *reinterpret_cast<const u32x4_v*>(valid ? static_cast<const void*>(p) : g.zero);
         }
     }
@@ -125,9 +128,9 @@ struct Shape {
 // Merged residues: the sum of row (a, b, n) and column col over the taps that the column's residue (rw, rh) has.  A NaN among
 // the terms ends it, so a cotangent that is NaN throughout costs one term per element.
 template <typename T>
-__device__ __forceinline__ float own_taps_sum(const Args<T>& g, const Sub& q, int a, int b, int n, int col, int rw, int rh) {
+__device__ __forceinline__ float own_taps_sum(const Args<T>& g, const Sub& q, const T* src, const T* wm, int a, int b, int n, int col, int rw, int rh) {
     const int nw = (g.kW - rw + g.os_w - 1) / g.os_w, nh = (g.kH - rh + g.os_h - 1) / g.os_h;
-    const T* wcol = g.wm + q.wm + (int64_t)col * q.Kpad;
+    const T* wcol = wm + q.wm + (int64_t)col * q.Kpad;
     float sum = 0.0f;
     for (int th = 0; th < nh; ++th) {
         const int sq = b * g.ss_h + q.h0 + th * q.hstep;
@@ -135,7 +138,7 @@ __device__ __forceinline__ float own_taps_sum(const Args<T>& g, const Sub& q, in
         for (int tw = 0; tw < nw; ++tw) {
             const int sp = a * g.ss_w + q.w0 + tw * q.wstep;
             if ((unsigned)sp >= (unsigned)g.SP) continue;
-            const T* x = g.src + (int64_t)((n * g.SQ + sq) * g.SP + sp) * g.Ctot;
+            const T* x = src + (int64_t)((n * g.SQ + sq) * g.SP + sp) * g.Ctot;
             const T* w = wcol + (th * q.TW + tw) * g.Cp;
 #pragma unroll 1
             for (int c = 0; c < g.Cp; ++c) sum = fmaf(ld(x + c), ld(w + c), sum);
@@ -155,7 +158,9 @@ __global__ __launch_bounds__(split::THREADS) void conv_any_kernel(Args<T> g) {
 #pragma unroll
     for (int i = 1; i < MAX_SUBS; ++i)
         if (i < g.subs && (int)blockIdx.x >= g.sub[i].first_block) q = g.sub[i];
-    const int id = (int)blockIdx.x - q.first_block;
+    const int id = (int)blockIdx.x - q.first_block, grp = blockIdx.y;
+    const T *const src = g.src + (int64_t)grp * g.Cp, *const wm = g.wm + grp * g.wm_group;
+    const int col_off = g.col_off + grp * g.Cch;
     const int tile = id / q.slices, slice = id - tile * q.slices;
     int tm, tn;
     tile_coords(tile, q.tiles_m, q.tiles_n, tm, tn);
@@ -163,9 +168,9 @@ __global__ __launch_bounds__(split::THREADS) void conv_any_kernel(Args<T> g) {
     static_assert(WM <= 2 && WN <= 2, "32 accumulator bits per i below");
     f32x16_v acc[WM][WN];
     {
-        const typename S::LA la(g, q, m0);
+        const typename S::LA la(g, q, src, m0);
         Operand<T> B;
-        B.p = g.wm + q.wm; B.sr = q.Kpad; B.sk = 1; B.vec_ok = 1;
+        B.p = wm + q.wm; B.sr = q.Kpad; B.sk = 1; B.vec_ok = 1;
         B.rows = g.Ncols - n0;                                         // the last tile clamps its rows
         B.p += (int64_t)n0 * q.Kpad;
         const typename S::LB lb(B, 0);
@@ -173,7 +178,8 @@ __global__ __launch_bounds__(split::THREADS) void conv_any_kernel(Args<T> g) {
         Core::run(la, lb, kbeg, min(kbeg + q.kslice, q.Kpad), reinterpret_cast<T*>(lds_raw), acc);
     }
     if (q.slices > 1) {
-        split::Plan p{q.slices, q.kslice, reinterpret_cast<float*>(g.partial + q.partial), g.counters + q.first_tile};
+        split::Plan p{q.slices, q.kslice, reinterpret_cast<float*>(g.partial + grp * g.partial_group + q.partial),
+                      g.counters + grp * g.sliced_tiles + q.first_tile};
         if (!Core::combine(p, tile, slice, acc)) return;
     }
     // rows -> output positions
@@ -203,8 +209,8 @@ __global__ __launch_bounds__(split::THREADS) void conv_any_kernel(Args<T> g) {
                 rh = res / g.res_w;
                 rw = res - rh * g.res_w;
             }
-            const float bv = g.bias ? ld(g.bias + g.col_off + ch) : 0.0f;
-            const int64_t coff = (int64_t)(g.col_off + ch) * g.PQ + (int64_t)rh * g.P + rw;
+            const float bv = g.bias ? ld(g.bias + col_off + ch) : 0.0f;
+            const int64_t coff = (int64_t)(col_off + ch) * g.PQ + (int64_t)rh * g.P + rw;
             float v[WM];
             bool st_ok[WM];
 #pragma unroll
@@ -245,7 +251,7 @@ __global__ __launch_bounds__(split::THREADS) void conv_any_kernel(Args<T> g) {
         const int res = (int)g.divCch.div((uint32_t)col), ch = col - res * g.Cch, rh = res / g.res_w, rw = res - rh * g.res_w;
         const int ow = a * g.os_w + q.ow0 + rw, oh = b * g.os_h + q.oh0 + rh;
         if ((unsigned)ow < (unsigned)g.P && (unsigned)oh < (unsigned)g.Q)
-            st(g.out + (int64_t)(n * g.Ctot_out + g.col_off + ch) * g.PQ + (int64_t)oh * g.P + ow, own_taps_sum<T>(g, q, a, b, n, col, rw, rh));
+            st(g.out + ((int64_t)n * g.Ctot_out + col_off + ch) * g.PQ + (int64_t)oh * g.P + ow, own_taps_sum<T>(g, q, src, wm, a, b, n, col, rw, rh));
     }
 }
 
@@ -336,12 +342,12 @@ __global__ __launch_bounds__(split::THREADS) void conv_any_wgrad_kernel(WgradArg
     });
 }
 
-// Tile and slices of a launch, and the bytes that its slices take (32 MiB at most)
+// Tile and slices of a launch over `groups` groups, and the bytes that its slices take per group (32 MiB in all at most)
 struct Choice { int tile, slices; size_t bytes; };
 template <typename T>
-Choice choose_any(Sub* sub, int subs, int Ncols, bool may_slice);                // conv_any_*.hip; fills in the tiling of sub[]
+Choice choose_any(Sub* sub, int subs, int Ncols, int groups, bool may_slice);    // conv_any_*.hip; fills in the tiling of sub[]
 template <typename T>
-int launch_any(hipStream_t s, Args<T>& a, size_t ws_front, bool dgrad, bool may_slice);
+int launch_any(hipStream_t s, Args<T>& a, int groups, size_t ws_front, bool dgrad, bool may_slice);
 template <typename T>
 int launch_any_wgrad(hipStream_t s, WgradArgs<T>& a, int slices, bool narrow);
 

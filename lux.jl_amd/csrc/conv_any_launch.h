@@ -18,17 +18,17 @@ inline const Tile* tiles() {
 }
 
 template <typename T, int WM, int WN, int NWM, int NWN>
-int launch_shape(hipStream_t s, Args<T>& a, int blocks, bool dgrad) {
+int launch_shape(hipStream_t s, Args<T>& a, int blocks, int groups, bool dgrad) {
     using S = Shape<T, WM, WN, NWM, NWN>;
     static const char* const names[2][2] = {{"conv_fprop_kernel<f32>", "conv_dgrad_kernel<f32>"}, {"conv_fprop_kernel<bf16>", "conv_dgrad_kernel<bf16>"}};
     ProfScope ps(names[sizeof(T) == 2][dgrad], s);
-    conv_any_kernel<T, WM, WN, NWM, NWN><<<dim3((unsigned)blocks), dim3(split::THREADS), S::Core::LDS_BYTES, s>>>(a);
+    conv_any_kernel<T, WM, WN, NWM, NWN><<<dim3((unsigned)blocks, (unsigned)groups), dim3(split::THREADS), S::Core::LDS_BYTES, s>>>(a);
     LUX_CHECK_LAUNCH();
     return LUXHIP_OK;
 }
 
 template <typename T>
-Choice choose_any(Sub* sub, int subs, int Ncols, bool may_slice) {
+Choice choose_any(Sub* sub, int subs, int Ncols, int groups, bool may_slice) {
     constexpr int BK = GemmTraits<T>::BK;
     constexpr size_t most_bytes = size_t(32) << 20;
     const int64_t cus = num_cus() > 0 ? num_cus() : 256;
@@ -42,8 +42,8 @@ Choice choose_any(Sub* sub, int subs, int Ncols, bool may_slice) {
         double work = 0.0;                                           // tiles x k
         for (int i = 0; i < subs; ++i) {
             const int64_t t = ceil_div(sub[i].M, tl[c].m) * ceil_div(Ncols, tl[c].n);
-            nt += t;
-            work += (double)t * (sub[i].Kpad + 100);
+            nt += t * groups;
+            work += (double)t * groups * (sub[i].Kpad + 100);
         }
         for (int sl = 1; sl <= 8; ++sl) {
             if (sl > 1 && (!may_slice || kmax / sl < 2 * BK || nt > 16384 || (size_t)(nt * sl) * tl[c].m * tl[c].n * sizeof(float) > most_bytes)) break;
@@ -67,8 +67,8 @@ Choice choose_any(Sub* sub, int subs, int Ncols, bool may_slice) {
 }
 
 template <typename T>
-int launch_any(hipStream_t s, Args<T>& a, size_t ws_front, bool dgrad, bool may_slice) {
-    const Choice c = choose_any<T>(a.sub, a.subs, a.Ncols, may_slice);
+int launch_any(hipStream_t s, Args<T>& a, int groups, size_t ws_front, bool dgrad, bool may_slice) {
+    const Choice c = choose_any<T>(a.sub, a.subs, a.Ncols, groups, may_slice);
     int blocks = 0, nt = 0;
     for (int i = 0; i < a.subs; ++i) {
         Sub& q = a.sub[i];
@@ -81,17 +81,19 @@ int launch_any(hipStream_t s, Args<T>& a, size_t ws_front, bool dgrad, bool may_
     }
     if (blocks == 0) return LUXHIP_OK;
     Workspace ws;
-    const int rc = get_workspace(s, ws_front + c.bytes, &ws);
+    const int rc = get_workspace(s, ws_front + c.bytes * groups, &ws);
     if (rc != LUXHIP_OK) return rc;
     a.partial = ws.data + ws_front;
+    a.partial_group = (int64_t)c.bytes;
+    a.sliced_tiles = nt;
     a.counters = ws.counters;
     a.zero = ws.zeros;
     switch (c.tile) {
-        case 0: return launch_shape<T, 1, 1, 2, 2>(s, a, blocks, dgrad);
-        case 1: return launch_shape<T, 2, 1, 2, 2>(s, a, blocks, dgrad);
-        case 2: return launch_shape<T, 2, 2, 2, 2>(s, a, blocks, dgrad);
-        case 3: return launch_shape<T, 2, 1, 4, 1>(s, a, blocks, dgrad);
-        default: return launch_shape<T, 1, 1, 4, 1>(s, a, blocks, dgrad);
+        case 0: return launch_shape<T, 1, 1, 2, 2>(s, a, blocks, groups, dgrad);
+        case 1: return launch_shape<T, 2, 1, 2, 2>(s, a, blocks, groups, dgrad);
+        case 2: return launch_shape<T, 2, 2, 2, 2>(s, a, blocks, groups, dgrad);
+        case 3: return launch_shape<T, 2, 1, 4, 1>(s, a, blocks, groups, dgrad);
+        default: return launch_shape<T, 1, 1, 4, 1>(s, a, blocks, groups, dgrad);
     }
 }
 

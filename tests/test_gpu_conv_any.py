@@ -27,6 +27,9 @@ CASES = [
     ((33, 34, 32, 2), (1, 1, 32, 24), 9, 0, 1, 1, False),            # one residue of 81 has taps
     ((20, 19, 33, 1), (3, 2, 33, 8), (7, 6), (2, 0, 1, 3), (2, 3), 1, True),   # 6 of 42, dilated; an odd number of bf16 elements
     ((6, 5, 4, 2), (2, 2, 2, 6), 1000, 0, 1, 2, False),              # stride far beyond the input
+    ((9, 8, 40, 2), (3, 3, 1, 40), 1, 1, 1, 40, False),              # depthwise: a group per block of the grid
+    ((9, 8, 40, 2), (5, 3, 1, 80), 2, 1, 1, 40, True),               # ... two channels out of one, merged residues
+    ((5, 4, 300, 1), (2, 2, 100, 21), 1, 0, 1, 3, False),            # groups with slices
 ]
 
 
@@ -127,3 +130,36 @@ def test_nonfinite_cotangent_reaches_its_window_only(gpu, dtype, xs, ws, stride,
     got = f64(gpu.conv_data_grad(dev(gpu, dy, dtype), dev(gpu, w, dtype), gd).to_numpy())
     np.testing.assert_array_equal(np.isfinite(got), ~seen)
     assert_close(np.where(seen, 0.0, got), np.where(seen, 0.0, want), dtype, f"{dtype} finite part of dx")
+
+
+@pytest.mark.parametrize("dtype,stride", [("f32", 1), ("f32", 2), ("bf16", 1), ("bf16", 2)])
+def test_depthwise_copies_take_no_more_than_the_tensor(gpu, dtype, stride):
+    """A depthwise layer above 64 MiB: its padded copies are made for a few groups at a time (channels stay apart, so a layer of
+    the same images with fewer channels gives each of them the same bits)."""
+    xs, ws = (280, 250, 96, 5) if dtype == "bf16" else (280, 250, 50, 5), (3, 3, 1, 96 if dtype == "bf16" else 50)
+    kw = dict(stride=stride, padding=1)
+    gd = gpu.DenseConvDims(xs, ws, groups=xs[2], **kw)
+    rng = np.random.default_rng(stable_seed("depthwise", dtype))
+    ints = lambda *s: rng.integers(-2, 3, size=s).astype(np.float32)
+    x, w, dy = ints(*xs), ints(*ws), ints(*gd.y_shape)
+    y, back = gpu.pullback(gpu.fused_conv_bias_activation, "identity", dev(gpu, w, dtype), dev(gpu, x, dtype), None, gd)
+    gw, gx, _ = back(dev(gpu, dy, dtype))
+    y, gw, gx = (a.to_numpy() for a in (y, gw, gx))
+    for c in (0, 11, 12, 49, xs[2] - 1):                     # first and last channels of the copies among them
+        od = O.ConvDims(xs[:2] + (1, xs[3]), (3, 3, 1, 1), **kw)
+        xc, wc, dc = f64(x[:, :, c:c + 1]), f64(w[:, :, :, c:c + 1]), f64(dy[:, :, c:c + 1])
+        np.testing.assert_array_equal(y[:, :, c:c + 1], O.conv(xc, wc, od))
+        np.testing.assert_array_equal(gx[:, :, c:c + 1], O.conv_data_grad(dc, wc, od))
+        want = O.conv_filter_grad(xc, dc, od)
+        np.testing.assert_array_equal(gw[:, :, :, c:c + 1], want if dtype == "f32" else O.round_to_bf16(want.astype(np.float32)))
+
+
+def test_groups_share_their_launches(gpu):
+    xs, ws = (12, 11, 24, 2), (3, 3, 2, 36)
+    gd = gpu.DenseConvDims(xs, ws, padding=1, groups=12)
+    rng = np.random.default_rng(3)
+    x, w, dy = (dev(gpu, rng.normal(size=s).astype(np.float32), "f32") for s in (xs, ws, gd.y_shape))
+    count = kernels_of(gpu, lambda: gpu.conv(x, w, gd))
+    assert count == {"whcn_to_cwhn_kernel": 1, "conv_fprop_kernel<f32>": 1}, count
+    count = kernels_of(gpu, lambda: gpu.conv_data_grad(dy, w, gd))
+    assert count == {"whcn_to_cwhn_kernel": 1, "conv_dgrad_kernel<f32>": 1}, count
