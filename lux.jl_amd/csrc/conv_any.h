@@ -58,7 +58,7 @@ struct Args {
     int res_w;                 // merged: residues along w
     int kW, kH;                // merged (dilation 1): tap t of residue r is filter tap t * os + r, where there is one
     int col_off, Ctot_out, act;
-    int subs, merged;
+    int subs, merged;          // merged: the residues are columns
     int64_t wm_group, partial_group;   // packed filter elements and bytes of partial sums per group
     int sliced_tiles;          // counters per group
     char* partial;
@@ -148,8 +148,11 @@ __device__ __forceinline__ float own_taps_sum(const Args<T>& g, const Sub& q, co
     return sum;
 }
 
-template <typename T, int WM, int WN, int NWM, int NWN>
-__global__ __launch_bounds__(split::THREADS) void conv_any_kernel(Args<T> g) {
+// MERGED: the residues of an input gradient are columns and a NaN among the sums is looked into.  A kernel of its own: the test
+// costs 3 to 5 %, and a register that takes a wave from every SIMD unless it is told to stay below (256 x 32 tiles of the first
+// layer, 78 us with four waves, 85 with three).
+template <typename T, int WM, int WN, int NWM, int NWN, bool MERGED>
+__global__ __launch_bounds__(split::THREADS, MERGED && WM * WN < 4 ? 4 : 1) void conv_any_kernel(Args<T> g) {
     using S = Shape<T, WM, WN, NWM, NWN>;
     using Core = typename S::Core;
     using ML = typename Core::ML;
@@ -219,7 +222,7 @@ __global__ __launch_bounds__(split::THREADS) void conv_any_kernel(Args<T> g) {
                 st_ok[i] = ok[i];
                 if (g.merged) {
                     st_ok[i] = ok[i] && (unsigned)(iw[i] + rw) < (unsigned)g.P && (unsigned)(ih[i] + rh) < (unsigned)g.Q;
-                    nan = nan || v[i] != v[i];
+                    if constexpr (MERGED) nan = nan || v[i] != v[i];
                 }
             }
             if (g.pre != nullptr) {
@@ -234,24 +237,26 @@ __global__ __launch_bounds__(split::THREADS) void conv_any_kernel(Args<T> g) {
                 if (st_ok[i]) st(g.out + coff + row[i], v[i]);
         }
     });
-    if (!nan) return;
-    uint64_t nans = 0;                 // bit 32 i + 16 j + r
-    static_for<WM * WN * 16>([&](auto E) {
-        constexpr int i = decltype(E)::value / (WN * 16), jr = decltype(E)::value % (WN * 16);
-        const float v = acc[i][jr / 16][jr % 16];
-        if (v != v) nans |= uint64_t(1) << (32 * i + jr);
-    });
-    while (nans != 0) {                // an input gradient: no bias, no activation
-        const int e = __builtin_ctzll(nans), r = e & 15;
-        nans &= nans - 1;
-        const int m = mb + (e & 32), col = nb + 2 * (e & 16) + ((r >> 2) << 3) + (r & 3);
-        if (m >= q.M || col >= g.Ncols) continue;
-        const int n = (int)q.divRAB.div((uint32_t)m), rem = m - n * q.RAB;
-        const int b = (int)q.divRA.div((uint32_t)rem), a = rem - b * q.RA;
-        const int res = (int)g.divCch.div((uint32_t)col), ch = col - res * g.Cch, rh = res / g.res_w, rw = res - rh * g.res_w;
-        const int ow = a * g.os_w + q.ow0 + rw, oh = b * g.os_h + q.oh0 + rh;
-        if ((unsigned)ow < (unsigned)g.P && (unsigned)oh < (unsigned)g.Q)
-            st(g.out + ((int64_t)n * g.Ctot_out + col_off + ch) * g.PQ + (int64_t)oh * g.P + ow, own_taps_sum<T>(g, q, src, wm, a, b, n, col, rw, rh));
+    if constexpr (MERGED) {
+        if (!nan) return;
+        uint64_t nans = 0;                 // bit 32 i + 16 j + r
+        static_for<WM * WN * 16>([&](auto E) {
+            constexpr int i = decltype(E)::value / (WN * 16), jr = decltype(E)::value % (WN * 16);
+            const float v = acc[i][jr / 16][jr % 16];
+            if (v != v) nans |= uint64_t(1) << (32 * i + jr);
+        });
+        while (nans != 0) {                // an input gradient: no bias, no activation
+            const int e = __builtin_ctzll(nans), r = e & 15;
+            nans &= nans - 1;
+            const int m = mb + (e & 32), col = nb + 2 * (e & 16) + ((r >> 2) << 3) + (r & 3);
+            if (m >= q.M || col >= g.Ncols) continue;
+            const int n = (int)q.divRAB.div((uint32_t)m), rem = m - n * q.RAB;
+            const int b = (int)q.divRA.div((uint32_t)rem), a = rem - b * q.RA;
+            const int res = (int)g.divCch.div((uint32_t)col), ch = col - res * g.Cch, rh = res / g.res_w, rw = res - rh * g.res_w;
+            const int ow = a * g.os_w + q.ow0 + rw, oh = b * g.os_h + q.oh0 + rh;
+            if ((unsigned)ow < (unsigned)g.P && (unsigned)oh < (unsigned)g.Q)
+                st(g.out + ((int64_t)n * g.Ctot_out + col_off + ch) * g.PQ + (int64_t)oh * g.P + ow, own_taps_sum<T>(g, q, src, wm, a, b, n, col, rw, rh));
+        }
     }
 }
 
