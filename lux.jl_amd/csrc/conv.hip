@@ -832,8 +832,9 @@ static int wgrad_plan(const ConvGeom& g, bool any, WgradPlan* p) {
     const int64_t tiles = ceil_div(p->Mrows, tile) * ceil_div(p->Ncols, tile);
     const int64_t Ktotal = (int64_t)g.OW * g.OH * g.N;
     // as many slices as keep every workgroup resident at once (two per compute unit): one more
-    // would add a whole round for a single straggler
-    int64_t want = std::max<int64_t>(1, 2 * (int64_t)std::max(1, num_cus()) / (tiles * g.groups));
+    // would add a whole round for a single straggler.  The groups of the padded kernel run one after the other and fill the
+    // chip each (28 x 28 x 96 x 8 fp32, depthwise 5 x 5: 115 us per group with the slices of a 96th of the chip)
+    int64_t want = std::max<int64_t>(1, 2 * (int64_t)std::max(1, num_cus()) / (tiles * (any ? 1 : g.groups)));
     int64_t ks = ceil_div(ceil_div(Ktotal, want), BK) * BK;
     ks = std::max<int64_t>(ks, 4 * BK);
     p->kslice = (int)ks;
