@@ -400,7 +400,9 @@ int luxhip_fused_dense_fwd(luxhip_stream_t s, int dtype, int act, int64_t M, int
  * dz = delta .* act'(y, pre); dbias = sum over the batch of dz; dW = dz * x'; dx = W' * dz.
  * delta, y, pre, dz: M x N contiguous; dW: M x K; dx: K x N contiguous.  dz is caller-
  * provided scratch of M*N elements (may alias delta when delta may be overwritten; may be
- * NULL for IDENTITY).  dbias, dW, dx may each be NULL to skip that output. */
+ * NULL for IDENTITY).  dbias, dW, dx may each be NULL to skip that output.  dx may be x's own memory
+ * (ldx = K: the two products then run one after the other, dW first); no other output may overlap an
+ * input or another output, as the two products otherwise run at the same time. */
 int luxhip_fused_dense_bwd(luxhip_stream_t s, int dtype, int act, int64_t M, int64_t K, int64_t N,
                            const void* delta, const void* y, const void* pre, const void* W, int64_t ldw,
                            const void* x, int64_t ldx, void* dz, void* dW, void* dx, void* dbias);

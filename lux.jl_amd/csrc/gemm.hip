@@ -55,6 +55,12 @@ template <typename T>
 static bool gradient_pair(hipStream_t s, int64_t M, int64_t K, int64_t N, const T* dz, const T* W, int64_t ldw, const T* x, int64_t ldx,
                           T* dW, T* dx, int* rc) {
     if (gemm_tile_override() != 0 || M < 1 || N < 1 || K < 1 || ldw < M || ldx < K) return false;
+    // one after the other dW is done with x before dx is written, so a caller may let dx take x's memory
+    auto apart = [](const T* a, int64_t na, const T* b, int64_t nb) {
+        const uintptr_t pa = reinterpret_cast<uintptr_t>(a), pb = reinterpret_cast<uintptr_t>(b);
+        return pa + (size_t)na * sizeof(T) <= pb || pb + (size_t)nb * sizeof(T) <= pa;
+    };
+    if (!apart(dx, K * N, x, (N - 1) * ldx + K)) return false;
     DenseArgs<T> a = dense_args<T>(false, false, M, K, N, dz, M, x, ldx, nullptr, dW, M, nullptr, LUXHIP_ACT_IDENTITY);
     DenseArgs<T> b = dense_args<T>(true, true, K, N, M, W, ldw, dz, M, nullptr, dx, K, nullptr, LUXHIP_ACT_IDENTITY);
     return launch_split_pair<T>(s, a, b, rc);

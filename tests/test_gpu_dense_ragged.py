@@ -125,3 +125,18 @@ def test_few_columns_and_many_rows(gpu, dtype, M, K, skinny):
     assert any("skinny" in n for n in names) == skinny, names
     want = W @ x
     np.testing.assert_array_equal(out[0].to_numpy(), want if dtype == "f32" else O.round_to_bf16(want))
+
+
+@pytest.mark.parametrize("dtype", ["f32", "bf16"])
+def test_input_gradient_in_the_inputs_own_memory(gpu, dtype):
+    """A caller that is done with x may have dx written over it: dW is finished before dx starts then."""
+    M, K, N = 130, 77, 301
+    rng = np.random.default_rng(stable_seed("alias", dtype))
+    W, x, dz = (dev(gpu, rng.integers(-2, 3, size=s).astype(np.float32), dtype) for s in ((M, K), (K, N), (M, N)))
+    want_W, want_x = (O.round_to_bf16(a) if dtype == "bf16" else a for a in (dz.to_numpy() @ x.to_numpy().T, W.to_numpy().T @ dz.to_numpy()))
+    dW = gpu.DeviceArray((M, K), dtype)
+    call = lambda: gpu._lib.call("luxhip_fused_dense_bwd", gpu.current_stream(), x.code, 0, M, K, N, dz.ptr, None, None, W.ptr, M, x.ptr, K, None,
+                                 dW.ptr, x.ptr, None)
+    assert not any("pair" in n for n in kernels_of(gpu, call))
+    np.testing.assert_array_equal(dW.to_numpy(), want_W)
+    np.testing.assert_array_equal(x.to_numpy(), want_x)
