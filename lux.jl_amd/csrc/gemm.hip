@@ -98,10 +98,10 @@ static int gemm_impl(hipStream_t s, int transA, int transB, int64_t M, int64_t N
         }
     }
     DenseArgs<T> a = dense_args<T>(a_kmajor, b_kmajor, M, N, K, A, lda, B, ldb, bias, C, ldc, pre, act);
-    if (gemm_tile_override() == 0 && !copied) {       // (operand copies occupy the workspace that these two would use)
+    if (gemm_tile_override() == 0 && !copied && ws_front == 0) {       // the workspace that these two use is free
         int rc = LUXHIP_OK;
-        if (launch_skinny<T>(s, a, a_kmajor, b_kmajor, ws_front, &rc)) return rc;
-        if (launch_split<T>(s, a, a_kmajor, b_kmajor, ws_front, &rc)) return rc;
+        if (launch_skinny<T>(s, a, a_kmajor, b_kmajor, &rc)) return rc;
+        if (launch_split<T>(s, a, a_kmajor, b_kmajor, &rc)) return rc;
     }
     if (a_kmajor && b_kmajor) return launch_layout<T, true, true>(s, a);
     if (a_kmajor) return launch_layout<T, true, false>(s, a);

@@ -44,10 +44,10 @@ int launch_batched_layout(hipStream_t s, DenseArgs<T>& a);
 
 // gemm_skinny.hip: at most 16 columns, A contiguous along m, B along k; false if the problem is another one
 template <typename T>
-bool launch_skinny(hipStream_t s, DenseArgs<T>& a, bool a_kmajor, bool b_kmajor, size_t ws_front, int* rc);
+bool launch_skinny(hipStream_t s, DenseArgs<T>& a, bool a_kmajor, bool b_kmajor, int* rc);
 // gemm_split_*.hip: products with few tiles or ragged operands; false if the problem is not theirs
 template <typename T>
-bool launch_split(hipStream_t s, DenseArgs<T>& a, bool a_kmajor, bool b_kmajor, size_t ws_front, int* rc);
+bool launch_split(hipStream_t s, DenseArgs<T>& a, bool a_kmajor, bool b_kmajor, int* rc);
 // two independent products in one launch: a with both operands contiguous along m / n, b with both along k
 template <typename T>
 bool launch_split_pair(hipStream_t s, DenseArgs<T>& a, DenseArgs<T>& b, int* rc);

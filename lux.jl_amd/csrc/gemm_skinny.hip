@@ -167,7 +167,7 @@ __global__ __launch_bounds__(THREADS) void skinny_gemm_kernel(Args<T> a) {
 }
 
 template <typename T>
-int launch(hipStream_t s, const DenseArgs<T>& d, size_t ws_front) {
+int launch(hipStream_t s, const DenseArgs<T>& d) {
     constexpr int V = Elem<T>::V, MT = 16 * V, KSTEP = 4 * V;
     Args<T> a;
     a.W = d.A.p; a.x = d.B.p; a.bias = d.bias; a.y = d.C; a.pre = d.pre;
@@ -178,15 +178,15 @@ int launch(hipStream_t s, const DenseArgs<T>& d, size_t ws_front) {
     // (11008 x 4096: 18.6 us against 20.4 with two in bf16, 29.7 against 38.2 in fp32); at least two steps of k per wave
     int64_t slices = std::max<int64_t>(1, std::min<int64_t>(cus / blocks, d.K / (2 * KSTEP * WAVES)));
     if (blocks > (int64_t)kWorkspaceCounters) slices = 1;
-    if (slices > 1 && !workspace_holds(s, ws_front + (size_t)blocks * slices * NMAX * MT * sizeof(float))) slices = 1;
+    if (slices > 1 && !workspace_holds(s, (size_t)blocks * slices * NMAX * MT * sizeof(float))) slices = 1;
     a.kwave = (int)(ceil_div(ceil_div(d.K, slices * WAVES), KSTEP) * KSTEP);
     a.slices = (int)ceil_div(d.K, (int64_t)a.kwave * WAVES);
     a.partial = nullptr; a.counters = nullptr;
     if (a.slices > 1) {
         Workspace ws;
-        const int rc = get_workspace(s, ws_front + (size_t)blocks * a.slices * NMAX * MT * sizeof(float), &ws);
+        const int rc = get_workspace(s, (size_t)blocks * a.slices * NMAX * MT * sizeof(float), &ws);
         if (rc != LUXHIP_OK) return rc;
-        a.partial = reinterpret_cast<float*>(ws.data + ws_front);
+        a.partial = reinterpret_cast<float*>(ws.data);
         a.counters = ws.counters;
     }
     ProfScope ps(sizeof(T) == 2 ? "skinny_gemm_kernel<bf16>" : "skinny_gemm_kernel<f32>", s);
@@ -213,12 +213,12 @@ static bool skinny_pays(int64_t M, int64_t K) {
 }
 
 template <typename T>
-bool launch_skinny(hipStream_t s, DenseArgs<T>& d, bool ak, bool bk, size_t ws_front, int* rc) {
+bool launch_skinny(hipStream_t s, DenseArgs<T>& d, bool ak, bool bk, int* rc) {
     if (ak || !bk || d.N > skinny::NMAX || d.N < 1 || d.M < 16 * skinny::Elem<T>::V || d.K < 1 || !skinny_pays<T>(d.M, d.K)) return false;
-    *rc = skinny::launch<T>(s, d, ws_front);
+    *rc = skinny::launch<T>(s, d);
     return true;
 }
-template bool launch_skinny<float>(hipStream_t, DenseArgs<float>&, bool, bool, size_t, int*);
-template bool launch_skinny<bf16_t>(hipStream_t, DenseArgs<bf16_t>&, bool, bool, size_t, int*);
+template bool launch_skinny<float>(hipStream_t, DenseArgs<float>&, bool, bool, int*);
+template bool launch_skinny<bf16_t>(hipStream_t, DenseArgs<bf16_t>&, bool, bool, int*);
 
 }  // namespace luxhip

@@ -64,9 +64,9 @@ inline void place(Plan& p, const Workspace& ws, int first_counter) {
 }
 
 template <typename T, int W, bool AK, bool BKM>
-int launch_cfg(hipStream_t s, DenseArgs<T>& a, int slices, size_t ws_front) {
+int launch_cfg(hipStream_t s, DenseArgs<T>& a, int slices) {
     using B = Body<T, W, AK, BKM>;
-    size_t bytes = ws_front;
+    size_t bytes = 0;
     Plan p = make_plan<T, W>(a, slices, &bytes);
     if (p.slices > 1 && !workspace_holds(s, bytes)) p = make_plan<T, W>(a, 1, &bytes);
     if (p.slices > 1) {
@@ -82,11 +82,11 @@ int launch_cfg(hipStream_t s, DenseArgs<T>& a, int slices, size_t ws_front) {
 }
 
 template <typename T, int W>
-int launch_layouts(hipStream_t s, DenseArgs<T>& a, bool ak, bool bk, int slices, size_t ws_front) {
-    if (ak && bk) return launch_cfg<T, W, true, true>(s, a, slices, ws_front);
-    if (ak) return launch_cfg<T, W, true, false>(s, a, slices, ws_front);
-    if (bk) return launch_cfg<T, W, false, true>(s, a, slices, ws_front);
-    return launch_cfg<T, W, false, false>(s, a, slices, ws_front);
+int launch_layouts(hipStream_t s, DenseArgs<T>& a, bool ak, bool bk, int slices) {
+    if (ak && bk) return launch_cfg<T, W, true, true>(s, a, slices);
+    if (ak) return launch_cfg<T, W, true, false>(s, a, slices);
+    if (bk) return launch_cfg<T, W, false, true>(s, a, slices);
+    return launch_cfg<T, W, false, false>(s, a, slices);
 }
 
 }  // namespace split
@@ -112,10 +112,10 @@ bool split_takes(const DenseArgs<T>& a) {
 }
 
 template <typename T>
-bool launch_split(hipStream_t s, DenseArgs<T>& a, bool ak, bool bk, size_t ws_front, int* rc) {
+bool launch_split(hipStream_t s, DenseArgs<T>& a, bool ak, bool bk, int* rc) {
     if (!split_takes(a)) return false;
     const split::Choice c = split::choose<T>(a.M, a.N, a.K);
-    *rc = c.w == 2 ? split::launch_layouts<T, 2>(s, a, ak, bk, c.slices, ws_front) : split::launch_layouts<T, 1>(s, a, ak, bk, c.slices, ws_front);
+    *rc = c.w == 2 ? split::launch_layouts<T, 2>(s, a, ak, bk, c.slices) : split::launch_layouts<T, 1>(s, a, ak, bk, c.slices);
     return true;
 }
 
