@@ -22,16 +22,8 @@ namespace skinny {
 constexpr int WAVES = 8, THREADS = WAVES * 64, NMAX = 16;
 typedef float f32x4_v __attribute__((ext_vector_type(4)));
 template <typename T>
-struct Elem;
-template <>
-struct Elem<float> {
-    static constexpr int V = 4;                 // elements per 16 bytes: m per lane, and k per quarter and step
-    typedef uint32_t vec __attribute__((ext_vector_type(4), aligned(4)));
-};
-template <>
-struct Elem<bf16_t> {
-    static constexpr int V = 8;
-    typedef uint32_t vec __attribute__((ext_vector_type(4), aligned(2)));
+struct Elem {
+    static constexpr int V = 16 / (int)sizeof(T);   // elements per 16 bytes: m per lane, and k per quarter and step
 };
 
 template <typename T>
@@ -47,7 +39,7 @@ struct Args {
 template <typename T>
 __global__ __launch_bounds__(THREADS) void skinny_gemm_kernel(Args<T> a) {
     constexpr int V = Elem<T>::V, MT = 16 * V, KSTEP = 4 * V;
-    using vec = typename Elem<T>::vec;
+    using vec = typename UnalignedVec<T>::type;
     __shared__ float sums[WAVES][NMAX * MT];
     __shared__ uint32_t flag;
     const int block = blockIdx.x / a.slices, slice = blockIdx.x - block * a.slices;

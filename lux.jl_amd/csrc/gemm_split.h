@@ -203,7 +203,7 @@ struct Core {
         if (!arrive_last(p.counters + tile, (uint32_t)p.slices, &flag)) return false;
         ML::zero(acc);
         const uint64_t* all = reinterpret_cast<const uint64_t*>(p.partial) + (size_t)tile * p.slices * (PAIRS * THREADS) + threadIdx.x;
-#pragma unroll (WM * WN == 1 ? 4 : 1)
+#pragma unroll WM * WN == 1 ? 4 : 1
         for (int s = 0; s < p.slices; ++s) {
             uint64_t v[PAIRS];
             static_for<PAIRS>([&](auto Q) {
