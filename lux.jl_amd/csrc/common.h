@@ -31,6 +31,7 @@ int64_t option_conv_tile();       // 0 automatic, else a tile code of the bf16 w
 // `flags`: kWorkspaceFlags words reserved for the resident kernels' (value, epoch) exchange words;
 // `epoch` is a value no earlier call on the stream has used, so the words never need clearing and
 // no other kernel writes this memory.
+constexpr int64_t kMostThreads = int64_t(1) << 32;      // a launch has fewer threads than this
 constexpr size_t kWorkspaceCounters = 65536;
 constexpr size_t kWorkspaceFlags = 16384;
 // Counters of different channels are spread over different cache lines where the channel count

@@ -643,7 +643,8 @@ struct AnyPlan {
         if (R > 1 && R * g.Cin_g <= 65536 && g.dw == 1 && g.dh == 1) {
             uw = unite(g.W, g.pw, g.sw, rw);
             uh = unite(g.H, g.ph, g.sh, rh);
-            together = (double)uw.count * uh.count * uw.taps * uh.taps * cols((double)R * g.Cin_g);
+            if ((double)uw.taps * uh.taps * Cp * R * g.Cin_g * sizeof(T) < 2147483648.0)
+                together = (double)uw.count * uh.count * uw.taps * uh.taps * cols((double)R * g.Cin_g);
         }
         if (together < apart) {
             merged = 1;
@@ -684,7 +685,7 @@ static int pad_and_pack(hipStream_t s, const T* in, T* out, int P, int Cin, int 
     const int tiles_p = (int)ceil_div(std::max(P, zeros), 64), tiles_c = (int)ceil_div(Ct, 64);
     if (out != nullptr) blocks = Ct == V ? ceil_div((int64_t)P * N + zeros, 256) : (int64_t)tiles_p * tiles_c * (N + (zeros > 0));
     const int64_t pack = wout != nullptr ? ceil_div(ps->total, 256) : 0;
-    LUX_UNSUPPORTED_IF(blocks + pack >= (int64_t(1) << 24), "conv: tensor too large for the layout transform");
+    LUX_UNSUPPORTED_IF((blocks + pack) * 256 >= kMostThreads, "conv: tensor too large for the layout transform");
     if (blocks + pack == 0) return LUXHIP_OK;
     ProfScope prof("whcn_to_cwhn_kernel", s);
     pad_to_cwhn_pack_kernel<T><<<(unsigned)(blocks + pack), 256, 0, s>>>(in, out, P, Cin, Cg, Cp, groups, N, zeros, tiles_p, tiles_c, (int)blocks, w, wout,
@@ -754,12 +755,24 @@ static int run_conv_any(hipStream_t s, const ConvGeom& g, bool dgrad, const AnyP
         if (!dgrad) { a.SP = g.W; a.SQ = g.H; a.ss_w = g.sw; a.ss_h = g.sh; a.P = g.OW; a.Q = g.OH; a.os_w = a.os_h = 1; a.Ctot_out = g.Cout; }
         else { a.SP = g.OW; a.SQ = g.OH; a.ss_w = a.ss_h = 1; a.P = g.W; a.Q = g.H; a.os_w = g.sw; a.os_h = g.sh; a.Ctot_out = g.Cin; }
         a.PQ = a.P * a.Q;
-        a.Ncols = plan.Ncols; a.Cch = plan.Cch; a.res_w = std::max(plan.res_w, 1); a.merged = plan.merged; a.kW = g.kW; a.kH = g.kH;
-        a.col_off = gr.first * plan.Cch; a.act = act; a.subs = l.n;
+        a.Cch = plan.Cch; a.res_w = std::max(plan.res_w, 1); a.merged = plan.merged; a.kW = g.kW; a.kH = g.kH;
+        a.act = act; a.subs = l.n;
         a.divCp = FastDiv((uint32_t)plan.Cp); a.divCch = FastDiv((uint32_t)plan.Cch);
-        for (int i = 0; i < l.n; ++i) a.sub[i] = l.sub[i];
-        const int rc = cany::launch_any<T>(s, a, gr.n, ws_front, dgrad, plan.slices);
-        if (rc != LUXHIP_OK) return rc;
+        int kmax = 0;
+        for (int i = 0; i < l.n; ++i) kmax = std::max(kmax, l.sub[i].Kpad);
+        // the kernel's offsets into a tile's filter columns have 32 bits: of filters of 4 GiB fewer columns at a time
+        const int most = plan.merged ? plan.Ncols : (int)std::min<int64_t>(plan.Ncols, std::max<int64_t>(1, ((int64_t(1) << 31) / (int64_t)sizeof(T)) / std::max(kmax, 1)));
+        const int at_a_time = most >= std::min(plan.Ncols, 128) ? plan.Ncols : most;
+        for (int col = 0; col < plan.Ncols; col += at_a_time) {
+            a.Ncols = std::min(at_a_time, plan.Ncols - col);
+            a.col_off = gr.first * plan.Cch + col;
+            for (int i = 0; i < l.n; ++i) {
+                a.sub[i] = l.sub[i];
+                a.sub[i].wm += (int64_t)col * l.sub[i].Kpad;
+            }
+            const int rc = cany::launch_any<T>(s, a, gr.n, ws_front, dgrad, plan.slices && at_a_time == plan.Ncols);
+            if (rc != LUXHIP_OK) return rc;
+        }
     }
     return LUXHIP_OK;
 }
@@ -840,6 +853,7 @@ static int wgrad_plan(const ConvGeom& g, bool any, WgradPlan* p) {
     p->kslice = (int)ks;
     p->slices = (int)ceil_div(Ktotal, ks);
     LUX_UNSUPPORTED_IF(p->slices > 65535, "conv wgrad: too many k slices");
+    LUX_UNSUPPORTED_IF((int64_t)p->Mrows * p->Ncols >= (int64_t(1) << 31), "conv wgrad: filter of 2^31 or more elements");
     return LUXHIP_OK;
 }
 
@@ -869,7 +883,7 @@ static size_t wgrad_partial_bytes(const ConvGeom& g) {
     size_t bytes = 0;
     for (int any = 0; any < 2; ++any) {
         WgradPlan p;
-        if (wgrad_plan<T>(g, any != 0, &p) != LUXHIP_OK) return 0;
+        if (wgrad_plan<T>(g, any != 0, &p) != LUXHIP_OK) continue;      // run_wgrad refuses it if it is the one
         if (wgrad_window_shape<T>(g))
             p.slices = std::max(p.slices, wpatch::image_lanes(g.N, (g.Cin_g / 64) * ((g.Cout_g + 63) / 64), num_cus() > 0 ? num_cus() : 256));
         bytes = std::max(bytes, (size_t)p.slices * p.Mrows * p.Ncols * sizeof(float));

@@ -35,7 +35,7 @@ Choice choose_any(Sub* sub, int subs, int Ncols, int groups, bool may_slice) {
     constexpr size_t most_bytes = size_t(32) << 20;
     const int64_t cus = num_cus() > 0 ? num_cus() : 256;
     const Tile* tl = tiles<T>();
-    Choice best{0, 1, 0};
+    Choice best{3, 1, 0};                                            // 256 rows: no output has more tiles than a launch
     double t_best = 1e30;
     int kmax = 0;
     for (int i = 0; i < subs; ++i) kmax = std::max(kmax, sub[i].Kpad);
@@ -48,6 +48,7 @@ Choice choose_any(Sub* sub, int subs, int Ncols, int groups, bool may_slice) {
             work += (double)t * groups * (sub[i].Kpad + 100);
         }
         for (int sl = 1; sl <= 8; ++sl) {
+            if (nt * sl * split::THREADS >= kMostThreads) break;
             if (sl > 1 && (!may_slice || kmax / sl < 2 * BK || nt > 16384 || (size_t)(nt * sl) * tl[c].m * tl[c].n * sizeof(float) > most_bytes)) break;
             const double k = (double)kmax / sl + 100;
             const double per_cu = nt * sl <= 4 * cus ? (double)ceil_div(nt * sl, cus) * k : work / cus;
@@ -77,7 +78,7 @@ int launch_any(hipStream_t s, Args<T>& a, int groups, size_t ws_front, bool dgra
         q.first_block = blocks;
         q.first_tile = nt;
         const int64_t t = (int64_t)q.tiles_m * q.tiles_n;
-        LUX_UNSUPPORTED_IF(blocks + t * q.slices >= (int64_t(1) << 31), "conv: too many tiles");
+        LUX_UNSUPPORTED_IF((blocks + t * q.slices) * groups * split::THREADS >= kMostThreads, "conv: too many tiles");
         blocks += (int)(t * q.slices);
         if (q.slices > 1) nt += (int)t;
     }

@@ -206,6 +206,7 @@ static bool skinny_pays(int64_t M, int64_t K) {
 
 template <typename T>
 bool launch_skinny(hipStream_t s, DenseArgs<T>& d, bool ak, bool bk, int* rc) {
+    if (ceil_div(d.M, 16 * skinny::Elem<T>::V) * skinny::THREADS >= kMostThreads) return false;      // the tiled kernels are persistent
     if (ak || !bk || d.N > skinny::NMAX || d.N < 1 || d.M < 16 * skinny::Elem<T>::V || d.K < 1 || !skinny_pays<T>(d.M, d.K)) return false;
     *rc = skinny::launch<T>(s, d);
     return true;

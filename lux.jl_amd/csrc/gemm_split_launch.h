@@ -106,6 +106,7 @@ bool split_takes(const DenseArgs<T>& a) {
     const int64_t lim = (int64_t(1) << 31) / (256 * (int64_t)sizeof(T));
     if (std::max(a.A.sr, a.A.sk) >= lim || std::max(a.B.sr, a.B.sk) >= lim) return false;
     const int64_t cus = num_cus() > 0 ? num_cus() : 256;
+    if (ceil_div(a.M, 64) * ceil_div(a.N, 64) * split::THREADS >= kMostThreads) return false;        // the big-tile kernels are persistent
     if (a.A.vec_ok && a.B.vec_ok && a.K <= 128 && std::min(a.M, a.N) < 64 && ceil_div(std::max(a.M, a.N), 64) > 4 * cus) return false;
     const int64_t busy = sizeof(T) == 2 && a.K >= 512 ? cus / 2 : cus * 3 / 4;
     return !(whole_tiles<T, 128, 128>(a) && (int64_t)(a.M / 128) * (a.N / 128) > busy);
@@ -141,7 +142,7 @@ bool launch_split_pair(hipStream_t s, DenseArgs<T>& a, DenseArgs<T>& b, int* rc)
     // one counter for each tile of a product with slices, those of b behind those of a
     const int64_t counters_a = pa.slices > 1 ? (int64_t)a.tiles_m * a.tiles_n : 0;
     const int64_t counters_b = pb.slices > 1 ? (int64_t)b.tiles_m * b.tiles_n : 0;
-    if (counters_a + counters_b > (int64_t)kWorkspaceCounters || na + nb >= (int64_t(1) << 31)) return false;
+    if (counters_a + counters_b > (int64_t)kWorkspaceCounters || (na + nb) * THREADS >= kMostThreads) return false;
     if (front > 0) {
         Workspace ws;
         *rc = get_workspace(s, front, &ws);
