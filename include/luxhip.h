@@ -426,7 +426,9 @@ typedef struct luxhip_conv_dims {
  * (bias == NULL, act identity) and Impl.conv_bias_act(::Type{Dev}, x, w, cdims, bias, act)
  * (src/impl/conv.jl:29-60,138-166).  pre (optional) receives conv .+ bias.  xt_keep (optional, as
  * large as x): receives the channel-contiguous copy of x that the kernels read; an rrule keeps it
- * next to x and hands it to luxhip_fused_conv_bwd, which then does not make it again. */
+ * next to x and hands it to luxhip_fused_conv_bwd, which then does not make it again.  Where the channels
+ * of a group are no multiple of 16 bytes the kernels read a padded copy of their own, and xt_keep costs a
+ * pass that saves none: an rrule passes NULL there. */
 int luxhip_conv_fwd(luxhip_stream_t s, int dtype, int act, const luxhip_conv_dims_t* d, const void* x,
                     const void* w, const void* bias, void* y, void* pre, void* xt_keep);
 /* dx = ∇conv_data(dy, w, cdims) (src/impl/conv.jl:128-131). */

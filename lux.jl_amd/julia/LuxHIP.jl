@@ -538,15 +538,17 @@ function Impl.∇conv_filter(x::HIPArray{T,4}, dy::HIPArray{T,4}, cdims::DenseCo
 end
 
 # CRC.rrule(fused_conv) + ∇fused_conv (impl/conv.jl:204-275) as one forward and one pullback call.  The forward
-# pass hands over the channel-contiguous copy of x that its kernels read (xt_keep); the pullback's filter
-# gradient reads it instead of transposing x again.
+# pass hands over the channel-contiguous copy of x that its kernels read (xt_keep), unless they pad it; the
+# pullback's filter gradient reads it instead of transposing x again.
 function CRC.rrule(::CRC.RuleConfig{>:CRC.HasReverseMode}, ::typeof(Impl.fused_conv), ::HIPOp, act::F, w::HIPArray{T,4}, x::HIPArray{T,4},
         bias::Union{Nothing,HIPArray{T,1}}, cdims::DenseConvDims{2}) where {F,T<:HIPFloat}
     id = act_id(act)
     id === nothing && throw(HIPFallbackError("the pullback of fused_conv with activation $(act)"))
     y = similar(x, T, (NNlib.output_size(cdims)..., NNlib.channels_out(cdims), size(x, 4)))
     pre = id in (4, 5, 6, 7, 8) ? similar(y) : nothing
-    xt = similar(x)
+    # where the kernels pad the channels of a group to whole 16-byte chunks their copy is not of x's size, and making it again
+    # in the pullback costs less than a second, unpadded one
+    xt = (size(x, 3) ÷ NNlib.groupcount(cdims)) * sizeof(T) % 16 == 0 ? similar(x) : nothing
     d = Ref(ConvDimsC(cdims, size(x, 4)))
     check(ccall((:luxhip_conv_fwd, libluxhip), Cint,
         (Ptr{Cvoid}, Cint, Cint, Ptr{ConvDimsC}, Ptr{Cvoid}, Ptr{Cvoid}, Ptr{Cvoid}, Ptr{Cvoid}, Ptr{Cvoid}, Ptr{Cvoid}),

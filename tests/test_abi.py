@@ -309,3 +309,11 @@ def test_julia_struct_mirrors_the_conv_descriptor():
     for (cn, jt_want, n), (jn, jt) in zip(flat, jfields):
         want = jt_want if n == 1 else f"NTuple{{{n},{jt_want}}}"
         assert jt.replace(" ", "") == want, f"field {cn}/{jn}: C {n} x {jt_want}, Julia {jt}"
+
+
+def test_both_hosts_keep_the_copy_of_x_under_the_same_rule():
+    """luxhip_conv_fwd's xt_keep costs a pass that saves none where the kernels pad a group's channels to 16 bytes: the
+    rrules of both host layers pass NULL there."""
+    python = open(os.path.join(ROOT, "lux.jl_amd", "luxlib.py")).read()
+    assert "if (cdims._c.Cin // cdims.groups) * x.itemsize % 16 == 0 else None" in python
+    assert "xt = (size(x, 3) ÷ NNlib.groupcount(cdims)) * sizeof(T) % 16 == 0 ? similar(x) : nothing" in open(JULIA_GLUE).read()
