@@ -1,13 +1,14 @@
 """Convolutions of any channel count and stride (conv_any.h) against the fp64 oracle: padded channels, the residues of a
-strided input gradient apart and merged, taps that some residues do not have, contractions shorter than a stage and cut into
-slices, and the kept copy of x whose channels the kernels would pad."""
+strided input gradient apart and merged, taps that some residues do not have and residues without taps, non-finite cotangents,
+groups in one launch and a few at a time, contractions shorter than a stage and cut into slices, and the kept copy of x whose
+channels the kernels would pad."""
 import ctypes as C
 
 import numpy as np
 import pytest
 
 from oracle import luxlib_oracle as O
-from tests.util import assert_close, dev, f64, host_inputs, kernels_of, stable_seed
+from tests.util import assert_close, dev, f64, host_inputs, kernels_of, rms, stable_seed
 
 pytestmark = pytest.mark.gpu
 
@@ -56,6 +57,35 @@ def test_conv_any(gpu, dtype, case):
     np.testing.assert_array_equal(fx.to_numpy(), gx.to_numpy())
     np.testing.assert_array_equal(fw.to_numpy(), gw.to_numpy())
     assert_close(fb.to_numpy(), f64(dy).sum(axis=(0, 1, 3)), dtype, tag + " db")
+
+
+@pytest.mark.parametrize("dtype", ["f32", "bf16"])
+@pytest.mark.parametrize("act", ["relu", "gelu"])
+@pytest.mark.parametrize("case", range(len(CASES)))
+def test_fused_pullback_with_an_activation(gpu, dtype, act, case):
+    """Derivatives from the output (relu) and from the pre-activation (gelu), through the dz pass of either kind (bf16 channels
+    in whole vectors: one pass writes both layouts, else a pass and a padding copy)."""
+    xs, ws, stride, pad, dil, groups, flip = CASES[case]
+    rng = np.random.default_rng(stable_seed("conv_any act", case, act))
+    kw = dict(stride=stride, padding=pad, dilation=dil, groups=groups, flipkernel=flip)
+    gd, od = gpu.DenseConvDims(xs, ws, **kw), O.ConvDims(xs, ws, **kw)
+    x, w, b, delta = host_inputs(dtype, rng.normal(size=xs), rng.normal(size=ws) / np.sqrt(ws[0] * ws[1] * ws[2]), 0.1 * rng.normal(size=ws[3]),
+                                 rng.normal(size=od.y_shape()))
+    y, back = gpu.pullback(gpu.fused_conv_bias_activation, act, dev(gpu, w, dtype), dev(gpu, x, dtype), dev(gpu, b, dtype), gd)
+    gw, gx, gb = back(dev(gpu, delta, dtype))
+    wy, wdw, wdx, wdb = O.fused_conv_pullback(act, f64(w), f64(x), f64(b), od, f64(delta))
+    if dtype == "bf16":                                     # y, the pre-activation and dz are stored in bf16 in between
+        pre = O.bias_add(O.conv(f64(x), f64(w), od), f64(b))
+        yq, preq = (f64(O.round_to_bf16(a.astype(np.float32))) for a in (wy, pre))
+        dzx = O.grad_activation(f64(delta), yq, act, preq)
+        dz = f64(O.round_to_bf16(dzx.astype(np.float32)))
+        wdw, wdx, wdb = O.conv_filter_grad(f64(x), dz, od), O.conv_data_grad(dz, f64(w), od), O.grad_bias_add(b, dzx)
+    tag = f"{dtype} {act} conv_any {case}"
+    per = np.sqrt(np.prod(od.y_shape()) / ws[3]) * rms(delta)          # terms of a sum over one channel's positions
+    assert_close(y.to_numpy(), wy, dtype, tag + " y")
+    assert_close(gw.to_numpy(), wdw, dtype, tag + " dw", scale=per * rms(x) * 0.5)
+    assert_close(gx.to_numpy(), wdx, dtype, tag + " dx", scale=np.sqrt(ws[0] * ws[1] * ws[3] / groups) * rms(delta) * rms(w) * 0.5)
+    assert_close(gb.to_numpy(), wdb, dtype, tag + " db", scale=per * 0.5)
 
 
 @pytest.mark.parametrize("xs,ws,stride,dil,launches", [
