@@ -48,6 +48,7 @@ template <typename T>
 struct Args {
     const T* src;              // channel-contiguous, first channel of the first group of the launch (one blockIdx.y each)
     const T* wm;               // its packed filter
+    int64_t wm_group;          // packed filter elements per group
     const void* zero;
     const T* bias;
     T *out, *pre;
@@ -56,15 +57,15 @@ struct Args {
     int os_w, os_h;
     int Ncols, Cch;            // columns; channels per residue (merged: Ncols = residues * Cch)
     int res_w;                 // merged: residues along w
-    int kW, kH;                // merged (dilation 1): tap t of residue r is filter tap t * os + r, where there is one
     int col_off, Ctot_out, act;
     int subs, merged;          // merged: the residues are columns
-    int64_t wm_group, partial_group;   // packed filter elements and bytes of partial sums per group
-    int sliced_tiles;          // counters per group
     char* partial;
     uint32_t* counters;
     FastDiv divCp, divCch;
     Sub sub[MAX_SUBS];
+    int64_t partial_group;     // bytes of partial sums per group
+    int sliced_tiles;          // counters per group
+    int kW, kH;                // merged (dilation 1): tap t of residue r is filter tap t * os + r, where there is one
 };
 
 // A: K-major rows of the im2col matrix
