@@ -490,7 +490,7 @@ static bool ln_ragged_vectors(int64_t L, int64_t nvec) {
 // x 512 11.6 / 14.6, x 4096 41.9 / 39.1).
 template <typename T>
 static bool ln_ragged_fused(int64_t L, int64_t R, int64_t nvec) {
-    if (sizeof(T) == 2 && L > 2048 && R >= 1024 && R < 3072) return false;
+    if (sizeof(T) == 2 && L > 2048 && R >= 768 && R < 3072) return false;
     return R <= 2048 || nvec >= (sizeof(T) == 2 ? 52 : 60);
 }
 
