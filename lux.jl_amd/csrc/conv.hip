@@ -149,14 +149,15 @@ struct PackSubs {
 template <typename T>
 __device__ __forceinline__ void pack_sub_element(const T* __restrict__ w, T* __restrict__ out, const ConvGeom& g, const PackSubs& ps, int64_t idx) {
     if (idx >= ps.total) return;
-    const int grp = (int)(idx / ps.per_group);
+    const bool small = ps.total < (int64_t(1) << 31);      // uniform; 64-bit divisions take longer than the rest
+    const int grp = small ? (int)((uint32_t)idx / (uint32_t)ps.per_group) : (int)(idx / ps.per_group);
     idx -= grp * ps.per_group;
     PackSub q = ps.sub[0];
 #pragma unroll
     for (int i = 1; i < cany::MAX_SUBS; ++i)
         if (i < ps.n && idx >= ps.sub[i].first) q = ps.sub[i];
     const int64_t e = idx - q.first;
-    const int col = (int)(e / q.Kpad), k = (int)(e - (int64_t)col * q.Kpad);
+    const int col = small ? (int)((uint32_t)e / (uint32_t)q.Kpad) : (int)(e / q.Kpad), k = (int)(e - (int64_t)col * q.Kpad);
     T v = T(0);
     const int t = k / ps.Cp, c = k - t * ps.Cp;
     const int th = t / q.TW, tw = t - th * q.TW;

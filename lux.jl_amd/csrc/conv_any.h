@@ -59,12 +59,12 @@ struct Args {
     int res_w;                 // merged: residues along w
     int col_off, Ctot_out, act;
     int subs, merged;          // merged: the residues are columns
+    int sliced_tiles;          // counters per group
     char* partial;
+    int64_t partial_group;     // bytes of partial sums per group
     uint32_t* counters;
     FastDiv divCp, divCch;
     Sub sub[MAX_SUBS];
-    int64_t partial_group;     // bytes of partial sums per group
-    int sliced_tiles;          // counters per group
     int kW, kH;                // merged (dilation 1): tap t of residue r is filter tap t * os + r, where there is one
 };
 
@@ -150,7 +150,7 @@ __device__ __forceinline__ float own_taps_sum(const Args<T>& g, const Sub& q, co
 }
 
 // MERGED: the residues of an input gradient are columns and a NaN among the sums is looked into.  A kernel of its own: the test
-// costs 3 to 5 %, and a register that takes a wave from every SIMD unless it is told to stay below (256 x 32 tiles of the first
+// costs 2 to 4 %, and a register that takes a wave from every SIMD unless it is told to stay below (256 x 32 tiles of the first
 // layer, 78 us with four waves, 85 with three).
 template <typename T, int WM, int WN, int NWM, int NWN, bool MERGED>
 __global__ __launch_bounds__(split::THREADS, MERGED && WM * WN < 4 ? 4 : 1) void conv_any_kernel(Args<T> g) {
@@ -186,6 +186,14 @@ __global__ __launch_bounds__(split::THREADS, MERGED && WM * WN < 4 ? 4 : 1) void
                       g.counters + grp * g.sliced_tiles + q.first_tile};
         if (!Core::combine(p, tile, slice, acc)) return;
     }
+    bool nan = false;                  // among this lane's sums (here, where no lane is masked off: two instructions per sum)
+    if constexpr (MERGED) {
+        static_for<WM * WN * 16>([&](auto E) {
+            constexpr int e = decltype(E)::value;
+            const float v = acc[e / (WN * 16)][e / 16 % WN][e % 16];
+            nan |= v != v;
+        });
+    }
     // rows -> output positions
     const int mb = ML::lane_m(m0), nb = ML::lane_n(n0);
     int64_t row[WM];
@@ -201,7 +209,6 @@ __global__ __launch_bounds__(split::THREADS, MERGED && WM * WN < 4 ? 4 : 1) void
         ih[i] = b * g.os_h + q.oh0;
         row[i] = (int64_t)n * g.Ctot_out * g.PQ + (int64_t)ih[i] * g.P + iw[i];
     }
-    bool nan = false;                  // merged: among this lane's sums
     static_for<WN * 16>([&](auto JR) {
         constexpr int j = decltype(JR)::value / 16, r = decltype(JR)::value % 16;
         const int col = nb + j * 32 + ((r >> 2) << 3) + (r & 3);
@@ -221,10 +228,7 @@ __global__ __launch_bounds__(split::THREADS, MERGED && WM * WN < 4 ? 4 : 1) void
             for (int i = 0; i < WM; ++i) {
                 v[i] = acc[i][j][r] + bv;
                 st_ok[i] = ok[i];
-                if (g.merged) {
-                    st_ok[i] = ok[i] && (unsigned)(iw[i] + rw) < (unsigned)g.P && (unsigned)(ih[i] + rh) < (unsigned)g.Q;
-                    if constexpr (MERGED) nan = nan || v[i] != v[i];
-                }
+                if (g.merged) st_ok[i] = ok[i] && (unsigned)(iw[i] + rw) < (unsigned)g.P && (unsigned)(ih[i] + rh) < (unsigned)g.Q;
             }
             if (g.pre != nullptr) {
 #pragma unroll
