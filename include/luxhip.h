@@ -297,6 +297,28 @@ int luxhip_attention_weights_pullback(luxhip_stream_t s, int dtype, int64_t S, i
                                       const int64_t* strides_o, const void* probs, double scale, void* dlogits,
                                       int64_t ldc, const int64_t* strides_c, int structure);
 
+/* scaled_dot_product_attention (src/impl/attention.jl:5-117) without a mask array, a bias or an fdrop, bf16 storage, in one
+ * kernel: the logits never go to memory.  probs (S, L, H, B): the weights, rounded; out (Ev, H, L, B): their product with v,
+ * rounded, and out_wide: the same unrounded (fp32), which the pullback reads.  batch_dims: query heads per key / value head,
+ * key / value heads, batches; strides_q, _k, _v: elements between tokens, heads (of q: query heads) and batches; features are
+ * contiguous.  scale and causal as in luxhip_attention_softmax_fwd.  LUXHIP_UNSUPPORTED (nothing is launched) where the
+ * kernels do not apply: more than 128 features, features or strides that are no multiples of 8, operands not 16-byte aligned
+ * (probs: any alignment), no keys, another dtype; luxhip_batched_matmul_strided and luxhip_attention_softmax_fwd take those. */
+int luxhip_attention_fwd(luxhip_stream_t s, int dtype, int64_t E, int64_t Ev, int64_t S, int64_t L,
+                         const int64_t* batch_dims, double scale, int causal, const void* q, const int64_t* strides_q,
+                         const void* k, const int64_t* strides_k, const void* v, const int64_t* strides_v, void* probs,
+                         void* out, float* out_wide);
+
+/* Its pullback (the batched products' rules, src/impl/batched_mul.jl:320-334, and the softmax rule), without the cotangent
+ * of the logits in memory: dq like q, dk and dv like k and v (the same strides) plus a stride of dk_repeat / dv_repeat
+ * elements between the query heads that share a key / value head (their sum is the caller's: luxhip_batch_sum).  probs and
+ * out_wide as the forward pass wrote them, d_out like out.  LUXHIP_UNSUPPORTED as above. */
+int luxhip_attention_bwd(luxhip_stream_t s, int dtype, int64_t E, int64_t Ev, int64_t S, int64_t L,
+                         const int64_t* batch_dims, double scale, int causal, const void* q, const int64_t* strides_q,
+                         const void* k, const int64_t* strides_k, const void* v, const int64_t* strides_v,
+                         const void* probs, const float* out_wide, const void* d_out, void* dq, void* dk,
+                         int64_t dk_repeat, void* dv, int64_t dv_repeat);
+
 /* ---------------------------------------------------------------- dropout ----------
  * The reference draws its noise with `rand!(rng, y)` from the array package's generator
  * (src/impl/dropout.jl:171-190); here a counter-based Philox4x32-10 stream stands in for it:

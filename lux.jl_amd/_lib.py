@@ -74,6 +74,9 @@ SIGNATURES = {
     "luxhip_instancenorm_running_stats": [_vp, _i, _i64, _i64, _i64, _fp, _fp, _d, _d, _vp, _vp, _vp, _vp],
     "luxhip_attention_softmax_fwd": [_vp, _i, _i64, _i64, _i64, _i64, _vp, _d, _i, _vp, _i64, _i64, _vp, _i64, _i64, _vp],
     "luxhip_attention_softmax_bwd": [_vp, _i, _i64, _i64, _i64, _i, _vp, _vp, _d, _vp],
+    "luxhip_attention_fwd": [_vp, _i, _i64, _i64, _i64, _i64, _ip64, _d, _i, _vp, _ip64, _vp, _ip64, _vp, _ip64, _vp, _vp, _fp],
+    "luxhip_attention_bwd": [_vp, _i, _i64, _i64, _i64, _i64, _ip64, _d, _i, _vp, _ip64, _vp, _ip64, _vp, _ip64, _vp, _fp, _vp, _vp, _vp,
+                             _i64, _vp, _i64],
     "luxhip_rand_uniform": [_vp, _i, _i64, _u64, _u64, _vp],
     "luxhip_dropout_fwd": [_vp, _i, _i64, _u64, _u64, _d, _d, _vp, _vp, _vp],
     "luxhip_dropout_mask": [_vp, _i, _i64, _d, _d, _vp],

@@ -274,6 +274,23 @@ __global__ __launch_bounds__(256) void attn_rowdot_quad_kernel(const T* __restri
     if (sub == 0 && col < cols) d[col] = acc;
 }
 
+template <typename T, typename TO>
+int attention_rowdot(hipStream_t s, const T* d_out, const TO* out, float* d, int64_t Ev, int64_t L, int64_t ldo, const int64_t* batch_dims,
+                     const int64_t* so) {
+    const int64_t cols = batch_dims[0] * batch_dims[1] * batch_dims[2] * L;
+    const int b0 = (int)batch_dims[0], b1 = (int)batch_dims[1];
+    const bool quad = Ev % 4 == 0 && ldo % 4 == 0 && so[0] % 4 == 0 && so[1] % 4 == 0 && so[2] % 4 == 0 &&
+                      reinterpret_cast<uintptr_t>(d_out) % (4 * sizeof(T)) == 0 && reinterpret_cast<uintptr_t>(out) % (4 * sizeof(TO)) == 0;
+    const unsigned grid = (unsigned)ceil_div(cols, quad ? 16 : 4);
+    ProfScope ps("attn_rowdot_kernel", s);
+    if (quad) attn_rowdot_quad_kernel<T, TO><<<grid, 256, 0, s>>>(d_out, out, d, (int)Ev, (int)L, ldo, b0, b1, so[0], so[1], so[2], cols);
+    else attn_rowdot_kernel<T, TO><<<grid, 256, 0, s>>>(d_out, out, d, (int)Ev, (int)L, ldo, b0, b1, so[0], so[1], so[2], cols);
+    LUX_CHECK_LAUNCH();
+    return LUXHIP_OK;
+}
+template int attention_rowdot<bf16_t, float>(hipStream_t, const bf16_t*, const float*, float*, int64_t, int64_t, int64_t, const int64_t*,
+                                             const int64_t*);
+
 static int gemm_check(int dtype, int act, int64_t M, int64_t N, int64_t K) {
     LUX_UNSUPPORTED_IF(dtype != LUXHIP_F32 && dtype != LUXHIP_BF16, "unsupported dtype %d", dtype);
     LUX_UNSUPPORTED_IF(act < 0 || act >= LUXHIP_ACT_COUNT, "unsupported activation id %d", act);
@@ -363,27 +380,10 @@ int luxhip_attention_weights_pullback(luxhip_stream_t s, int dtype, int64_t S, i
     rc = get_workspace((hipStream_t)s, (size_t)cols * sizeof(float), &ws);
     if (rc != LUXHIP_OK) return rc;
     float* d = reinterpret_cast<float*>(ws.data);
-    {
-        ProfScope ps("attn_rowdot_kernel", (hipStream_t)s);
-        const int b0 = (int)batch_dims[0], b1 = (int)batch_dims[1];
-        const int64_t* so = strides_o;
-        const size_t eo = dtype == LUXHIP_F32 || wide ? 4 : 2, ed = dtype == LUXHIP_F32 ? 4 : 2;      // element sizes of out and d_out
-        const bool quad = Ev % 4 == 0 && ldo % 4 == 0 && so[0] % 4 == 0 && so[1] % 4 == 0 && so[2] % 4 == 0 &&
-                          reinterpret_cast<uintptr_t>(d_out) % (4 * ed) == 0 && reinterpret_cast<uintptr_t>(out) % (4 * eo) == 0;
-        const unsigned grid = (unsigned)ceil_div(cols, quad ? 16 : 4);
-#define ROWDOT(T, TO)                                                                                                                   \
-    do {                                                                                                                                \
-        if (quad) attn_rowdot_quad_kernel<T, TO><<<grid, 256, 0, (hipStream_t)s>>>((const T*)d_out, (const TO*)out, d, (int)Ev, (int)L, ldo, \
-                                                                                   b0, b1, so[0], so[1], so[2], cols);                  \
-        else attn_rowdot_kernel<T, TO><<<grid, 256, 0, (hipStream_t)s>>>((const T*)d_out, (const TO*)out, d, (int)Ev, (int)L, ldo, b0, b1, \
-                                                                         so[0], so[1], so[2], cols);                                   \
-    } while (0)
-        if (dtype == LUXHIP_F32) ROWDOT(float, float);
-        else if (wide) ROWDOT(bf16_t, float);
-        else ROWDOT(bf16_t, bf16_t);
-#undef ROWDOT
-        LUX_CHECK_LAUNCH();
-    }
+    if (dtype == LUXHIP_F32) rc = attention_rowdot((hipStream_t)s, (const float*)d_out, (const float*)out, d, Ev, L, ldo, batch_dims, strides_o);
+    else if (wide) rc = attention_rowdot((hipStream_t)s, (const bf16_t*)d_out, (const float*)out, d, Ev, L, ldo, batch_dims, strides_o);
+    else rc = attention_rowdot((hipStream_t)s, (const bf16_t*)d_out, (const bf16_t*)out, d, Ev, L, ldo, batch_dims, strides_o);
+    if (rc != LUXHIP_OK) return rc;
     // dprobs (S x L) = v' (S x Ev) * d_out (Ev x L), with the softmax rule as its epilogue
     if (dtype == LUXHIP_F32)
         return batched_impl<float>((hipStream_t)s, 1, 0, S, L, Ev, batch_dims, (const float*)v, ldv, strides_v, (const float*)d_out, ldo,

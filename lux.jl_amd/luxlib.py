@@ -658,6 +658,12 @@ class _AttnLayout:
         self.batch = a.size // self.sb if self.sb else 0
 
 
+def _attention_spans(lq, lk, lv, Ev, H, B) -> bool:
+    """What the fused kernels address with 32-bit byte offsets inside a head, and their grid."""
+    span = max(lq.tokens * lq.st, lk.tokens * lk.st, lv.tokens * lv.st, lq.tokens * H * Ev)
+    return 2 * span < 1 << 31 and H * B < 1 << 23 and -(-max(lq.tokens, lk.tokens) // 128) * H * B < 1 << 23
+
+
 def _permute_leading3(a: DeviceArray, perm) -> DeviceArray:
     """permutedims(a, (perm..., 4:N...))."""
     out = DeviceArray(tuple(a.shape[p - 1] for p in perm) + tuple(a.shape[3:]), a.dtype)
@@ -737,33 +743,61 @@ def rrule_scaled_dot_product_attention(q, k, v, head_dim=1, token_dim=3, scale=N
     # (a logit rounded to bf16 is off by 2^-9 |logit|, the weight then by that relative amount)
     wide = "f32" if dt == "bf16" else dt
     sm_code = _BF16_WIDE if dt == "bf16" else None
-    logits = DeviceArray((S, L, H) + bshape, wide)
     sC = (S * L, S * L * r, S * L * H)
     # a causal mask (keep s <= l) leaves whole tiles of the logits unused and makes the weights and every
     # cotangent of the same shape triangular: the products skip what is known to be zero or unused
     causal = bool(is_causal)
     tri = causal and fdrop is None       # an arbitrary fdrop need not keep the masked weights at zero
-    _bmm_strided(True, False, S, L, E, bdims, k, lk.st, (0, lk.sh, lk.sb), q, lq.st, (lq.sh, lq.sh * r, lq.sb), logits, S, sC,
-                 1 if causal else 0)
-    probs = DeviceArray((S, L, H) + bshape, dt)
-    _lib.call("luxhip_attention_softmax_fwd", current_stream(), probs.code if sm_code is None else sm_code, S, L, H, B, logits.ptr, scale_inv,
-              int(causal), _p(mask_a), mask_sh, mask_sb, _p(bias_a), bias_sh, bias_sb, probs.ptr)
-    softmax_out, fdrop_back = probs, None
-    if fdrop is not None:
-        probs, fdrop_back = fdrop(softmax_out)         # impl/attention.jl:88-104: fdrop(softmax(...))
     so = (Ev, Ev * r, Ev * H * L)
-    # bf16 without an fdrop: the product is written unrounded (fp32) and kept for the pullback, whose softmax rule takes
+    probs = DeviceArray((S, L, H) + bshape, dt)
+    # bf16 without an fdrop: the product is also kept unrounded (fp32) for the pullback, whose softmax rule takes
     # its inner product from it; the array that is returned is its rounded copy
     out_wide = DeviceArray((Ev, H, L) + bshape, wide) if (fdrop is None and wide != dt) else None
-    out = out_wide if out_wide is not None else DeviceArray((Ev, H, L) + bshape, dt)
-    _bmm_strided(False, False, Ev, L, S, bdims, v, lv.st, (0, lv.sh, lv.sb), probs, S, sC, out, Ev * H, so, 2 if tri else 0)
-    if out_wide is not None:
-        out = _convert(out_wide, dt)
+    # one kernel each way where it applies (bf16, whole 16-byte vectors of at most 128 features): luxhip_attention_fwd / _bwd
+    fused = (out_wide is not None and mask_a is None and bias_a is None and 0 < E <= 128 and 0 < Ev <= 128 and E % 8 == 0 and Ev % 8 == 0
+             and S > 0 and L > 0 and H > 0 and B > 0 and (q.ptr | k.ptr | v.ptr) % 16 == 0
+             and _attention_spans(lq, lk, lv, Ev, H, B))
+    logits, softmax_out, fdrop_back = None, probs, None
+    out = DeviceArray((Ev, H, L) + bshape, dt)
+    strides = (_i64x3((lq.st, lq.sh, lq.sb)), _i64x3((lk.st, lk.sh, lk.sb)), _i64x3((lv.st, lv.sh, lv.sb)))
+    if fused:
+        _lib.call("luxhip_attention_fwd", current_stream(), probs.code, E, Ev, S, L, _i64x3(bdims), scale_inv, int(causal), q.ptr, strides[0],
+                  k.ptr, strides[1], v.ptr, strides[2], probs.ptr, out.ptr, out_wide.ptr)
+    else:
+        logits = DeviceArray((S, L, H) + bshape, wide)
+        _bmm_strided(True, False, S, L, E, bdims, k, lk.st, (0, lk.sh, lk.sb), q, lq.st, (lq.sh, lq.sh * r, lq.sb), logits, S, sC,
+                     1 if causal else 0)
+        _lib.call("luxhip_attention_softmax_fwd", current_stream(), probs.code if sm_code is None else sm_code, S, L, H, B, logits.ptr, scale_inv,
+                  int(causal), _p(mask_a), mask_sh, mask_sb, _p(bias_a), bias_sh, bias_sb, probs.ptr)
+        if fdrop is not None:
+            probs, fdrop_back = fdrop(softmax_out)         # impl/attention.jl:88-104: fdrop(softmax(...))
+        product = out if out_wide is None else out_wide
+        _bmm_strided(False, False, Ev, L, S, bdims, v, lv.st, (0, lv.sh, lv.sb), probs, S, sC, product, Ev * H, so, 2 if tri else 0)
+        if out_wide is not None:
+            _lib.call("luxhip_convert", current_stream(), out_wide.code, out.code, out.size, out_wide.ptr, out.ptr)
 
     def back(d_out: DeviceArray, d_probs: Optional[DeviceArray] = None):
         if d_probs is not None:
             raise _lib.Unsupported(_lib.UNSUPPORTED, "attention: a cotangent for the returned weights")
-        dlogits = logits if logits.dtype == dt else DeviceArray(logits.shape, dt)   # the logits are no longer needed
+
+        def repeats(like):       # one gradient per query head; those that share a key/value group are summed afterwards
+            return DeviceArray(((r,) if r > 1 else ()) + tuple(like.shape), dt)
+
+        def summed(full, like):  # pullback of repeat_inner_gqa
+            if r == 1:
+                return full
+            red = DeviceArray(like.shape, dt)
+            _lib.call("luxhip_batch_sum", current_stream(), red.code, like.size, r, full.ptr, red.ptr)
+            return red
+
+        if fused and d_out.dtype == dt and d_out.ptr % 16 == 0:
+            dq, dk, dv = DeviceArray(q.shape, dt), repeats(k), repeats(v)
+            _lib.call("luxhip_attention_bwd", current_stream(), softmax_out.code, E, Ev, S, L, _i64x3(bdims), scale_inv, int(causal), q.ptr,
+                      strides[0], k.ptr, strides[1], v.ptr, strides[2], softmax_out.ptr, out_wide.ptr, d_out.ptr, dq.ptr, dk.ptr,
+                      k.size if r > 1 else 0, dv.ptr, v.size if r > 1 else 0)
+            return dq, summed(dk, k), summed(dv, v)
+        # the logits are no longer needed
+        dlogits = logits if logits is not None and logits.dtype == dt else DeviceArray(softmax_out.shape, dt)
         if fdrop_back is None:
             # the cotangent of the weights (v' d_out) and the softmax rule in one: the cotangent stays in the product's
             # fp32 accumulators, its inner product with the weights comes from d_out and out
@@ -786,16 +820,11 @@ def rrule_scaled_dot_product_attention(q, k, v, head_dim=1, token_dim=3, scale=N
                      (lq.sh, lq.sh * r, lq.sb), 2 if tri else 0)
 
         def kv_grad(like, lay, A, lda, sA, Bm):
-            # (rows of `like`) x S = A (rows x L) * Bm' (L x S), one product per head; the heads that share
-            # a key/value group are summed afterwards (pullback of repeat_inner_gqa)
-            full = DeviceArray(((r,) if r > 1 else ()) + tuple(like.shape), dt)
+            # (rows of `like`) x S = A (rows x L) * Bm' (L x S), one product per head
+            full = repeats(like)
             _bmm_strided(False, True, lay.E, S, L, bdims, A, lda, sA, Bm, S, sC, full, lay.st,
                          (like.size if r > 1 else 0, lay.sh, lay.sb), 3 if tri else 0)
-            if r == 1:
-                return full
-            red = DeviceArray(like.shape, dt)
-            _lib.call("luxhip_batch_sum", current_stream(), red.code, like.size, r, full.ptr, red.ptr)
-            return red
+            return summed(full, like)
 
         dv = kv_grad(v, lv, d_out, Ev * H, so, probs)
         dk = kv_grad(k, lk, q, lq.st, (lq.sh, lq.sh * r, lq.sb), dlogits)

@@ -1,0 +1,77 @@
+"""The fused attention kernels (bf16, no mask array, bias or fdrop) at the edges of their tiles: 128 columns per
+workgroup, 32 per wave, 64 (32) rows per tile, 32 features per accumulator tile, eight heads per turn over the XCDs."""
+import numpy as np
+import pytest
+
+from oracle import luxlib_oracle as O
+from tests.util import assert_close, dev, f64, host_inputs, kernels_of, stable_seed
+
+pytestmark = pytest.mark.gpu
+
+CASES = [
+    # E, Ev, H, G, L, S, B, token_dim, causal
+    (8, 8, 1, 1, 1, 1, 1, 3, False), (32, 32, 2, 2, 31, 33, 1, 3, False), (40, 16, 2, 1, 65, 63, 2, 3, True),
+    (64, 64, 8, 2, 129, 127, 1, 3, False), (64, 72, 3, 3, 257, 193, 1, 2, True), (96, 96, 4, 4, 128, 256, 2, 3, True),
+    (80, 48, 2, 2, 160, 100, 1, 3, True), (128, 128, 8, 8, 256, 256, 1, 2, False), (128, 128, 2, 1, 384, 385, 1, 3, True),
+    (128, 104, 16, 8, 97, 300, 1, 3, False), (16, 128, 8, 1, 200, 130, 2, 3, True),
+]
+
+
+@pytest.mark.parametrize("case", range(len(CASES)))
+def test_edges_of_the_tiles(gpu, case):
+    E, Ev, H, G, L, S, B, token_dim, causal = CASES[case]
+    rng = np.random.default_rng(stable_seed("attn-fused", case))
+    shape = (lambda e, h, t: ((e, h, t) if token_dim == 3 else (e, t, h)) + (B,))
+    q, k, v = host_inputs("bf16", rng.normal(size=shape(E, H, L)), rng.normal(size=shape(E, G, S)), rng.normal(size=shape(Ev, G, S)))
+    dq_, dk_, dv_ = (dev(gpu, a, "bf16") for a in (q, k, v))
+    # memory that no kernel wrote would show up as NaN
+    poison = [dev(gpu, np.full(n, np.nan, np.float32), "bf16") for n in (S * L * H * B, 2 * Ev * H * L * B, q.size, k.size * (H // G), v.size * (H // G))]
+    del poison
+    run = lambda: gpu.pullback(gpu.scaled_dot_product_attention, dq_, dk_, dv_, 1, token_dim, None, None, True if causal else None)
+    (out, w), back = run()
+    wout, ww = O.scaled_dot_product_attention(f64(q), f64(k), f64(v), token_dim, None, None, True if causal else None)
+    assert_close(w.to_numpy(), ww, "bf16", "weights")
+    stored = f64(w.to_numpy())
+    if causal:
+        assert not stored[np.arange(S)[:, None] > np.arange(L)[None, :]].any()
+    wout, _ = O.scaled_dot_product_attention(f64(q), f64(k), f64(v), token_dim, None, None, True if causal else None, weights=stored)
+    assert_close(out.to_numpy(), wout, "bf16", "out")
+    (d_out,) = host_inputs("bf16", rng.normal(size=wout.shape))
+    got = back(dev(gpu, d_out, "bf16"))
+    want = O.scaled_dot_product_attention_pullback(f64(q), f64(k), f64(v), f64(d_out), token_dim, None, None, True if causal else None,
+                                                   weights=stored, stored=lambda a: f64(O.round_to_bf16(np.asarray(a, np.float32))))
+    # dlogits are differences: where the softmax is saturated they are far below the terms they are made of
+    for g, x, name in zip(got, want, ("dq", "dk", "dv")):
+        assert_close(g.to_numpy(), x, "bf16", name, scale=1e-3)
+    names = kernels_of(gpu, lambda: run()[1](dev(gpu, d_out, "bf16")))
+    assert {"attn_fwd_kernel", "attn_dkv_kernel", "attn_dq_kernel"} <= set(names)
+
+
+def test_an_unaligned_cotangent_takes_the_step_by_step_pullback(gpu):
+    """Both pullbacks start from the same stored weights and give the same gradients up to the order of their sums."""
+    E, H, L, B = 64, 2, 130, 2
+    rng = np.random.default_rng(stable_seed("attn-fused-unaligned"))
+    q, k, v, d = host_inputs("bf16", *(rng.normal(size=(E, H, L, B)) for _ in range(4)))
+    _, back = gpu.pullback(gpu.scaled_dot_product_attention, dev(gpu, q, "bf16"), dev(gpu, k, "bf16"), dev(gpu, v, "bf16"), 1, 3, None, None, True)
+    a = back(dev(gpu, d, "bf16"))
+    base = dev(gpu, np.concatenate([np.zeros(1, np.float32), d.ravel(order="F")]), "bf16")
+    off = gpu.DeviceArray(d.shape, "bf16", ptr=base.ptr + 2, base=base)
+    names = kernels_of(gpu, lambda: back(off))
+    assert "attn_dq_kernel" not in names
+    for x, y in zip(a, back(off)):
+        assert_close(x.to_numpy(), f64(y.to_numpy()), "bf16", "gradients", rel=2.0 ** -7)      # one unit in the last place of either
+
+
+def test_columns_with_infinite_logits(gpu):
+    """A query with an infinite logit: its whole column of weights is NaN, masked positions included, and so is its output;
+    the columns beside it are not touched."""
+    E, H, L = 64, 2, 200
+    rng = np.random.default_rng(stable_seed("attn-fused-inf"))
+    q, k, v = host_inputs("bf16", *(rng.normal(size=(E, H, L, 1)) for _ in range(3)))
+    q[:, 1, 70, 0] = 3e38
+    k[:, 1, 3, 0] = 3e38
+    d = lambda a: dev(gpu, a, "bf16")
+    y, w = gpu.scaled_dot_product_attention(d(q), d(k), d(v), 1, 3, None, None, True)
+    y, w = y.to_numpy(), w.to_numpy()
+    assert np.isnan(w[:, 70, 1, 0]).all() and np.isnan(y[:, 1, 70, 0]).all()
+    assert np.isfinite(w[:, :, 0]).all() and np.isfinite(w[:, :3, 1]).all() and np.isfinite(y[:, 0]).all() and np.isfinite(y[:, 1, :3]).all()
