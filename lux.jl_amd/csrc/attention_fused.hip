@@ -12,7 +12,8 @@
 // everything else is arranged to hide behind that stream.  Two sweeps over the keys (column maxima and sums, then weights
 // and output) cost a second product k'q but no traffic.  The pullback forms v' d_out twice, once per sweep (over queries
 // for dk, dv; over keys for dq), because handing dS from one to the other would write and read it.
-// Measured at 128 x 2048 x 32 x 4, causal (step-by-step path before): forward 1.15 ms -> 0.53 ms, pullback 0.85 ms -> 0.69 ms.
+// Measured at 128 x 2048 x 32 x 4, causal (step-by-step path before): forward 1.15 ms -> 0.48 ms, pullback 0.85 ms -> 0.59 ms
+// (dq 0.285, dk and dv 0.305; without the loads and stores of the weights 0.32, 0.21 and 0.26).
 //
 // Layout of the work: a workgroup is four waves; a wave owns 32 columns (queries in the forward and dq kernels, keys in the
 // dk / dv kernel) and walks the other dimension.  Every product is v_mfma_f32_32x32x16_bf16 with the walked dimension (or
@@ -20,21 +21,22 @@
 //   * a column of the softmax lies in two lanes (l and l + 32), its reductions are in-lane plus one exchange;
 //   * the accumulator of one product is the B operand of the next without a shuffle: accumulator register r of half-wave h
 //     holds row 8 (r / 4) + 4 h + r % 4, and the A operand's k slots are read in the same order (frag_t).
-// Tiles of 64 (32 in the dk / dv kernel) rows go global -> registers -> LDS, double buffered with one barrier per tile.
-// An LDS row is 256 bytes = sixteen 16-byte chunks; chunk c of row r is stored at c ^ f(r), f(r) = (r % 4) * 4 + (r / 4) % 4:
-// sixteen consecutive rows then lie in sixteen different chunks for the row-wise reads, and the four rows of a transposing
-// read (ds_read_b64_tr_b16) in four different 64-byte granules.
+// Tiles of 32 rows go global -> registers -> LDS, double buffered with one barrier per tile.  An LDS row is 256 bytes in a
+// pitch of 336 = 5 x 64 + 16: sixteen consecutive rows start in sixteen different 16-byte chunks of the 256-byte bank period
+// (row-wise reads: no conflict), the four rows of a transposing read (ds_read_b64_tr_b16) 80 bytes apart (at most two lanes
+// on a bank).  XOR-swizzled rows have no conflicts at all, but every fragment address is then an XOR and an addition where
+// it is an immediate here: 234 vector instructions per 32 x 32 tile of the dk / dv kernel, which had become its bound.
 #include <algorithm>
+#include <cmath>
 
 #include "common.h"
 #include "gemm_core.h"
-#include "gemm_dense_decl.h"
 
 namespace luxhip {
 namespace attn {
 
 constexpr int WAVES = 4, THREADS = WAVES * 64, COLS = 32 * WAVES;      // columns of a workgroup
-constexpr int PITCH = 256;                                             // bytes of an LDS row
+constexpr int ROWS = 32, PITCH = 336, TILE = ROWS * PITCH;              // a tile in LDS: rows, bytes of a row, bytes
 constexpr int MAX_E = 128;
 
 struct Args {
@@ -47,27 +49,27 @@ struct Args {
     int heads;                // H * batches
     int blocks;               // column blocks per head
     int causal;
-    float c, scale;           // scale * log2(e), scale
+    int negative;             // the sign of the scale, which the forward kernel moves to q
+    float c, scale;           // |scale| log2(e), scale
+    float* dsum;              // where the dq kernel leaves d for the dk / dv kernel
     int64_t qt, qh, qb, kt, kh, kb, vt, vh, vb, dkr, dvr;   // strides in elements: token, head, batch; repeat (dk, dv)
 };
 
 // ------------------------------------------------------------------------------------------------ who works on what
-// Heads are dealt to the XCDs (consecutive workgroups go to different ones), all blocks of a head to one: its k and v then
-// stay in one L2.  Fewer heads than that: block by block over all heads.  Causal work grows with the query block, so the
-// long blocks come first (`reverse`: the last block is the longest).
+// Block by block over all heads: consecutive workgroups go to different XCDs, so with a multiple of eight heads all blocks
+// of a head share one XCD's L2.  Under a causal mask the work grows with the query block and the masked part, which the
+// forward kernel fills, shrinks:
+//   REVERSE: the long blocks of all heads first (head by head, the last head's long blocks ran on while most compute units
+//     were done: 70 % of the wave slots in use over the kernel);
+//   ALTERNATE: last, first, second last, ...: blocks that compute and blocks that fill run side by side.
+enum Order { FORWARD, REVERSE, ALTERNATE };
 struct Where {
     int head, block, h, b, g, i0;
-    __device__ __forceinline__ Where(const Args& a, bool reverse) {
-        const int id = blockIdx.x;
-        if ((a.heads & 7) == 0) {
-            const int idx = id >> 3;
-            block = idx % a.blocks;
-            head = (idx / a.blocks) * 8 + (id & 7);
-        } else {
-            block = id / a.heads;
-            head = id - block * a.heads;
-        }
-        if (reverse) block = a.blocks - 1 - block;
+    __device__ __forceinline__ Where(const Args& a, Order order) {
+        block = blockIdx.x / a.heads;
+        head = blockIdx.x - block * a.heads;
+        if (order == REVERSE) block = a.blocks - 1 - block;
+        if (order == ALTERNATE) block = (block & 1) ? block >> 1 : a.blocks - 1 - (block >> 1);
         h = head % a.H;
         b = head / a.H;
         g = h / a.r;
@@ -76,72 +78,81 @@ struct Where {
 };
 
 // ------------------------------------------------------------------------------------------------ tiles
-__device__ __forceinline__ int swz(int row) { return ((row & 3) << 2) | ((row >> 2) & 3); }
-
-// ROWS rows of a (tokens x features) operand, feature chunks past E and rows past `rows` as zeros
-template <int ROWS, int ET>
+// 32 rows of a (tokens x features) operand, one tile after the other; features past E and rows past the last as zeros.
+// SETS tiles are on their way at a time, in register sets 0, 1 in turn.  Every load is issued unconditionally (past the end: the
+// last row once more): a load under a condition, even a uniform one, makes the compiler's wait for an older load a wait for all.
+template <int ET, int SETS>
 struct Tile {
     static constexpr int NCH = ET == 1 ? 4 : ET == 2 ? 8 : 16;          // chunks of a row that are loaded
     static constexpr int STEP = THREADS / NCH;                           // rows per pass
     static constexpr int N = (ROWS + STEP - 1) / STEP;
-    raw16_t reg[N];
-    uint32_t row, chunk_bytes, lds;
+    raw16_t reg[SETS][N];
+    const char* p;
+    uint32_t pitch, off, last, lds;      // off: this thread's chunk in its first row of the next tile; last: in the last row
+    int row;
     bool live;
-    __device__ __forceinline__ explicit Tile(int E) {
+    __device__ __forceinline__ Tile(const bf16_t* p_, int64_t stride, int E, int rows, int first)
+        : p(reinterpret_cast<const char*>(p_)), pitch((uint32_t)(stride * 2)) {
         const int ch = threadIdx.x % NCH;
         row = threadIdx.x / NCH;
-        live = ch * 8 < E;
-        chunk_bytes = live ? ch * 16 : 0;
-        lds = row * PITCH + ((ch ^ swz(row)) << 4);                      // STEP is a multiple of 16: the same f for every pass
-        static_assert(STEP % 16 == 0, "rows of the passes must share their swizzle");
+        live = row < ROWS && ch * 8 < E;
+        const uint32_t cb = ch * 8 < E ? ch * 16 : 0;
+        off = (uint32_t)(ROWS * first + row) * pitch + cb;
+        last = (uint32_t)(rows - 1) * pitch + cb;
+        lds = row * PITCH + ch * 16;
     }
-    __device__ __forceinline__ bool mine(int i) const { return ROWS % STEP == 0 || row + i * STEP < (uint32_t)ROWS; }
-    // rows r0 .. r0 + ROWS - 1 of the operand at p; `rows` > 0
-    __device__ __forceinline__ void load(const bf16_t* p, uint32_t pitch_bytes, int r0, int rows) {
+    // chunks that no tile fills
+    __device__ __forceinline__ void clear(char* tile) const {
+        const raw16_t zero = {0u, 0u, 0u, 0u};
 #pragma unroll
-        for (int i = 0; i < N; ++i) {
-            const int r = min(r0 + (int)row + i * STEP, rows - 1);
-            reg[i] = *reinterpret_cast<const raw16_t*>(reinterpret_cast<const char*>(p) + ((uint32_t)r * pitch_bytes + chunk_bytes));
-        }
+        for (int i = 0; i < N; ++i)
+            if (row < ROWS && !live) *reinterpret_cast<raw16_t*>(tile + lds + i * STEP * PITCH) = zero;
     }
-    __device__ __forceinline__ void store(char* tile, int r0, int rows) const {
+    __device__ __forceinline__ void load(int set) {
 #pragma unroll
-        for (int i = 0; i < N; ++i) {
-            const bool in = live && r0 + (int)row + i * STEP < rows;
+        for (int i = 0; i < N; ++i) reg[set][i] = *reinterpret_cast<const raw16_t*>(p + min(off + i * STEP * pitch, last));
+        off += ROWS * pitch;
+    }
+    // tile t of an operand of `rows` rows
+    __device__ __forceinline__ void store(char* tile, int set, int t, int rows) const {
+        if (ROWS * (t + 1) <= rows) {      // uniform
+#pragma unroll
+            for (int i = 0; i < N; ++i)
+                if (live) *reinterpret_cast<raw16_t*>(tile + lds + i * STEP * PITCH) = reg[set][i];
+        } else {
             const raw16_t zero = {0u, 0u, 0u, 0u};
-            if (mine(i)) *reinterpret_cast<raw16_t*>(tile + lds + i * STEP * PITCH) = in ? reg[i] : zero;
+#pragma unroll
+            for (int i = 0; i < N; ++i)
+                if (live) *reinterpret_cast<raw16_t*>(tile + lds + i * STEP * PITCH) = ROWS * t + row + i * STEP < rows ? reg[set][i] : zero;
         }
     }
 };
 
-// Row-wise fragment (A operand): rows r0 .. r0 + 31 of the tile, features 16 kk .. 16 kk + 15
+// Row-wise fragment (A operand): the tile's rows, features 16 kk .. 16 kk + 15
 struct FragRow {
-    uint32_t off, h;
+    uint32_t off;
     __device__ __forceinline__ FragRow() {
         const int l = threadIdx.x & 63;
-        h = l >> 5;
-        off = (l & 31) * PITCH + ((h ^ swz(l & 31)) << 4);
+        off = (l & 31) * PITCH + (l >> 5) * 16;
     }
-    __device__ __forceinline__ bf16x8_v get(const char* tile, int r0, int kk) const {     // r0: a multiple of 32
-        return __builtin_bit_cast(bf16x8_v, *reinterpret_cast<const raw16_t*>(tile + r0 * PITCH + (off ^ (kk << 5))));
+    __device__ __forceinline__ bf16x8_v get(const char* tile, int kk) const {
+        return __builtin_bit_cast(bf16x8_v, *reinterpret_cast<const raw16_t*>(tile + off + 32 * kk));
     }
 };
 // Transposed fragment (A operand): features 32 t .. 32 t + 31 as rows, tile rows r0 + {4h .. 4h + 3, 8 + 4h ..} as k slots
-// (the order in which an accumulator holds its rows).  r0: a multiple of 16.
+// (the order in which an accumulator holds its rows)
 struct FragT {
-    uint32_t lo;
+    uint32_t off;
     __device__ __forceinline__ FragT() {
-        const int l = threadIdx.x & 63, b = l >> 4, s = l & 15, h = b >> 1;
-        const int row = 4 * h + (s >> 2), chunk = 2 * (b & 1) + ((s & 3) >> 1);
-        lo = row * PITCH + ((chunk ^ swz(row)) << 4) + (s & 1) * 8;
+        const int l = threadIdx.x & 63, b = l >> 4, s = l & 15;
+        off = (4 * (b >> 1) + (s >> 2)) * PITCH + (b & 1) * 32 + (s & 3) * 8;
     }
     __device__ __forceinline__ static s16x4_v tr(const char* p) {
         typedef __attribute__((address_space(3))) s16x4_v* lds_ptr;
         return __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_ptr)(p));
     }
     __device__ __forceinline__ bf16x8_v get(const char* tile, int r0, int t) const {
-        // row + 8: (row / 4) % 4 changes by 2, one XOR
-        const s16x4_v a = tr(tile + r0 * PITCH + (lo ^ (t << 6))), b = tr(tile + (r0 + 8) * PITCH + (lo ^ (t << 6) ^ (2 << 4)));
+        const s16x4_v a = tr(tile + off + r0 * PITCH + 64 * t), b = tr(tile + off + (r0 + 8) * PITCH + 64 * t);
         const s16x8_v v = {a[0], a[1], a[2], a[3], b[0], b[1], b[2], b[3]};
         return __builtin_bit_cast(bf16x8_v, v);
     }
@@ -176,7 +187,7 @@ __device__ __forceinline__ raw16_t reorder(raw16_t w) {
     return raw16_t{a[0], b[0], a[1], b[1]};
 }
 
-typedef uint32_t raw16_u __attribute__((ext_vector_type(4), aligned(2)));
+typedef uint32_t raw16_u __attribute__((ext_vector_type(4), aligned(2)));       // anywhere in a row of weights
 // Eight consecutive bf16 at p + at, of which only those below `end` exist (ragged rows: any alignment)
 __device__ __forceinline__ void store8(bf16_t* p, int at, int end, raw16_t w) {
     if (at + 8 <= end) {
@@ -198,6 +209,36 @@ __device__ __forceinline__ raw16_t load8(const bf16_t* p, int at, int end) {
     }
     return w;
 }
+
+// 32 columns (one per lane of a half-wave) x 64 keys of weights between the lanes that own a column and full lines of memory:
+// a wave's own 4 KiB of LDS, 128 bytes per column, its eight chunks XORed with column % 8.  Straight from the lanes a store
+// instruction touches 32 lines with 32 bytes each; this way eight whole ones.
+constexpr int PT_BYTES = 32 * 128;
+struct WeightTile {
+    char* lds;
+    int lane;
+    __device__ __forceinline__ WeightTile(void* p, int w) : lds((char*)p + w * PT_BYTES), lane(threadIdx.x & 63) {}
+    // keys 16 n + {4h .. 4h + 3, 8 + 4h ..} of this lane's column (accumulator order)
+    __device__ __forceinline__ void put(int n, raw16_t w) const {
+        const int c = lane & 31, h = lane >> 5;
+        char* row = lds + c * 128 + 8 * h;
+        *reinterpret_cast<uint2*>(row + (((2 * n) ^ (c & 7)) << 4)) = make_uint2(w[0], w[1]);
+        *reinterpret_cast<uint2*>(row + (((2 * n + 1) ^ (c & 7)) << 4)) = make_uint2(w[2], w[3]);
+    }
+    __device__ __forceinline__ raw16_t get(int n) const {
+        const int c = lane & 31, h = lane >> 5;
+        const char* row = lds + c * 128 + 8 * h;
+        const uint2 a = *reinterpret_cast<const uint2*>(row + (((2 * n) ^ (c & 7)) << 4));
+        const uint2 b = *reinterpret_cast<const uint2*>(row + (((2 * n + 1) ^ (c & 7)) << 4));
+        return raw16_t{a.x, a.y, b.x, b.y};
+    }
+    // line side, i < 4: column 8 i + lane / 8, keys 8 (lane % 8) ...
+    __device__ __forceinline__ int column(int i) const { return 8 * i + (lane >> 3); }
+    __device__ __forceinline__ int key() const { return 8 * (lane & 7); }
+    __device__ __forceinline__ raw16_t* line(int i) const {
+        return reinterpret_cast<raw16_t*>(lds + column(i) * 128 + (((lane & 7) ^ (lane >> 3)) << 4));
+    }
+};
 
 // rows (features) x columns (the wave's tokens) accumulators to a (tokens x features) tensor
 template <int ET>
@@ -222,38 +263,53 @@ __device__ __forceinline__ f32x16_v zero16() {
 // accumulator register i of half-wave h: its row
 __device__ __forceinline__ int acc_row(int i, int h) { return 8 * (i >> 2) + 4 * h + (i & 3); }
 
+// (32 rows of the tile) x (the wave's 32 columns), contracted over the features
+// G: fragments that are on their way before the first product waits for one
+template <int ET, int G>
+__device__ __forceinline__ f32x16_v product(const FragRow& fr, const char* tile, const bf16x8_v (&cols)[2 * ET]) {
+    f32x16_v z = zero16();
+#pragma unroll
+    for (int k0 = 0; k0 < 2 * ET; k0 += G) {
+        bf16x8_v f[G];
+#pragma unroll
+        for (int i = 0; i < G; ++i)
+            if (k0 + i < 2 * ET) f[i] = fr.get(tile, k0 + i);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int i = 0; i < G; ++i)
+            if (k0 + i < 2 * ET) z = __builtin_amdgcn_mfma_f32_32x32x16_bf16(f[i], cols[k0 + i], z, 0, 0, 0);
+    }
+    return z;
+}
+
 // ------------------------------------------------------------------------------------------------ forward
-constexpr int KB = 64;                                  // keys per tile
-constexpr int TILE_BYTES = KB * PITCH;                  // 16 KiB
-constexpr size_t FWD_LDS = 4 * TILE_BYTES;              // k and v, two of each
+constexpr size_t FWD_LDS = 4 * TILE + WAVES * PT_BYTES;     // k and v, two tiles of each, and the waves' weights: 58 KiB
 
 template <int ET>
 __global__ __launch_bounds__(THREADS, 2) void fwd_kernel(Args a) {
     extern __shared__ __align__(16) unsigned char lds_raw[];
-    char* const kt = reinterpret_cast<char*>(lds_raw);
-    char* const vt = kt + 2 * TILE_BYTES;
-    const Where wh(a, a.causal != 0);
+    char* const lds = reinterpret_cast<char*>(lds_raw);     // k 0, k 1, v 0, v 1, weights
+    const Where wh(a, a.causal ? ALTERNATE : FORWARD);
     const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), h = lane >> 5;
     const int l0 = wh.block * COLS, wl0 = l0 + 32 * w, l = wl0 + (lane & 31);
     const bf16_t* const kp = a.k + wh.g * a.kh + wh.b * a.kb;
     const bf16_t* const vp = a.v + wh.g * a.vh + wh.b * a.vb;
-    const uint32_t kpitch = (uint32_t)(a.kt * 2), vpitch = (uint32_t)(a.vt * 2);
     const int s_end = a.causal ? min(a.S, l0 + COLS) : a.S;                    // keys that any query of the workgroup sees
-    const int tiles = (s_end + KB - 1) / KB;
+    const int tiles = 2 * ((s_end + 2 * ROWS - 1) / (2 * ROWS));               // in pairs; rows past the end are zeros
     const int w_end = wl0 >= a.L ? 0 : a.causal ? min(a.S, wl0 + 32) : a.S;    // ... of the wave
     const int limit = a.causal ? min(l, a.S - 1) : a.S - 1;
     const FragRow fr;
     const FragT ft;
     bf16x8_v qf[2 * ET];
     load_columns<ET>(qf, a.q + wh.h * a.qh + wh.b * a.qb, (uint32_t)(a.qt * 2), l, a.L, a.E);
+    if (a.negative) {
+#pragma unroll
+        for (int kk = 0; kk < 2 * ET; ++kk) qf[kk] = __builtin_bit_cast(bf16x8_v, __builtin_bit_cast(raw16_t, qf[kk]) ^ 0x80008000u);
+    }
 
-    // scaled logits (times log2 e) of keys s0 .. s0 + 31 of tile buffer `tile`, -inf where masked
-    auto logits = [&](const char* tile, int j, int s0) {
-        f32x16_v z = zero16();
-#pragma unroll
-        for (int kk = 0; kk < 2 * ET; ++kk) z = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fr.get(tile, 32 * j, kk), qf[kk], z, 0, 0, 0);
-#pragma unroll
-        for (int i = 0; i < 16; ++i) z[i] *= a.c;
+    // unscaled logits of keys s0 .. s0 + 31: -inf where masked
+    auto logits = [&](const char* tile, int s0) {
+        f32x16_v z = product<ET, 2 * ET>(fr, tile, qf);
         if (s0 + 31 > (a.causal ? min(wl0, a.S - 1) : a.S - 1)) {
 #pragma unroll
             for (int i = 0; i < 16; ++i)
@@ -262,97 +318,110 @@ __global__ __launch_bounds__(THREADS, 2) void fwd_kernel(Args a) {
         return z;
     };
 
-    Tile<KB, ET> tk(a.E);
     // sweep 1: maximum and sum of exponentials, per lane (half of the keys of its column).  A column of which nothing but
     // -inf has been seen keeps the sum 0 (the subtrahend is 0 then).
     float m = -INFINITY, sum = 0.0f;
-    tk.load(kp, kpitch, 0, a.S);
-    tk.store(kt, 0, a.S);
-    __syncthreads();
-    for (int t = 0; t < tiles; ++t) {
-        const char* cur = kt + (t & 1) * TILE_BYTES;
-        if (t + 1 < tiles) tk.load(kp, kpitch, (t + 1) * KB, a.S);
-#pragma unroll
-        for (int j = 0; j < 2; ++j) {
-            const int s0 = t * KB + 32 * j;
-            if (s0 < w_end) {
-                const f32x16_v z = logits(cur, j, s0);
-                float mt = z[0];
-#pragma unroll
-                for (int i = 1; i < 16; ++i) mt = fmaxf(mt, z[i]);
-                const float mn = fmaxf(m, mt), ms = mn == -INFINITY ? 0.0f : mn;
-                float add = 0.0f;
-#pragma unroll
-                for (int i = 0; i < 16; ++i) add += __builtin_amdgcn_exp2f(z[i] - ms);
-                sum = sum * __builtin_amdgcn_exp2f(m - ms) + add;
-                m = mn;
-            }
-        }
-        if (t + 1 < tiles) tk.store(kt + ((t + 1) & 1) * TILE_BYTES, (t + 1) * KB, a.S);
+    {
+        Tile<ET, 2> tk(kp, a.kt, a.E, a.S, 0);
+        tk.load(0);
+        tk.load(1);                                         // past the end: the last row once more
+        tk.clear(lds);
+        tk.clear(lds + TILE);
+        tk.store(lds, 0, 0, a.S);
         __syncthreads();
+        for (int t0 = 0; t0 < tiles; t0 += 2) {
+            static_for<2>([&](auto U) {
+                constexpr int u = decltype(U)::value;
+                const int t = t0 + u;
+                tk.load(u);
+                if (ROWS * t < w_end) {
+                    const f32x16_v z = logits(lds + u * TILE, ROWS * t);
+                    float mt = z[0];
+#pragma unroll
+                    for (int i = 1; i < 16; ++i) mt = fmaxf(mt, z[i]);
+                    const float mn = fmaxf(m, mt * a.c), ms = mn == -INFINITY ? 0.0f : mn;
+                    float add = 0.0f;
+#pragma unroll
+                    for (int i = 0; i < 16; ++i) add += __builtin_amdgcn_exp2f(fmaf(z[i], a.c, -ms));
+                    sum = sum * __builtin_amdgcn_exp2f(m - ms) + add;
+                    m = mn;
+                }
+                tk.store(lds + (1 - u) * TILE, 1 - u, t + 1, a.S);
+                __syncthreads();
+            });
+        }
     }
-    float mx;
-    float inv;
+    // weight = exp2(c z - base), base = maximum + log2(sum)
+    float base;
     {
         const float mo = __shfl_xor(m, 32), so = __shfl_xor(sum, 32);
-        mx = fmaxf(m, mo);
-        const float ms = mx == -INFINITY ? 0.0f : mx;
-        inv = 1.0f / (sum * __builtin_amdgcn_exp2f(m - ms) + so * __builtin_amdgcn_exp2f(mo - ms));
+        const float mx = fmaxf(m, mo), ms = mx == -INFINITY ? 0.0f : mx;
+        base = mx == -INFINITY ? NAN : mx + __builtin_amdgcn_logf(sum * __builtin_amdgcn_exp2f(m - ms) + so * __builtin_amdgcn_exp2f(mo - ms));
     }
-
-    // the tiles of sweep 2 on their way while the masked part of the columns is filled
-    Tile<KB, ET> tv(a.Ev);
-    tk.load(kp, kpitch, 0, a.S);
-    tv.load(vp, vpitch, 0, a.S);
-    bf16_t* const wrow0 = a.probs + ((int64_t)wh.head * a.L + wl0) * a.S;        // row wl0 of this head
-    if (wl0 < a.L) {
-        const int rows = min(32, a.L - wl0);
-        for (int i = 0; i < rows; ++i) {                                         // a masked weight: 0 times 1 / sum
-            const float z0 = 0.0f * __shfl(inv, i);
-            const uint32_t zz = f32x2_to_bf16x2(z0, z0);
-            const raw16_t zw = {zz, zz, zz, zz};
-            for (int s = w_end + 8 * lane; s < a.S; s += 512) store8(wrow0 + (int64_t)i * a.S, s, a.S, zw);
-        }
-    }
-    tk.store(kt, 0, a.S);
-    tv.store(vt, 0, a.S);
-    __syncthreads();
 
     // sweep 2: the weights, rounded, to memory and into the product with v
+    bf16_t* const wrow0 = a.probs + ((int64_t)wh.head * a.L + wl0) * a.S;        // row wl0 of this head
+    const WeightTile pt(lds + 4 * TILE, w);
     f32x16_v o[ET];
 #pragma unroll
     for (int t = 0; t < ET; ++t) o[t] = zero16();
-    bf16_t* const wrow = wrow0 + (int64_t)(lane & 31) * a.S;
-    for (int t = 0; t < tiles; ++t) {
-        const char *kc = kt + (t & 1) * TILE_BYTES, *vc = vt + (t & 1) * TILE_BYTES;
-        if (t + 1 < tiles) {
-            tk.load(kp, kpitch, (t + 1) * KB, a.S);
-            tv.load(vp, vpitch, (t + 1) * KB, a.S);
+    {
+        Tile<ET, 2> tk(kp, a.kt, a.E, a.S, 0), tv(vp, a.vt, a.Ev, a.S, 0);
+#pragma unroll
+        for (int b = 0; b < 2; ++b) {
+            tk.load(b);
+            tv.load(b);
+            tv.clear(lds + (2 + b) * TILE);
         }
-#pragma unroll
-        for (int j = 0; j < 2; ++j) {
-            const int s0 = t * KB + 32 * j;
-            if (s0 < w_end) {
-                f32x16_v z = logits(kc, j, s0);
-#pragma unroll
-                for (int i = 0; i < 16; ++i) z[i] = __builtin_amdgcn_exp2f(z[i] - mx) * inv;
-#pragma unroll
-                for (int n = 0; n < 2; ++n) {
-                    const raw16_t pw = pack8(z, n);
-                    const raw16_t mem = reorder(pw);
-                    if (l < a.L) store8(wrow, s0 + 16 * n + 8 * h, w_end, mem);
-                    const bf16x8_v pb = __builtin_bit_cast(bf16x8_v, pw);
-#pragma unroll
-                    for (int e = 0; e < ET; ++e)
-                        o[e] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ft.get(vc, 32 * j + 16 * n, e), pb, o[e], 0, 0, 0);
-                }
-            }
-        }
-        if (t + 1 < tiles) {
-            tk.store(kt + ((t + 1) & 1) * TILE_BYTES, (t + 1) * KB, a.S);
-            tv.store(vt + ((t + 1) & 1) * TILE_BYTES, (t + 1) * KB, a.S);
-        }
+        tk.store(lds, 0, 0, a.S);
+        tv.store(lds + 2 * TILE, 0, 0, a.S);
         __syncthreads();
+        // the finished 64 keys (or the first 32 of them) from s0 on
+        auto store_weights = [&](int s0) {
+            const int end = min(w_end, s0 + 64);
+            if (end == s0 + 64 && wl0 + 32 <= a.L) {        // uniform
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+                    *reinterpret_cast<raw16_u*>(wrow0 + (int64_t)pt.column(i) * a.S + s0 + pt.key()) = *pt.line(i);
+            } else {
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+                    if (wl0 + pt.column(i) < a.L && s0 + pt.key() < end)
+                        store8(wrow0 + (int64_t)pt.column(i) * a.S, s0 + pt.key(), end, *pt.line(i));
+            }
+        };
+        for (int t0 = 0; t0 < tiles; t0 += 2) {
+            static_for<2>([&](auto U) {
+                constexpr int u = decltype(U)::value;
+                const int t = t0 + u;
+                tk.load(u);
+                tv.load(u);
+                if (ROWS * t < w_end) {
+                    f32x16_v z = logits(lds + u * TILE, ROWS * t);
+                    bf16x8_v vf[2][ET];                 // read while the exponentials are computed
+#pragma unroll
+                    for (int n = 0; n < 2; ++n)
+#pragma unroll
+                        for (int e = 0; e < ET; ++e) vf[n][e] = ft.get(lds + (2 + u) * TILE, 16 * n, e);
+                    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                    for (int i = 0; i < 16; ++i) z[i] = __builtin_amdgcn_exp2f(fmaf(z[i], a.c, -base));
+#pragma unroll
+                    for (int n = 0; n < 2; ++n) {
+                        const raw16_t pw = pack8(z, n);
+                        pt.put(2 * u + n, pw);
+#pragma unroll
+                        for (int e = 0; e < ET; ++e)
+                            o[e] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf[n][e], __builtin_bit_cast(bf16x8_v, pw), o[e], 0, 0, 0);
+                    }
+                }
+                // the next tile first: its wait must not include this tile's stores
+                tk.store(lds + (1 - u) * TILE, 1 - u, t + 1, a.S);
+                tv.store(lds + (3 - u) * TILE, 1 - u, t + 1, a.S);
+                if (u == 1 && ROWS * t0 < w_end) store_weights(ROWS * t0);
+                __syncthreads();
+            });
+        }
     }
     // out (Ev, H, L, B), rounded and unrounded
     const int64_t orow = (((int64_t)wh.b * a.L + l) * a.H + wh.h) * a.Ev;
@@ -367,179 +436,223 @@ __global__ __launch_bounds__(THREADS, 2) void fwd_kernel(Args a) {
                     *reinterpret_cast<float4*>(a.out_wide + orow + e) = make_float4(o[t][4 * g], o[t][4 * g + 1], o[t][4 * g + 2], o[t][4 * g + 3]);
             }
     }
+    // the masked part of the columns, last: nothing waits for these stores.  0, or NaN where the sum is none.
+    const int rows = min(32, a.L - wl0);
+    if (w_end < a.S) {
+        for (int i = 0; i < rows; ++i) {
+            const float z0 = __shfl(base, i) != __shfl(base, i) ? NAN : 0.0f;
+            const uint32_t zz = f32x2_to_bf16x2(z0, z0);
+            const raw16_t zw = {zz, zz, zz, zz};
+            for (int s = w_end + 8 * lane; s < a.S; s += 512) store8(wrow0 + (int64_t)i * a.S, s, a.S, zw);
+        }
+    }
 }
 
 // ------------------------------------------------------------------------------------------------ pullback
-// scale weights .* (dP - d) of 16 rows, as the B operand of the next product: pw as loaded (bf16 pairs in accumulator order)
-__device__ __forceinline__ raw16_t softmax_rule(raw16_t pw, const f32x16_v& dp, int n, const float (&d)[8], float scale) {
+// weights .* (scale dP - scale d) of 16 rows, as the B operand of the next product: pw as loaded (bf16 pairs in accumulator
+// order), sd = scale d of each row
+__device__ __forceinline__ raw16_t softmax_rule(raw16_t pw, const f32x16_v& dp, int n, const float (&sd)[8], float scale) {
     raw16_t out;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
         const float p0 = __uint_as_float(pw[i] << 16), p1 = __uint_as_float(pw[i] & 0xffff0000u);
-        out[i] = f32x2_to_bf16x2(scale * p0 * (dp[8 * n + 2 * i] - d[2 * i]), scale * p1 * (dp[8 * n + 2 * i + 1] - d[2 * i + 1]));
+        out[i] = f32x2_to_bf16x2(p0 * fmaf(dp[8 * n + 2 * i], scale, -sd[2 * i]), p1 * fmaf(dp[8 * n + 2 * i + 1], scale, -sd[2 * i + 1]));
     }
     return out;
 }
 
-// dq: a wave owns 32 queries and walks the keys
-template <int ET>
+// dq: a wave owns 32 queries and walks the keys.  VEC: rows of weights are whole 16-byte vectors (S a multiple of 8).
+template <int ET, bool VEC>
 __global__ __launch_bounds__(THREADS, 2) void dq_kernel(Args a) {
     extern __shared__ __align__(16) unsigned char lds_raw[];
-    char* const kt = reinterpret_cast<char*>(lds_raw);
-    char* const vt = kt + 2 * TILE_BYTES;
-    const Where wh(a, a.causal != 0);
+    char* const lds = reinterpret_cast<char*>(lds_raw);     // k 0, k 1, v 0, v 1, weights
+    const Where wh(a, a.causal ? REVERSE : FORWARD);
     const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), h = lane >> 5;
     const int l0 = wh.block * COLS, wl0 = l0 + 32 * w, l = wl0 + (lane & 31);
-    const bf16_t* const kp = a.k + wh.g * a.kh + wh.b * a.kb;
-    const bf16_t* const vp = a.v + wh.g * a.vh + wh.b * a.vb;
-    const uint32_t kpitch = (uint32_t)(a.kt * 2), vpitch = (uint32_t)(a.vt * 2);
     const int s_end = a.causal ? min(a.S, l0 + COLS) : a.S;
-    const int tiles = (s_end + KB - 1) / KB;
+    const int tiles = 2 * ((s_end + 2 * ROWS - 1) / (2 * ROWS));               // in pairs; rows past the end are zeros
     const int w_end = wl0 >= a.L ? 0 : a.causal ? min(a.S, wl0 + 32) : a.S;
     const int lc = min(l, a.L - 1);
     const FragRow fr;
     const FragT ft;
+    // the weights of 64 keys, as they lie in memory, one such step ahead of their use
+    const WeightTile pt(lds + 4 * TILE, w);
+    raw16_t pw[4];
+    const bf16_t* const wplane = a.probs + (int64_t)wh.head * a.L * a.S;
+    const bf16_t* wrow[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) wrow[i] = wplane + (int64_t)min(wl0 + pt.column(i), a.L - 1) * a.S;
+    auto load_weights = [&](int s0) {
+        const int key = s0 + pt.key();
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            if constexpr (VEC) pw[i] = *reinterpret_cast<const raw16_u*>(wrow[i] + min(key, a.S - 8));     // past the end: masked below
+            else pw[i] = load8(wrow[i], key, w_end);
+        }
+    };
+    Tile<ET, 2> tk(a.k + wh.g * a.kh + wh.b * a.kb, a.kt, a.E, a.S, 0), tv(a.v + wh.g * a.vh + wh.b * a.vb, a.vt, a.Ev, a.S, 0);
+#pragma unroll
+    for (int b = 0; b < 2; ++b) {
+        tk.load(b);
+        tv.load(b);
+    }
+    load_weights(0);
     bf16x8_v df[2 * ET];
     load_columns<ET>(df, a.d_out + ((int64_t)wh.b * a.L * a.H + wh.h) * a.Ev, (uint32_t)(a.H * a.Ev * 2), l, a.L, a.Ev);
-    const float dl = a.d[(int64_t)wh.head * a.L + lc];
-    const bf16_t* const wrow = a.probs + ((int64_t)wh.head * a.L + lc) * a.S;
-    raw16_t pw[4];                        // the weights of the tile about to be used: 64 keys of the lane's query
-    auto load_weights = [&](int s0) {
+    // d = sum over the features of d_out .* out, half of them in each of a query's two lanes
+    float dl = 0.0f;
+    {
+        const float* orow = a.out_wide + (((int64_t)wh.b * a.L + lc) * a.H + wh.h) * a.Ev;
 #pragma unroll
-        for (int n = 0; n < 4; ++n) pw[n] = load8(wrow, s0 + 16 * n + 8 * h, w_end);
-    };
-    Tile<KB, ET> tk(a.E), tv(a.Ev);
-    tk.load(kp, kpitch, 0, a.S);
-    tv.load(vp, vpitch, 0, a.S);
-    load_weights(0);
+        for (int kk = 0; kk < 2 * ET; ++kk) {
+            const int e = 16 * kk + 8 * h;
+            const float* p = orow + (e < a.Ev ? e : 0);
+            const float4 x = *reinterpret_cast<const float4*>(p), y = *reinterpret_cast<const float4*>(p + 4);
+            const float ov[8] = {x.x, x.y, x.z, x.w, y.x, y.y, y.z, y.w};
+            float dv[8];
+            Vec<bf16_t>::unpack(__builtin_bit_cast(raw16_t, df[kk]), dv);
+            if (e < a.Ev) {
+#pragma unroll
+                for (int i = 0; i < 8; ++i) dl = fmaf(dv[i], ov[i], dl);
+            }
+        }
+        dl += __shfl_xor(dl, 32);
+        if (h == 0 && l < a.L) a.dsum[(int64_t)wh.head * a.L + l] = dl;
+    }
+    const float sd = a.scale * dl, dd[8] = {sd, sd, sd, sd, sd, sd, sd, sd};
     f32x16_v acc[ET];
 #pragma unroll
     for (int t = 0; t < ET; ++t) acc[t] = zero16();
-    const float dd[8] = {dl, dl, dl, dl, dl, dl, dl, dl};
-    tk.store(kt, 0, a.S);
-    tv.store(vt, 0, a.S);
+    tk.clear(lds);
+    tk.clear(lds + TILE);
+    tv.clear(lds + 2 * TILE);
+    tv.clear(lds + 3 * TILE);
+    tk.store(lds, 0, 0, a.S);
+    tv.store(lds + 2 * TILE, 0, 0, a.S);
     __syncthreads();
-    for (int t = 0; t < tiles; ++t) {
-        const char *kc = kt + (t & 1) * TILE_BYTES, *vc = vt + (t & 1) * TILE_BYTES;
-        raw16_t pc[4];
+    for (int t0 = 0; t0 < tiles; t0 += 2) {
 #pragma unroll
-        for (int n = 0; n < 4; ++n) pc[n] = pw[n];
-        if (t + 1 < tiles) {
-            tk.load(kp, kpitch, (t + 1) * KB, a.S);
-            tv.load(vp, vpitch, (t + 1) * KB, a.S);
-            load_weights((t + 1) * KB);
+        for (int i = 0; i < 4; ++i) {
+            const raw16_t zero = {0u, 0u, 0u, 0u};
+            *pt.line(i) = !VEC || ROWS * t0 + pt.key() < w_end ? pw[i] : zero;
         }
+        static_for<2>([&](auto U) {
+            constexpr int u = decltype(U)::value;
+            const int t = t0 + u;
+            tk.load(u);
+            tv.load(u);
+            if (u == 0) load_weights(ROWS * (t + 2));
+            if (ROWS * t < w_end) {
+                const f32x16_v dp = product<ET, 2 * ET>(fr, lds + (2 + u) * TILE, df);
+                bf16x8_v kf[2][ET];                     // read while the softmax rule is computed
 #pragma unroll
-        for (int j = 0; j < 2; ++j) {
-            if (t * KB + 32 * j < w_end) {
-                f32x16_v dp = zero16();
+                for (int n = 0; n < 2; ++n)
 #pragma unroll
-                for (int kk = 0; kk < 2 * ET; ++kk) dp = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fr.get(vc, 32 * j, kk), df[kk], dp, 0, 0, 0);
+                    for (int e = 0; e < ET; ++e) kf[n][e] = ft.get(lds + u * TILE, 16 * n, e);
+                __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
                 for (int n = 0; n < 2; ++n) {
-                    const bf16x8_v ds = __builtin_bit_cast(bf16x8_v, softmax_rule(reorder(pc[2 * j + n]), dp, n, dd, a.scale));
+                    const bf16x8_v ds = __builtin_bit_cast(bf16x8_v, softmax_rule(pt.get(2 * u + n), dp, n, dd, a.scale));
 #pragma unroll
-                    for (int e = 0; e < ET; ++e)
-                        acc[e] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ft.get(kc, 32 * j + 16 * n, e), ds, acc[e], 0, 0, 0);
+                    for (int e = 0; e < ET; ++e) acc[e] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf[n][e], ds, acc[e], 0, 0, 0);
                 }
             }
-        }
-        if (t + 1 < tiles) {
-            tk.store(kt + ((t + 1) & 1) * TILE_BYTES, (t + 1) * KB, a.S);
-            tv.store(vt + ((t + 1) & 1) * TILE_BYTES, (t + 1) * KB, a.S);
-        }
-        __syncthreads();
+            tk.store(lds + (1 - u) * TILE, 1 - u, t + 1, a.S);
+            tv.store(lds + (3 - u) * TILE, 1 - u, t + 1, a.S);
+            __syncthreads();
+        });
     }
     store_features<ET>(acc, a.dq + wh.h * a.qh + wh.b * a.qb + (int64_t)lc * a.qt, l < a.L, a.E);
 }
 
-// dk, dv: a wave owns 32 keys and walks the queries
-constexpr int LB = 32;                                          // queries per tile
-constexpr int LTILE = LB * PITCH;                               // 8 KiB: 32 queries x (128 features | 128 keys of the workgroup)
-constexpr size_t DKV_LDS = 2 * (3 * LTILE + LB * 4);            // q, d_out, weights and d, two of each
+// dk, dv: a wave owns 32 keys and walks the queries.  VEC as above.
+constexpr size_t DKV_LDS = 2 * (3 * TILE + ROWS * 4);           // q, d_out, weights (32 queries x 128 keys) and d, two of each: 63 KiB
 
-template <int ET>
+template <int ET, bool VEC>
 __global__ __launch_bounds__(THREADS, 2) void dkv_kernel(Args a) {
     extern __shared__ __align__(16) unsigned char lds_raw[];
-    char* const qt = reinterpret_cast<char*>(lds_raw);
-    char* const ot = qt + 2 * LTILE;
-    char* const pt = ot + 2 * LTILE;
-    float* const dt = reinterpret_cast<float*>(pt + 2 * LTILE);
-    const Where wh(a, false);                                   // causal: the first block of keys is seen by every query
+    char* const lds = reinterpret_cast<char*>(lds_raw);         // q 0, q 1, d_out 0, 1, weights 0, 1, d 0, 1
+    float* const dt = reinterpret_cast<float*>(lds + 6 * TILE);
+    const Where wh(a, FORWARD);                                 // causal: the first block of keys is seen by every query
     const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), h = lane >> 5;
     const int s0 = wh.block * COLS, ws0 = s0 + 32 * w, s = ws0 + (lane & 31);
-    const bf16_t* const qp = a.q + wh.h * a.qh + wh.b * a.qb;
-    const bf16_t* const op = a.d_out + ((int64_t)wh.b * a.L * a.H + wh.h) * a.Ev;
-    const bf16_t* const pp = a.probs + (int64_t)wh.head * a.L * a.S;
-    const float* const dp_ = a.d + (int64_t)wh.head * a.L;
-    const uint32_t qpitch = (uint32_t)(a.qt * 2), opitch = (uint32_t)(a.H * a.Ev * 2);
-    const int first = a.causal ? s0 / LB : 0, tiles = (a.L + LB - 1) / LB;
-    const int w_first = ws0 >= a.S ? tiles : a.causal ? ws0 / LB : 0;
+    const int first = a.causal ? s0 / ROWS : 0, tiles = 2 * ((a.L + 2 * ROWS - 1) / (2 * ROWS));     // first is even
+    const int w_first = ws0 >= a.S ? tiles : a.causal ? ws0 / ROWS : 0;
     const FragRow fr;
     const FragT ft;
+    Tile<ET, 1> tq(a.q + wh.h * a.qh + wh.b * a.qb, a.qt, a.E, a.L, first);
+    Tile<ET, 1> to(a.d_out + ((int64_t)wh.b * a.L * a.H + wh.h) * a.Ev, (int64_t)a.H * a.Ev, a.Ev, a.L, first);
+    // weights: 32 queries x 128 keys, two chunks of eight keys per thread
+    raw16_t pw[2][2];
+    float dv[2] = {0.0f, 0.0f};
+    const int prow = threadIdx.x >> 4, pch = threadIdx.x & 15;
+    const bf16_t* const wplane = a.probs + (int64_t)wh.head * a.L * a.S;
+    const float* const dplane = a.d + (int64_t)wh.head * a.L;
+    const int pkey = s0 + 8 * pch;
+    auto load_weights = [&](int t, int set) {
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            const int r = t * ROWS + prow + 16 * i;
+            const bf16_t* row = wplane + (int64_t)min(r, a.L - 1) * a.S;
+            if constexpr (VEC) pw[set][i] = *reinterpret_cast<const raw16_u*>(row + min(pkey, a.S - 8));    // past the end: masked below
+            else pw[set][i] = load8(row, pkey, r < a.L ? a.S : 0);
+        }
+        dv[set] = dplane[min(t * ROWS + ((int)threadIdx.x & 31), a.L - 1)];
+    };
+    auto store = [&](int t, int b) {
+        tq.store(lds + b * TILE, 0, t, a.L);
+        to.store(lds + (2 + b) * TILE, 0, t, a.L);
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            const raw16_t zero = {0u, 0u, 0u, 0u};
+            const bool in = !VEC || (pkey < a.S && t * ROWS + prow + 16 * i < a.L);
+            *reinterpret_cast<raw16_t*>(lds + (4 + b) * TILE + (prow + 16 * i) * PITCH + pch * 16) = in ? pw[b][i] : zero;
+        }
+        // 0 past the end: a non-finite d must not reach the keys through absent queries
+        if (threadIdx.x < ROWS) dt[b * ROWS + threadIdx.x] = t * ROWS + (int)threadIdx.x < a.L ? a.scale * dv[b] : 0.0f;
+    };
+    tq.load(0);
+    to.load(0);
+    load_weights(first, 0);
+    load_weights(first + 1, 1);
     bf16x8_v vf[2 * ET];
     load_columns<ET>(vf, a.v + wh.g * a.vh + wh.b * a.vb, (uint32_t)(a.vt * 2), s, a.S, a.Ev);
     f32x16_v ak[ET], av[ET];
 #pragma unroll
     for (int t = 0; t < ET; ++t) { ak[t] = zero16(); av[t] = zero16(); }
-
-    Tile<LB, ET> tq(a.E), to(a.Ev);
-    // weights: 32 queries x 128 keys, two chunks of eight keys per thread
-    raw16_t pw[2];
-    float dv = 0.0f;
-    const int prow = threadIdx.x >> 4, pch = threadIdx.x & 15;
-    const uint32_t plds = prow * PITCH + ((pch ^ swz(prow)) << 4);
-    auto load = [&](int t) {
-        tq.load(qp, qpitch, t * LB, a.L);
-        to.load(op, opitch, t * LB, a.L);
 #pragma unroll
-        for (int i = 0; i < 2; ++i) {
-            const int r = t * LB + prow + 16 * i;
-            pw[i] = load8(pp + (int64_t)min(r, a.L - 1) * a.S, s0 + 8 * pch, r < a.L ? a.S : 0);
-        }
-        if (threadIdx.x < LB) {                     // 0 past the end: a non-finite d must not reach the keys through absent queries
-            const int r = t * LB + (int)threadIdx.x;
-            dv = r < a.L ? dp_[r] : 0.0f;
-        }
-    };
-    auto store = [&](int t) {
-        const int b = t & 1;
-        tq.store(qt + b * LTILE, t * LB, a.L);
-        to.store(ot + b * LTILE, t * LB, a.L);
-#pragma unroll
-        for (int i = 0; i < 2; ++i) *reinterpret_cast<raw16_t*>(pt + b * LTILE + plds + i * 16 * PITCH) = pw[i];
-        if (threadIdx.x < LB) dt[b * LB + threadIdx.x] = dv;
-    };
-    if (first < tiles) {
-        load(first);
-        store(first);
+    for (int b = 0; b < 2; ++b) {
+        tq.clear(lds + b * TILE);
+        to.clear(lds + (2 + b) * TILE);
     }
+    if (first < tiles) store(first, 0);
     __syncthreads();
-    for (int t = first; t < tiles; ++t) {
-        const int b = t & 1;
-        const char *qc = qt + b * LTILE, *oc = ot + b * LTILE, *pc = pt + b * LTILE;
-        if (t + 1 < tiles) load(t + 1);
-        if (t >= w_first) {
-            f32x16_v dp = zero16();
+    for (int t0 = first; t0 < tiles; t0 += 2) {
+        static_for<2>([&](auto U) {
+            constexpr int u = decltype(U)::value;
+            const int t = t0 + u;
+            const char *qc = lds + u * TILE, *oc = lds + (2 + u) * TILE, *pc = lds + (4 + u) * TILE;
+            tq.load(0);
+            to.load(0);
+            load_weights(t + 2, u);             // these come from memory, the others mostly from caches
+            if (t >= w_first) {
+                const f32x16_v dp = product<ET, 2>(fr, oc, vf);
 #pragma unroll
-            for (int kk = 0; kk < 2 * ET; ++kk) dp = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fr.get(oc, 0, kk), vf[kk], dp, 0, 0, 0);
+                for (int n = 0; n < 2; ++n) {
+                    const bf16x8_v pb = ft.get(pc, 16 * n, w);       // the wave's 32 keys are "features" 32 w .. of the weights' tile
 #pragma unroll
-            for (int n = 0; n < 2; ++n) {
-                const bf16x8_v pb = ft.get(pc, 16 * n, w);       // the wave's 32 keys are "features" 32 w .. of the weights' tile
+                    for (int e = 0; e < ET; ++e) av[e] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ft.get(oc, 16 * n, e), pb, av[e], 0, 0, 0);
+                    const float4 d0 = *reinterpret_cast<const float4*>(dt + u * ROWS + 16 * n + 4 * h);
+                    const float4 d1 = *reinterpret_cast<const float4*>(dt + u * ROWS + 16 * n + 8 + 4 * h);
+                    const float dd[8] = {d0.x, d0.y, d0.z, d0.w, d1.x, d1.y, d1.z, d1.w};
+                    const bf16x8_v ds = __builtin_bit_cast(bf16x8_v, softmax_rule(__builtin_bit_cast(raw16_t, pb), dp, n, dd, a.scale));
 #pragma unroll
-                for (int e = 0; e < ET; ++e) av[e] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ft.get(oc, 16 * n, e), pb, av[e], 0, 0, 0);
-                float dd[8];
-                const float4 d0 = *reinterpret_cast<const float4*>(dt + b * LB + 16 * n + 4 * h);
-                const float4 d1 = *reinterpret_cast<const float4*>(dt + b * LB + 16 * n + 8 + 4 * h);
-                dd[0] = d0.x; dd[1] = d0.y; dd[2] = d0.z; dd[3] = d0.w;
-                dd[4] = d1.x; dd[5] = d1.y; dd[6] = d1.z; dd[7] = d1.w;
-                const bf16x8_v ds = __builtin_bit_cast(bf16x8_v, softmax_rule(__builtin_bit_cast(raw16_t, pb), dp, n, dd, a.scale));
-#pragma unroll
-                for (int e = 0; e < ET; ++e) ak[e] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ft.get(qc, 16 * n, e), ds, ak[e], 0, 0, 0);
+                    for (int e = 0; e < ET; ++e) ak[e] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ft.get(qc, 16 * n, e), ds, ak[e], 0, 0, 0);
+                }
             }
-        }
-        if (t + 1 < tiles) store(t + 1);
-        __syncthreads();
+            store(t + 1, 1 - u);
+            __syncthreads();
+        });
     }
     const int sc = min(s, a.S - 1);
     store_features<ET>(ak, a.dk + wh.i0 * a.dkr + wh.g * a.kh + wh.b * a.kb + (int64_t)sc * a.kt, s < a.S, a.E);
@@ -561,27 +674,31 @@ static int launch_fwd(hipStream_t s, Args& a) {
     LUX_CHECK_LAUNCH();
     return LUXHIP_OK;
 }
-template <int ET>
-static int launch_bwd(hipStream_t s, Args& a) {
+template <int ET, bool VEC>
+static int launch_bwd_as(hipStream_t s, Args& a) {
     static ResidentOnce ro;
     ro.get([&](hipError_t& err) {
-        err = hipFuncSetAttribute(reinterpret_cast<const void*>(dq_kernel<ET>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)FWD_LDS);
+        err = hipFuncSetAttribute(reinterpret_cast<const void*>(dq_kernel<ET, VEC>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)FWD_LDS);
         if (err == hipSuccess)
-            err = hipFuncSetAttribute(reinterpret_cast<const void*>(dkv_kernel<ET>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)DKV_LDS);
+            err = hipFuncSetAttribute(reinterpret_cast<const void*>(dkv_kernel<ET, VEC>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)DKV_LDS);
         return 1;
     });
     LUX_CHECK_HIP(ro.error);
-    a.blocks = (int)ceil_div(a.S, COLS);
     {
-        ProfScope ps("attn_dkv_kernel", s);
-        dkv_kernel<ET><<<dim3((unsigned)a.blocks * (unsigned)a.heads), dim3(THREADS), DKV_LDS, s>>>(a);
+        a.blocks = (int)ceil_div(a.L, COLS);
+        ProfScope ps("attn_dq_kernel", s);
+        dq_kernel<ET, VEC><<<dim3((unsigned)a.blocks * (unsigned)a.heads), dim3(THREADS), FWD_LDS, s>>>(a);
         LUX_CHECK_LAUNCH();
     }
-    a.blocks = (int)ceil_div(a.L, COLS);
-    ProfScope ps("attn_dq_kernel", s);
-    dq_kernel<ET><<<dim3((unsigned)a.blocks * (unsigned)a.heads), dim3(THREADS), FWD_LDS, s>>>(a);
+    a.blocks = (int)ceil_div(a.S, COLS);
+    ProfScope ps("attn_dkv_kernel", s);
+    dkv_kernel<ET, VEC><<<dim3((unsigned)a.blocks * (unsigned)a.heads), dim3(THREADS), DKV_LDS, s>>>(a);
     LUX_CHECK_LAUNCH();
     return LUXHIP_OK;
+}
+template <int ET>
+static int launch_bwd(hipStream_t s, Args& a) {
+    return a.S % 8 == 0 ? launch_bwd_as<ET, true>(s, a) : launch_bwd_as<ET, false>(s, a);
 }
 
 // Offsets inside one head's operand are 32-bit bytes, a grid has fewer than 2^31 / 256 workgroups, loads are 16 bytes wide
@@ -624,7 +741,10 @@ static int attention_args(attn::Args& a, int dtype, int64_t E, int64_t Ev, int64
     a.vt = sv[0]; a.vh = sv[1]; a.vb = sv[2];
     a.causal = causal != 0;
     a.scale = (float)scale;
-    a.c = (float)(scale * 1.4426950408889634);
+    // at least the smallest normal number: a masked logit is -inf before it is scaled
+    a.negative = scale < 0;
+    a.c = (float)(std::abs(scale) * 1.4426950408889634);
+    if (a.c < 1.2e-38f) a.c = 1.2e-38f;
     if (S == 0 || L == 0 || a.H == 0 || batch_dims[2] == 0) return LUXHIP_OK;
     LUX_INVALID_IF(q == nullptr || k == nullptr || v == nullptr, "attention: null operand");
     LUX_UNSUPPORTED_IF(!aligned16(q) || !aligned16(k) || !aligned16(v), "fused attention: operands must be 16-byte aligned");
@@ -681,11 +801,9 @@ int luxhip_attention_bwd(luxhip_stream_t s, int dtype, int64_t E, int64_t Ev, in
     Workspace ws;
     rc = get_workspace((hipStream_t)s, (size_t)a.heads * a.L * sizeof(float), &ws);
     if (rc != LUXHIP_OK) return rc;
-    const int64_t so[3] = {a.Ev, (int64_t)a.Ev * a.r, (int64_t)a.Ev * a.H * a.L};
-    rc = attention_rowdot((hipStream_t)s, (const bf16_t*)d_out, out_wide, reinterpret_cast<float*>(ws.data), a.Ev, a.L, (int64_t)a.Ev * a.H,
-                          batch_dims, so);
-    if (rc != LUXHIP_OK) return rc;
-    a.d = reinterpret_cast<const float*>(ws.data);
+    a.dsum = reinterpret_cast<float*>(ws.data);
+    a.d = a.dsum;
+    a.out_wide = const_cast<float*>(out_wide);
     a.probs = const_cast<bf16_t*>((const bf16_t*)probs);
     a.d_out = (const bf16_t*)d_out;
     a.dq = (bf16_t*)dq;

@@ -275,7 +275,7 @@ __global__ __launch_bounds__(256) void attn_rowdot_quad_kernel(const T* __restri
 }
 
 template <typename T, typename TO>
-int attention_rowdot(hipStream_t s, const T* d_out, const TO* out, float* d, int64_t Ev, int64_t L, int64_t ldo, const int64_t* batch_dims,
+static int attention_rowdot(hipStream_t s, const T* d_out, const TO* out, float* d, int64_t Ev, int64_t L, int64_t ldo, const int64_t* batch_dims,
                      const int64_t* so) {
     const int64_t cols = batch_dims[0] * batch_dims[1] * batch_dims[2] * L;
     const int b0 = (int)batch_dims[0], b1 = (int)batch_dims[1];
@@ -288,9 +288,6 @@ int attention_rowdot(hipStream_t s, const T* d_out, const TO* out, float* d, int
     LUX_CHECK_LAUNCH();
     return LUXHIP_OK;
 }
-template int attention_rowdot<bf16_t, float>(hipStream_t, const bf16_t*, const float*, float*, int64_t, int64_t, int64_t, const int64_t*,
-                                             const int64_t*);
-
 static int gemm_check(int dtype, int act, int64_t M, int64_t N, int64_t K) {
     LUX_UNSUPPORTED_IF(dtype != LUXHIP_F32 && dtype != LUXHIP_BF16, "unsupported dtype %d", dtype);
     LUX_UNSUPPORTED_IF(act < 0 || act >= LUXHIP_ACT_COUNT, "unsupported activation id %d", act);

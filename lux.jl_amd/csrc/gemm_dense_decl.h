@@ -52,9 +52,4 @@ bool launch_split(hipStream_t s, DenseArgs<T>& a, bool a_kmajor, bool b_kmajor, 
 template <typename T>
 bool launch_split_pair(hipStream_t s, DenseArgs<T>& a, DenseArgs<T>& b, int* rc);
 
-// gemm.hip: d[b * L + n] = sum_e d_out[e, n] out[e, n] of product b (attention pullback)
-template <typename T, typename TO>
-int attention_rowdot(hipStream_t s, const T* d_out, const TO* out, float* d, int64_t Ev, int64_t L, int64_t ldo, const int64_t* batch_dims,
-                     const int64_t* so);
-
 }  // namespace luxhip

@@ -658,10 +658,20 @@ class _AttnLayout:
         self.batch = a.size // self.sb if self.sb else 0
 
 
-def _attention_spans(lq, lk, lv, Ev, H, B) -> bool:
-    """What the fused kernels address with 32-bit byte offsets inside a head, and their grid."""
-    span = max(lq.tokens * lq.st, lk.tokens * lk.st, lv.tokens * lv.st, lq.tokens * H * Ev)
-    return 2 * span < 1 << 31 and H * B < 1 << 23 and -(-max(lq.tokens, lk.tokens) // 128) * H * B < 1 << 23
+def _attention_fused(lq, lk, lv, E, Ev, H, B) -> bool:
+    """Whether the fused kernels (luxhip_attention_fwd / _bwd) can and should take the call: whole 16-byte vectors of at most
+    128 features, 32-bit byte offsets inside a head, and enough workgroups (one per 128 tokens and head).  Few long heads
+    leave most of the chip idle there, while the step-by-step products cut both token dims into tiles: with 128 features
+    2 heads of 2048 tokens took 222 against 133 us, 8 heads 225 against 189, 12 heads (192 workgroups) 226 against 255;
+    with 64 features 2 heads 162 against 135, 8 heads (128 workgroups) 164 against 187.  Up to 512 tokens and on ragged
+    key counts (step by step 195 us for 2 x 583 tokens, fused 113) the fused kernels are ahead at any number of heads."""
+    L, S = lq.tokens, lk.tokens
+    if not (0 < E <= 128 and 0 < Ev <= 128 and E % 8 == 0 and Ev % 8 == 0 and S > 0 and L > 0 and H > 0 and B > 0):
+        return False
+    span, groups = max(L * lq.st, S * lk.st, S * lv.st, L * H * Ev), -(-max(L, S) // 128) * H * B
+    if 2 * span >= 1 << 31 or H * B >= 1 << 23 or groups >= 1 << 23:
+        return False
+    return max(L, S) <= 512 or S % 8 != 0 or groups >= (144 if max(E, Ev) > 64 else 56)
 
 
 def _permute_leading3(a: DeviceArray, perm) -> DeviceArray:
@@ -753,10 +763,8 @@ def rrule_scaled_dot_product_attention(q, k, v, head_dim=1, token_dim=3, scale=N
     # bf16 without an fdrop: the product is also kept unrounded (fp32) for the pullback, whose softmax rule takes
     # its inner product from it; the array that is returned is its rounded copy
     out_wide = DeviceArray((Ev, H, L) + bshape, wide) if (fdrop is None and wide != dt) else None
-    # one kernel each way where it applies (bf16, whole 16-byte vectors of at most 128 features): luxhip_attention_fwd / _bwd
-    fused = (out_wide is not None and mask_a is None and bias_a is None and 0 < E <= 128 and 0 < Ev <= 128 and E % 8 == 0 and Ev % 8 == 0
-             and S > 0 and L > 0 and H > 0 and B > 0 and (q.ptr | k.ptr | v.ptr) % 16 == 0
-             and _attention_spans(lq, lk, lv, Ev, H, B))
+    fused = (out_wide is not None and mask_a is None and bias_a is None and (q.ptr | k.ptr | v.ptr) % 16 == 0
+             and _attention_fused(lq, lk, lv, E, Ev, H, B))
     logits, softmax_out, fdrop_back = None, probs, None
     out = DeviceArray((Ev, H, L) + bshape, dt)
     strides = (_i64x3((lq.st, lq.sh, lq.sb)), _i64x3((lk.st, lk.sh, lk.sb)), _i64x3((lv.st, lv.sh, lv.sb)))

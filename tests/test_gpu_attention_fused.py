@@ -13,8 +13,17 @@ CASES = [
     (8, 8, 1, 1, 1, 1, 1, 3, False), (32, 32, 2, 2, 31, 33, 1, 3, False), (40, 16, 2, 1, 65, 63, 2, 3, True),
     (64, 64, 8, 2, 129, 127, 1, 3, False), (64, 72, 3, 3, 257, 193, 1, 2, True), (96, 96, 4, 4, 128, 256, 2, 3, True),
     (80, 48, 2, 2, 160, 100, 1, 3, True), (128, 128, 8, 8, 256, 256, 1, 2, False), (128, 128, 2, 1, 384, 385, 1, 3, True),
-    (128, 104, 16, 8, 97, 300, 1, 3, False), (16, 128, 8, 1, 200, 130, 2, 3, True),
+    (128, 104, 16, 8, 97, 300, 1, 3, False), (16, 128, 8, 1, 200, 130, 2, 3, True), (64, 64, 2, 2, 33, 8, 1, 3, False),
+    (96, 80, 2, 2, 72, 200, 2, 3, False), (128, 128, 3, 3, 161, 136, 1, 3, True), (72, 64, 1, 1, 40, 16, 3, 2, True),
 ]
+
+
+def test_few_long_heads_stay_on_the_step_by_step_products(gpu):
+    """2 heads of 1024 tokens are 16 workgroups of the fused kernels; the same tokens in 16 heads are 128."""
+    for heads, fused in ((2, False), (16, True)):
+        d = dev(gpu, np.zeros((64, heads, 1024, 1), np.float32), "bf16")
+        names = kernels_of(gpu, lambda: gpu.scaled_dot_product_attention(d, d, d))
+        assert ("attn_fwd_kernel" in names) == fused
 
 
 @pytest.mark.parametrize("case", range(len(CASES)))
