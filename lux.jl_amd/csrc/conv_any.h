@@ -111,10 +111,10 @@ struct RowLoader {
             reg[i] = *reinterpret_cast<const u32x4_v*>(valid ? static_cast<const void*>(p) : g.zero);
         }
     }
+    template <bool SPLIT>
     __device__ __forceinline__ void store(u32x4_v (&reg)[PER], T* lds, int) const {
 #pragma unroll
-        for (int i = 0; i < PER; ++i)
-            *reinterpret_cast<u32x4_v*>(lds + lds_chunk_offset<T, true, ROWS>((int)threadIdx.x / CPR + i * STEP, chunk)) = reg[i];
+        for (int i = 0; i < PER; ++i) put_chunk<T, true, ROWS, SPLIT>(lds, (int)threadIdx.x / CPR + i * STEP, chunk, reg[i]);
     }
 };
 
@@ -153,7 +153,7 @@ __device__ __forceinline__ float own_taps_sum(const Args<T>& g, const Sub& q, co
 // costs 2 to 4 %, and a register that takes a wave from every SIMD unless it is told to stay below (256 x 32 tiles of the first
 // layer, 78 us with four waves, 85 with three).
 template <typename T, int WM, int WN, int NWM, int NWN, bool MERGED>
-__global__ __launch_bounds__(split::THREADS, MERGED && WM * WN < 4 ? 4 : 1) void conv_any_kernel(Args<T> g) {
+__global__ __launch_bounds__(split::THREADS, MERGED && WM * WN < 4 ? (sizeof(T) == 4 && WM * WN == 2 ? 3 : 4) : (split_waves<T, WM, WN>())) void conv_any_kernel(Args<T> g) {
     using S = Shape<T, WM, WN, NWM, NWN>;
     using Core = typename S::Core;
     using ML = typename Core::ML;
@@ -312,12 +312,13 @@ struct WgradRowLoader {
             reg[i] = *reinterpret_cast<const u32x4_v*>(valid ? static_cast<const void*>(p) : g.zero);
         }
     }
+    template <bool SPLIT>
     __device__ __forceinline__ void store(u32x4_v (&reg)[PER], T* lds, int skip) const {
 #pragma unroll
         for (int i = 0; i < PER; ++i) {
             const int k = (int)threadIdx.x / CPR + i * STEP;
             const u32x4_v v = k < skip ? u32x4_v{0u, 0u, 0u, 0u} : reg[i];
-            *reinterpret_cast<u32x4_v*>(lds + lds_chunk_offset<T, false, ROWS>(r, k)) = v;
+            put_chunk<T, false, ROWS, SPLIT>(lds, r, k, v);
         }
     }
 };
@@ -331,7 +332,7 @@ struct WgradShape {
 };
 
 template <typename T, int WM, int WN, int NWM, int NWN>
-__global__ __launch_bounds__(split::THREADS) void conv_any_wgrad_kernel(WgradArgs<T> g) {
+__global__ __launch_bounds__(split::THREADS, (split_waves<T, WM, WN>())) void conv_any_wgrad_kernel(WgradArgs<T> g) {
     using S = WgradShape<T, WM, WN, NWM, NWN>;
     using Core = typename S::Core;
     using ML = typename Core::ML;

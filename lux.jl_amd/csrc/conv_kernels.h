@@ -216,11 +216,12 @@ struct ConvTapLoaderK {
             reg[i] = *p;
         }
     }
+    template <bool SPLIT>
     __device__ __forceinline__ void store(T* lds) const {
 #pragma unroll
         for (int i = 0; i < PER_THREAD; ++i) {
             const int r = threadIdx.x / CPR + i * STEP;
-            *reinterpret_cast<u32x4_v*>(lds + lds_chunk_offset<T, true, ROWS>(r, chunk_el)) = reg[i];
+            put_chunk<T, true, ROWS, SPLIT>(lds, r, chunk_el, reg[i]);
         }
     }
 };
@@ -241,7 +242,7 @@ struct ConvTapArgs {
 // Persistent: workgroup b handles tiles b, b + gridDim.x, ...  On the direct-to-LDS path the
 // first stages of the next tile are issued before the epilogue of the current one.
 template <typename T, int WM, int WN, int NWN, int NST, int NWM>
-__global__ __launch_bounds__(NWM * NWN * 64) void conv_tap_kernel(ConvTapArgs<T> a) {
+__global__ __launch_bounds__(NWM * NWN * 64, (split_waves<T, WM, WN>())) void conv_tap_kernel(ConvTapArgs<T> a) {
     constexpr bool DIRECT = sizeof(T) == 2;
     using ML = GemmMainloop<T, WM, WN, true, true, DIRECT, NWN, NST, NWM>;
     extern __shared__ __align__(16) unsigned char lds_raw[];

@@ -9,7 +9,8 @@
 // lane.
 //
 // Storage types:  bf16 -> v_mfma_f32_32x32x16_bf16 (BK = 32 per stage),
-//                 fp32 -> v_mfma_f32_32x32x2_f32   (BK = 16 per stage).
+//                 fp32 -> v_mfma_f32_32x32x2_f32   (BK = 16 per stage), or three bf16 parts per value on
+//                 v_mfma_f32_32x32x16_bf16 (split_f32, put_chunk).
 //
 // Each operand tile is staged global -> registers -> LDS (double buffered, one barrier per
 // stage) in the layout that matches how it lies in memory:
@@ -102,9 +103,19 @@ struct GemmTraits<float> {
 //       32-byte granules).
 __host__ __device__ constexpr int mn_swizzle_shift(int rows) { return rows >= 128 ? 5 : 4; }
 
+// fp32 contractions on the bf16 matrix cores (put_chunk): waves of 2 or 4 accumulators.  One accumulator per wave spends as much
+// on the cutting as it saves (64 x 64 tiles: 0 to 7 % slower than the fp32 instruction).  Four accumulators take 128 registers
+// with the smaller partial products, and the compiler would go on to give the kernel all 512: split_waves is the launch bound that
+// keeps two waves on a SIMD (59.2 GFLOP of a 3 x 3 convolution: 545 us with one wave, 371 with two, 531 on the fp32 instruction).
+template <typename T, int WM, int WN>
+__host__ __device__ constexpr bool split_f32() { return sizeof(T) == 4 && (WM * WN == 2 || WM * WN == 4); }
+template <typename T, int WM, int WN>
+__host__ __device__ constexpr int split_waves() { return split_f32<T, WM, WN>() && WM * WN == 4 ? 2 : 1; }
+
 // elements of one LDS stage of an operand tile with `rows` rows
 template <typename T, bool KMAJOR>
-__host__ __device__ constexpr int lds_tile_elems(int rows) {
+__host__ __device__ constexpr int lds_tile_elems(int rows, bool split) {
+    if (split) return rows * (3 * GemmTraits<T>::BK / 2);                // three bf16 planes (put_chunk); the plain layouts are smaller
     return KMAJOR ? rows * GemmTraits<T>::kmajor_stride() : GemmTraits<T>::BK * (rows + GemmTraits<T>::PAD_MN);
 }
 
@@ -128,6 +139,44 @@ __device__ __forceinline__ int lds_chunk_offset(int r, int k) {
     } else {
         if constexpr (sizeof(T) == 2) return k * ROWS + (r ^ ((k & 3) << mn_swizzle_shift(ROWS)));   // r is a multiple of 8
         else return k * (ROWS + Tr::PAD_MN) + r;
+    }
+}
+
+// fp32 on the bf16 matrix cores.  v_mfma_f32_32x32x2_f32 runs at 1/16 of the bf16 rate, so an fp32 value is cut into three bf16
+// values (8 + 8 + 8 significand bits: hi + mid + lo is the value exactly, down to 2^-110) on its way into LDS, and a product
+// into the six partial products of at least 2^-18 of it; what is left out is below 2^-26.  Partial products are exact and are
+// added in fp32, hi * hi (one instruction per 16 k, where the fp32 instruction takes eight) apart from the five smaller ones,
+// so the sum is rounded less often, not more.
+// Values for which the parts do not carry the value are left to the fp32 instruction: a tile whose result holds an infinity or
+// a NaN (an infinite operand times an absent part, or a value that rounds to a bf16 infinity), or a number below 2^-80 (operands
+// so small that their parts underflow) is computed again, see GemmMainloop::run.
+//
+// A 16-byte chunk that starts at (row r, column k) of a tile -> LDS.  SPLIT: three bf16 planes of ROWS x 16, each K-major
+// [row][16] with the two 16-byte halves of a row exchanged in rows 8 .. 15 of sixteen (sixteen rows then fall into sixteen
+// different chunks of the bank period), or MN-major [k][ROWS] as for bf16 operands.
+template <int ROWS>
+__host__ __device__ constexpr int plane_elems() { return ROWS * 8; }      // in floats
+template <typename T, bool KMAJOR, int ROWS, bool SPLIT>
+__device__ __forceinline__ void put_chunk(T* lds, int r, int k, u32x4_v v) {
+    if constexpr (SPLIT) {
+        static_assert(sizeof(T) == 4 && GemmTraits<T>::BK == 16, "planes of 16 k");
+        bf16_t* p = reinterpret_cast<bf16_t*>(lds) + (KMAJOR ? r * 16 + (k ^ (r & 8)) : k * ROWS + (r ^ ((k & 3) << mn_swizzle_shift(ROWS))));
+        float f[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) f[i] = __uint_as_float(v[i]);
+#pragma unroll
+        for (int q = 0; q < 3; ++q) {
+            const uint32_t a = f32x2_to_bf16x2(f[0], f[1]), b = f32x2_to_bf16x2(f[2], f[3]);
+            *reinterpret_cast<uint2*>(p + q * 2 * plane_elems<ROWS>()) = make_uint2(a, b);
+            if (q < 2) {
+                f[0] -= __uint_as_float(a << 16);
+                f[1] -= __uint_as_float(a & 0xffff0000u);
+                f[2] -= __uint_as_float(b << 16);
+                f[3] -= __uint_as_float(b & 0xffff0000u);
+            }
+        }
+    } else {
+        *reinterpret_cast<u32x4_v*>(lds + lds_chunk_offset<T, KMAJOR, ROWS>(r, k)) = v;
     }
 }
 
@@ -196,12 +245,13 @@ struct TileLoader {
         }
     }
 
+    template <bool SPLIT>
     __device__ __forceinline__ void store(T* lds) const {
 #pragma unroll
         for (int i = 0; i < PER_THREAD; ++i) {
             int r, k;
             coords(threadIdx.x + i * THREADS, r, k);
-            *reinterpret_cast<u32x4_v*>(lds + lds_chunk_offset<T, KMAJOR, ROWS>(r, k)) = reg[i];
+            put_chunk<T, KMAJOR, ROWS, SPLIT>(lds, r, k, reg[i]);
         }
     }
 };
@@ -360,6 +410,82 @@ __device__ __forceinline__ void load_frag_f32(const float* lds, int rbase, int k
     }
 }
 
+// Fragment (32 rows x 16 k) of part `plane` of a split tile
+template <bool KMAJOR, int ROWS>
+__device__ __forceinline__ bf16x8_v load_frag_part(const float* tile, int rbase, int plane) {
+    const bf16_t* p = reinterpret_cast<const bf16_t*>(tile + plane * plane_elems<ROWS>());
+    if constexpr (KMAJOR) {
+        const int l = threadIdx.x & 63, r = rbase + (l & 31);
+        return __builtin_bit_cast(bf16x8_v, *reinterpret_cast<const u32x4_v*>(p + r * 16 + (((l >> 5) << 3) ^ (r & 8))));
+    } else {
+        return load_frag_bf16<false, ROWS>(p, rbase, 0);
+    }
+}
+// neither zero nor a finite number of at least 2^-80
+__device__ __forceinline__ bool split_suspect(float v) {
+    const uint32_t u = __float_as_uint(v) & 0x7fffffffu;
+    return u - 1u < 0x17800000u - 1u || u >= 0x7f800000u;
+}
+
+template <int WM, int WN>
+__device__ __forceinline__ bool split_suspect(const f32x16_v (&acc)[WM][WN]) {
+    bool any = false;
+#pragma unroll
+    for (int i = 0; i < WM; ++i)
+#pragma unroll
+        for (int j = 0; j < WN; ++j)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) any |= split_suspect(acc[i][j][r]);
+    return any;
+}
+// One stage (16 k) of a wave's WM x WN accumulators; SPLIT: on the bf16 matrix cores, the smaller partial products in `small`
+template <bool SPLIT, bool A_KMAJOR, bool B_KMAJOR, int TILE_M, int TILE_N, int WM, int WN>
+__device__ __forceinline__ void mfma_stage_f32(const float* As, const float* Bs, int wave_m, int wave_n, f32x16_v (&acc)[WM][WN],
+                                               f32x16_v (&small)[WM][WN]) {
+    if constexpr (SPLIT) {
+        bf16x8_v fa[3][WM], fb[3][WN];
+#pragma unroll
+        for (int q = 0; q < 3; ++q) {
+#pragma unroll
+            for (int j = 0; j < WN; ++j) fb[q][j] = load_frag_part<B_KMAJOR, TILE_N>(Bs, wave_n + j * 32, q);
+#pragma unroll
+            for (int i = 0; i < WM; ++i) fa[q][i] = load_frag_part<A_KMAJOR, TILE_M>(As, wave_m + i * 32, q);
+        }
+        auto term = [&](auto QA, auto QB, f32x16_v (&to)[WM][WN]) {
+#pragma unroll
+            for (int i = 0; i < WM; ++i)
+#pragma unroll
+                for (int j = 0; j < WN; ++j)
+                    to[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fb[decltype(QB)::value][j], fa[decltype(QA)::value][i], to[i][j], 0, 0, 0);
+        };
+        using std::integral_constant;
+        const integral_constant<int, 0> hi{};
+        const integral_constant<int, 1> mid{};
+        const integral_constant<int, 2> lo{};
+        term(hi, hi, acc);                 // in the order in which the parts arrive from LDS
+        term(hi, mid, small);
+        term(mid, hi, small);
+        term(mid, mid, small);
+        term(hi, lo, small);
+        term(lo, hi, small);
+    } else {
+#pragma unroll
+        for (int kw = 0; kw < 2; ++kw) {
+            float fa[WM][4], fb[WN][4];
+#pragma unroll
+            for (int i = 0; i < WM; ++i) load_frag_f32<A_KMAJOR, TILE_M>(As, wave_m + i * 32, kw, fa[i]);
+#pragma unroll
+            for (int j = 0; j < WN; ++j) load_frag_f32<B_KMAJOR, TILE_N>(Bs, wave_n + j * 32, kw, fb[j]);
+#pragma unroll
+            for (int s = 0; s < 4; ++s)
+#pragma unroll
+                for (int i = 0; i < WM; ++i)
+#pragma unroll
+                    for (int j = 0; j < WN; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(fb[j][s], fa[i][s], acc[i][j], 0, 0, 0);
+        }
+    }
+}
+
 // ----------------------------------------------------------------------------- tile -> C coordinates
 // Tile `id` of `nb` = tiles_m * tiles_n tiles -> (tm, tn).  Workgroups walk the tiles in
 // strides of the grid size (a multiple of 8 whenever there are more tiles than workgroups), so
@@ -403,17 +529,20 @@ struct GemmMainloop {
     static constexpr int TILE_M = NWM * WM * 32, TILE_N = NWN * WN * 32;
     using PlainLoaderA = TileLoader<T, A_KMAJOR, TILE_M, FULL, THREADS>;
     using PlainLoaderB = TileLoader<T, B_KMAJOR, TILE_N, FULL, THREADS>;
-    static constexpr int A_ELEMS = lds_tile_elems<T, A_KMAJOR>(TILE_M);
-    static constexpr int B_ELEMS = lds_tile_elems<T, B_KMAJOR>(TILE_N);
+    static constexpr int A_ELEMS = lds_tile_elems<T, A_KMAJOR>(TILE_M, split_f32<T, WM, WN>());
+    static constexpr int B_ELEMS = lds_tile_elems<T, B_KMAJOR>(TILE_N, split_f32<T, WM, WN>());
     static constexpr int STAGE_ELEMS = A_ELEMS + B_ELEMS;
     static constexpr bool DIRECT = FULL && sizeof(T) == 2;     // global -> LDS without registers
     static constexpr int NST = NSTAGES > 0 ? NSTAGES : (DIRECT ? 4 : 2);   // LDS stages
     static constexpr size_t LDS_BYTES = NST * (size_t)STAGE_ELEMS * sizeof(T);
+    static constexpr bool SPLIT_F32 = split_f32<T, WM, WN>();
     static constexpr int PERM_A = (PERMUTE && DIRECT && A_KMAJOR && WM > 1 && (THREADS / 4) % (32 * WM) == 0) ? WM : 0;
     static constexpr int M_STEP = PERM_A ? 1 : 32;            // distance in m between acc[i] and acc[i + 1] of a lane
     using DirectLoaderA = DirectLoader<A_KMAJOR, TILE_M, THREADS, false, PERM_A>;
     using DirectLoaderB = DirectLoader<B_KMAJOR, TILE_N, THREADS>;
 
+    // MAY_SPLIT: fp32 products may take the bf16 matrix cores (split_f32)
+    template <bool MAY_SPLIT = true>
     __device__ __forceinline__ static void run(const Operand<T>& A, const Operand<T>& B, int K, int m0, int n0, T* lds,
                                                f32x16_v (&acc)[WM][WN]) {
         if constexpr (FULL && sizeof(T) == 2) {
@@ -421,7 +550,7 @@ struct GemmMainloop {
         } else {
             PlainLoaderA la(A, m0, K);
             PlainLoaderB lb(B, n0, K);
-            run(la, lb, K, lds, acc);
+            run<MAY_SPLIT>(la, lb, K, lds, acc);
         }
     }
 
@@ -580,18 +709,24 @@ struct GemmMainloop {
     }
 
     // k range [0, K) in stages of BK; the loaders decide what a stage contains
-    template <class LoaderA, class LoaderB>
+    template <bool MAY_SPLIT = true, class LoaderA, class LoaderB>
     __device__ __forceinline__ static void run(LoaderA& la, LoaderB& lb, int K, T* lds, f32x16_v (&acc)[WM][WN]) {
         static_assert(LoaderA::KMAJOR == A_KMAJOR && LoaderB::KMAJOR == B_KMAJOR, "loader layout mismatch");
+        if constexpr (MAY_SPLIT && SPLIT_F32) {
+            run_as<true>(la, lb, K, lds, acc);
+            if (__syncthreads_or(split_suspect(acc)) == 0) return;
+        }
+        run_as<false>(la, lb, K, lds, acc);
+    }
+
+    // SPLIT: fp32 operands as three bf16 parts each
+    template <bool SPLIT, class LoaderA, class LoaderB>
+    __device__ __forceinline__ static void run_as(LoaderA& la, LoaderB& lb, int K, T* lds, f32x16_v (&acc)[WM][WN]) {
         const int w = threadIdx.x >> 6;
         const int wave_m = (w % NWM) * (WM * 32), wave_n = (w / NWM) * (WN * 32);
-#pragma unroll
-        for (int i = 0; i < WM; ++i)
-#pragma unroll
-            for (int j = 0; j < WN; ++j)
-#pragma unroll
-                for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.0f;
-
+        zero(acc);
+        f32x16_v small[WM][WN];                                 // SPLIT: the smaller partial products
+        if constexpr (SPLIT) zero(small);
         const int KT = (K + Tr::BK - 1) / Tr::BK;
         auto compute = [&](const T* As, const T* Bs) {
             if constexpr (sizeof(T) == 2) {
@@ -609,55 +744,68 @@ struct GemmMainloop {
                             acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fb[j], fa[i], acc[i][j], 0, 0, 0);
                 }
             } else {
-#pragma unroll
-                for (int kw = 0; kw < Tr::BK / 8; ++kw) {
-                    float fa[WM][4], fb[WN][4];
-#pragma unroll
-                    for (int i = 0; i < WM; ++i) load_frag_f32<A_KMAJOR, TILE_M>(As, wave_m + i * 32, kw, fa[i]);
-#pragma unroll
-                    for (int j = 0; j < WN; ++j) load_frag_f32<B_KMAJOR, TILE_N>(Bs, wave_n + j * 32, kw, fb[j]);
-#pragma unroll
-                    for (int s = 0; s < 4; ++s)
-#pragma unroll
-                        for (int i = 0; i < WM; ++i)
-#pragma unroll
-                            for (int j = 0; j < WN; ++j)
-                                acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(fb[j][s], fa[i][s], acc[i][j], 0, 0, 0);
-                }
+                mfma_stage_f32<SPLIT, A_KMAJOR, B_KMAJOR, TILE_M, TILE_N>(As, Bs, wave_m, wave_n, acc, small);
             }
         };
-        // Global loads run two stages ahead of the MFMAs (two register sets), LDS is double
-        // buffered: while stage kt is consumed from one LDS buffer, stage kt+1 waits in the
-        // first register set for its LDS slot and stage kt+2 is in flight into the second.
-        LoaderA la2 = la;
-        LoaderB lb2 = lb;
         T* buf0 = lds;
         T* buf1 = lds + STAGE_ELEMS;
-        la.load(0);
-        lb.load(0);
-        la.store(buf0);
-        lb.store(buf0 + A_ELEMS);
-        if (KT > 1) { la.load(Tr::BK); lb.load(Tr::BK); }
-        if (KT > 2) { la2.load(2 * Tr::BK); lb2.load(2 * Tr::BK); }
-        __syncthreads();
-        int kt = 0;
-        for (; kt + 2 <= KT; kt += 2) {
-            // even stage: buf0 holds kt, set 1 holds kt+1, set 2 holds kt+2
-            compute(buf0, buf0 + A_ELEMS);
-            la.store(buf1);
-            lb.store(buf1 + A_ELEMS);
-            if (kt + 3 < KT) { la.load((kt + 3) * Tr::BK); lb.load((kt + 3) * Tr::BK); }
+        if constexpr (SPLIT) {
+            // Global loads run one stage ahead in one register set (a second one does not fit beside 128 accumulators at two
+            // waves per SIMD), LDS is double buffered.
+            la.load(0);
+            lb.load(0);
+            la.template store<true>(buf0);
+            lb.template store<true>(buf0 + A_ELEMS);
+            if (KT > 1) { la.load(Tr::BK); lb.load(Tr::BK); }
             __syncthreads();
-            // odd stage: buf1 holds kt+1, set 2 holds kt+2, set 1 holds kt+3
-            compute(buf1, buf1 + A_ELEMS);
-            if (kt + 2 < KT) {
-                la2.store(buf0);
-                lb2.store(buf0 + A_ELEMS);
-                if (kt + 4 < KT) { la2.load((kt + 4) * Tr::BK); lb2.load((kt + 4) * Tr::BK); }
+            for (int kt = 0; kt < KT; ++kt) {
+                compute(buf0, buf0 + A_ELEMS);
+                if (kt + 1 < KT) {
+                    la.template store<true>(buf1);
+                    lb.template store<true>(buf1 + A_ELEMS);
+                    if (kt + 2 < KT) { la.load((kt + 2) * Tr::BK); lb.load((kt + 2) * Tr::BK); }
+                }
+                __syncthreads();                                // the last one: a second pass refills the stages
+                T* const t = buf0;
+                buf0 = buf1;
+                buf1 = t;
             }
+#pragma unroll
+            for (int i = 0; i < WM; ++i)
+#pragma unroll
+                for (int j = 0; j < WN; ++j) acc[i][j] += small[i][j];
+        } else {
+            // Global loads run two stages ahead of the MFMAs (two register sets), LDS is double
+            // buffered: while stage kt is consumed from one LDS buffer, stage kt+1 waits in the
+            // first register set for its LDS slot and stage kt+2 is in flight into the second.
+            LoaderA la2 = la;
+            LoaderB lb2 = lb;
+            la.load(0);
+            lb.load(0);
+            la.template store<false>(buf0);
+            lb.template store<false>(buf0 + A_ELEMS);
+            if (KT > 1) { la.load(Tr::BK); lb.load(Tr::BK); }
+            if (KT > 2) { la2.load(2 * Tr::BK); lb2.load(2 * Tr::BK); }
             __syncthreads();
+            int kt = 0;
+            for (; kt + 2 <= KT; kt += 2) {
+                // even stage: buf0 holds kt, set 1 holds kt+1, set 2 holds kt+2
+                compute(buf0, buf0 + A_ELEMS);
+                la.template store<false>(buf1);
+                lb.template store<false>(buf1 + A_ELEMS);
+                if (kt + 3 < KT) { la.load((kt + 3) * Tr::BK); lb.load((kt + 3) * Tr::BK); }
+                __syncthreads();
+                // odd stage: buf1 holds kt+1, set 2 holds kt+2, set 1 holds kt+3
+                compute(buf1, buf1 + A_ELEMS);
+                if (kt + 2 < KT) {
+                    la2.template store<false>(buf0);
+                    lb2.template store<false>(buf0 + A_ELEMS);
+                    if (kt + 4 < KT) { la2.load((kt + 4) * Tr::BK); lb2.load((kt + 4) * Tr::BK); }
+                }
+                __syncthreads();
+            }
+            if (kt < KT) compute(buf0, buf0 + A_ELEMS);   // odd number of stages: the last one sits in buf0
         }
-        if (kt < KT) compute(buf0, buf0 + A_ELEMS);   // odd number of stages: the last one sits in buf0
     }
 
     // First m and n of this lane inside the tile at (m0, n0); element acc[i][j][r] belongs to

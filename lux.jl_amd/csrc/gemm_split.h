@@ -73,6 +73,7 @@ struct Loader {
             reg[i] = *reinterpret_cast<const typename UnalignedVec<T>::type*>(p + voff[i]);
     }
     // skip: leading k of the stage that are to count as zero
+    template <bool SPLIT>
     __device__ __forceinline__ void store(u32x4_v (&reg)[PER], T* lds, int skip) const {
 #pragma unroll
         for (int i = 0; i < PER; ++i) {
@@ -99,7 +100,7 @@ struct Loader {
                     if (k < skip) v = u32x4_v{0u, 0u, 0u, 0u};
                 }
             }
-            *reinterpret_cast<u32x4_v*>(lds + lds_chunk_offset<T, KMAJOR, ROWS>(r, k)) = v;
+            put_chunk<T, KMAJOR, ROWS, SPLIT>(lds, r, k, v);
         }
     }
 };
@@ -120,7 +121,9 @@ struct Core {
     static constexpr size_t LDS_BYTES = (size_t)U * ML::STAGE_ELEMS * sizeof(T);
     static_assert(NWM * NWN * 64 == THREADS, "four waves");
 
-    __device__ __forceinline__ static void compute(const T* As, const T* Bs, int wave_m, int wave_n, f32x16_v (&acc)[WM][WN]) {
+    template <bool SPLIT>
+    __device__ __forceinline__ static void compute(const T* As, const T* Bs, int wave_m, int wave_n, f32x16_v (&acc)[WM][WN],
+                                                   f32x16_v (&small)[WM][WN]) {
         if constexpr (sizeof(T) == 2) {
 #pragma unroll
             for (int kk = 0; kk < Tr::BK / 16; ++kk) {
@@ -135,29 +138,25 @@ struct Core {
                     for (int j = 0; j < WN; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fb[j], fa[i], acc[i][j], 0, 0, 0);
             }
         } else {
-#pragma unroll
-            for (int kw = 0; kw < Tr::BK / 8; ++kw) {
-                float fa[WM][4], fb[WN][4];
-#pragma unroll
-                for (int i = 0; i < WM; ++i) load_frag_f32<AK, ML::TILE_M>(As, wave_m + i * 32, kw, fa[i]);
-#pragma unroll
-                for (int j = 0; j < WN; ++j) load_frag_f32<BKM, ML::TILE_N>(Bs, wave_n + j * 32, kw, fb[j]);
-#pragma unroll
-                for (int s = 0; s < 4; ++s)
-#pragma unroll
-                    for (int i = 0; i < WM; ++i)
-#pragma unroll
-                        for (int j = 0; j < WN; ++j)
-                            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(fb[j][s], fa[i][s], acc[i][j], 0, 0, 0);
-            }
+            mfma_stage_f32<SPLIT, AK, BKM, ML::TILE_M, ML::TILE_N>(As, Bs, wave_m, wave_n, acc, small);
         }
     }
 
     // k range [kbeg, kend)
     __device__ __forceinline__ static void run(const LA& la, const LB& lb, int kbeg, int kend, T* lds, f32x16_v (&acc)[WM][WN]) {
+        if constexpr (ML::SPLIT_F32) {
+            run_as<true>(la, lb, kbeg, kend, lds, acc);
+            if (__syncthreads_or(split_suspect(acc)) == 0) return;
+        }
+        run_as<false>(la, lb, kbeg, kend, lds, acc);
+    }
+    template <bool SPLIT>
+    __device__ __forceinline__ static void run_as(const LA& la, const LB& lb, int kbeg, int kend, T* lds, f32x16_v (&acc)[WM][WN]) {
         const int w = threadIdx.x >> 6;
         const int wave_m = (w % NWM) * (WM * 32), wave_n = (w / NWM) * (WN * 32);
         ML::zero(acc);
+        f32x16_v small[WM][WN];                                 // SPLIT: the smaller partial products
+        if constexpr (SPLIT) ML::zero(small);
         u32x4_v ra[U][LA::PER], rb[U][LB::PER];
         int skip[U];
         auto fetch_stages = [&](int k0) {
@@ -177,15 +176,21 @@ struct Core {
 #pragma unroll
             for (int u = 0; u < U; ++u)
                 if (k0 + u * Tr::BK < kend) {
-                    la.store(ra[u], lds + u * ML::STAGE_ELEMS, skip[u]);
-                    lb.store(rb[u], lds + u * ML::STAGE_ELEMS + ML::A_ELEMS, skip[u]);
+                    la.template store<SPLIT>(ra[u], lds + u * ML::STAGE_ELEMS, skip[u]);
+                    lb.template store<SPLIT>(rb[u], lds + u * ML::STAGE_ELEMS + ML::A_ELEMS, skip[u]);
                 }
             __syncthreads();
             if (k0 + U * Tr::BK < kend) fetch_stages(k0 + U * Tr::BK);
 #pragma unroll
             for (int u = 0; u < U; ++u)
-                if (k0 + u * Tr::BK < kend) compute(lds + u * ML::STAGE_ELEMS, lds + u * ML::STAGE_ELEMS + ML::A_ELEMS, wave_m, wave_n, acc);
+                if (k0 + u * Tr::BK < kend) compute<SPLIT>(lds + u * ML::STAGE_ELEMS, lds + u * ML::STAGE_ELEMS + ML::A_ELEMS, wave_m, wave_n, acc, small);
             __syncthreads();
+        }
+        if constexpr (SPLIT) {
+#pragma unroll
+            for (int i = 0; i < WM; ++i)
+#pragma unroll
+                for (int j = 0; j < WN; ++j) acc[i][j] += small[i][j];
         }
     }
 
@@ -244,7 +249,7 @@ __device__ __forceinline__ void tile_slice(const DenseArgs<T>& a, const Plan& p,
 }
 
 template <typename T, int W, bool AK, bool BKM>
-__global__ __launch_bounds__(THREADS) void split_gemm_kernel(DenseArgs<T> a, Plan p) {
+__global__ __launch_bounds__(THREADS, (split_waves<T, W, W>())) void split_gemm_kernel(DenseArgs<T> a, Plan p) {
     extern __shared__ __align__(16) unsigned char lds_raw[];
     tile_slice<T, W, AK, BKM>(a, p, blockIdx.x, reinterpret_cast<T*>(lds_raw));
 }

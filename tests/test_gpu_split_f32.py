@@ -1,0 +1,82 @@
+"""fp32 contractions whose values are cut into three bf16 parts: errors of fp32 size, and the values that have no such parts
+(infinities, NaN, numbers near the ends of the range), which take the fp32 instruction."""
+import numpy as np
+import pytest
+
+from tests.util import assert_close, dev, stable_seed
+
+pytestmark = pytest.mark.gpu
+
+# M, N, K: whole 128 x 128 tiles, ragged ones that fill the chip, slices of a long contraction; M x N all above a 64 x 64 tile per compute unit
+SIZES = [(2048, 2048, 64), (2047, 2050, 40), (1280, 1152, 1031), (2048, 1664, 16)]
+
+
+def product(gpu, w, x):
+    return gpu.matmul(dev(gpu, w, "f32"), dev(gpu, x, "f32")).to_numpy()
+
+
+@pytest.mark.parametrize("size", range(len(SIZES)))
+def test_error_is_that_of_fp32(gpu, size):
+    """Rounding a partial sum of k terms leaves an error uniform in 2^-24 of it, 2^-24 / sqrt(3) of sqrt(k / K) of the result in
+    the mean square; at most K independent ones add up to 2^-24 sqrt(K / 6), twice of which is allowed.  The products are exact
+    to 2^-26 of the terms, whose 2-norm is the result's."""
+    M, N, K = SIZES[size]
+    rng = np.random.default_rng(stable_seed("split", size))
+    w, x = rng.normal(size=(M, K)).astype(np.float32), rng.normal(size=(K, N)).astype(np.float32)
+    want = w.astype(np.float64) @ x.astype(np.float64)
+    err = product(gpu, w, x).astype(np.float64) - want
+    assert np.linalg.norm(err) <= (2.0 ** -23 * np.sqrt(K / 6) + 2.0 ** -26) * np.linalg.norm(want)
+
+
+@pytest.mark.parametrize("size", range(len(SIZES)))
+def test_values_without_parts(gpu, size):
+    M, N, K = SIZES[size]
+    rng = np.random.default_rng(stable_seed("split-special", size))
+    # multiples of 1/4 up to 2: a value with one bf16 part, so an infinite partner meets parts that are zero
+    w, x = (rng.integers(1, 9, size=s).astype(np.float32) / 4 for s in ((M, K), (K, N)))
+    big = np.finfo(np.float32).max
+    w[3, 1], w[140, 2], w[141, 0], w[M - 1, 3] = np.inf, -np.inf, np.nan, big
+    w[M - 1, :3] = w[M - 1, 4:] = 0
+    x[3] = 0.5
+    got = product(gpu, w, x)
+    want = w.astype(np.float64) @ x.astype(np.float64)
+    assert (got[3] == np.inf).all() and (got[140] == -np.inf).all() and np.isnan(got[141]).all()
+    np.testing.assert_allclose(got[M - 1], 0.5 * big, rtol=1e-6)
+    rows = np.setdiff1d(np.arange(M), (3, 140, 141, M - 1))
+    np.testing.assert_allclose(got[rows], want[rows], rtol=1e-6)
+
+
+@pytest.mark.parametrize("scale", [1e-35, 1e-30, 1e30])
+def test_numbers_near_the_ends_of_the_range(gpu, scale):
+    M, N, K = 2048, 2048, 64
+    rng = np.random.default_rng(stable_seed("split-scale", scale))
+    w, x = (rng.normal(size=(M, K)) * scale).astype(np.float32), rng.normal(size=(K, N)).astype(np.float32)
+    assert_close(product(gpu, w, x) / np.float64(scale), (w.astype(np.float64) @ x.astype(np.float64)) / scale, "f32", "scaled", rel=1e-5)
+
+
+@pytest.mark.parametrize("channels", [(128, 128), (80, 112), (48, 64)])
+def test_convolution_with_an_infinite_input(gpu, channels):
+    """Both gradients and the output of a 3 x 3 convolution: an infinity stays inside the windows that see it."""
+    cin, cout = channels
+    W = H = 30
+    n = 8
+    rng = np.random.default_rng(stable_seed("split-conv", channels))
+    x = rng.normal(size=(W, H, cin, n)).astype(np.float32)
+    w = np.abs(rng.normal(size=(3, 3, cin, cout)) * 0.1).astype(np.float32)
+    x[10, 12, 5, 3] = np.inf
+    cd = gpu.DenseConvDims(x.shape, w.shape, padding=1)
+    y = gpu.conv(dev(gpu, x, "f32"), dev(gpu, w, "f32"), cd).to_numpy()
+    inside = np.zeros(y.shape, bool)
+    inside[9:12, 11:14, :, 3] = True
+    assert (y[inside] == np.inf).all() and np.isfinite(y[~inside]).all()
+    x[10, 12, 5, 3] = 0
+    clean = gpu.conv(dev(gpu, x, "f32"), dev(gpu, w, "f32"), cd).to_numpy()
+    assert_close(y[~inside], clean[~inside].astype(np.float64), "f32", "outside the windows")
+    dy = rng.normal(size=y.shape).astype(np.float32)
+    dy[4, 4, 7, 2] = np.inf
+    dx = gpu.conv_data_grad(dev(gpu, dy, "f32"), dev(gpu, w, "f32"), cd).to_numpy()
+    inside = np.zeros(dx.shape, bool)
+    inside[3:6, 3:6, :, 2] = True
+    assert (dx[inside] == np.inf).all() and np.isfinite(dx[~inside]).all()
+    dw = gpu.conv_filter_grad(dev(gpu, x, "f32"), dev(gpu, dy, "f32"), cd).to_numpy()
+    assert np.isfinite(dw[:, :, :, np.arange(cout) != 7]).all() and not np.isfinite(dw[:, :, :, 7]).any()
