@@ -226,6 +226,34 @@ struct ConvTapLoaderK {
     }
 };
 
+// The filter matrix through registers: K-major rows, K in whole stages.  Rows past the last are the last one again (columns that
+// are not stored), so every load is one unconditional instruction.
+template <typename T, int ROWS, int THREADS>
+struct FilterLoaderK {
+    using Tr = GemmTraits<T>;
+    static constexpr bool KMAJOR = true;
+    static constexpr int CPR = Tr::BK / Tr::VEC;
+    static constexpr int PER_THREAD = ROWS * CPR / THREADS, STEP = THREADS / CPR;
+    static_assert(PER_THREAD >= 1 && (ROWS * CPR) % THREADS == 0, "tile must split evenly over the workgroup");
+    u32x4_v reg[PER_THREAD];
+    const T* p[PER_THREAD];
+    __device__ __forceinline__ FilterLoaderK(const Operand<T>& op, int n0) {
+#pragma unroll
+        for (int i = 0; i < PER_THREAD; ++i)
+            p[i] = op.p + (int64_t)min(n0 + (int)threadIdx.x / CPR + i * STEP, op.rows - 1) * op.sr + (threadIdx.x % CPR) * Tr::VEC;
+    }
+    __device__ __forceinline__ void load(int k0) {
+#pragma unroll
+        for (int i = 0; i < PER_THREAD; ++i) reg[i] = *reinterpret_cast<const typename UnalignedVec<T>::type*>(p[i] + k0);
+    }
+    template <bool SPLIT>
+    __device__ __forceinline__ void store(T* lds) const {
+#pragma unroll
+        for (int i = 0; i < PER_THREAD; ++i)
+            put_chunk<T, true, ROWS, SPLIT>(lds, threadIdx.x / CPR + i * STEP, (threadIdx.x % CPR) * Tr::VEC, reg[i]);
+    }
+};
+
 template <typename T>
 struct ConvTapArgs {
     TapGeom<T> tap;
@@ -280,7 +308,7 @@ __global__ __launch_bounds__(NWM * NWN * 64, (split_waves<T, WM, WN>())) void co
             tile_coords(t, a.tiles_m, a.tiles_n, tm, tn);
             const int m0 = a.m_begin + tm * ML::TILE_M, n0 = tn * ML::TILE_N;
             ConvTapLoaderK<T, ML::TILE_M, ML::THREADS> la(g, m0);
-            typename ML::PlainLoaderB lb(a.Wm, n0, a.K);
+            FilterLoaderK<T, ML::TILE_N, ML::THREADS> lb(a.Wm, n0);
             ML::run(la, lb, a.K, lds, acc);
             conv_epilogue<ML, T, WM, WN>(acc, m0, n0, g.M, g.PQ, g.divPQ, a.Ncols, a.col_off, a.Ctot_out, a.bias, a.out, a.pre, a.act);
             __syncthreads();   // every wave is done with the LDS stages before the next tile refills them
