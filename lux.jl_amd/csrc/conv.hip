@@ -244,6 +244,65 @@ __global__ __launch_bounds__(256) void pad_to_cwhn_pack_kernel(const T* __restri
     }
 }
 
+// The first layer of an image network (bf16, at most four channels, a window of 5 to 8 positions along w): x is copied with four
+// channels per position and the rows' padding in place, so that the positions of a window in one source row are one run of at
+// most 32 elements.  A stage of the contraction is such a run: kH stages instead of kW kH / 4 over channels padded to eight (7 x 7:
+// 224 against 392; 224 x 224 x 3 x 32 -> 64 channels at stride 2: output 66 -> 58 us, filter gradient 78 -> 47, each copy of x 12.5 -> 7).
+struct Runs {
+    int W2 = 0;                // positions of a copied row, even; 0: not this kind of layer
+    static constexpr int EL = 32;
+};
+template <typename T>
+static Runs runs_of(const ConvGeom& g) {
+    Runs r;
+    const int64_t w2 = ((int64_t)(g.OW - 1) * g.sw + Runs::EL / 4 + 1) / 2 * 2;
+    if (sizeof(T) == 2 && g.groups == 1 && g.Cin <= 4 && g.kW >= 5 && g.kW <= Runs::EL / 4 && g.dw == 1 &&
+        w2 * g.H * g.N < (int64_t(1) << 28))
+        r.W2 = (int)w2;
+    return r;
+}
+// Blocks behind the copy's pack the filter: wout[co][kb][ka][4 channels], 32 elements per kb
+__global__ __launch_bounds__(256) void runs_copy_pack_kernel(const bf16_t* __restrict__ x, bf16_t* __restrict__ out, FastDiv div_half, FastDiv divH,
+                                                             uint32_t pairs, int W2, int blocks, const bf16_t* __restrict__ w, bf16_t* __restrict__ wout,
+                                                             ConvGeom g) {
+    if ((int)blockIdx.x >= blocks) {
+        const int e = ((int)blockIdx.x - blocks) * 256 + (int)threadIdx.x, K = g.kH * Runs::EL;
+        if (e >= g.Cout * K) return;
+        const int co = e / K, k = e - co * K, kb = k / Runs::EL, ka = (k - kb * Runs::EL) / 4, ci = k & 3;
+        bf16_t v = 0;
+        if (ka < g.kW && ci < g.Cin) {
+            const int a = g.flip ? ka : g.kW - 1 - ka, b = g.flip ? kb : g.kH - 1 - kb;
+            v = w[a + (int64_t)g.kW * (b + g.kH * (ci + g.Cin * co))];
+        }
+        wout[e] = v;
+        return;
+    }
+    const uint32_t idx = blockIdx.x * 256u + threadIdx.x;
+    if (idx >= pairs) return;
+    const uint32_t row = div_half.div(idx), n = divH.div(row), h = row - n * (uint32_t)g.H;
+    const int p = (int)(idx - row * div_half.d) * 2 - g.pw;
+    bf16_t e[8];
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+            const bool in = c < g.Cin && (unsigned)(p + j) < (unsigned)g.W;
+            e[4 * j + c] = x[in ? (((int64_t)n * g.Cin + c) * g.H + h) * g.W + p + j : 0];
+            if (!in) e[4 * j + c] = 0;
+        }
+    *reinterpret_cast<raw16_t*>(out + (size_t)idx * 8) = *reinterpret_cast<const raw16_t*>(e);
+}
+static int runs_copy_pack(hipStream_t s, const ConvGeom& g, Runs r, const bf16_t* x, bf16_t* out, const bf16_t* w, bf16_t* wout) {
+    const int64_t pairs = (int64_t)g.N * g.H * (r.W2 / 2), blocks = ceil_div(pairs, 256);
+    const int64_t pack = wout != nullptr ? ceil_div((int64_t)g.Cout * g.kH * Runs::EL, 256) : 0;
+    LUX_UNSUPPORTED_IF((int64_t)g.Cout * g.kH * Runs::EL >= (int64_t(1) << 30), "conv: filter too large");
+    ProfScope ps("whcn_to_cwhn_kernel", s);
+    runs_copy_pack_kernel<<<(unsigned)(blocks + pack), 256, 0, s>>>(x, out, FastDiv((uint32_t)(r.W2 / 2)), FastDiv((uint32_t)g.H), (uint32_t)pairs, r.W2,
+                                                                    (int)blocks, w, wout, g);
+    LUX_CHECK_LAUNCH();
+    return LUXHIP_OK;
+}
+
 // First pass of the fused pullback (bf16; P and C multiples of 8, 16-byte aligned pointers): one pass over delta
 // writes dz = delta .* act'(y, pre) as it lies (p contiguous: what the window and the direct filter-gradient kernels
 // read), its channel-contiguous copy dzT (what the input-gradient kernels read) and the bias gradient's partial sums,
@@ -351,13 +410,13 @@ __global__ __launch_bounds__(256) void conv_dbias_finalize_kernel(const float* _
 // added in order.
 template <typename T>
 __global__ __launch_bounds__(256) void wgrad_reduce_kernel(const float* __restrict__ partial, T* __restrict__ dw, ConvGeom g,
-                                                           int grp, int slices, int reduce_blocks, int Cp, int64_t slice_stride,
+                                                           int grp, int slices, int reduce_blocks, int Mrows, int Cp, int run, int64_t slice_stride,
                                                            BiasPartials bp) {
     if ((int)blockIdx.x >= reduce_blocks) {       // workgroups behind the reduction: one channel of the bias gradient each
         conv_dbias_finalize_channel(bp.partial, bp.dbias, bp.C, bp.slices, (int)blockIdx.x - reduce_blocks);
         return;
     }
-    const int Mrows = g.kW * g.kH * Cp;                // Cp: channels per tap in the partial sums (padded)
+    // Cp: channels per tap in the partial sums (padded); run > 0: rows are [kb][run / 4 positions][4 channels] instead
     const int total = Mrows * g.Cout_g;
     const int idx = (blockIdx.x * blockDim.x + threadIdx.x) * 4;
     if (idx >= total) return;
@@ -386,8 +445,8 @@ __global__ __launch_bounds__(256) void wgrad_reduce_kernel(const float* __restri
         if (id >= total) break;
         const int m = id % Mrows, col = id / Mrows;
         const int t = m / Cp, ci = m - t * Cp;
-        if (ci >= g.Cin_g) continue;
-        const int ka = t % g.kW, kb = t / g.kW;
+        const int taps = run > 0 ? run / 4 : g.kW, ka = t % taps, kb = t / taps;
+        if (ci >= g.Cin_g || ka >= g.kW) continue;
         const int a = g.flip ? ka : g.kW - 1 - ka, b = g.flip ? kb : g.kH - 1 - kb;
         st(dw + a + g.kW * (b + g.kH * (ci + g.Cin_g * (grp * g.Cout_g + col))), acc[e]);
     }
@@ -584,6 +643,7 @@ struct AnyPlan {
     struct Launch { cany::Sub sub[cany::MAX_SUBS]; PackSub pack[cany::MAX_SUBS]; int n; };
     std::vector<Launch> launches;
     int Ncols = 0, Cch = 0, res_w = 0, merged = 0, Cp = 0;
+    Runs runs;                                               // fprop: stages are runs of positions
     bool zero_first = false;                                 // some positions of dx belong to no sub-problem: clear it before
     int64_t wm_elems = 0;                                    // packed filter of one group
     bool slices = true;                                      // contractions may be cut (workspace for the partial sums)
@@ -618,7 +678,13 @@ struct AnyPlan {
         Ncols = Cch = dgrad ? g.Cin_g : g.Cout_g;
         const Residue none{0, 0, 0, 0, 1, 0};
         if (!dgrad) {
-            add(none, g.OW, none, g.OH, g.N, -g.pw, g.dw, g.kW, -g.ph, g.dh, g.kH, 0, 0);
+            runs = runs_of<T>(g);
+            if (runs.W2 > 0) {
+                Cp = Runs::EL;
+                add(none, g.OW, none, g.OH, g.N, 0, 0, 1, -g.ph, g.dh, g.kH, 0, 0);
+            } else {
+                add(none, g.OW, none, g.OH, g.N, -g.pw, g.dw, g.kW, -g.ph, g.dh, g.kH, 0, 0);
+            }
             return;
         }
         // Where all residues fit one launch, those without taps write their zeros in it; of more (a stride of 32 has 1024)
@@ -755,6 +821,8 @@ static int run_conv_any(hipStream_t s, const ConvGeom& g, bool dgrad, const AnyP
         a.Ctot = (alone ? gr.n : g.groups) * plan.Cp; a.Cp = plan.Cp;
         if (!dgrad) { a.SP = g.W; a.SQ = g.H; a.ss_w = g.sw; a.ss_h = g.sh; a.P = g.OW; a.Q = g.OH; a.os_w = a.os_h = 1; a.Ctot_out = g.Cout; }
         else { a.SP = g.OW; a.SQ = g.OH; a.ss_w = a.ss_h = 1; a.P = g.W; a.Q = g.H; a.os_w = g.sw; a.os_h = g.sh; a.Ctot_out = g.Cin; }
+        a.run = 0;
+        if (plan.runs.W2 > 0) { a.Ctot = 4; a.SP = plan.runs.W2; a.run = 4 * g.kW; }
         a.PQ = a.P * a.Q;
         a.Cch = plan.Cch; a.res_w = std::max(plan.res_w, 1); a.merged = plan.merged; a.kW = g.kW; a.kH = g.kH;
         a.act = act; a.subs = l.n;
@@ -837,9 +905,9 @@ static int run_conv_gemm(hipStream_t s, const ConvGeom& g, bool dgrad, const T* 
 // Rows (taps x padded channels), columns and slices of the filter gradient's partial sums
 struct WgradPlan { int Mrows, Ncols, slices, kslice; bool narrow; };
 template <typename T>
-static int wgrad_plan(const ConvGeom& g, bool any, WgradPlan* p) {
+static int wgrad_plan(const ConvGeom& g, bool any, Runs runs, WgradPlan* p) {
     constexpr int BK = GemmTraits<T>::BK;
-    p->Mrows = g.kW * g.kH * (any ? padded<T>(g.Cin_g) : g.Cin_g);
+    p->Mrows = any && runs.W2 > 0 ? g.kH * Runs::EL : g.kW * g.kH * (any ? padded<T>(g.Cin_g) : g.Cin_g);
     p->Ncols = any ? padded<T>(g.Cout_g) : g.Cout_g;
     p->narrow = p->Mrows <= 64 || p->Ncols <= 64;
     const int tile = p->narrow ? 64 : 128;
@@ -882,9 +950,9 @@ static bool wgrad_direct_ok(const ConvGeom& g, const void* xT, const void* dy) {
 template <typename T>
 static size_t wgrad_partial_bytes(const ConvGeom& g) {
     size_t bytes = 0;
-    for (int any = 0; any < 2; ++any) {
+    for (int any = 0; any < 3; ++any) {
         WgradPlan p;
-        if (wgrad_plan<T>(g, any != 0, &p) != LUXHIP_OK) continue;      // run_wgrad refuses it if it is the one
+        if (wgrad_plan<T>(g, any != 0, any == 2 ? runs_of<T>(g) : Runs(), &p) != LUXHIP_OK) continue;      // run_wgrad refuses it if it is the one
         if (wgrad_window_shape<T>(g))
             p.slices = std::max(p.slices, wpatch::image_lanes(g.N, (g.Cin_g / 64) * ((g.Cout_g + 63) / 64), num_cus() > 0 ? num_cus() : 256));
         bytes = std::max(bytes, (size_t)p.slices * p.Mrows * p.Ncols * sizeof(float));
@@ -892,16 +960,16 @@ static size_t wgrad_partial_bytes(const ConvGeom& g) {
     return align256(bytes);
 }
 
-// dy: WHCN cotangent (used by the window and the direct bf16 kernels); dyT: its channel-contiguous copy with padded channels,
+// runs: xT is the copy of runs_copy_pack.  dy: WHCN cotangent (used by the window and the direct bf16 kernels); dyT: its channel-contiguous copy with padded channels,
 // followed by BK positions of zeros where there are fewer than BK positions in all (used by the general kernel).  Where
 // channels are padded, xT / dyT hold the groups `gr` alone, else all of them.
 template <typename T>
-static int run_wgrad(hipStream_t s, const ConvGeom& g, Groups gr, const T* xT, const T* dy, const T* dyT, float* partial, T* dw,
+static int run_wgrad(hipStream_t s, const ConvGeom& g, Groups gr, Runs runs, const T* xT, const T* dy, const T* dyT, float* partial, T* dw,
                      const void* zeros, const BiasPartials* bias = nullptr) {
     const bool direct = wgrad_direct_ok<T>(g, xT, dy);
     const bool window = wgrad_window_shape<T>(g) && aligned16(xT) && aligned16(dy) && aligned16(partial);
     WgradPlan plan;
-    int rc = wgrad_plan<T>(g, !direct && !window, &plan);
+    int rc = wgrad_plan<T>(g, !direct && !window, runs, &plan);
     if (rc != LUXHIP_OK) return rc;
     int slices = plan.slices;
     const int kslice = plan.kslice;
@@ -947,6 +1015,9 @@ static int run_wgrad(hipStream_t s, const ConvGeom& g, Groups gr, const T* xT, c
             a.OW = g.OW; a.OWOH = g.OW * g.OH; a.SP = g.W; a.SQ = g.H;
             a.kW = g.kW; a.sw = g.sw; a.sh = g.sh; a.pw = g.pw; a.ph = g.ph; a.dw = g.dw; a.dh = g.dh;
             a.divOW = FastDiv((uint32_t)a.OW); a.divOWOH = FastDiv((uint32_t)a.OWOH); a.divCp = FastDiv((uint32_t)Cp); a.divkW = FastDiv((uint32_t)g.kW);
+            if (runs.W2 > 0) {                                 // xT holds runs of positions
+                a.Ctot = 4; a.Cp = Runs::EL; a.divCp = FastDiv((uint32_t)Runs::EL); a.kW = 1; a.divkW = FastDiv(1); a.pw = 0; a.SP = runs.W2;
+            }
             a.positions = g.OW * g.OH * g.N;
             a.Ktotal = std::max(a.positions, GemmTraits<T>::BK);
             a.kslice = kslice; a.partial = partial;
@@ -958,7 +1029,8 @@ static int run_wgrad(hipStream_t s, const ConvGeom& g, Groups gr, const T* xT, c
         const int reduce_blocks = (int)ceil_div(total, 1024);
         BiasPartials bp;
         if (bias != nullptr && grp == g.groups - 1) bp = *bias;       // the bias gradient's channels ride on the last group's launch
-        wgrad_reduce_kernel<T><<<(unsigned)(reduce_blocks + bp.C), 256, 0, s>>>(partial, dw, g, grp, slices, reduce_blocks, Mrows / (g.kW * g.kH),
+        wgrad_reduce_kernel<T><<<(unsigned)(reduce_blocks + bp.C), 256, 0, s>>>(partial, dw, g, grp, slices, reduce_blocks, Mrows,
+                                                                           runs.W2 > 0 ? 4 : Mrows / (g.kW * g.kH), runs.W2 > 0 ? Runs::EL : 0,
                                                                            (int64_t)Mrows * plan.Ncols, bp);
         LUX_CHECK_LAUNCH();
     }
@@ -976,7 +1048,8 @@ static int dy_zeros(const ConvGeom& g) {
 template <typename T>
 static size_t xt_bytes(const ConvGeom& g, int n) {       // n: groups at a time, where padded
     const int Cp = padded<T>(g.Cin_g);
-    return align256((size_t)g.W * g.H * g.N * (Cp != g.Cin_g ? n : g.groups) * Cp * sizeof(T));
+    const size_t runs = (size_t)runs_of<T>(g).W2 * g.H * g.N * 4 * sizeof(T);      // either form
+    return align256(std::max(runs, (size_t)g.W * g.H * g.N * (Cp != g.Cin_g ? n : g.groups) * Cp * sizeof(T)));
 }
 template <typename T>
 static size_t dyt_bytes(const ConvGeom& g, int n) {
@@ -1030,7 +1103,13 @@ static int conv_fwd_t(hipStream_t s, int act, const ConvGeom& g, const T* x, con
         const bool first = gr.first == 0;
         if (plan.Cp != g.Cin_g || first) {
             const int copied = plan.Cp != g.Cin_g ? gr.n : g.groups;
-            rc = pad_and_pack<T>(s, x + (size_t)gr.first * g.Cin_g * g.W * g.H, xT, g.W * g.H, g.Cin, g.Cin_g, copied, g.N, 0, w, first ? wF : nullptr, g, &ps);
+            if constexpr (sizeof(T) == 2) {
+                if (plan.runs.W2 > 0) {
+                    if ((rc = runs_copy_pack(s, g, plan.runs, x, xT, w, wF)) != LUXHIP_OK) return rc;
+                }
+            }
+            if (plan.runs.W2 == 0)
+                rc = pad_and_pack<T>(s, x + (size_t)gr.first * g.Cin_g * g.W * g.H, xT, g.W * g.H, g.Cin, g.Cin_g, copied, g.N, 0, w, first ? wF : nullptr, g, &ps);
             if (rc != LUXHIP_OK) return rc;
         }
         if ((rc = run_conv_any<T>(s, g, false, plan, gr, xT, w, wF, true, bias, y, pre, act, xb + wb)) != LUXHIP_OK) return rc;
@@ -1068,7 +1147,10 @@ static int dy_copy_and_pack(hipStream_t s, const ConvGeom& g, bool any, const An
 }
 // xT of the groups `gr`, likewise; from the caller's unpadded copy where x is not given
 template <typename T>
-static int x_copy(hipStream_t s, const ConvGeom& g, Groups gr, const T* x, const T* unpadded, T* xT) {
+static int x_copy(hipStream_t s, const ConvGeom& g, Groups gr, Runs runs, const T* x, const T* unpadded, T* xT) {
+    if constexpr (sizeof(T) == 2) {
+        if (runs.W2 > 0) return runs_copy_pack(s, g, runs, x, xT, nullptr, nullptr);
+    }
     const int Cp = padded<T>(g.Cin_g);
     const bool alone = Cp != g.Cin_g;
     if (!alone && gr.first > 0) return LUXHIP_OK;
@@ -1111,12 +1193,13 @@ static int conv_bwd_filter_t(hipStream_t s, const ConvGeom& g, const T* x, const
     T* xT = reinterpret_cast<T*>(ws.data);
     T* dyT = reinterpret_cast<T*>(ws.data + xb);
     float* partial = reinterpret_cast<float*>(ws.data + xb + yb);
+    const Runs runs = runs_of<T>(g);
     for (Groups gr{0, 0}; gr.first < g.groups; gr.first += gr.n) {
         gr.n = std::min(n, g.groups - gr.first);
-        if ((rc = x_copy<T>(s, g, gr, x, nullptr, xT)) != LUXHIP_OK) return rc;
+        if ((rc = x_copy<T>(s, g, gr, runs, x, nullptr, xT)) != LUXHIP_OK) return rc;
         // the direct kernel reads dy as it is
         if (!wgrad_direct_ok<T>(g, xT, dy) && (rc = dy_copy<T>(s, g, gr, dy, dyT)) != LUXHIP_OK) return rc;
-        if ((rc = run_wgrad<T>(s, g, gr, xT, dy, dyT, partial, dw, ws.zeros)) != LUXHIP_OK) return rc;
+        if ((rc = run_wgrad<T>(s, g, gr, runs, xT, dy, dyT, partial, dw, ws.zeros)) != LUXHIP_OK) return rc;
     }
     return LUXHIP_OK;
 }
@@ -1178,8 +1261,9 @@ static int fused_conv_bwd_t(hipStream_t s, int dtype, int act, const ConvGeom& g
             if ((rc = run_dgrad<T>(s, g, any, plan, gr, dzT, w, wD, packed, dx, xb + yb + wb + pb + bb, ws.zeros)) != LUXHIP_OK) return rc;
         }
         if (dw != nullptr) {
-            if (!kept && (rc = x_copy<T>(s, g, gr, x, xt_kept, reinterpret_cast<T*>(ws.data))) != LUXHIP_OK) return rc;
-            rc = run_wgrad<T>(s, g, gr, xT, dzp, dzT, partial, dw, ws.zeros, bias_later.dbias != nullptr ? &bias_later : nullptr);
+            const Runs runs = !kept && x != nullptr ? runs_of<T>(g) : Runs();
+            if (!kept && (rc = x_copy<T>(s, g, gr, runs, x, xt_kept, reinterpret_cast<T*>(ws.data))) != LUXHIP_OK) return rc;
+            rc = run_wgrad<T>(s, g, gr, runs, xT, dzp, dzT, partial, dw, ws.zeros, bias_later.dbias != nullptr ? &bias_later : nullptr);
             if (rc != LUXHIP_OK) return rc;
         }
     }

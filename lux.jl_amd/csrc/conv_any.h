@@ -66,10 +66,12 @@ struct Args {
     FastDiv divCp, divCch;
     Sub sub[MAX_SUBS];
     int kW, kH;                // merged (dilation 1): tap t of residue r is filter tap t * os + r, where there is one
+    int run;                   // RUNS: elements of a stage that belong to the row's window, the rest count as zero
 };
 
-// A: K-major rows of the im2col matrix
-template <typename T, int ROWS>
+// A: K-major rows of the im2col matrix.  RUNS: a stage is the window's positions of one source row (see Runs in conv.hip); what
+// lies behind them in memory is data of other windows, and is cut off here (a zero in the filter would turn an infinity into NaN).
+template <typename T, int ROWS, bool RUNS>
 struct RowLoader {
     using Tr = GemmTraits<T>;
     static constexpr bool KMAJOR = true;
@@ -114,14 +116,21 @@ struct RowLoader {
     template <bool SPLIT>
     __device__ __forceinline__ void store(u32x4_v (&reg)[PER], T* lds, int) const {
 #pragma unroll
-        for (int i = 0; i < PER; ++i) put_chunk<T, true, ROWS, SPLIT>(lds, (int)threadIdx.x / CPR + i * STEP, chunk, reg[i]);
+        for (int i = 0; i < PER; ++i) {
+            u32x4_v v = reg[i];
+            if constexpr (RUNS) {
+#pragma unroll
+                for (int e = 0; e < 4; ++e) v[e] = chunk + e * (Tr::VEC / 4) < g.run ? v[e] : 0u;
+            }
+            put_chunk<T, true, ROWS, SPLIT>(lds, (int)threadIdx.x / CPR + i * STEP, chunk, v);
+        }
     }
 };
 
-template <typename T, int WM, int WN, int NWM, int NWN>
+template <typename T, int WM, int WN, int NWM, int NWN, bool RUNS = false>
 struct Shape {
     static constexpr int TILE_M = NWM * WM * 32, TILE_N = NWN * WN * 32;
-    using LA = RowLoader<T, TILE_M>;
+    using LA = RowLoader<T, TILE_M, RUNS>;
     using LB = split::Loader<T, true, TILE_N>;
     using Core = split::Core<T, WM, WN, NWM, NWN, LA, LB>;
 };
@@ -152,9 +161,9 @@ __device__ __forceinline__ float own_taps_sum(const Args<T>& g, const Sub& q, co
 // MERGED: the residues of an input gradient are columns and a NaN among the sums is looked into.  A kernel of its own: the test
 // costs 2 to 4 %, and a register that takes a wave from every SIMD unless it is told to stay below (256 x 32 tiles of the first
 // layer, 78 us with four waves, 85 with three).
-template <typename T, int WM, int WN, int NWM, int NWN, bool MERGED>
+template <typename T, int WM, int WN, int NWM, int NWN, bool MERGED, bool RUNS = false>
 __global__ __launch_bounds__(split::THREADS, MERGED && WM * WN < 4 ? (sizeof(T) == 4 && WM * WN == 2 ? 3 : 4) : (split_waves<T, WM, WN>())) void conv_any_kernel(Args<T> g) {
-    using S = Shape<T, WM, WN, NWM, NWN>;
+    using S = Shape<T, WM, WN, NWM, NWN, RUNS>;
     using Core = typename S::Core;
     using ML = typename Core::ML;
     extern __shared__ __align__(16) unsigned char lds_raw[];

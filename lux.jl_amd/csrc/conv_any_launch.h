@@ -23,6 +23,13 @@ int launch_shape(hipStream_t s, Args<T>& a, int blocks, int groups, bool dgrad) 
     static const char* const names[2][2] = {{"conv_fprop_kernel<f32>", "conv_dgrad_kernel<f32>"}, {"conv_fprop_kernel<bf16>", "conv_dgrad_kernel<bf16>"}};
     ProfScope ps(names[sizeof(T) == 2][dgrad], s);
     const dim3 grid((unsigned)blocks, (unsigned)groups);
+    if constexpr (sizeof(T) == 2) {
+        if (a.run > 0) {
+            conv_any_kernel<T, WM, WN, NWM, NWN, false, true><<<grid, dim3(split::THREADS), S::Core::LDS_BYTES, s>>>(a);
+            LUX_CHECK_LAUNCH();
+            return LUXHIP_OK;
+        }
+    }
     if (a.merged) conv_any_kernel<T, WM, WN, NWM, NWN, true><<<grid, dim3(split::THREADS), S::Core::LDS_BYTES, s>>>(a);
     else conv_any_kernel<T, WM, WN, NWM, NWN, false><<<grid, dim3(split::THREADS), S::Core::LDS_BYTES, s>>>(a);
     LUX_CHECK_LAUNCH();
