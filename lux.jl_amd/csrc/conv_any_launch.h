@@ -76,8 +76,20 @@ Choice choose_any(Sub* sub, int subs, int Ncols, int groups, bool may_slice) {
     return best;
 }
 
+// conv_any_bf16.hip
+bool launch_few(hipStream_t s, const Args<bf16_t>& a, int* rc);
+
 template <typename T>
 int launch_any(hipStream_t s, Args<T>& a, int groups, size_t ws_front, bool dgrad, bool may_slice) {
+    if constexpr (sizeof(T) == 2) {
+        if (dgrad && groups == 1 && a.merged) {
+            Workspace ws;
+            int rc = get_workspace(s, ws_front, &ws);
+            if (rc != LUXHIP_OK) return rc;
+            a.zero = ws.zeros;
+            if (launch_few(s, a, &rc)) return rc;
+        }
+    }
     const Choice c = choose_any<T>(a.sub, a.subs, a.Ncols, groups, may_slice);
     int blocks = 0, nt = 0;
     for (int i = 0; i < a.subs; ++i) {

@@ -1,4 +1,4 @@
-"""First layers (bf16, at most four channels, windows of 5 to 8 along w): the positions of a window in one row of the copied input
+"""Layers next to an image (few channels).  First layers (bf16, at most four channels, windows of 5 to 8 along w): the positions of a window in one row of the copied input
 are one stage of the contraction.  Every channel count and window width, odd strides (8-byte alignment of the windows), padding
 on either side alone, dilation along h, more rows and columns than a tile."""
 import numpy as np
@@ -51,3 +51,29 @@ def test_an_infinity_stays_inside_its_windows(gpu, width):
     dy = host_inputs("bf16", rng.normal(size=y.shape))[0]
     gw = gpu.conv_filter_grad(dev(gpu, x, "bf16"), dev(gpu, dy, "bf16"), cd).to_numpy()
     assert np.isfinite(gw[:, :, [0, 2]]).all() and not np.isfinite(gw[:, :, 1]).any()
+
+
+FEW = [
+    # x shape, w shape, stride, pad, flip: rows and residues that end inside a tile, 1 .. 4 taps, 16 .. 64 channels, up to 32 columns
+    ((70, 36, 3, 8), (7, 7, 3, 64), 2, 3, False), ((65, 67, 2, 16), (5, 3, 2, 16), 2, 2, True), ((66, 34, 8, 20), (4, 4, 8, 48), 2, 1, False),
+    ((97, 99, 1, 8), (9, 9, 1, 32), 3, 4, False), ((64, 40, 1, 33), (8, 6, 1, 64), (4, 2), (2, 2), False), ((34, 33, 3, 40), (2, 2, 3, 64), 2, 0, False),
+]
+
+
+@pytest.mark.parametrize("case", range(len(FEW)))
+def test_input_gradient_with_few_channels(gpu, case):
+    """All residues as columns, the cotangents of a tile in LDS (conv_few.h), and infinite cotangents: they reach the positions
+    that see them and no others."""
+    xs, ws, stride, pad, flip = FEW[case]
+    rng = np.random.default_rng(stable_seed("conv_few", case))
+    gd, od = (D(xs, ws, stride=stride, padding=pad, flipkernel=flip) for D in (gpu.DenseConvDims, O.ConvDims))
+    w, dy = host_inputs("bf16", rng.normal(size=ws) / np.sqrt(ws[0] * ws[1] * ws[3]), rng.normal(size=od.y_shape()))
+    want = O.conv_data_grad(f64(dy), f64(w), od)
+    got = gpu.conv_data_grad(dev(gpu, dy, "bf16"), dev(gpu, w, "bf16"), gd).to_numpy()
+    assert_close(got, want, "bf16", "dx")
+    one = np.zeros(dy.shape)
+    one[3, 5, 1, 2] = 1.0
+    sees = O.conv_data_grad(one, np.ones(ws), od) != 0
+    dy[3, 5, 1, 2] = np.inf
+    bad = gpu.conv_data_grad(dev(gpu, dy, "bf16"), dev(gpu, np.abs(w) + 0.01, "bf16"), gd).to_numpy()
+    assert (bad[sees] == np.inf).all() and np.isfinite(bad[~sees]).all()
