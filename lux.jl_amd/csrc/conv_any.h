@@ -162,7 +162,7 @@ __device__ __forceinline__ float own_taps_sum(const Args<T>& g, const Sub& q, co
 // costs 2 to 4 %, and a register that takes a wave from every SIMD unless it is told to stay below (256 x 32 tiles of the first
 // layer, 78 us with four waves, 85 with three).
 template <typename T, int WM, int WN, int NWM, int NWN, bool MERGED, bool RUNS = false>
-__global__ __launch_bounds__(split::THREADS, MERGED && WM * WN < 4 ? (sizeof(T) == 4 && WM * WN == 2 ? 3 : 4) : (split_waves<T, WM, WN>())) void conv_any_kernel(Args<T> g) {
+__global__ __launch_bounds__(split::THREADS, MERGED && WM * WN < 4 ? 4 : (split_waves<T, WM, WN>())) void conv_any_kernel(Args<T> g) {
     using S = Shape<T, WM, WN, NWM, NWN, RUNS>;
     using Core = typename S::Core;
     using ML = typename Core::ML;

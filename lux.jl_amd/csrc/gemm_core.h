@@ -103,14 +103,17 @@ struct GemmTraits<float> {
 //       32-byte granules).
 __host__ __device__ constexpr int mn_swizzle_shift(int rows) { return rows >= 128 ? 5 : 4; }
 
-// fp32 contractions on the bf16 matrix cores (put_chunk): waves of 2 or 4 accumulators.  One accumulator per wave spends as much
-// on the cutting as it saves (64 x 64 tiles: 0 to 7 % slower than the fp32 instruction).  Four accumulators take 128 registers
-// with the smaller partial products, and the compiler would go on to give the kernel all 512: split_waves is the launch bound that
-// keeps two waves on a SIMD (59.2 GFLOP of a 3 x 3 convolution: 545 us with one wave, 371 with two, 531 on the fp32 instruction).
+// fp32 contractions on the bf16 matrix cores (put_chunk): waves of 4 accumulators.  A value is cut once for every accumulator
+// column or row of its wave, so smaller waves spend as much on the cutting as they save: 64 x 64 tiles (one accumulator) are 0 to
+// 7 % slower than the fp32 instruction; 128 x 64 and 256 x 32 (two) win up to 4 % where the contraction is long and lose up to
+// 11 % where it is short (3 x 3 windows of 16 channels, 64 columns, 280000 rows: 102 us, 91 on the fp32 instruction).  Four
+// accumulators take 128 registers with the smaller partial products, and the compiler would go on to give the kernel all 512:
+// split_waves is the launch bound that keeps two waves on a SIMD (59.2 GFLOP of a 3 x 3 convolution: 545 us with one wave, 371
+// with two, 531 on the fp32 instruction).
 template <typename T, int WM, int WN>
-__host__ __device__ constexpr bool split_f32() { return sizeof(T) == 4 && (WM * WN == 2 || WM * WN == 4); }
+__host__ __device__ constexpr bool split_f32() { return sizeof(T) == 4 && WM * WN == 4; }
 template <typename T, int WM, int WN>
-__host__ __device__ constexpr int split_waves() { return split_f32<T, WM, WN>() && WM * WN == 4 ? 2 : 1; }
+__host__ __device__ constexpr int split_waves() { return split_f32<T, WM, WN>() ? 2 : 1; }
 
 // elements of one LDS stage of an operand tile with `rows` rows
 template <typename T, bool KMAJOR>
