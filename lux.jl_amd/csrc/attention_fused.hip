@@ -318,8 +318,10 @@ __global__ __launch_bounds__(THREADS, 2) void fwd_kernel(Args a) {
         return z;
     };
 
-    // sweep 1: maximum and sum of exponentials, per lane (half of the keys of its column).  A column of which nothing but
-    // -inf has been seen keeps the sum 0 (the subtrahend is 0 then).
+    // sweep 1: maximum of the unscaled logits and sum of exponentials, per lane (half of the keys of its column).  A column of which
+    // nothing but -inf has been seen keeps the sum 0 (the subtrahend is 0 then).  The maximum is subtracted before the scale: the
+    // difference is exact where it matters.  fma(z, c, -c m) is an instruction less, but carries the rounding of c m, half a unit
+    // of a number that may be of any size: logits of 1e6 gave 100 equal keys weights 4 % off, those of 1e9 overflowed.
     float m = -INFINITY, sum = 0.0f;
     {
         Tile<ET, 2> tk(kp, a.kt, a.E, a.S, 0);
@@ -339,11 +341,11 @@ __global__ __launch_bounds__(THREADS, 2) void fwd_kernel(Args a) {
                     float mt = z[0];
 #pragma unroll
                     for (int i = 1; i < 16; ++i) mt = fmaxf(mt, z[i]);
-                    const float mn = fmaxf(m, mt * a.c), ms = mn == -INFINITY ? 0.0f : mn;
+                    const float mn = fmaxf(m, mt), ms = mn == -INFINITY ? 0.0f : mn;
                     float add = 0.0f;
 #pragma unroll
-                    for (int i = 0; i < 16; ++i) add += __builtin_amdgcn_exp2f(fmaf(z[i], a.c, -ms));
-                    sum = sum * __builtin_amdgcn_exp2f(m - ms) + add;
+                    for (int i = 0; i < 16; ++i) add += __builtin_amdgcn_exp2f((z[i] - ms) * a.c);
+                    sum = sum * __builtin_amdgcn_exp2f((m - ms) * a.c) + add;
                     m = mn;
                 }
                 tk.store(lds + (1 - u) * TILE, 1 - u, t + 1, a.S);
@@ -351,12 +353,13 @@ __global__ __launch_bounds__(THREADS, 2) void fwd_kernel(Args a) {
             });
         }
     }
-    // weight = exp2(c z - base), base = maximum + log2(sum)
-    float base;
+    // weight = exp2(c (z - top)) inv, top = maximum, inv = 1 / sum (infinite where no key counts: the weights are NaN)
+    float top, inv;
     {
         const float mo = __shfl_xor(m, 32), so = __shfl_xor(sum, 32);
-        const float mx = fmaxf(m, mo), ms = mx == -INFINITY ? 0.0f : mx;
-        base = mx == -INFINITY ? NAN : mx + __builtin_amdgcn_logf(sum * __builtin_amdgcn_exp2f(m - ms) + so * __builtin_amdgcn_exp2f(mo - ms));
+        const float mx = fmaxf(m, mo);
+        top = mx == -INFINITY ? 0.0f : mx;
+        inv = 1.0f / (sum * __builtin_amdgcn_exp2f((m - top) * a.c) + so * __builtin_amdgcn_exp2f((mo - top) * a.c));
     }
 
     // sweep 2: the weights, rounded, to memory and into the product with v
@@ -405,7 +408,7 @@ __global__ __launch_bounds__(THREADS, 2) void fwd_kernel(Args a) {
                         for (int e = 0; e < ET; ++e) vf[n][e] = ft.get(lds + (2 + u) * TILE, 16 * n, e);
                     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-                    for (int i = 0; i < 16; ++i) z[i] = __builtin_amdgcn_exp2f(fmaf(z[i], a.c, -base));
+                    for (int i = 0; i < 16; ++i) z[i] = __builtin_amdgcn_exp2f((z[i] - top) * a.c) * inv;
 #pragma unroll
                     for (int n = 0; n < 2; ++n) {
                         const raw16_t pw = pack8(z, n);
@@ -436,11 +439,11 @@ __global__ __launch_bounds__(THREADS, 2) void fwd_kernel(Args a) {
                     *reinterpret_cast<float4*>(a.out_wide + orow + e) = make_float4(o[t][4 * g], o[t][4 * g + 1], o[t][4 * g + 2], o[t][4 * g + 3]);
             }
     }
-    // the masked part of the columns, last: nothing waits for these stores.  0, or NaN where the sum is none.
+    // the masked part of the columns, last: nothing waits for these stores.  0, or NaN where 1 / sum is no number.
     const int rows = min(32, a.L - wl0);
     if (w_end < a.S) {
         for (int i = 0; i < rows; ++i) {
-            const float z0 = __shfl(base, i) != __shfl(base, i) ? NAN : 0.0f;
+            const float z0 = 0.0f * __shfl(inv, i);
             const uint32_t zz = f32x2_to_bf16x2(z0, z0);
             const raw16_t zw = {zz, zz, zz, zz};
             for (int s = w_end + 8 * lane; s < a.S; s += 512) store8(wrow0 + (int64_t)i * a.S, s, a.S, zw);

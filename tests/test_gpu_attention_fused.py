@@ -84,3 +84,22 @@ def test_columns_with_infinite_logits(gpu):
     y, w = y.to_numpy(), w.to_numpy()
     assert np.isnan(w[:, 70, 1, 0]).all() and np.isnan(y[:, 1, 70, 0]).all()
     assert np.isfinite(w[:, :, 0]).all() and np.isfinite(w[:, :3, 1]).all() and np.isfinite(y[:, 0]).all() and np.isfinite(y[:, 1, :3]).all()
+
+
+@pytest.mark.parametrize("scale", [1.0, -1.0, 1e3, 1e-3])
+def test_weights_of_large_logits_add_up_to_one(gpu, scale):
+    """Equal keys share a column equally, whatever the size of their logits, and so do the largest ones of a column.  The weights are
+    fp32 quotients rounded to bf16 (2^-9 of the value); bf16 operands of few bits make the logits themselves exact."""
+    E, H, L, S = 64, 16, 130, 100
+    rng = np.random.default_rng(stable_seed("attn-fused-large", scale))
+    q = rng.integers(1, 9, size=(E, H, L, 1)) * 64.0                 # products of 2^15 and more, sums of up to 2^24: exact in fp32
+    k = np.repeat(rng.integers(1, 9, size=(E, H, 1, 1)) * 64.0, S, axis=2)
+    k[:, :, 60:] = -k[:, :, 60:] if scale > 0 else k[:, :, 60:]     # a scale below 0: all keys equal still
+    v = rng.normal(size=(E, H, S, 1))
+    d = lambda a: dev(gpu, a.astype(np.float32), "bf16")
+    run = lambda: gpu.scaled_dot_product_attention(d(q), d(k), d(v), 1, 3, 1.0 / scale)
+    assert "attn_fwd_kernel" in kernels_of(gpu, run)
+    n = 60 if scale > 0 else S
+    want = np.zeros((S, L, H, 1))
+    want[:n] = 1.0 / n
+    np.testing.assert_allclose(run()[1].to_numpy(), want, rtol=2.0 ** -8, atol=0)
