@@ -13,6 +13,7 @@ Julia's column-major layout and logical shapes (W, H, C, N) / (features, batch).
 from __future__ import annotations
 
 import ctypes as C
+import functools
 import math
 from dataclasses import dataclass, field
 from typing import Optional, Sequence, Tuple
@@ -658,20 +659,49 @@ class _AttnLayout:
         self.batch = a.size // self.sb if self.sb else 0
 
 
-def _attention_fused(lq, lk, lv, E, Ev, H, B) -> bool:
-    """Whether the fused kernels (luxhip_attention_fwd / _bwd) can and should take the call: whole 16-byte vectors of at most
-    128 features, 32-bit byte offsets inside a head, and enough workgroups (one per 128 tokens and head).  Few long heads
-    leave most of the chip idle there, while the step-by-step products cut both token dims into tiles: with 128 features
-    2 heads of 2048 tokens took 222 against 133 us, 8 heads 225 against 189, 12 heads (192 workgroups) 226 against 255;
-    with 64 features 2 heads 162 against 135, 8 heads (128 workgroups) 164 against 187.  Up to 512 tokens and on ragged
-    key counts (step by step 195 us for 2 x 583 tokens, fused 113) the fused kernels are ahead at any number of heads."""
-    L, S = lq.tokens, lk.tokens
+@functools.lru_cache(maxsize=512)
+def _attention_fused(L, S, E, Ev, H, B, stride_q, stride_k, stride_v, causal):
+    """Whether the fused kernels (luxhip_attention_fwd, luxhip_attention_bwd) can and should take the forward pass and the pullback (two
+    truth values) of L queries on S keys in H query heads and B batches.  They can with whole 16-byte vectors of at most 128 features,
+    32-bit byte offsets inside a head (strides: elements between tokens) and fewer than 2^23 workgroups.
+
+    They should where they are faster than the step-by-step products, by an estimate of both in us.  A workgroup of the forward and the dq kernel owns
+    128 queries of a head and walks all keys, one of the dk / dv kernel 128 keys and all queries: with fewer workgroups than compute
+    units the time is that of one walk, however many heads there are, while the products cut both token dims into tiles.  The walk's
+    time per 32 tokens and the products' times are fitted to 502 calls (1 to 512 heads, 1 to 8192 queries and keys in all
+    proportions, 32 to 128 features, causal or not; 31 and 34 us are the products' launches by this host): what the estimate takes
+    is 0.2 % behind the faster way in the mean, 13 % at worst.
+    Forward at 64 features, us fused / step by step: 1 query, 2048 keys, 32 heads 64 / 38, 512 heads 67 / 92; 512 queries, 2048 keys,
+    8 heads 69 / 50, 32 heads 71 / 107; 1024 x 1024, 2 heads 37 / 32, 8 heads 39 / 41.  Pullback at 128 features: 2048 x 2048, 8 heads
+    137 / 118, 32 heads 243 / 383; 8192 queries, 128 keys, 32 heads 365 / 292; 128 queries, 2048 keys, 32 heads 77 / 62, 256
+    heads 263 / 312.
+    Rows that are no whole vectors cost the products more than the kernels (32 x 2047 forward 64 / 80, 583 x 583 pullback 77 / 125):
+    from 32 tokens on either side the kernels take those whatever the number of heads."""
     if not (0 < E <= 128 and 0 < Ev <= 128 and E % 8 == 0 and Ev % 8 == 0 and S > 0 and L > 0 and H > 0 and B > 0):
-        return False
-    span, groups = max(L * lq.st, S * lk.st, S * lv.st, L * H * Ev), -(-max(L, S) // 128) * H * B
-    if 2 * span >= 1 << 31 or H * B >= 1 << 23 or groups >= 1 << 23:
-        return False
-    return max(L, S) <= 512 or S % 8 != 0 or groups >= (144 if max(E, Ev) > 64 else 56)
+        return False, False
+    heads, f = H * B, 32 * -(-max(E, Ev) // 32)
+    groups_q, groups_k = -(-L // 128) * heads, -(-S // 128) * heads
+    if 2 * max(L * stride_q, S * stride_k, S * stride_v, L * H * Ev) >= 1 << 31 or max(groups_q, groups_k) >= 1 << 23:
+        return False, False
+    # tokens of the longest walk and of the average one; logits that are computed
+    keys, mean_keys, mean_queries, logits = S, S, L, L * S * heads
+    if causal:
+        keys = min(S, -(-L // 128) * 128)
+        mean_keys = min(keys, (S - S * S / (2 * L) if S < L else L / 2) + 64)
+        mean_queries = min(L, (L - S / 2 if S < L else L * L / (2 * S)) + 64)
+        logits *= min(1.0, 0.6 + 160 / S)
+    # a workgroup of few queries has idle waves and leaves its compute unit to others
+    fwd = 6 + (0.72 + 0.005 * f) * (1.12 if causal else 1) * max(keys, mean_keys * groups_q * min(4, -(-L // 32)) / 1024) / 32
+    bwd = (8 + (0.35 + 0.0031 * f) * max(keys, mean_keys * groups_q / 256) / 32 +
+           (0.5 + 0.0057 * f) * (2.2 if S % 8 else 1) * max(L, 32, (max(mean_queries, 64) + 64) * groups_k / 256) / 32)
+    steps_fwd = max(31, 10 + 0.018 * keys + 5e-5 * S * heads + 1.45e-6 * logits, 16 + 2.9e-6 * logits)
+    steps_bwd = max(34, 15 + 0.0105 * keys + 0.019 * L + max(1.7e-6 * logits, 3.7e-6 * f * max(L, S) * heads), 2.7e-6 * logits)
+    many = min(L, S) >= 32
+    if S % 8 != 0:
+        steps_fwd, steps_bwd = 1.3 * steps_fwd, 1.3 * steps_bwd
+    elif L % 8 != 0 and many:
+        steps_fwd *= 1.2
+    return (many and S % 8 != 0) or fwd < steps_fwd, (many and (S % 8 != 0 or L % 8 != 0)) or bwd < steps_bwd
 
 
 def _permute_leading3(a: DeviceArray, perm) -> DeviceArray:
@@ -763,8 +793,9 @@ def rrule_scaled_dot_product_attention(q, k, v, head_dim=1, token_dim=3, scale=N
     # bf16 without an fdrop: the product is also kept unrounded (fp32) for the pullback, whose softmax rule takes
     # its inner product from it; the array that is returned is its rounded copy
     out_wide = DeviceArray((Ev, H, L) + bshape, wide) if (fdrop is None and wide != dt) else None
-    fused = (out_wide is not None and mask_a is None and bias_a is None and (q.ptr | k.ptr | v.ptr) % 16 == 0
-             and _attention_fused(lq, lk, lv, E, Ev, H, B))
+    fused, fused_back = False, False
+    if out_wide is not None and mask_a is None and bias_a is None and (q.ptr | k.ptr | v.ptr) % 16 == 0:
+        fused, fused_back = _attention_fused(L, S, E, Ev, H, B, lq.st, lk.st, lv.st, causal)
     logits, softmax_out, fdrop_back = None, probs, None
     out = DeviceArray((Ev, H, L) + bshape, dt)
     strides = (_i64x3((lq.st, lq.sh, lq.sb)), _i64x3((lk.st, lk.sh, lk.sb)), _i64x3((lv.st, lv.sh, lv.sb)))
@@ -798,7 +829,7 @@ def rrule_scaled_dot_product_attention(q, k, v, head_dim=1, token_dim=3, scale=N
             _lib.call("luxhip_batch_sum", current_stream(), red.code, like.size, r, full.ptr, red.ptr)
             return red
 
-        if fused and d_out.dtype == dt and d_out.ptr % 16 == 0:
+        if fused_back and d_out.dtype == dt and d_out.ptr % 16 == 0:
             dq, dk, dv = DeviceArray(q.shape, dt), repeats(k), repeats(v)
             _lib.call("luxhip_attention_bwd", current_stream(), softmax_out.code, E, Ev, S, L, _i64x3(bdims), scale_inv, int(causal), q.ptr,
                       strides[0], k.ptr, strides[1], v.ptr, strides[2], softmax_out.ptr, out_wide.ptr, d_out.ptr, dq.ptr, dk.ptr,
