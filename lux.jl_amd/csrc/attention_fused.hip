@@ -212,12 +212,19 @@ __device__ __forceinline__ raw16_t load8(const bf16_t* p, int at, int end) {
 
 // 32 columns (one per lane of a half-wave) x 64 keys of weights between the lanes that own a column and full lines of memory:
 // a wave's own 4 KiB of LDS, 128 bytes per column, its eight chunks XORed with column % 8.  Straight from the lanes a store
-// instruction touches 32 lines with 32 bytes each; this way eight whole ones.
+// instruction touches 32 lines with 32 bytes each; this way eight whole ones.  No workgroup barrier is between the lanes that write
+// and those that read: the LDS takes a wave's accesses in their order, and exchange() keeps the compiler to that order.
 constexpr int PT_BYTES = 32 * 128;
 struct WeightTile {
     char* lds;
     int lane;
     __device__ __forceinline__ WeightTile(void* p, int w) : lds((char*)p + w * PT_BYTES), lane(threadIdx.x & 63) {}
+    // between one side's accesses and the other's
+    __device__ __forceinline__ static void exchange() {
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront", "local");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront", "local");
+    }
     // keys 16 n + {4h .. 4h + 3, 8 + 4h ..} of this lane's column (accumulator order)
     __device__ __forceinline__ void put(int n, raw16_t w) const {
         const int c = lane & 31, h = lane >> 5;
@@ -382,6 +389,7 @@ __global__ __launch_bounds__(THREADS, 2) void fwd_kernel(Args a) {
         // the finished 64 keys (or the first 32 of them) from s0 on
         auto store_weights = [&](int s0) {
             const int end = min(w_end, s0 + 64);
+            pt.exchange();
             if (end == s0 + 64 && wl0 + 32 <= a.L) {        // uniform
 #pragma unroll
                 for (int i = 0; i < 4; ++i)
@@ -422,7 +430,7 @@ __global__ __launch_bounds__(THREADS, 2) void fwd_kernel(Args a) {
                 tk.store(lds + (1 - u) * TILE, 1 - u, t + 1, a.S);
                 tv.store(lds + (3 - u) * TILE, 1 - u, t + 1, a.S);
                 if (u == 1 && ROWS * t0 < w_end) store_weights(ROWS * t0);
-                __syncthreads();
+                __syncthreads();                        // and an exchange(): the next weights go over these
             });
         }
     }
@@ -539,6 +547,7 @@ __global__ __launch_bounds__(THREADS, 2) void dq_kernel(Args a) {
             const raw16_t zero = {0u, 0u, 0u, 0u};
             *pt.line(i) = !VEC || ROWS * t0 + pt.key() < w_end ? pw[i] : zero;
         }
+        pt.exchange();
         static_for<2>([&](auto U) {
             constexpr int u = decltype(U)::value;
             const int t = t0 + u;
@@ -562,7 +571,7 @@ __global__ __launch_bounds__(THREADS, 2) void dq_kernel(Args a) {
             }
             tk.store(lds + (1 - u) * TILE, 1 - u, t + 1, a.S);
             tv.store(lds + (3 - u) * TILE, 1 - u, t + 1, a.S);
-            __syncthreads();
+            __syncthreads();                            // and an exchange(): the next weights go over these
         });
     }
     store_features<ET>(acc, a.dq + wh.h * a.qh + wh.b * a.qb + (int64_t)lc * a.qt, l < a.L, a.E);
