@@ -146,19 +146,24 @@ __device__ __forceinline__ int lds_chunk_offset(int r, int k) {
 }
 
 // fp32 on the bf16 matrix cores.  v_mfma_f32_32x32x2_f32 runs at 1/16 of the bf16 rate, so an fp32 value is cut into three bf16
-// values (8 + 8 + 8 significand bits: hi + mid + lo is the value exactly, down to 2^-110) on its way into LDS, and a product
-// into the six partial products of at least 2^-18 of it; what is left out is below 2^-26.  Partial products are exact and are
-// added in fp32, hi * hi (one instruction per 16 k, where the fp32 instruction takes eight) apart from the five smaller ones,
-// so the sum is rounded less often, not more.
-// Values for which the parts do not carry the value are left to the fp32 instruction: a tile whose result holds an infinity or
-// a NaN (an infinite operand times an absent part, or a value that rounds to a bf16 infinity), or a number below 2^-80 (operands
-// so small that their parts underflow) is computed again, see GemmMainloop::run.
+// values (8 + 8 + 8 significand bits) on its way into LDS, and a product into the six partial products of at least 2^-18 of it;
+// what is left out is below 2^-26.  Partial products are exact and are added in fp32, hi * hi (one instruction per 16 k, where
+// the fp32 instruction takes eight) apart from the five smaller ones, so the sum is rounded less often, not more.
+// Values are multiplied by 2^24 before they are cut and sums by 2^-48 at the end (finish_parts), both exact: fp32 numbers are
+// multiples of 2^-149, so that all their parts are multiples of 2^-125, normal bf16 numbers or zero, and hi + mid + lo is the value
+// exactly, subnormal numbers included; a partial product that counts for a normal result (2^-26 of 2^-126) is 2^-104, far from the
+// end of the range.  (Without the factor the lower parts of values below 2^-110 underflow, which a large partner brings to light:
+// operands of 1e-37 and 1e25 gave products 3e-4 off, 1e-41 and 1e30 gave 0.)
+// The other end of the range is left to the fp32 instruction: an infinite or NaN operand, one of 2^104 or more (2e31) and a sum of
+// 2^80 or more (1e24) make the accumulators of their rows or columns infinite or NaN, and such a tile is computed again, see
+// GemmMainloop::run.  It then costs both passes (fp32 2048^3: 346 + 484 us for all tiles).
 //
 // A 16-byte chunk that starts at (row r, column k) of a tile -> LDS.  SPLIT: three bf16 planes of ROWS x 16, each K-major
 // [row][16] with the two 16-byte halves of a row exchanged in rows 8 .. 15 of sixteen (sixteen rows then fall into sixteen
 // different chunks of the bank period), or MN-major [k][ROWS] as for bf16 operands.
 template <int ROWS>
 __host__ __device__ constexpr int plane_elems() { return ROWS * 8; }      // in floats
+constexpr float PART_SCALE = 0x1p24f, PART_UNSCALE = 0x1p-48f;            // of an operand's values, of a sum of products
 template <typename T, bool KMAJOR, int ROWS, bool SPLIT>
 __device__ __forceinline__ void put_chunk(T* lds, int r, int k, u32x4_v v) {
     if constexpr (SPLIT) {
@@ -166,7 +171,7 @@ __device__ __forceinline__ void put_chunk(T* lds, int r, int k, u32x4_v v) {
         bf16_t* p = reinterpret_cast<bf16_t*>(lds) + (KMAJOR ? r * 16 + (k ^ (r & 8)) : k * ROWS + (r ^ ((k & 3) << mn_swizzle_shift(ROWS))));
         float f[4];
 #pragma unroll
-        for (int i = 0; i < 4; ++i) f[i] = __uint_as_float(v[i]);
+        for (int i = 0; i < 4; ++i) f[i] = __uint_as_float(v[i]) * PART_SCALE;
 #pragma unroll
         for (int q = 0; q < 3; ++q) {
             const uint32_t a = f32x2_to_bf16x2(f[0], f[1]), b = f32x2_to_bf16x2(f[2], f[3]);
@@ -424,22 +429,21 @@ __device__ __forceinline__ bf16x8_v load_frag_part(const float* tile, int rbase,
         return load_frag_bf16<false, ROWS>(p, rbase, 0);
     }
 }
-// neither zero nor a finite number of at least 2^-80
-__device__ __forceinline__ bool split_suspect(float v) {
-    const uint32_t u = __float_as_uint(v) & 0x7fffffffu;
-    return u - 1u < 0x17800000u - 1u || u >= 0x7f800000u;
-}
-
+// The sums of all partial products, without the operands' factors; false if one of them is no finite number
 template <int WM, int WN>
-__device__ __forceinline__ bool split_suspect(const f32x16_v (&acc)[WM][WN]) {
-    bool any = false;
+__device__ __forceinline__ bool finish_parts(f32x16_v (&acc)[WM][WN], const f32x16_v (&small)[WM][WN]) {
+    bool finite = true;
 #pragma unroll
     for (int i = 0; i < WM; ++i)
 #pragma unroll
         for (int j = 0; j < WN; ++j)
 #pragma unroll
-            for (int r = 0; r < 16; ++r) any |= split_suspect(acc[i][j][r]);
-    return any;
+            for (int r = 0; r < 16; ++r) {
+                const float v = acc[i][j][r] + small[i][j][r];
+                finite &= fabsf(v) < INFINITY;
+                acc[i][j][r] = v * PART_UNSCALE;
+            }
+    return finite;
 }
 // One stage (16 k) of a wave's WM x WN accumulators; SPLIT: on the bf16 matrix cores, the smaller partial products in `small`
 template <bool SPLIT, bool A_KMAJOR, bool B_KMAJOR, int TILE_M, int TILE_N, int WM, int WN>
@@ -716,15 +720,14 @@ struct GemmMainloop {
     __device__ __forceinline__ static void run(LoaderA& la, LoaderB& lb, int K, T* lds, f32x16_v (&acc)[WM][WN]) {
         static_assert(LoaderA::KMAJOR == A_KMAJOR && LoaderB::KMAJOR == B_KMAJOR, "loader layout mismatch");
         if constexpr (MAY_SPLIT && SPLIT_F32) {
-            run_as<true>(la, lb, K, lds, acc);
-            if (__syncthreads_or(split_suspect(acc)) == 0) return;
+            if (__syncthreads_and(run_as<true>(la, lb, K, lds, acc))) return;
         }
         run_as<false>(la, lb, K, lds, acc);
     }
 
-    // SPLIT: fp32 operands as three bf16 parts each
+    // SPLIT: fp32 operands as three bf16 parts each; false if a result is no finite number then
     template <bool SPLIT, class LoaderA, class LoaderB>
-    __device__ __forceinline__ static void run_as(LoaderA& la, LoaderB& lb, int K, T* lds, f32x16_v (&acc)[WM][WN]) {
+    __device__ __forceinline__ static bool run_as(LoaderA& la, LoaderB& lb, int K, T* lds, f32x16_v (&acc)[WM][WN]) {
         const int w = threadIdx.x >> 6;
         const int wave_m = (w % NWM) * (WM * 32), wave_n = (w / NWM) * (WN * 32);
         zero(acc);
@@ -773,10 +776,7 @@ struct GemmMainloop {
                 buf0 = buf1;
                 buf1 = t;
             }
-#pragma unroll
-            for (int i = 0; i < WM; ++i)
-#pragma unroll
-                for (int j = 0; j < WN; ++j) acc[i][j] += small[i][j];
+            return finish_parts(acc, small);
         } else {
             // Global loads run two stages ahead of the MFMAs (two register sets), LDS is double
             // buffered: while stage kt is consumed from one LDS buffer, stage kt+1 waits in the
@@ -808,6 +808,7 @@ struct GemmMainloop {
                 __syncthreads();
             }
             if (kt < KT) compute(buf0, buf0 + A_ELEMS);   // odd number of stages: the last one sits in buf0
+            return true;
         }
     }
 

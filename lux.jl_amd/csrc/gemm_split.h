@@ -145,13 +145,12 @@ struct Core {
     // k range [kbeg, kend)
     __device__ __forceinline__ static void run(const LA& la, const LB& lb, int kbeg, int kend, T* lds, f32x16_v (&acc)[WM][WN]) {
         if constexpr (ML::SPLIT_F32) {
-            run_as<true>(la, lb, kbeg, kend, lds, acc);
-            if (__syncthreads_or(split_suspect(acc)) == 0) return;
+            if (__syncthreads_and(run_as<true>(la, lb, kbeg, kend, lds, acc))) return;
         }
         run_as<false>(la, lb, kbeg, kend, lds, acc);
     }
-    template <bool SPLIT>
-    __device__ __forceinline__ static void run_as(const LA& la, const LB& lb, int kbeg, int kend, T* lds, f32x16_v (&acc)[WM][WN]) {
+    template <bool SPLIT>          // false: see GemmMainloop::run_as
+    __device__ __forceinline__ static bool run_as(const LA& la, const LB& lb, int kbeg, int kend, T* lds, f32x16_v (&acc)[WM][WN]) {
         const int w = threadIdx.x >> 6;
         const int wave_m = (w % NWM) * (WM * 32), wave_n = (w / NWM) * (WN * 32);
         ML::zero(acc);
@@ -186,12 +185,8 @@ struct Core {
                 if (k0 + u * Tr::BK < kend) compute<SPLIT>(lds + u * ML::STAGE_ELEMS, lds + u * ML::STAGE_ELEMS + ML::A_ELEMS, wave_m, wave_n, acc, small);
             __syncthreads();
         }
-        if constexpr (SPLIT) {
-#pragma unroll
-            for (int i = 0; i < WM; ++i)
-#pragma unroll
-                for (int j = 0; j < WN; ++j) acc[i][j] += small[i][j];
-        }
+        if constexpr (SPLIT) return finish_parts(acc, small);
+        return true;
     }
 
     // hand-off of a slice's accumulators; true in the workgroup that holds the sum and runs the epilogue

@@ -3,6 +3,7 @@
 import numpy as np
 import pytest
 
+from oracle import luxlib_oracle as O
 from tests.util import assert_close, dev, stable_seed
 
 pytestmark = pytest.mark.gpu
@@ -80,3 +81,48 @@ def test_convolution_with_an_infinite_input(gpu, channels):
     assert (dx[inside] == np.inf).all() and np.isfinite(dx[~inside]).all()
     dw = gpu.conv_filter_grad(dev(gpu, x, "f32"), dev(gpu, dy, "f32"), cd).to_numpy()
     assert np.isfinite(dw[:, :, :, np.arange(cout) != 7]).all() and not np.isfinite(dw[:, :, :, 7]).any()
+
+
+# Scales of the two operands.  Nothing of an fp32 number may be lost that a large partner brings to light, subnormal numbers included; the last ones
+# leave the range that the parts carry (operands from 2^104, sums from 2^80)
+PAIRS = [(1e-35, 1e20), (1e20, 1e-36), (1e-37, 1e25), (1e-39, 1e30), (1e30, 1e-41), (1e-41, 1e3), (1e-26, 1.0), (1e30, 1e-30), (1e33, 1e-33), (1e15, 1e15)]
+
+
+def scaled(rng, scale, shape):
+    return (rng.normal(size=shape) * scale).astype(np.float32)
+
+
+def error(got, want):
+    scale = np.linalg.norm(want)
+    return np.linalg.norm(got.astype(np.float64) / scale - want / scale)
+
+
+@pytest.mark.parametrize("a,b", PAIRS)
+def test_small_operands_with_large_partners(gpu, a, b):
+    """Whole tiles and ragged ones, the bound of test_error_is_that_of_fp32."""
+    for M, N, K in ((2048, 2048, 64), (1921, 2047, 100)):
+        rng = np.random.default_rng(stable_seed("split-pair", a, b, M))
+        w, x = scaled(rng, a, (M, K)), scaled(rng, b, (K, N))
+        assert error(product(gpu, w, x), w.astype(np.float64) @ x.astype(np.float64)) <= 2.0 ** -23 * np.sqrt(K / 6) + 2.0 ** -26
+
+
+@pytest.mark.parametrize("channels", [(96, 96), (72, 128), (128, 72)])
+@pytest.mark.parametrize("a,b", [(1e-37, 1e25), (1e30, 1e-41)])
+def test_convolutions_of_small_operands_with_large_partners(gpu, channels, a, b):
+    """The three directions of a 3 x 3 convolution that fills the chip; images stand for themselves in the output and the input
+    gradient, so only the last one is compared."""
+    cin, cout = channels
+    xs, ws = (64, 64, cin, 8), (3, 3, cin, cout)
+    rng = np.random.default_rng(stable_seed("split-pair-conv", a, b, channels))
+    x, w, dy = scaled(rng, a, xs), scaled(rng, b, ws), scaled(rng, a, (64, 64, cout, 8))
+    gd, od = gpu.DenseConvDims(xs, ws, padding=1), O.ConvDims(xs[:3] + (1,), ws, padding=1)
+    last = lambda t: t[..., -1:].astype(np.float64)
+    bound = lambda K: 2.0 ** -23 * np.sqrt(K / 6) + 2.0 ** -26
+    got = gpu.conv(dev(gpu, x, "f32"), dev(gpu, w, "f32"), gd).to_numpy()
+    assert error(last(got), O.conv(last(x), w.astype(np.float64), od)) <= bound(9 * cin)
+    got = gpu.conv_data_grad(dev(gpu, dy, "f32"), dev(gpu, w, "f32"), gd).to_numpy()
+    assert error(last(got), O.conv_data_grad(last(dy), w.astype(np.float64), od)) <= bound(9 * cout)
+    x, dy = np.ascontiguousarray(x[:32, :32, :, :2]), scaled(rng, b, (32, 32, cout, 2))
+    gd, od = (D(x.shape, ws, padding=1) for D in (gpu.DenseConvDims, O.ConvDims))
+    got = gpu.conv_filter_grad(dev(gpu, x, "f32"), dev(gpu, dy, "f32"), gd).to_numpy()
+    assert error(got, O.conv_filter_grad(x.astype(np.float64), dy.astype(np.float64), od)) <= bound(2 * 32 * 32)
