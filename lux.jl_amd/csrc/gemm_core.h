@@ -528,28 +528,27 @@ inline int persistent_grid(Kernel kernel, int threads, size_t lds_bytes, int64_t
 // NWM x NWN waves per workgroup (along m, along n); wave w sits at (w % NWM, w / NWM).
 // PERMUTE: on the direct-to-LDS path with a K-major A, the A rows of each wave are permuted
 // (DirectLoader PERM_WM = WM) so that a lane owns WM consecutive m: m = lane_m + i.
+// MAY_SPLIT: fp32 products may take the bf16 matrix cores (split_f32), whose stages are larger.
 template <typename T, int WM, int WN, bool A_KMAJOR, bool B_KMAJOR, bool FULL = false, int NWN = 2, int NSTAGES = 0,
-          int NWM = 2, bool PERMUTE = false>
+          int NWM = 2, bool PERMUTE = false, bool MAY_SPLIT = true>
 struct GemmMainloop {
     using Tr = GemmTraits<T>;
     static constexpr int THREADS = NWM * NWN * 64;
     static constexpr int TILE_M = NWM * WM * 32, TILE_N = NWN * WN * 32;
     using PlainLoaderA = TileLoader<T, A_KMAJOR, TILE_M, FULL, THREADS>;
     using PlainLoaderB = TileLoader<T, B_KMAJOR, TILE_N, FULL, THREADS>;
-    static constexpr int A_ELEMS = lds_tile_elems<T, A_KMAJOR>(TILE_M, split_f32<T, WM, WN>());
-    static constexpr int B_ELEMS = lds_tile_elems<T, B_KMAJOR>(TILE_N, split_f32<T, WM, WN>());
+    static constexpr bool SPLIT_F32 = MAY_SPLIT && split_f32<T, WM, WN>();
+    static constexpr int A_ELEMS = lds_tile_elems<T, A_KMAJOR>(TILE_M, SPLIT_F32);
+    static constexpr int B_ELEMS = lds_tile_elems<T, B_KMAJOR>(TILE_N, SPLIT_F32);
     static constexpr int STAGE_ELEMS = A_ELEMS + B_ELEMS;
     static constexpr bool DIRECT = FULL && sizeof(T) == 2;     // global -> LDS without registers
     static constexpr int NST = NSTAGES > 0 ? NSTAGES : (DIRECT ? 4 : 2);   // LDS stages
     static constexpr size_t LDS_BYTES = NST * (size_t)STAGE_ELEMS * sizeof(T);
-    static constexpr bool SPLIT_F32 = split_f32<T, WM, WN>();
     static constexpr int PERM_A = (PERMUTE && DIRECT && A_KMAJOR && WM > 1 && (THREADS / 4) % (32 * WM) == 0) ? WM : 0;
     static constexpr int M_STEP = PERM_A ? 1 : 32;            // distance in m between acc[i] and acc[i + 1] of a lane
     using DirectLoaderA = DirectLoader<A_KMAJOR, TILE_M, THREADS, false, PERM_A>;
     using DirectLoaderB = DirectLoader<B_KMAJOR, TILE_N, THREADS>;
 
-    // MAY_SPLIT: fp32 products may take the bf16 matrix cores (split_f32)
-    template <bool MAY_SPLIT = true>
     __device__ __forceinline__ static void run(const Operand<T>& A, const Operand<T>& B, int K, int m0, int n0, T* lds,
                                                f32x16_v (&acc)[WM][WN]) {
         if constexpr (FULL && sizeof(T) == 2) {
@@ -557,7 +556,7 @@ struct GemmMainloop {
         } else {
             PlainLoaderA la(A, m0, K);
             PlainLoaderB lb(B, n0, K);
-            run<MAY_SPLIT>(la, lb, K, lds, acc);
+            run(la, lb, K, lds, acc);
         }
     }
 
@@ -716,10 +715,10 @@ struct GemmMainloop {
     }
 
     // k range [0, K) in stages of BK; the loaders decide what a stage contains
-    template <bool MAY_SPLIT = true, class LoaderA, class LoaderB>
+    template <class LoaderA, class LoaderB>
     __device__ __forceinline__ static void run(LoaderA& la, LoaderB& lb, int K, T* lds, f32x16_v (&acc)[WM][WN]) {
         static_assert(LoaderA::KMAJOR == A_KMAJOR && LoaderB::KMAJOR == B_KMAJOR, "loader layout mismatch");
-        if constexpr (MAY_SPLIT && SPLIT_F32) {
+        if constexpr (SPLIT_F32) {
             if (__syncthreads_and(run_as<true>(la, lb, K, lds, acc))) return;
         }
         run_as<false>(la, lb, K, lds, acc);

@@ -403,11 +403,16 @@ struct SoftmaxRuleOperands {
 };
 struct NoOperands {};
 
+// fp32 products of batches stay on the fp32 instruction, in its smaller stages: their contractions are short and ragged, and in
+// three bf16 parts fp32 attention of twenty sizes ran at 0.72 to 1.36 of this speed, at 0.94 in the mean.
+template <typename T, int WM, int WN, bool A_KMAJOR, bool B_KMAJOR, bool FULL, int NWN, int NWM>
+using BatchedMainloop = GemmMainloop<T, WM, WN, A_KMAJOR, B_KMAJOR, FULL, NWN, 0, NWM, true, false>;
+
 // EP: the variant with the softmax rule as its epilogue (a.ep_probs), a kernel of its own so that the plain products
 // keep their register budget (and with it two workgroups per compute unit)
 template <typename T, int WM, int WN, bool A_KMAJOR, bool B_KMAJOR, bool FULL, int NWN, int NWM, bool EP = false>
 __global__ __launch_bounds__(NWM * NWN * 64, (EP && FULL) ? 2 : 1) void batched_gemm_kernel(DenseArgs<T> a) {
-    using ML = GemmMainloop<T, WM, WN, A_KMAJOR, B_KMAJOR, FULL, NWN, 0, NWM, true>;
+    using ML = BatchedMainloop<T, WM, WN, A_KMAJOR, B_KMAJOR, FULL, NWN, NWM>;
     extern __shared__ __align__(16) unsigned char lds_raw[];
     T* lds = reinterpret_cast<T*>(lds_raw);
     const int tiles = a.tiles_m * a.tiles_n;
@@ -463,9 +468,7 @@ __global__ __launch_bounds__(NWM * NWN * 64, (EP && FULL) ? 2 : 1) void batched_
             const BatchTile<T> cur = batch_tile<T, ML::TILE_M, ML::TILE_N>(a, t, tiles);
             if (!cur.store) continue;          // uniform
             if constexpr (EP) ep.load(a, cur.coff, cur.product, cur.m0, cur.n0);
-            // on the fp32 instruction: the short, ragged contractions of batches gain nothing on the bf16 matrix cores (fp32 attention
-            // 0.72 to 1.36 of its time either way, 0.94 over twenty sizes)
-            ML::template run<false>(cur.A, cur.B, cur.K, cur.m0, cur.n0, lds, acc);
+            ML::run(cur.A, cur.B, cur.K, cur.m0, cur.n0, lds, acc);
             DenseArgs<T> out = a;
             out.C = cur.C;
             if constexpr (EP) ep.store(acc, a, cur.coff, cur.m0, cur.n0);
@@ -478,7 +481,7 @@ __global__ __launch_bounds__(NWM * NWN * 64, (EP && FULL) ? 2 : 1) void batched_
 
 template <typename T, int WM, int WN, bool AK, bool BKM, bool FULL, bool EP = false>
 int launch_batched_cfg(hipStream_t s, DenseArgs<T>& a) {
-    using ML = GemmMainloop<T, WM, WN, AK, BKM, FULL, 2, 0, 2>;
+    using ML = BatchedMainloop<T, WM, WN, AK, BKM, FULL, 2, 2>;
     a.tiles_m = (int)ceil_div(a.M, ML::TILE_M);
     a.tiles_n = (int)ceil_div(a.N, ML::TILE_N);
     const int64_t total = (int64_t)a.tiles_m * a.tiles_n * a.batch;
