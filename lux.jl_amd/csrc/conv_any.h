@@ -69,6 +69,10 @@ struct Args {
     int run;                   // RUNS: elements of a stage that belong to the row's window, the rest count as zero
 };
 
+// A chunk of a row.  Runs of positions (see Runs in conv.hip) start at any position, and one of four bf16 channels is eight bytes; the
+// load is the same instruction as an aligned one.
+typedef uint32_t chunk8_t __attribute__((ext_vector_type(4), aligned(8)));
+
 // A: K-major rows of the im2col matrix.  RUNS: a stage is the window's positions of one source row (see Runs in conv.hip); what
 // lies behind them in memory is data of other windows, and is cut off here (a zero in the filter would turn an infinity into NaN).
 template <typename T, int ROWS, bool RUNS>
@@ -110,7 +114,7 @@ struct RowLoader {
             const int sp = ps[i] + dp, sq = qs[i] + dq;
             const bool valid = tap && (unsigned)sp < (unsigned)g.SP && (unsigned)sq < (unsigned)g.SQ;
             const T* p = src + ((int64_t)((pos[i] + sq) * g.SP + sp) * g.Ctot + c);
-            reg[i] = *reinterpret_cast<const u32x4_v*>(valid ? static_cast<const void*>(p) : g.zero);
+            reg[i] = *reinterpret_cast<const chunk8_t*>(valid ? static_cast<const void*>(p) : g.zero);
         }
     }
     template <bool SPLIT>
@@ -318,7 +322,7 @@ struct WgradRowLoader {
             const int sp = ow * g.sw + dp, sq = oh * g.sh + dq;
             const bool valid = in && kp < g.positions && (unsigned)sp < (unsigned)g.SP && (unsigned)sq < (unsigned)g.SQ;
             const T* p = g.src + ((int64_t)((n * g.SQ + sq) * g.SP + sp) * g.Ctot + c);
-            reg[i] = *reinterpret_cast<const u32x4_v*>(valid ? static_cast<const void*>(p) : g.zero);
+            reg[i] = *reinterpret_cast<const chunk8_t*>(valid ? static_cast<const void*>(p) : g.zero);
         }
     }
     template <bool SPLIT>
