@@ -100,8 +100,8 @@ int luxhip_event_destroy(luxhip_event_t e);
  * streaming kernels (bias_activation, batchnorm, groupnorm, layernorm) hand two events to their
  * dispatch, which signals them at the begin and at the end of the kernel itself: the duration a
  * kernel trace reports.  The other launches are bracketed by events recorded around them (the
- * kernel plus the gap to the launch before it).  luxhip_profile_report synchronises, writes a JSON array of {kernel, count, total_ms, min_ms,
- * max_ms} into buf and clears the log. */
+ * kernel plus the gap to the launch before it).  luxhip_profile_report synchronises, writes a JSON array of {kernel, count, parts, total_ms,
+ * min_ms, max_ms} into buf and clears the log; parts: launches that computed fp32 products as three bf16 parts per value. */
 int luxhip_profile_enable(int on);
 /* Tuning switches (no counterpart in LuxLib; tests use them to reach every code path):
  *   "bn_resident"   1 (default) / 0: single-pass batchnorm kernels that keep the tensor in registers

@@ -83,6 +83,7 @@ struct ProfScope {
     hipEvent_t start = nullptr, stop = nullptr;
     ProfScope(const char* n, hipStream_t s, bool exact = false);
     ~ProfScope();
+    void in_parts(bool yes);     // the launch computes fp32 products in bf16 parts (gemm_core.h): the report counts such launches
 };
 
 // kernel<<<grid, block, lds, s>>>(args...) of an exact scope

@@ -22,6 +22,7 @@ int launch_shape(hipStream_t s, Args<T>& a, int blocks, int groups, bool dgrad) 
     using S = Shape<T, WM, WN, NWM, NWN>;
     static const char* const names[2][2] = {{"conv_fprop_kernel<f32>", "conv_dgrad_kernel<f32>"}, {"conv_fprop_kernel<bf16>", "conv_dgrad_kernel<bf16>"}};
     ProfScope ps(names[sizeof(T) == 2][dgrad], s);
+    ps.in_parts(split_f32<T, WM, WN>());
     const dim3 grid((unsigned)blocks, (unsigned)groups);
     if constexpr (sizeof(T) == 2) {
         if (a.run > 0) {
@@ -125,6 +126,7 @@ int launch_wgrad_shape(hipStream_t s, WgradArgs<T>& a, int slices) {
     a.tiles_m = (int)ceil_div(a.Mrows, S::TILE_M);
     a.tiles_n = (int)ceil_div(a.Ncols, S::TILE_N);
     ProfScope ps(sizeof(T) == 2 ? "conv_wgrad_kernel<bf16>" : "conv_wgrad_kernel<f32>", s);
+    ps.in_parts(split_f32<T, WM, WN>());
     conv_any_wgrad_kernel<T, WM, WN, NWM, NWN><<<dim3((unsigned)(a.tiles_m * a.tiles_n * slices)), dim3(split::THREADS), S::Core::LDS_BYTES, s>>>(a);
     LUX_CHECK_LAUNCH();
     return LUXHIP_OK;

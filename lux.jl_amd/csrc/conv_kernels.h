@@ -343,6 +343,7 @@ int launch_conv_tap(hipStream_t s, ConvTapArgs<T>& a) {
         {{"conv_fprop_kernel<f32>", "conv_fprop_kernel<f32>+tail"}, {"conv_dgrad_kernel<f32>", "conv_dgrad_kernel<f32>+tail"}},
         {{"conv_fprop_kernel<bf16>", "conv_fprop_kernel<bf16>+tail"}, {"conv_dgrad_kernel<bf16>", "conv_dgrad_kernel<bf16>+tail"}}};
     ProfScope ps(names[sizeof(T) == 2][a.tap.dgrad ? 1 : 0][a.m_begin > 0], s);
+    ps.in_parts(ML::SPLIT_F32);
     kernel<<<dim3((unsigned)grid), dim3(ML::THREADS), ML::LDS_BYTES, s>>>(a);
     LUX_CHECK_LAUNCH();
     return LUXHIP_OK;

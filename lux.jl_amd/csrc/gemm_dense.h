@@ -131,6 +131,7 @@ int launch_cfg_full(hipStream_t s, DenseArgs<T>& a) {
     const int grid = (int)std::min<int64_t>((int64_t)a.tiles_m * a.tiles_n, resident);
     ProfScope ps(sizeof(T) == 2 ? (a.tail ? "dense_gemm_kernel<bf16>+tail" : "dense_gemm_kernel<bf16>")
                                 : (a.tail ? "dense_gemm_kernel<f32>+tail" : "dense_gemm_kernel<f32>"), s);
+    ps.in_parts(ML::SPLIT_F32);
     kernel<<<dim3((unsigned)grid), dim3(ML::THREADS), ML::LDS_BYTES, s>>>(a);
     LUX_CHECK_LAUNCH();
     return LUXHIP_OK;

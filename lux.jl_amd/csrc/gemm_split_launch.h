@@ -76,6 +76,7 @@ int launch_cfg(hipStream_t s, DenseArgs<T>& a, int slices) {
         place(p, ws, 0);
     }
     ProfScope ps(sizeof(T) == 2 ? "split_gemm_kernel<bf16>" : "split_gemm_kernel<f32>", s);
+    ps.in_parts(split_f32<T, W, W>());
     split_gemm_kernel<T, W, AK, BKM><<<dim3((unsigned)(a.tiles_m * a.tiles_n * p.slices)), dim3(THREADS), B::LDS_BYTES, s>>>(a, p);
     LUX_CHECK_LAUNCH();
     return LUXHIP_OK;

@@ -56,6 +56,7 @@ struct ProfEntry {
     const char* name;
     hipStream_t stream;
     int a, b;   // indices into g_prof_events, b < 0 while the scope is open
+    bool parts = false;
 };
 bool g_prof = false;
 std::vector<ProfEntry> g_prof_entries;
@@ -103,6 +104,13 @@ ProfScope::~ProfScope() {
     // the matching entry is the last one with this name still open
     for (auto it = g_prof_entries.rbegin(); it != g_prof_entries.rend(); ++it)
         if (it->name == name && it->b < 0) { it->b = prof_record(stream); break; }
+}
+
+void ProfScope::in_parts(bool yes) {
+    if (!active || !yes) return;
+    std::lock_guard<std::mutex> lk(g_mu);
+    for (auto it = g_prof_entries.rbegin(); it != g_prof_entries.rend(); ++it)
+        if (it->name == name && it->b < 0) { it->parts = true; break; }
 }
 
 int set_error(int status, const char* fmt, ...) {
@@ -433,13 +441,13 @@ int luxhip_profile_report(char* buf, size_t len) {
     LUX_INVALID_IF(buf == nullptr || len < 3, "profile_report: buffer too small");
     LUX_CHECK_HIP(hipDeviceSynchronize());
     std::lock_guard<std::mutex> lk(g_mu);
-    struct Agg { int count = 0; double total = 0, mn = 1e30, mx = 0; };
+    struct Agg { int count = 0, parts = 0; double total = 0, mn = 1e30, mx = 0; };
     std::map<std::string, Agg> agg;
     for (auto& e : g_prof_entries) {
         float ms = 0.0f;
         if (e.a >= 0 && e.b >= 0 && hipEventElapsedTime(&ms, g_prof_events[e.a], g_prof_events[e.b]) == hipSuccess) {
             Agg& a = agg[e.name];
-            a.count++; a.total += ms;
+            a.count++; a.parts += e.parts; a.total += ms;
             if (ms < a.mn) a.mn = ms;
             if (ms > a.mx) a.mx = ms;
         }
@@ -452,8 +460,8 @@ int luxhip_profile_report(char* buf, size_t len) {
     bool first = true;
     for (auto& kv : agg) {
         if (off + 200 >= len) break;
-        off += snprintf(buf + off, len - off, "%s{\"kernel\": \"%s\", \"count\": %d, \"total_ms\": %.6f, \"min_ms\": %.6f, \"max_ms\": %.6f}",
-                        first ? "" : ", ", kv.first.c_str(), kv.second.count, kv.second.total, kv.second.mn, kv.second.mx);
+        off += snprintf(buf + off, len - off, "%s{\"kernel\": \"%s\", \"count\": %d, \"parts\": %d, \"total_ms\": %.6f, \"min_ms\": %.6f, \"max_ms\": %.6f}",
+                        first ? "" : ", ", kv.first.c_str(), kv.second.count, kv.second.parts, kv.second.total, kv.second.mn, kv.second.mx);
         first = false;
     }
     snprintf(buf + off, len - off, "]");

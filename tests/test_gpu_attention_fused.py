@@ -136,3 +136,22 @@ def test_weights_of_large_logits_add_up_to_one(gpu, scale):
     want = np.zeros((S, L, H, 1))
     want[:n] = 1.0 / n
     np.testing.assert_allclose(run()[1].to_numpy(), want, rtol=2.0 ** -8, atol=0)
+
+
+@pytest.mark.parametrize("scale", [-3.0, np.inf])
+def test_negative_and_zero_scale(gpu, scale):
+    """A negative divisor turns the softmax round (the kernels flip q's sign), an infinite one makes all logits equal, masked ones still
+    -inf."""
+    E, H, L, S = 64, 2, 97, 130
+    rng = np.random.default_rng(stable_seed("attn-fused-scale", scale))
+    q, k, v, d_out = host_inputs("bf16", *(rng.normal(size=(E, H, t, 1)) for t in (L, S, S, L)))
+    (out, w), back = gpu.pullback(gpu.scaled_dot_product_attention, *(dev(gpu, a, "bf16") for a in (q, k, v)), 1, 3, scale, None, True)
+    stored = f64(w.to_numpy())
+    assert_close(stored, O.scaled_dot_product_attention(f64(q), f64(k), f64(v), 3, scale, None, True)[1], "bf16", "weights")
+    assert_close(out.to_numpy(), O.scaled_dot_product_attention(f64(q), f64(k), f64(v), 3, scale, None, True, weights=stored)[0], "bf16", "out")
+    grads = []
+    assert "attn_dq_kernel" in kernels_of(gpu, lambda: grads.extend(back(dev(gpu, d_out, "bf16"))))
+    want = O.scaled_dot_product_attention_pullback(f64(q), f64(k), f64(v), f64(d_out), 3, scale, None, True, weights=stored,
+                                                   stored=lambda a: f64(O.round_to_bf16(np.asarray(a, np.float32))))
+    for g, x, name in zip(grads, want, ("dq", "dk", "dv")):
+        assert_close(g.to_numpy(), x, "bf16", name, scale=1e-3)

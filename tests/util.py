@@ -80,8 +80,8 @@ def stable_seed(*parts):
     return zlib.crc32(repr(parts).encode()) & 0x7FFFFFFF
 
 
-def kernels_of(gpu, f):
-    """The kernels that f launches, with their number."""
+def profile_of(gpu, f):
+    """The profile's entries of the kernels that f launches."""
     import ctypes
     import json
     buf = ctypes.create_string_buffer(1 << 16)
@@ -91,4 +91,14 @@ def kernels_of(gpu, f):
         gpu._lib.call("luxhip_profile_report", buf, len(buf))
     finally:
         gpu._lib.call("luxhip_profile_enable", 0)
-    return {k["kernel"]: k["count"] for k in json.loads(buf.value.decode())}
+    return json.loads(buf.value.decode())
+
+
+def kernels_of(gpu, f):
+    """The kernels that f launches, with their number."""
+    return {k["kernel"]: k["count"] for k in profile_of(gpu, f)}
+
+
+def in_parts(gpu, f):
+    """The kernels among them that computed fp32 products as three bf16 parts per value, with the number of those launches."""
+    return {k["kernel"]: k["parts"] for k in profile_of(gpu, f) if k["parts"]}
