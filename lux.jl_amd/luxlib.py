@@ -669,14 +669,16 @@ def _attention_fused(L, S, E, Ev, H, B, stride_q, stride_k, stride_v, causal):
     128 queries of a head and walks all keys, one of the dk / dv kernel 128 keys and all queries: with fewer workgroups than compute
     units the time is that of one walk, however many heads there are, while the products cut both token dims into tiles.  The walk's
     time per 32 tokens and the products' times are fitted to 502 calls (1 to 512 heads, 1 to 8192 queries and keys in all
-    proportions, 32 to 128 features, causal or not; 31 and 34 us are the products' launches by this host): what the estimate takes
-    is 0.2 % behind the faster way in the mean, 13 % at worst.
+    proportions, 32 to 128 features, causal or not; 31 and 34 us are the products' launches by this host), those of ragged keys to another
+    835.  Over 1666 calls, half of them with ragged keys, what the estimate takes is 0.3 % (forward) and 0.5 % (pullback) behind the faster
+    way in the mean; six pullbacks are more than 5 % slower than step by step, 20 % at worst.
     Forward at 64 features, us fused / step by step: 1 query, 2048 keys, 32 heads 64 / 38, 512 heads 67 / 92; 512 queries, 2048 keys,
     8 heads 69 / 50, 32 heads 71 / 107; 1024 x 1024, 2 heads 37 / 32, 8 heads 39 / 41.  Pullback at 128 features: 2048 x 2048, 8 heads
     137 / 118, 32 heads 243 / 383; 8192 queries, 128 keys, 32 heads 365 / 292; 128 queries, 2048 keys, 32 heads 77 / 62, 256
     heads 263 / 312.
-    Rows that are no whole vectors cost the products more than the kernels (32 x 2047 forward 64 / 80, 583 x 583 pullback 77 / 125):
-    from 32 tokens on either side the kernels take those whatever the number of heads."""
+    Weights in rows that are no whole vectors cost the products more than the kernels: forward, from 32 tokens on either side, at any
+    number of heads (32 x 2047 64 / 80, none of 835 calls slower).  The pullback's walk of few blocks of keys over many queries loses
+    nevertheless: 2047 queries, 47 keys, 2 heads 153 / 98; 2688 queries, 214 keys, 1 head 174 / 142; 583 x 583 77 / 125."""
     if not (0 < E <= 128 and 0 < Ev <= 128 and E % 8 == 0 and Ev % 8 == 0 and S > 0 and L > 0 and H > 0 and B > 0):
         return False, False
     heads, f = H * B, 32 * -(-max(E, Ev) // 32)
@@ -692,16 +694,17 @@ def _attention_fused(L, S, E, Ev, H, B, stride_q, stride_k, stride_v, causal):
         logits *= min(1.0, 0.6 + 160 / S)
     # a workgroup of few queries has idle waves and leaves its compute unit to others
     fwd = 6 + (0.72 + 0.005 * f) * (1.12 if causal else 1) * max(keys, mean_keys * groups_q * min(4, -(-L // 32)) / 1024) / 32
-    bwd = (8 + (0.35 + 0.0031 * f) * max(keys, mean_keys * groups_q / 256) / 32 +
-           (0.5 + 0.0057 * f) * (2.2 if S % 8 else 1) * max(L, 32, (max(mean_queries, 64) + 64) * groups_k / 256) / 32)
     steps_fwd = max(31, 10 + 0.018 * keys + 5e-5 * S * heads + 1.45e-6 * logits, 16 + 2.9e-6 * logits)
-    steps_bwd = max(34, 15 + 0.0105 * keys + 0.019 * L + max(1.7e-6 * logits, 3.7e-6 * f * max(L, S) * heads), 2.7e-6 * logits)
-    many = min(L, S) >= 32
-    if S % 8 != 0:
-        steps_fwd, steps_bwd = 1.3 * steps_fwd, 1.3 * steps_bwd
-    elif L % 8 != 0 and many:
-        steps_fwd *= 1.2
-    return (many and S % 8 != 0) or fwd < steps_fwd, (many and (S % 8 != 0 or L % 8 != 0)) or bwd < steps_bwd
+    # ragged rows of weights: a walk over queries waits for guarded loads, the products' logits take an element at a time
+    ragged = S % 8 != 0
+    bwd = (8 + (0.35 + 0.0031 * f) * max(keys, mean_keys * groups_q / 256) / 32 +
+           (0.5 + 0.0057 * f) * max((2.6 if ragged else 1) * max(L, 32), (max(mean_queries, 64) + 64) * groups_k / 256) / 32)
+    rows = 3.7e-6 * f * max(L, S) * heads
+    if ragged:
+        steps_bwd = max(41, 15 + 0.07 * keys + 0.034 * L + max(2.65e-5 * logits, rows))
+    else:
+        steps_bwd = max(34, 15 + 0.0105 * keys + 0.019 * L + max(1.7e-6 * logits, rows), 2.7e-6 * logits)
+    return (ragged and min(L, S) >= 32) or fwd < steps_fwd, bwd < steps_bwd
 
 
 def _permute_leading3(a: DeviceArray, perm) -> DeviceArray:

@@ -31,6 +31,9 @@ ROUTES = [
     (64, 64, 32, 32, 1, 4096, 1, False, False, False), (128, 128, 8, 2, 16, 2048, 1, False, False, False), (64, 64, 4, 4, 8, 1024, 1, False, False, True),
     (128, 128, 1, 1, 1024, 16, 2, False, True, False), (128, 64, 4, 2, 1024, 128, 1, True, True, False), (96, 96, 2, 2, 512, 512, 1, True, True, False),
     (64, 64, 2, 2, 1, 512, 1, False, True, True), (64, 64, 2, 1, 33, 1031, 1, False, True, True), (64, 64, 8, 8, 64, 2048, 1, True, True, True),
+    # ragged tokens: many queries on few keys, the reverse, and either side of the pullback's line
+    (96, 96, 2, 2, 2047, 47, 1, False, True, False), (128, 128, 4, 2, 1605, 52, 1, True, True, False), (64, 64, 1, 1, 635, 3072, 1, False, False, False),
+    (64, 64, 2, 2, 1023, 130, 1, False, True, False), (64, 64, 12, 12, 256, 111, 7, False, True, True),
 ]
 
 
