@@ -360,13 +360,13 @@ __global__ __launch_bounds__(THREADS, 2) void fwd_kernel(Args a) {
             });
         }
     }
-    // weight = exp2(c (z - top) + less), top = maximum, less = -log2(sum) (infinite where no key counts: the weights are NaN)
-    float top, less;
+    // weight = exp2(c (z - top)) inv, top = maximum, inv = 1 / sum (infinite where no key counts: the weights are NaN)
+    float top, inv;
     {
         const float mo = __shfl_xor(m, 32), so = __shfl_xor(sum, 32);
         const float mx = fmaxf(m, mo);
         top = mx == -INFINITY ? 0.0f : mx;
-        less = -__builtin_amdgcn_logf(sum * __builtin_amdgcn_exp2f((m - top) * a.c) + so * __builtin_amdgcn_exp2f((mo - top) * a.c));
+        inv = 1.0f / (sum * __builtin_amdgcn_exp2f((m - top) * a.c) + so * __builtin_amdgcn_exp2f((mo - top) * a.c));
     }
 
     // sweep 2: the weights, rounded, to memory and into the product with v
@@ -416,7 +416,7 @@ __global__ __launch_bounds__(THREADS, 2) void fwd_kernel(Args a) {
                         for (int e = 0; e < ET; ++e) vf[n][e] = ft.get(lds + (2 + u) * TILE, 16 * n, e);
                     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-                    for (int i = 0; i < 16; ++i) z[i] = __builtin_amdgcn_exp2f(fmaf(z[i] - top, a.c, less));
+                    for (int i = 0; i < 16; ++i) z[i] = __builtin_amdgcn_exp2f((z[i] - top) * a.c) * inv;
 #pragma unroll
                     for (int n = 0; n < 2; ++n) {
                         const raw16_t pw = pack8(z, n);
@@ -447,11 +447,11 @@ __global__ __launch_bounds__(THREADS, 2) void fwd_kernel(Args a) {
                     *reinterpret_cast<float4*>(a.out_wide + orow + e) = make_float4(o[t][4 * g], o[t][4 * g + 1], o[t][4 * g + 2], o[t][4 * g + 3]);
             }
     }
-    // the masked part of the columns, last: nothing waits for these stores.  0, or NaN where log2(sum) is no number.
+    // the masked part of the columns, last: nothing waits for these stores.  0, or NaN where 1 / sum is no number.
     const int rows = min(32, a.L - wl0);
     if (w_end < a.S) {
         for (int i = 0; i < rows; ++i) {
-            const float l0 = __shfl(less, i), z0 = l0 - l0;
+            const float z0 = 0.0f * __shfl(inv, i);
             const uint32_t zz = f32x2_to_bf16x2(z0, z0);
             const raw16_t zw = {zz, zz, zz, zz};
             for (int s = w_end + 8 * lane; s < a.S; s += 512) store8(wrow0 + (int64_t)i * a.S, s, a.S, zw);
