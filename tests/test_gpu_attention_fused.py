@@ -158,3 +158,49 @@ def test_negative_and_zero_scale(gpu, scale):
                                                    stored=lambda a: f64(O.round_to_bf16(np.asarray(a, np.float32))))
     for g, x, name in zip(grads, want, ("dq", "dk", "dv")):
         assert_close(g.to_numpy(), x, "bf16", name, scale=1e-3)
+
+
+@pytest.mark.parametrize("E,size", [(64, 1.0), (96, 1.0), (64, 0.25)])
+def test_weights_carry_the_errors_of_fp32_and_no_more(gpu, E, size):
+    """How many weights round to another bf16 number than their exact values: an error of r (relative) moves a value of mantissa f in
+    [1, 2) past a boundary with probability r f 2^7, 185 r in the mean.  Exponents up to 8 are off by 2^-22 at most, 9.5e-8 of a weight in the root
+    mean square; exp2, the reciprocal of the sum, the sum and the product are half a unit in the last place each (3.4e-8).  1.2e-7
+    together, 9.5e-8 in the mean of the absolute values: 1.8e-5 of the weights; half as many again are allowed."""
+    H, T = 12, 745
+    rng = np.random.default_rng(stable_seed("attn-fused-fp32", E, size))
+    q, k, v = host_inputs("bf16", *(rng.normal(size=(E, H, T, 1)) * s for s in (size, 1, 1)))
+    d = lambda a: dev(gpu, a, "bf16")
+    out = []
+    assert "attn_fwd_kernel" in kernels_of(gpu, lambda: out.append(gpu.scaled_dot_product_attention(d(q), d(k), d(v))))
+    got = f64(out[0][1].to_numpy())[:, :, :, 0]                                     # keys, queries, heads
+    off = 0
+    for h in range(H):
+        z = f64(k[:, h, :, 0]).T @ f64(q[:, h, :, 0]) / np.sqrt(E)
+        w = np.exp(z - z.max(axis=0))
+        m, e = np.frexp(w / w.sum(axis=0))
+        off += np.count_nonzero(got[:, :, h] != np.ldexp(np.rint(m * 256), e - 8))
+    assert off <= 1.5 * 1.8e-5 * H * T * T
+
+
+@pytest.mark.parametrize("causal", [False, True])
+def test_columns_of_every_size_beside_each_other(gpu, causal):
+    """Logits from 2^-6 to 2^24 in the lanes of one wave, whose maxima grow from tile to tile or lie in the first or the last one: sums change their
+    offsets, some columns' because of others'.  Operands of few bits make the logits exact in fp32."""
+    E, H, L, S = 64, 16, 130, 200
+    rng = np.random.default_rng(stable_seed("attn-fused-offsets", causal))
+    q = rng.integers(-2, 3, size=(E, H, L, 1)) * 2.0 ** rng.integers(-6, 21, size=(1, H, L, 1))
+    k = rng.integers(-3, 4, size=(E, H, S, 1)).astype(np.float64)
+    ramp = 1.0 + np.arange(S) // 20                                  # up to 10: four bits
+    for h in range(H):
+        k[:, h, :, 0] = k[:, h, [0], 0] * (ramp, ramp[::-1], -ramp, 1.0 + 0 * ramp)[h % 4] if h % 8 < 4 else k[:, h, :, 0]
+    d = lambda a: dev(gpu, a.astype(np.float32), "bf16")
+    out = []
+    assert "attn_fwd_kernel" in kernels_of(gpu, lambda: out.append(gpu.scaled_dot_product_attention(d(q), d(k), d(k), 1, 3, None, None, True if causal else None)))
+    got = out[0][1].to_numpy()
+    for h in range(H):
+        z = k[:, h, :, 0].T @ q[:, h, :, 0] / 8.0
+        if causal:
+            z = np.where(np.arange(S)[:, None] <= np.arange(L)[None, :], z, -np.inf)
+        w = np.exp(z - z.max(axis=0))
+        # exponents of 150 at most count, rounded once: 2^-17 of a weight
+        np.testing.assert_allclose(got[:, :, h, 0], w / w.sum(axis=0), rtol=2.0 ** -8 + 2.0 ** -16, atol=1e-36)
