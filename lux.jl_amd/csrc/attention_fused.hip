@@ -489,14 +489,14 @@ __global__ __launch_bounds__(THREADS, 2) void fwd_kernel(Args a) {
 }
 
 // ------------------------------------------------------------------------------------------------ pullback
-// weights .* (scale dP - scale d) of 16 rows, as the B operand of the next product: pw as loaded (bf16 pairs in accumulator
-// order), sd = scale d of each row
-__device__ __forceinline__ raw16_t softmax_rule(raw16_t pw, const f32x16_v& dp, int n, const float (&sd)[8], float scale) {
+// scale weights .* (dP - d) of 16 rows, as the B operand of the next product: pw as loaded (bf16 pairs in accumulator
+// order), d of each row.  The difference first: it may cancel, and fma(dP, scale, -scale d), an instruction less, leaves the rounding of scale d.
+__device__ __forceinline__ raw16_t softmax_rule(raw16_t pw, const f32x16_v& dp, int n, const float (&d)[8], float scale) {
     raw16_t out;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
         const float p0 = __uint_as_float(pw[i] << 16), p1 = __uint_as_float(pw[i] & 0xffff0000u);
-        out[i] = f32x2_to_bf16x2(p0 * fmaf(dp[8 * n + 2 * i], scale, -sd[2 * i]), p1 * fmaf(dp[8 * n + 2 * i + 1], scale, -sd[2 * i + 1]));
+        out[i] = f32x2_to_bf16x2(scale * p0 * (dp[8 * n + 2 * i] - d[2 * i]), scale * p1 * (dp[8 * n + 2 * i + 1] - d[2 * i + 1]));
     }
     return out;
 }
@@ -540,8 +540,9 @@ __global__ __launch_bounds__(THREADS, 2) void dq_kernel(Args a) {
     bf16x8_v df[2 * ET];
     load_columns<ET>(df, a.d_out + ((int64_t)wh.b * a.L * a.H + wh.h) * a.Ev, (uint32_t)(a.H * a.Ev * 2), l, a.L, a.Ev);
     // d = sum over the features of d_out .* out, half of them in each of a query's two lanes
-    float dl = 0.0f;
+    float dl;
     {
+        float part[8] = {};                             // a long chain of additions would round as often
         const float* orow = a.out_wide + (((int64_t)wh.b * a.L + lc) * a.H + wh.h) * a.Ev;
 #pragma unroll
         for (int kk = 0; kk < 2 * ET; ++kk) {
@@ -553,13 +554,14 @@ __global__ __launch_bounds__(THREADS, 2) void dq_kernel(Args a) {
             Vec<bf16_t>::unpack(__builtin_bit_cast(raw16_t, df[kk]), dv);
             if (e < a.Ev) {
 #pragma unroll
-                for (int i = 0; i < 8; ++i) dl = fmaf(dv[i], ov[i], dl);
+                for (int i = 0; i < 8; ++i) part[i] = fmaf(dv[i], ov[i], part[i]);
             }
         }
+        dl = ((part[0] + part[1]) + (part[2] + part[3])) + ((part[4] + part[5]) + (part[6] + part[7]));
         dl += __shfl_xor(dl, 32);
         if (h == 0 && l < a.L) a.dsum[(int64_t)wh.head * a.L + l] = dl;
     }
-    const float sd = a.scale * dl, dd[8] = {sd, sd, sd, sd, sd, sd, sd, sd};
+    const float dd[8] = {dl, dl, dl, dl, dl, dl, dl, dl};
     f32x16_v acc[ET];
 #pragma unroll
     for (int t = 0; t < ET; ++t) acc[t] = zero16();
@@ -650,7 +652,7 @@ __global__ __launch_bounds__(THREADS, 2) void dkv_kernel(Args a) {
             *reinterpret_cast<raw16_t*>(lds + (4 + b) * TILE + (prow + 16 * i) * PITCH + pch * 16) = in ? pw[b][i] : zero;
         }
         // 0 past the end: a non-finite d must not reach the keys through absent queries
-        if (threadIdx.x < ROWS) dt[b * ROWS + threadIdx.x] = t * ROWS + (int)threadIdx.x < a.L ? a.scale * dv[b] : 0.0f;
+        if (threadIdx.x < ROWS) dt[b * ROWS + threadIdx.x] = t * ROWS + (int)threadIdx.x < a.L ? dv[b] : 0.0f;
     };
     tq.load(0);
     to.load(0);

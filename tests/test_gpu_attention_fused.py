@@ -204,3 +204,19 @@ def test_columns_of_every_size_beside_each_other(gpu, causal):
         w = np.exp(z - z.max(axis=0))
         # exponents of 150 at most count, rounded once: 2^-17 of a weight
         np.testing.assert_allclose(got[:, :, h, 0], w / w.sum(axis=0), rtol=2.0 ** -8 + 2.0 ** -16, atol=1e-36)
+
+
+@pytest.mark.parametrize("E", [24, 96, 128])
+def test_gradients_that_cancel_are_zero(gpu, E):
+    """Equal values for all keys: the cotangents of the weights are all their mean, so dq and dk are 0.  Small integers make every sum exact, and a
+    weight of one or of a power of two, so they are exactly 0 where nothing else rounds (the scale is no power of two)."""
+    H, L, S = 4, 300, 64
+    rng = np.random.default_rng(stable_seed("attn-fused-cancel", E))
+    q, v, d_out = (rng.integers(-4, 5, size=(E, H, t, 1)).astype(np.float64) for t in (L, 1, L))
+    k = np.ones((E, H, S, 1))                                        # equal logits: 64 weights of 1 / 64
+    d = lambda a: dev(gpu, a.astype(np.float32), "bf16")
+    _, back = gpu.pullback(gpu.scaled_dot_product_attention, d(q), d(k), d(np.repeat(v, S, axis=2)), 1, 3)
+    grads = []
+    assert "attn_dq_kernel" in kernels_of(gpu, lambda: grads.extend(back(d(d_out))))
+    assert not grads[0].to_numpy().any() and not grads[1].to_numpy().any()
+    np.testing.assert_allclose(grads[2].to_numpy(), np.broadcast_to(d_out.sum(axis=2, keepdims=True) / S, (E, H, S, 1)), rtol=2.0 ** -8)
