@@ -719,7 +719,8 @@ struct GemmMainloop {
     __device__ __forceinline__ static void run(LoaderA& la, LoaderB& lb, int K, T* lds, f32x16_v (&acc)[WM][WN]) {
         static_assert(LoaderA::KMAJOR == A_KMAJOR && LoaderB::KMAJOR == B_KMAJOR, "loader layout mismatch");
         if constexpr (SPLIT_F32) {
-            if (__syncthreads_and(run_as<true>(la, lb, K, lds, acc))) return;
+            // (one term: the fp32 instruction rounds it once, the sum of its parts would be rounded twice)
+            if (K > 1 && __syncthreads_and(run_as<true>(la, lb, K, lds, acc))) return;
         }
         run_as<false>(la, lb, K, lds, acc);
     }

@@ -38,6 +38,14 @@ def test_error_is_that_of_fp32(gpu, size):
     assert np.linalg.norm(err) <= (2.0 ** -23 * np.sqrt(K / 6) + 2.0 ** -26) * np.linalg.norm(want)
 
 
+@pytest.mark.parametrize("M,N", [(2048, 2048), (1921, 2047)])
+def test_an_outer_product_is_rounded_once(gpu, M, N):
+    """Whole and ragged 128 x 128 tiles."""
+    rng = np.random.default_rng(stable_seed("split-outer", M))
+    w, x = rng.normal(size=(M, 1)).astype(np.float32), rng.normal(size=(1, N)).astype(np.float32)
+    np.testing.assert_array_equal(product(gpu, w, x), w * x)
+
+
 @pytest.mark.parametrize("size", range(len(SIZES)))
 def test_values_without_parts(gpu, size):
     M, N, K, kernel = SIZES[size]
