@@ -145,7 +145,7 @@ struct Core {
     // k range [kbeg, kend)
     __device__ __forceinline__ static void run(const LA& la, const LB& lb, int kbeg, int kend, T* lds, f32x16_v (&acc)[WM][WN]) {
         if constexpr (ML::SPLIT_F32) {
-            if (kend > kbeg + 1 && __syncthreads_and(run_as<true>(la, lb, kbeg, kend, lds, acc))) return;      // one term: see GemmMainloop::run
+            if (__syncthreads_and(run_as<true>(la, lb, kbeg, kend, lds, acc))) return;
         }
         run_as<false>(la, lb, kbeg, kend, lds, acc);
     }
