@@ -12,8 +12,8 @@
 // everything else is arranged to hide behind that stream.  Two sweeps over the keys (column maxima and sums, then weights
 // and output) cost a second product k'q but no traffic.  The pullback forms v' d_out twice, once per sweep (over queries
 // for dk, dv; over keys for dq), because handing dS from one to the other would write and read it.
-// Measured at 128 x 2048 x 32 x 4, causal (step-by-step path before): forward 1.15 ms -> 0.48 ms, pullback 0.85 ms -> 0.59 ms
-// (dq 0.285, dk and dv 0.305; without the loads and stores of the weights 0.32, 0.21 and 0.26).
+// Measured at 128 x 2048 x 32 x 4, causal (step-by-step path before): forward 1.15 ms -> 0.46 ms, pullback 0.85 ms -> 0.56 ms
+// (dq 0.28, dk and dv 0.28; without the loads and stores of the weights 0.32, 0.21 and 0.26 of 0.48, 0.285 and 0.305).
 //
 // Layout of the work: a workgroup is four waves; a wave owns 32 columns (queries in the forward and dq kernels, keys in the
 // dk / dv kernel) and walks the other dimension.  Every product is v_mfma_f32_32x32x16_bf16 with the walked dimension (or

@@ -247,7 +247,7 @@ __global__ __launch_bounds__(256) void pad_to_cwhn_pack_kernel(const T* __restri
 // The first layer of an image network (bf16, at most four channels, a window of 5 to 8 positions along w): x is copied with four
 // channels per position and the rows' padding in place, so that the positions of a window in one source row are one run of at
 // most 32 elements.  A stage of the contraction is such a run: kH stages instead of kW kH / 4 over channels padded to eight (7 x 7:
-// 224 against 392; 224 x 224 x 3 x 32 -> 64 channels at stride 2: output 66 -> 58 us, filter gradient 78 -> 47, each copy of x 12.5 -> 7).
+// 224 against 392; 224 x 224 x 3 x 32 -> 64 channels at stride 2: output 66 -> 53 us, filter gradient 75 -> 42, each copy of x 12 -> 7).
 struct Runs {
     int W2 = 0;                // positions of a copied row, even; 0: not this kind of layer
     static constexpr int EL = 32;
@@ -594,7 +594,7 @@ static bool window_shape(const ConvGeom& g, bool dgrad) {
 // The whole-tap kernels: channels per group in whole stages, for the input gradient a unit stride, and enough work to fill
 // the chip with their large tiles.  Below that the kernels of conv_any.h are ahead: bf16 5 x 5, 192 -> 16 channels on 25 x 25
 // x 18 107 us against 33, fp32 5 x 5, 208 -> 40 on 66 x 66 x 4 417 against 162; with the chip full they are not: bf16 3 x 3,
-// 128 channels on 56 x 56 x 64 63 us (window kernel) against 132, fp32 541 against 550.
+// 128 channels on 56 x 56 x 64 63 us (window kernel) against 132, fp32 541 against 550 (both on the fp32 instruction then).
 template <typename T>
 static bool tap_shape(const ConvGeom& g, bool dgrad) {
     const int Cg = dgrad ? g.Cout_g : g.Cin_g, Ncols = dgrad ? g.Cin_g : g.Cout_g;

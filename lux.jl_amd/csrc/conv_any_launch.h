@@ -8,7 +8,8 @@ namespace cany {
 
 // Cost of one k of a tile in us: with the compute unit to itself (latency), and of a full compute unit's time.  Fitted to
 // forced launches of 24 problems (M from 196 to 400000 rows, 16 to 208 columns, K from 16 to 5200); a tile's prologue and
-// epilogue count as another 100 k.
+// epilogue count as another 100 k.  (fp32 128 x 128: of the fp32 instruction, on which the other fp32 tiles still are.  In three bf16 parts
+// those take about 0.65 of it, so that sizes near the line go to smaller tiles that no longer are the faster ones.)
 struct Tile { int m, n; double alone, shared; };
 template <typename T>
 inline const Tile* tiles() {

@@ -108,8 +108,8 @@ __host__ __device__ constexpr int mn_swizzle_shift(int rows) { return rows >= 12
 // 7 % slower than the fp32 instruction; 128 x 64 and 256 x 32 (two) win up to 4 % where the contraction is long and lose up to
 // 11 % where it is short (3 x 3 windows of 16 channels, 64 columns, 280000 rows: 102 us, 91 on the fp32 instruction).  Four
 // accumulators take 128 registers with the smaller partial products, and the compiler would go on to give the kernel all 512:
-// split_waves is the launch bound that keeps two waves on a SIMD (59.2 GFLOP of a 3 x 3 convolution: 545 us with one wave, 371
-// with two, 531 on the fp32 instruction).
+// split_waves is the launch bound that keeps two waves on a SIMD (58 GFLOP of a 3 x 3 convolution: 0.68 of the time with one wave;
+// 311 to 332 us, 512 on the fp32 instruction).
 template <typename T, int WM, int WN>
 __host__ __device__ constexpr bool split_f32() { return sizeof(T) == 4 && WM * WN == 4; }
 template <typename T, int WM, int WN>

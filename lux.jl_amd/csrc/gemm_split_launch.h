@@ -11,7 +11,8 @@ struct Choice { int w, slices; };
 // Time of a product in microseconds with tiles of 64 w and `slices` slices: one k of a tile costs `alone` ns when the
 // workgroup has its compute unit to itself (the latency of a stage) and `shared` ns of the compute unit's time when it is
 // full; a hand-off costs a round trip, a trip per slice for the workgroup that adds them, and the partial sums' bytes.
-// The constants are fitted to sweeps over tile, slices and sizes from 256 x 64 x 128 to 3651 x 2048 x 1350.
+// The constants are fitted to sweeps over tile, slices and sizes from 256 x 64 x 128 to 3651 x 2048 x 1350, in fp32 on the fp32
+// instruction: w = 2 computes in three bf16 parts since and is faster than these say (2048^3 0.71 of the time).
 template <typename T>
 double estimate(int w, int slices, int64_t M, int64_t N, int64_t K) {
     const int64_t cus = num_cus() > 0 ? num_cus() : 256;
@@ -100,7 +101,7 @@ extern template int launch_layouts<float, 2>(hipStream_t, DenseArgs<float>&, boo
 // (us, big tiles against these: 1920 x 2048 x 2048 27.4 / 36.3, 1280 x 2048 x 4096 46.9 / 62.0), with 128 they are not
 // (1024 x 2048 x 4096 45.5 / 41.9; 1024^3 13.3 / 9.2), nor where K is short (1536 x 2048 x 128 5.6 / 5.3 up to 192 tiles,
 // 1920 x 2048 x 128 6.0 / 6.6).  In fp32 the line lies between 192 tiles (1536 x 2048 x 1024 80.4 / 73.0) and 208
-// (1664 x 2048 x 1024 81.3 / 88.1).  Aligned operands of less than a tile in one dimension and many tiles in the other are
+// (1664 x 2048 x 1024 81.3 / 88.1; both sides before 128 x 128 tiles took to three bf16 parts).  Aligned operands of less than a tile in one dimension and many tiles in the other are
 // streamed by the big-tile kernels as well while K is short (fp32 1000000 x 9 x 100 178.9 / 193.1, bf16 300000 x 9 x 32
 // 14.2 / 15.8; but 24 x 200000 x 512 38.7 / 33.8).
 template <typename T>
