@@ -6,7 +6,8 @@
 
 namespace luxhip {
 
-template <typename T, int ACT, int VEC>
+// RAGGED: any alignment (common.h, row_load)
+template <typename T, int ACT, int VEC, bool RAGGED = false>
 __device__ __forceinline__ void dx_vec(const T* delta, const T* out, const T* pre, size_t off, float (&dx)[VEC]) {
     float d[VEC], o[VEC], p[VEC];
     if constexpr (VEC == 1) {
@@ -14,9 +15,9 @@ __device__ __forceinline__ void dx_vec(const T* delta, const T* out, const T* pr
         if constexpr (ACT != LUXHIP_ACT_IDENTITY && !Act<ACT>::needs_pre) o[0] = ld(out + off);
         if constexpr (Act<ACT>::needs_pre) p[0] = ld(pre + off);
     } else {
-        Vec<T>::load(delta + off, d);
-        if constexpr (ACT != LUXHIP_ACT_IDENTITY && !Act<ACT>::needs_pre) Vec<T>::load(out + off, o);
-        if constexpr (Act<ACT>::needs_pre) Vec<T>::load(pre + off, p);
+        row_load<T, VEC, RAGGED>(delta, off, d);
+        if constexpr (ACT != LUXHIP_ACT_IDENTITY && !Act<ACT>::needs_pre) row_load<T, VEC, RAGGED>(out, off, o);
+        if constexpr (Act<ACT>::needs_pre) row_load<T, VEC, RAGGED>(pre, off, p);
     }
 #pragma unroll
     for (int k = 0; k < VEC; ++k) {

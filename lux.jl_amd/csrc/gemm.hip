@@ -5,6 +5,7 @@
 #include <algorithm>
 
 #include "common.h"
+#include "gemm_copies.h"
 #include "gemm_dense_decl.h"
 
 namespace luxhip {
@@ -13,8 +14,9 @@ int bias_act_bwd_dispatch(hipStream_t s, int dtype, int act, int64_t I, int64_t 
                           const void* out, const void* pre, void* dx, void* dbias);   // elementwise.hip
 
 int transpose_matrix_bf16(hipStream_t s, const bf16_t* in, bf16_t* out, int64_t P, int64_t C);   // conv.hip
-int dense_dz_transposed(hipStream_t s, int act, int64_t M, int64_t N, const bf16_t* delta, const bf16_t* out, const bf16_t* pre,
-                        bf16_t* dz, bf16_t* dzT, float* partial, bf16_t* dbias);                 // elementwise.hip
+int launch_kk256_sliced(hipStream_t s, DenseArgs<bf16_t>& a, int slices, float* partial);   // gemm_inst_bf16_kk.hip
+size_t kk256_partial_bytes(int64_t M, int64_t N, int slices);
+double split_time_bf16(int64_t M, int64_t N, int64_t K);                                    // gemm_split_bf16.hip
 
 int gemm_tile_override() { return (int)option_gemm_tile(); }
 static inline size_t align256(size_t b) { return (b + 255) & ~size_t(255); }
@@ -48,6 +50,109 @@ static DenseArgs<T> dense_args(bool a_kmajor, bool b_kmajor, int64_t M, int64_t 
     a.C = C; a.ldc = ldc; a.bias = bias; a.pre = pre; a.act = act;
     a.c_vec = (reinterpret_cast<uintptr_t>(C) & 7u) == 0 && (reinterpret_cast<uintptr_t>(pre) & 7u) == 0 && ldc % 4 == 0;
     return a;
+}
+
+// ------------------------------------------------------------------------------- ragged products on the 256 x 256 kernel
+// An operand of a large bf16 product as the caller has it, or (`ready`) as the kernel reads it: k contiguous, rows of whole steps.
+struct Side {
+    const bf16_t* p;
+    int64_t ld, rows;
+    bool kmajor, ready;
+};
+static Side side(const bf16_t* p, int64_t ld, int64_t rows, bool kmajor, int64_t K) {
+    return Side{p, ld, rows, kmajor, kmajor && K % 64 == 0 && ld % 8 == 0 && aligned16(p)};
+}
+static int64_t whole_steps(int64_t K) { return ceil_div(K, 64) * 64; }
+static size_t copy_bytes(const Side& a, int64_t K) { return a.ready ? 0 : align256((size_t)a.rows * whole_steps(K) * sizeof(bf16_t)); }
+
+// Time of the 256 x 256 kernel with its copies, in microseconds: a k of a tile takes 17 ns where few compute units work and 23 where all do
+// (the clock and the caches), a round of tiles 7 us for its ends, slices a pass over 256 KiB of partial sums each, a copy a launch
+// and its bytes.  Fitted to 171 products of 256 to 12288 in every dimension and layout with 1 to 8 slices (9 % rms).
+static double big_time(int64_t M, int64_t N, int64_t K, const Side& A, const Side& B, int slices) {
+    const int64_t cus = num_cus() > 0 ? num_cus() : 256, units = ceil_div(M, 256) * ceil_div(N, 256) * slices;
+    const double k_us = 16.6e-3 + 6.2e-3 * std::min(1.0, (double)units / (double)cus);
+    double t = 1.3 + (double)ceil_div(units, cus) * ((double)ceil_div(ceil_div(K, 64), slices) * 64.0 * k_us + 7.2);
+    if (slices > 1) t += 3.7 + 0.07 * (double)units;
+    for (const Side* o : {&A, &B})
+        if (!o->ready) t += 3.5 + (double)o->rows * (double)whole_steps(K) * 4.0 / 5e6;
+    return t;
+}
+
+// Slices of the contraction (1: whole) if the product goes to the 256 x 256 kernel, else 0.  It goes there where the two estimates say that it is faster so than
+// on the kernels that load at any alignment (gemm_split.h), whose k of a 128 x 128 tile takes 12.5 ns of a compute unit: 50 for the 256 x 256
+// that take 23 here.  Of the 171 products none was slower for it; on either side of the line (us, there / here): 3135 x 6144 x 745 59 / 58,
+// 2449 x 1304 x 1216 26 / 38, 1629 x 3835 x 9408 243 / 139 in two slices, 2368 x 11200 x 6400 499 / 355.  Whole aligned tiles of 256 that fill the chip
+// have their own rule (pretranspose_pays, launch_layout).
+static int ragged_slices(hipStream_t s, int64_t M, int64_t N, int64_t K, const Side& A, const Side& B, size_t front) {
+    if (option_gemm_pretranspose() == 0 || gemm_tile_override() != 0 || M < 256 || N < 256 || K < 128) return 0;
+    const int64_t Kp = whole_steps(K), tiles = ceil_div(M, 256) * ceil_div(N, 256), chunk_limit = (int64_t(1) << 31) - 2048;
+    if (256 * Kp * 2 >= (int64_t(1) << 31) || tiles >= (int64_t(1) << 27) || M * (Kp / 8) >= chunk_limit || N * (Kp / 8) >= chunk_limit ||
+        (M + 8) * N >= (int64_t(1) << 33) || ceil_div(K, 64) > 65535) return 0;
+    const bool whole = M % 256 == 0 && N % 256 == 0 && K % 32 == 0 && aligned16(A.p) && A.ld % 8 == 0 && aligned16(B.p) && B.ld % 8 == 0;
+    if (whole && tiles >= 128) return 0;
+    int best = 0;
+    // 3: the launch, which this estimate counts; less what the two may be wrong by (1664 x 576 x 6400 in eight slices: 0.94 by the estimates, and slower)
+    const double there = split_time_bf16(M, N, K) + 3.0;
+    double t_best = 1e30;
+    for (int slices = 1; slices <= 8 && slices <= Kp / 128; ++slices) {
+        const double t = big_time(M, N, K, A, B, slices);
+        if (t < t_best && t < (slices == 1 ? 0.97 : 0.93) * there) { t_best = t; best = slices; }
+    }
+    if (best > 0 && !workspace_holds(s, front + copy_bytes(A, K) + copy_bytes(B, K) + kk256_partial_bytes(M, N, best))) return 0;
+    return best;
+}
+
+// C = act(A B + bias) on the 256 x 256 kernel; copies of the operands that are not ready go to the workspace behind `front` bytes, the
+// partial sums of the slices behind them
+static int ragged_product(hipStream_t s, int64_t M, int64_t N, int64_t K, Side A, Side B, const bf16_t* bias, bf16_t* C, int64_t ldc, bf16_t* pre,
+                          int act, int slices, size_t front = 0) {
+    const int64_t Kp = whole_steps(K);
+    const size_t bytes = copy_bytes(A, K) + copy_bytes(B, K) + kk256_partial_bytes(M, N, slices);
+    float* partial = nullptr;
+    if (bytes > 0) {
+        Workspace ws;
+        int rc = get_workspace(s, front + bytes, &ws);
+        if (rc != LUXHIP_OK) return rc;
+        char* at = ws.data + front;
+        for (Side* o : {&A, &B}) {
+            if (o->ready) continue;
+            bf16_t* copy = reinterpret_cast<bf16_t*>(at);
+            at += copy_bytes(*o, K);
+            rc = o->kmajor ? kmajor_rows(s, o->p, o->ld, o->rows, K, copy, Kp) : kmajor_transposed(s, o->p, o->ld, o->rows, K, copy, Kp);
+            if (rc != LUXHIP_OK) return rc;
+            *o = Side{copy, Kp, o->rows, true, true};
+        }
+        partial = reinterpret_cast<float*>(at);
+    }
+    DenseArgs<bf16_t> a = dense_args<bf16_t>(true, true, M, N, Kp, A.p, A.ld, B.p, B.ld, bias, C, ldc, pre, act);
+    return launch_kk256_sliced(s, a, slices, partial);
+}
+
+// The pullback of a dense layer whose two gradient products both go to the 256 x 256 kernel: the pass over delta writes dz as both
+// of them read it, with the bias gradient's partial sums.  *done: false if it is a problem of other kernels (nothing was launched).
+static int ragged_gradients(hipStream_t s, int act, int64_t M, int64_t K, int64_t N, const bf16_t* delta, const bf16_t* y, const bf16_t* pre,
+                            const bf16_t* W, int64_t ldw, const bf16_t* x, int64_t ldx, bf16_t* dz, bf16_t* dW, bf16_t* dx, bf16_t* dbias, bool* done) {
+    *done = false;
+    if (ldw < M || ldx < K || M < 1 || N < 1) return LUXHIP_OK;
+    const int64_t Mp = whole_steps(M), Np = whole_steps(N);
+    const bf16_t* dz_dense = act == LUXHIP_ACT_IDENTITY ? delta : dz;
+    const bool padded = M % 64 != 0 || !aligned16(dz_dense);            // dz goes to the workspace, in rows of whole steps
+    const size_t zb = padded ? align256((size_t)N * Mp * 2) : 0, tb = align256((size_t)M * Np * 2);
+    const size_t pb = dbias != nullptr ? align256((size_t)ceil_div(N, 64) * M * sizeof(float)) : 0, front = zb + tb + pb;
+    const Side dzT{nullptr, Np, M, true, true}, sx = side(x, ldx, K, false, N), sw = side(W, ldw, K, true, M), dzN{nullptr, Mp, N, true, true};
+    const int slices_w = ragged_slices(s, M, K, N, dzT, sx, front), slices_x = ragged_slices(s, K, N, M, sw, dzN, front);
+    if (slices_w == 0 || slices_x == 0) return LUXHIP_OK;
+    *done = true;
+    Workspace ws;
+    int rc = get_workspace(s, front + std::max(copy_bytes(sx, N) + kk256_partial_bytes(M, K, slices_w), copy_bytes(sw, M) + kk256_partial_bytes(K, N, slices_x)), &ws);
+    if (rc != LUXHIP_OK) return rc;
+    bf16_t* const out = padded ? reinterpret_cast<bf16_t*>(ws.data) : act == LUXHIP_ACT_IDENTITY ? nullptr : dz;
+    bf16_t* const outT = reinterpret_cast<bf16_t*>(ws.data + zb);
+    rc = dense_dz_kmajor(s, act, M, N, delta, y, pre, out, padded ? Mp : M, outT, Np, reinterpret_cast<float*>(ws.data + zb + tb), dbias);
+    if (rc != LUXHIP_OK) return rc;
+    rc = ragged_product(s, M, K, N, Side{outT, Np, M, true, true}, sx, nullptr, dW, M, nullptr, LUXHIP_ACT_IDENTITY, slices_w, front);
+    if (rc != LUXHIP_OK) return rc;
+    return ragged_product(s, K, N, M, sw, Side{padded ? out : dz_dense, padded ? Mp : M, N, true, true}, nullptr, dx, K, nullptr, LUXHIP_ACT_IDENTITY, slices_x, front);
 }
 
 // dW (M x K) = dz (M x N) * x' and dx (K x N) = W' * dz in one launch; false if they are not small enough for it
@@ -98,8 +203,13 @@ static int gemm_impl(hipStream_t s, int transA, int transB, int64_t M, int64_t N
         }
     }
     DenseArgs<T> a = dense_args<T>(a_kmajor, b_kmajor, M, N, K, A, lda, B, ldb, bias, C, ldc, pre, act);
-    if (gemm_tile_override() == 0 && !copied && ws_front == 0) {       // the workspace that these two use is free
+    if (gemm_tile_override() == 0 && !copied && ws_front == 0) {       // the workspace that these use is free
         int rc = LUXHIP_OK;
+        if constexpr (sizeof(T) == 2) {
+            const Side sa = side(A, lda, M, a_kmajor, K), sb = side(B, ldb, N, b_kmajor, K);
+            const int slices = ragged_slices(s, M, N, K, sa, sb, 0);
+            if (slices > 0) return ragged_product(s, M, N, K, sa, sb, bias, C, ldc, pre, act, slices);
+        }
         if (launch_skinny<T>(s, a, a_kmajor, b_kmajor, &rc)) return rc;
         if (launch_split<T>(s, a, a_kmajor, b_kmajor, &rc)) return rc;
     }
@@ -435,8 +545,8 @@ int luxhip_fused_dense_bwd(luxhip_stream_t s, int dtype, int act, int64_t M, int
         if (rc != LUXHIP_OK) return rc;
         bf16_t* dzT = reinterpret_cast<bf16_t*>(ws.data);
         void* dz_out = act == LUXHIP_ACT_IDENTITY ? nullptr : dz;
-        rc = dense_dz_transposed((hipStream_t)s, act, M, N, (const bf16_t*)delta, (const bf16_t*)y, (const bf16_t*)pre, (bf16_t*)dz_out,
-                                 dzT, reinterpret_cast<float*>(ws.data + tb), (bf16_t*)dbias);
+        rc = dense_dz_kmajor((hipStream_t)s, act, M, N, (const bf16_t*)delta, (const bf16_t*)y, (const bf16_t*)pre, (bf16_t*)dz_out, M, dzT, N,
+                             reinterpret_cast<float*>(ws.data + tb), (bf16_t*)dbias);
         if (rc != LUXHIP_OK) return rc;
         if (dz_out) dzp = dz_out;
         // dW (M x K) = dz (M x N) * x' (N x K) with dz given as its transpose (N contiguous)
@@ -444,6 +554,12 @@ int luxhip_fused_dense_bwd(luxhip_stream_t s, int dtype, int act, int64_t M, int
                            LUXHIP_ACT_IDENTITY, tb + pb);
         if (rc != LUXHIP_OK) return rc;
     } else {
+    if (dtype == LUXHIP_BF16 && dW != nullptr && dx != nullptr && W != nullptr && x != nullptr && M * N < (int64_t(1) << 31)) {
+        bool done = false;
+        rc = ragged_gradients((hipStream_t)s, act, M, K, N, (const bf16_t*)delta, (const bf16_t*)y, (const bf16_t*)pre, (const bf16_t*)W, ldw,
+                              (const bf16_t*)x, ldx, (bf16_t*)dz, (bf16_t*)dW, (bf16_t*)dx, (bf16_t*)dbias, &done);
+        if (done) return rc;
+    }
     if (act != LUXHIP_ACT_IDENTITY || dbias != nullptr) {
         // dz = delta .* act'(y, pre) and dbias = sum over the batch, one pass (dense layout: I = 1)
         void* dz_out = act == LUXHIP_ACT_IDENTITY ? nullptr : dz;

@@ -500,16 +500,21 @@ __device__ __forceinline__ void mfma_stage_f32(const float* As, const float* Bs,
 // different XCDs, 8 of them, each with its own L2).  Ids are therefore first regrouped per XCD
 // and then walked in groups of 8 tiles along m, which keeps the operand rows and columns that
 // one L2 sees close together.
-__device__ __forceinline__ void tile_coords(int id, int tiles_m, int tiles_n, int& tm, int& tn) {
-    const int nb = tiles_m * tiles_n;
+// `id` of `nb` -> its position when every XCD has consecutive ones
+__device__ __forceinline__ int xcd_regroup(int id, int nb) {
     const int per = nb >> 3;
-    const int lid = id < (per << 3) ? (id & 7) * per + (id >> 3) : id;
+    return id < (per << 3) ? (id & 7) * per + (id >> 3) : id;
+}
+__device__ __forceinline__ void tile_walk(int lid, int tiles_m, int tiles_n, int& tm, int& tn) {
     constexpr int GROUP = 8;
     const int in_group = GROUP * tiles_n;
     const int first_m = (lid / in_group) * GROUP;
     const int gsize = min(tiles_m - first_m, GROUP);
     tm = first_m + (lid % in_group) % gsize;
     tn = (lid % in_group) / gsize;
+}
+__device__ __forceinline__ void tile_coords(int id, int tiles_m, int tiles_n, int& tm, int& tn) {
+    tile_walk(xcd_regroup(id, tiles_m * tiles_n), tiles_m, tiles_n, tm, tn);
 }
 
 // Workgroups of a persistent tile kernel: as many as stay resident at once, at most one per tile.

@@ -43,6 +43,10 @@ struct Args {
     bf16_t *C, *pre;
     int64_t lda, ldb, ldc;      // elements
     int K, act, tiles_m, tiles_n;
+    int m_last, n_last;         // where the last tile of a dimension starts: M - 256, N - 256
+    int slices;                 // SPLIT: of the contraction, every one at least two steps
+    float* partial;             // SPLIT: [slice][n][m], columns ldp apart
+    int64_t ldp, slice_stride;
 };
 
 // Keeps the compiler from hoisting everything derived from `v` out of the loops (it would hold one
@@ -89,7 +93,7 @@ __device__ __forceinline__ void epilogue_as(const f32x4_v (&acc)[SM][SN], const 
     const int nb = n0 + (w >> 1) * 64 + 4 * (l >> 4);
     float bv[SM];
     if (a.bias) {
-        Vec<bf16_t>::load(a.bias + mb, bv);
+        row_load<bf16_t, SM, true>(a.bias, mb, bv);
     } else {
 #pragma unroll
         for (int i = 0; i < SM; ++i) bv[i] = 0.0f;
@@ -101,10 +105,10 @@ __device__ __forceinline__ void epilogue_as(const f32x4_v (&acc)[SM][SN], const 
         float v[SM];
 #pragma unroll
         for (int i = 0; i < SM; ++i) v[i] = acc[i][j][r] + bv[i];
-        if constexpr (HAS_PRE) Vec<bf16_t>::store(a.pre + (int64_t)n * a.ldc + mb, v);
+        if constexpr (HAS_PRE) row_store<bf16_t, SM, true>(a.pre, (size_t)n * a.ldc + mb, v, 0);
         if constexpr (ACT_MODE == 1) act_vec_as<LUXHIP_ACT_RELU>(v);
         else if constexpr (ACT_MODE == 2) act_vec(act, v);
-        Vec<bf16_t>::store(a.C + (int64_t)n * a.ldc + mb, v);
+        row_store<bf16_t, SM, true>(a.C, (size_t)n * a.ldc + mb, v, 0);
     });
 }
 __device__ __forceinline__ void epilogue(const f32x4_v (&acc)[SM][SN], const Args& a, int m0, int n0) {
@@ -112,6 +116,21 @@ __device__ __forceinline__ void epilogue(const f32x4_v (&acc)[SM][SN], const Arg
     else if (a.act == LUXHIP_ACT_IDENTITY) epilogue_as<0, false>(acc, a, m0, n0);
     else if (a.act == LUXHIP_ACT_RELU) epilogue_as<1, false>(acc, a, m0, n0);
     else epilogue_as<2, false>(acc, a, m0, n0);
+}
+
+// A slice's sums as they are, for slices_reduce_kernel
+__device__ __forceinline__ void store_partial(const f32x4_v (&acc)[SM][SN], const Args& a, int slice, int m0, int n0) {
+    const int l = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const int mb = m0 + (w & 1) * 128 + 8 * (l & 15);
+    const int nb = n0 + (w >> 1) * 64 + 4 * (l >> 4);
+    float* const out = a.partial + (size_t)slice * a.slice_stride;
+    static_for<SN * 4>([&](auto JR) {
+        constexpr int j = decltype(JR)::value / 4, r = decltype(JR)::value % 4;
+        const size_t off = (size_t)(nb + 16 * j + r) * a.ldp + mb;
+        const float lo[4] = {acc[0][j][r], acc[1][j][r], acc[2][j][r], acc[3][j][r]}, hi[4] = {acc[4][j][r], acc[5][j][r], acc[6][j][r], acc[7][j][r]};
+        row_store<float, 4, true>(out, off, lo, 0);
+        row_store<float, 4, true>(out, off + 4, hi, 0);
+    });
 }
 
 // Persistent: workgroup b takes tiles b, b + gridDim.x, ...; the first blocks of the next tile are
@@ -125,23 +144,39 @@ __device__ __forceinline__ void epilogue(const f32x4_v (&acc)[SM][SN], const Arg
 //   columns (valid memory, a free slot, never read): no special cases for the tail.
 //   boundary, before the last k group: every wave's reads of step kt have returned and the blocks of step
 //   kt + 1 have landed (loads return in order: at most the four instructions of block 2 kt + 4 are left).
+//
+// SPLIT: the units of work are slices of tiles.  Those of one slice are neighbours on an XCD (they read the same k of the operands).  Their sums
+// go to memory for a pass of their own (slices_reduce_kernel): with the sums of a tile added by the workgroup that arrives last, 896 x 5924 x 6272
+// in two slices took 139 us, as long as whole (134); with the pass 94.
+template <bool SPLIT>
 __global__ __launch_bounds__(THREADS) void dense_gemm_kk256_kernel(Args a) {
     extern __shared__ __align__(16) unsigned char lds_raw[];
     char* lds = reinterpret_cast<char*>(lds_raw);
-    const int total = a.tiles_m * a.tiles_n;
+    const int tiles = a.tiles_m * a.tiles_n, total = SPLIT ? tiles * a.slices : tiles;
     const int w = threadIdx.x >> 6;
     const int wave_m = (w & 1) * 128, wave_n = (w >> 1) * 64;
-    const int KT = a.K / BK;
+    int KT = a.K / BK;                                         // steps of this unit
     const int64_t lda_b = a.lda * 2, ldb_b = a.ldb * 2;
-    const int klast = (KT - 1) * BK * 2;                       // byte offset of the last step's columns
 
-    int t = blockIdx.x, tm, tn;
-    tile_coords(t, a.tiles_m, a.tiles_n, tm, tn);
-    int m0 = tm * TILE, n0 = tn * TILE;
+    int t = blockIdx.x, tm, tn, slice = 0, k0b = 0;            // k0b: byte offset of the unit's first columns
+    auto locate = [&](int unit) {
+        if constexpr (SPLIT) {
+            const int lid = xcd_regroup(unit, total), steps = a.K / BK;
+            slice = lid / tiles;
+            tile_walk(lid - slice * tiles, a.tiles_m, a.tiles_n, tm, tn);
+            const int first = (int)((int64_t)steps * slice / a.slices), end = (int)((int64_t)steps * (slice + 1) / a.slices);
+            KT = end - first;
+            k0b = first * BK * 2;
+        } else {
+            tile_coords(unit, a.tiles_m, a.tiles_n, tm, tn);
+        }
+    };
+    locate(t);
+    int m0 = min(tm * TILE, a.m_last), n0 = min(tn * TILE, a.n_last);
     const BlockLoader<true> la(a.lda);
     const BlockLoader<false> lb(a.ldb);
-    const char* ga = reinterpret_cast<const char*>(a.A) + (int64_t)m0 * lda_b;      // uniform: the tile's rows, k = 0
-    const char* gb = reinterpret_cast<const char*>(a.B) + (int64_t)n0 * ldb_b;
+    const char* ga = reinterpret_cast<const char*>(a.A) + (int64_t)m0 * lda_b + k0b;      // uniform: the tile's rows, the unit's first k
+    const char* gb = reinterpret_cast<const char*>(a.B) + (int64_t)n0 * ldb_b + k0b;
     // blocks 0, 1, 2 and the first half of block 3 of the tile at (ga, gb)
     auto issue_prologue = [&]() {
 #pragma unroll
@@ -214,6 +249,8 @@ __global__ __launch_bounds__(THREADS) void dense_gemm_kk256_kernel(Args a) {
 #define KK256_FENCE() __builtin_amdgcn_sched_barrier(0)
         const int tnext = t + gridDim.x;
         int m0n = 0, n0n = 0;
+        const int steps = KT, slice_now = slice;
+        const int klast = (steps - 1) * BK * 2;                // byte offset of the last step's columns
         // ring slots (byte offsets) of the blocks of the current step and of those being loaded
         uint32_t sA = 0, sB = BLOCK_BYTES;                     // blocks 2 kt, 2 kt + 1
         auto next_slot = [](uint32_t s_, int by) {             // (slot + by) % RING in bytes, by < RING
@@ -223,7 +260,7 @@ __global__ __launch_bounds__(THREADS) void dense_gemm_kk256_kernel(Args a) {
         int k1 = 128, k2 = 256;                                // byte offsets of the columns of steps kt + 1, kt + 2
         reads_1(sA, sB, 0, 0);
         reads_2(sA, 0, 0);
-        for (int kt = 0; kt < KT; ++kt) {
+        for (int kt = 0; kt < steps; ++kt) {
             const int k1c = min(k1, klast), k2c = min(k2, klast);
             char* const d3 = lds + next_slot(sA, 3);           // block 2 kt + 3: B of step kt + 1
             char* const d4 = lds + next_slot(sA, 4);           // block 2 kt + 4: A of step kt + 2
@@ -245,7 +282,7 @@ __global__ __launch_bounds__(THREADS) void dense_gemm_kk256_kernel(Args a) {
             KK256_FENCE(); mfmas(1, 2); KK256_FENCE();
             // Boundary (the MFMAs stay outside every branch: accumulator tuples that differ between the arms
             // of a branch end up copied or spilled).
-            if (kt + 1 < KT) {
+            if (kt + 1 < steps) {
                 __builtin_amdgcn_s_waitcnt(4 | (0x7 << 4));     // vmcnt(4) lgkmcnt(0)
                 __builtin_amdgcn_s_barrier();
                 // block 2 kt + 5 (B of step kt + 2) takes the slot of the A block just released
@@ -263,11 +300,11 @@ __global__ __launch_bounds__(THREADS) void dense_gemm_kk256_kernel(Args a) {
                 __builtin_amdgcn_s_waitcnt(0 | (0x7 << 4));     // vmcnt(0) lgkmcnt(0)
                 __builtin_amdgcn_s_barrier();
                 if (tnext < total) {
-                    tile_coords(tnext, a.tiles_m, a.tiles_n, tm, tn);
-                    m0n = tm * TILE;
-                    n0n = tn * TILE;
-                    ga = reinterpret_cast<const char*>(a.A) + (int64_t)m0n * lda_b;
-                    gb = reinterpret_cast<const char*>(a.B) + (int64_t)n0n * ldb_b;
+                    locate(tnext);
+                    m0n = min(tm * TILE, a.m_last);
+                    n0n = min(tn * TILE, a.n_last);
+                    ga = reinterpret_cast<const char*>(a.A) + (int64_t)m0n * lda_b + k0b;
+                    gb = reinterpret_cast<const char*>(a.B) + (int64_t)n0n * ldb_b + k0b;
                     issue_prologue();
                 }
                 KK256_FENCE(); mfmas(1, 4); KK256_FENCE();
@@ -278,39 +315,102 @@ __global__ __launch_bounds__(THREADS) void dense_gemm_kk256_kernel(Args a) {
         }
 #undef KK256_READY
 #undef KK256_FENCE
-        epilogue(acc, a, m0, n0);
+        if constexpr (SPLIT) {
+            store_partial(acc, a, slice_now, m0, n0);
+        } else {
+            epilogue(acc, a, m0, n0);
+        }
         if (tnext >= total) break;
         t = tnext; m0 = m0n; n0 = n0n;
     }
 }
 
-// The kernel's conditions: whole tiles, K in whole steps and long enough to fill the ring, 16-byte
-// loads of the bias and stores of eight consecutive m.
+// The kernel's conditions: a tile in either dimension, K in whole steps and long enough to fill the ring, operands in 16-byte loads.
+// The last tile of a dimension that is no multiple of 256 is moved back until it ends with the matrix; what it repeats is
+// computed twice, with the same result.  The results and the bias need no more alignment than their elements.
 inline bool applicable(const DenseArgs<bf16_t>& a) {
-    const auto al16 = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; };
-    return a.M % TILE == 0 && a.N % TILE == 0 && a.K % BK == 0 && a.K >= 2 * BK && a.A.sk == 1 && a.B.sk == 1 && a.A.vec_ok &&
-           a.B.vec_ok && al16(a.C) && al16(a.pre) && al16(a.bias) && a.ldc % 8 == 0 &&
-           256 * a.A.sr * 2 < (int64_t(1) << 31) && 256 * a.B.sr * 2 < (int64_t(1) << 31);
+    return a.M >= TILE && a.N >= TILE && a.K % BK == 0 && a.K >= 2 * BK && a.A.sk == 1 && a.B.sk == 1 && a.A.vec_ok && a.B.vec_ok &&
+           256 * a.A.sr * 2 < (int64_t(1) << 31) && 256 * a.B.sr * 2 < (int64_t(1) << 31) && ceil_div(a.M, TILE) * ceil_div(a.N, TILE) < (int64_t(1) << 31);
 }
 
-inline int launch(hipStream_t s, DenseArgs<bf16_t>& a) {
-    a.tiles_m = a.M / TILE;
-    a.tiles_n = a.N / TILE;
+// C = act(sum over slices of the partial sums + bias), eight m of a column per thread, slices in order.
+__global__ __launch_bounds__(256) void slices_reduce_kernel(Args a, int M, FastDiv chunks, uint32_t total) {
+    const uint32_t idx = blockIdx.x * 256u + threadIdx.x;
+    if (idx >= total) return;
+    const uint32_t n = chunks.div(idx), m = (idx - n * chunks.d) * 8;
+    float v[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) v[e] = 0.0f;
+    const float* p = a.partial + (size_t)n * a.ldp + m;
+#pragma unroll 4
+    for (int s = 0; s < a.slices; ++s) {
+        float lo[4], hi[4];
+        Vec<float>::load(p + (size_t)s * a.slice_stride, lo);
+        Vec<float>::load(p + (size_t)s * a.slice_stride + 4, hi);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) { v[e] += lo[e]; v[4 + e] += hi[e]; }
+    }
+    const size_t off = (size_t)n * a.ldc + m;
+    const int have = M - (int)m;
+    if (a.bias != nullptr) {
+#pragma unroll
+        for (int e = 0; e < 8; ++e)
+            if (e < have) v[e] += ld(a.bias + m + e);
+    }
+    float y[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) y[e] = v[e];
+    act_vec(a.act, y);
+    if (have >= 8) {
+        if (a.pre != nullptr) row_store<bf16_t, 8, true>(a.pre, off, v, 0);
+        row_store<bf16_t, 8, true>(a.C, off, y, 0);
+    } else {
+#pragma unroll
+        for (int e = 0; e < 8; ++e)
+            if (e < have) {
+                if (a.pre != nullptr) st(a.pre + off + e, v[e]);
+                st(a.C + off + e, y[e]);
+            }
+    }
+}
+
+inline int64_t partial_ld(int64_t M) { return ceil_div(M, 8) * 8; }
+inline size_t partial_bytes(int64_t M, int64_t N, int slices) { return slices > 1 ? (size_t)partial_ld(M) * N * slices * sizeof(float) : 0; }
+
+template <bool SPLIT>
+int launch_as(hipStream_t s, const Args& k, int64_t units, const char* name) {
+    auto kernel = dense_gemm_kk256_kernel<SPLIT>;
     static ResidentOnce ro;
     ro.get([&](hipError_t& err) {
-        err = hipFuncSetAttribute(reinterpret_cast<const void*>(dense_gemm_kk256_kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                  (int)LDS_BYTES);
+        err = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)LDS_BYTES);
         return 1;
     });
     LUX_CHECK_HIP(ro.error);
-    const int64_t cus = num_cus() > 0 ? num_cus() : 256;
-    const int grid = (int)std::min<int64_t>((int64_t)a.tiles_m * a.tiles_n, cus);   // the ring fills the LDS: one workgroup per compute unit
+    const int64_t cus = num_cus() > 0 ? num_cus() : 256;       // the ring fills the LDS: one workgroup per compute unit
+    ProfScope ps(name, s);
+    kernel<<<dim3((unsigned)std::min(units, cus)), dim3(THREADS), LDS_BYTES, s>>>(k);
+    LUX_CHECK_LAUNCH();
+    return LUXHIP_OK;
+}
+
+// slices > 1 (at most K / 128): `partial` holds partial_bytes()
+inline int launch(hipStream_t s, DenseArgs<bf16_t>& a, int slices = 1, float* partial = nullptr) {
+    a.tiles_m = (int)ceil_div(a.M, TILE);
+    a.tiles_n = (int)ceil_div(a.N, TILE);
     Args k;
     k.A = a.A.p; k.B = a.B.p; k.bias = a.bias; k.C = a.C; k.pre = a.pre;
     k.lda = a.A.sr; k.ldb = a.B.sr; k.ldc = a.ldc;
-    k.K = a.K; k.act = a.act; k.tiles_m = a.tiles_m; k.tiles_n = a.tiles_n;
-    ProfScope ps(a.tail ? "dense_gemm_kernel<bf16>+tail" : "dense_gemm_kernel<bf16>", s);
-    dense_gemm_kk256_kernel<<<dim3((unsigned)grid), dim3(THREADS), LDS_BYTES, s>>>(k);
+    k.K = a.K; k.act = a.act; k.tiles_m = a.tiles_m; k.tiles_n = a.tiles_n; k.m_last = a.M - TILE; k.n_last = a.N - TILE;
+    k.slices = slices; k.partial = partial; k.ldp = partial_ld(a.M); k.slice_stride = k.ldp * a.N;
+    const int64_t tiles = (int64_t)a.tiles_m * a.tiles_n;
+    const char* const name = a.tail ? "dense_gemm_kernel<bf16>+tail" : "dense_gemm_kernel<bf16>";
+    if (slices == 1) return launch_as<false>(s, k, tiles, name);
+    const int64_t total = (k.ldp / 8) * a.N;
+    LUX_INVALID_IF(total >= (int64_t(1) << 31), "dense_gemm_kk256: too many partial sums");
+    const int rc = launch_as<true>(s, k, tiles * slices, name);
+    if (rc != LUXHIP_OK) return rc;
+    ProfScope ps("slices_reduce_kernel", s);
+    slices_reduce_kernel<<<(unsigned)ceil_div(total, 256), 256, 0, s>>>(k, a.M, FastDiv((uint32_t)(k.ldp / 8)), (uint32_t)total);
     LUX_CHECK_LAUNCH();
     return LUXHIP_OK;
 }
