@@ -406,39 +406,51 @@ __global__ __launch_bounds__(256) void conv_dbias_finalize_kernel(const float* _
 }
 
 // dw[a, b, ci, g*Cout_g + col] = sum over slices of partial[slice][m' = t*Cin_g + ci][col].
-// A thread owns 4 consecutive m' (one 16-byte load per slice, eight slices in flight); slices are
-// added in order.
+// A thread owns 4 consecutive m' (one 16-byte load per slice, eight slices in flight) of every `parts`-th slice; the parts of a
+// workgroup's values are added in order through LDS.  Bound by the latency of its trips to memory: with a thread per value (parts = 1) a filter of
+// few values on many slices is a handful of workgroups with 64 trips each (64 x 51 values, 419 slices: 23.0 us, in 32 parts 6.9).
 template <typename T>
 __global__ __launch_bounds__(256) void wgrad_reduce_kernel(const float* __restrict__ partial, T* __restrict__ dw, ConvGeom g,
-                                                           int grp, int slices, int reduce_blocks, int Mrows, int Cp, int run, int64_t slice_stride,
+                                                           int grp, int slices, int parts, int reduce_blocks, int Mrows, int Cp, int run, int64_t slice_stride,
                                                            BiasPartials bp) {
     if ((int)blockIdx.x >= reduce_blocks) {       // workgroups behind the reduction: one channel of the bias gradient each
         conv_dbias_finalize_channel(bp.partial, bp.dbias, bp.C, bp.slices, (int)blockIdx.x - reduce_blocks);
         return;
     }
     // Cp: channels per tap in the partial sums (padded); run > 0: rows are [kb][run / 4 positions][4 channels] instead
+    __shared__ float sums[256 * 4];
     const int total = Mrows * g.Cout_g;
-    const int idx = (blockIdx.x * blockDim.x + threadIdx.x) * 4;
-    if (idx >= total) return;
+    const int quads = 256 / parts, part = (int)threadIdx.x / quads;
+    const int idx = ((int)blockIdx.x * quads + (int)threadIdx.x % quads) * 4;
     float acc[4] = {0.0f, 0.0f, 0.0f, 0.0f};
     const bool vec = (total & 3) == 0 && (slice_stride & 3) == 0;   // then idx + 3 < total and every slice row is 16-byte aligned
-    if (vec) {
-        int sl = 0;
-        for (; sl + 8 <= slices; sl += 8) {
+    if (vec && idx < total) {
+        int sl = part;
+        for (; sl + 7 * parts < slices; sl += 8 * parts) {
             float4 v[8];
 #pragma unroll
-            for (int u = 0; u < 8; ++u) v[u] = *reinterpret_cast<const float4*>(partial + (size_t)(sl + u) * slice_stride + idx);
+            for (int u = 0; u < 8; ++u) v[u] = *reinterpret_cast<const float4*>(partial + (size_t)(sl + u * parts) * slice_stride + idx);
 #pragma unroll
             for (int u = 0; u < 8; ++u) { acc[0] += v[u].x; acc[1] += v[u].y; acc[2] += v[u].z; acc[3] += v[u].w; }
         }
-        for (; sl < slices; ++sl) {
+#pragma unroll 4
+        for (; sl < slices; sl += parts) {
             const float4 v = *reinterpret_cast<const float4*>(partial + (size_t)sl * slice_stride + idx);
             acc[0] += v.x; acc[1] += v.y; acc[2] += v.z; acc[3] += v.w;
         }
     } else {
-        for (int sl = 0; sl < slices; ++sl)
+        for (int sl = part; sl < slices; sl += parts)
             for (int e = 0; e < 4; ++e)
                 if (idx + e < total) acc[e] += partial[(size_t)sl * slice_stride + idx + e];
+    }
+    if (parts > 1) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) sums[threadIdx.x * 4 + e] = acc[e];
+        __syncthreads();
+        if (part != 0) return;
+        for (int p = 1; p < parts; ++p)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) acc[e] += sums[(threadIdx.x + p * quads) * 4 + e];
     }
     for (int e = 0; e < 4; ++e) {
         const int id = idx + e;
@@ -1026,10 +1038,13 @@ static int run_wgrad(hipStream_t s, const ConvGeom& g, Groups gr, Runs runs, con
         if (rc != LUXHIP_OK) return rc;
         ProfScope ps("wgrad_reduce_kernel", s);
         const int total = Mrows * g.Cout_g;
-        const int reduce_blocks = (int)ceil_div(total, 1024);
+        // parts of at least four slices, as many as give every compute unit a workgroup: beyond that they cost (36864 threads in one part 8.4 us, in two 9.8)
+        int parts = 1;
+        while (parts < 64 && (int64_t)total / 4 * parts * 2 <= 256 * (int64_t)std::max(1, num_cus()) && parts * 8 <= slices) parts *= 2;
+        const int reduce_blocks = (int)ceil_div(ceil_div(total, 4), 256 / parts);
         BiasPartials bp;
         if (bias != nullptr && grp == g.groups - 1) bp = *bias;       // the bias gradient's channels ride on the last group's launch
-        wgrad_reduce_kernel<T><<<(unsigned)(reduce_blocks + bp.C), 256, 0, s>>>(partial, dw, g, grp, slices, reduce_blocks, Mrows,
+        wgrad_reduce_kernel<T><<<(unsigned)(reduce_blocks + bp.C), 256, 0, s>>>(partial, dw, g, grp, slices, parts, reduce_blocks, Mrows,
                                                                            runs.W2 > 0 ? 4 : Mrows / (g.kW * g.kH), runs.W2 > 0 ? Runs::EL : 0,
                                                                            (int64_t)Mrows * plan.Ncols, bp);
         LUX_CHECK_LAUNCH();
