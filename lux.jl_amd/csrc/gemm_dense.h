@@ -502,6 +502,10 @@ int launch_batched_cfg(hipStream_t s, DenseArgs<T>& a) {
 
 template <typename T, bool AK, bool BKM>
 int launch_batched_layout(hipStream_t s, DenseArgs<T>& a) {
+    if constexpr (sizeof(T) == 4) {
+        int rc = LUXHIP_OK;
+        if (launch_split_batched(s, a, AK, BKM, &rc)) return rc;
+    }
     // 128 x 128 tiles when a product has at least one whole tile of them, 64 x 64 otherwise;
     // the variant without bounds checks when every product is made of whole, aligned tiles
     if (a.ep_probs != nullptr) {

@@ -52,4 +52,7 @@ bool launch_split(hipStream_t s, DenseArgs<T>& a, bool a_kmajor, bool b_kmajor, 
 template <typename T>
 bool launch_split_pair(hipStream_t s, DenseArgs<T>& a, DenseArgs<T>& b, int* rc);
 
+// gemm_split_batched_f32.hip: batched fp32 products that are faster there; false if the problem is another one
+bool launch_split_batched(hipStream_t s, DenseArgs<float>& a, bool a_kmajor, bool b_kmajor, int* rc);
+
 }  // namespace luxhip

@@ -46,8 +46,9 @@ struct Loader {
         if constexpr (KMAJOR) { r = id / CPR; k = (id % CPR) * Tr::VEC; }
         else { k = id / CPR; r = (id % CPR) * Tr::VEC; }
     }
-    __device__ __forceinline__ Loader(const Operand<T>& op, int r0) {
-        base = reinterpret_cast<const char*>(op.p + (KMAJOR ? (int64_t)r0 * op.sr : (int64_t)r0));
+    // back: an MN-major operand of fewer rows than a chunk (the end of a larger one) is read from `back` elements before its first row on, VEC - rows
+    __device__ __forceinline__ Loader(const Operand<T>& op, int r0, int back = 0) {
+        base = reinterpret_cast<const char*>(op.p + (KMAJOR ? (int64_t)r0 * op.sr : (int64_t)r0 - back));
         k_bytes = KMAJOR ? (int64_t)sizeof(T) : op.sk * (int64_t)sizeof(T);
         bounded = op.rows < ROWS;
 #pragma unroll
@@ -60,7 +61,7 @@ struct Loader {
                     r = min(r, op.rows - 1);
                 } else if (r + Tr::VEC > op.rows) {
                     sh[i] = r + Tr::VEC - op.rows;
-                    r = op.rows - Tr::VEC;
+                    r = op.rows - Tr::VEC + back;
                 }
             }
             voff[i] = (uint32_t)(((int64_t)r * op.sr + (int64_t)k * op.sk) * (int64_t)sizeof(T));
