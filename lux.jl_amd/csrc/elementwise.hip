@@ -19,43 +19,37 @@ constexpr int kThreads = 256;
 constexpr int kUnroll = 4;  // 16-byte vectors per thread; all of a thread's loads are issued before the first use
 
 // ------------------------------------------------------------------------------- forward
-template <typename T, int ACT, int VEC, bool HAS_BIAS, bool WRITE_PRE>
+// RAGGED: rows of I elements that are no multiple of a vector, or pointers that are not aligned to one (RowVec, common.h): every access stays
+// one 16-byte instruction, where an element per thread took eight of two bytes.
+// Bound by HBM: the pullback of 70 x 70 x 117 x 39 in bf16 70.9 -> 25.0 us (134 MB), fp32 51 x 51 x 128 x 40 with tanh 29.8 -> 27.4.
+template <typename T, int ACT, int VEC, bool HAS_BIAS, bool WRITE_PRE, bool RAGGED>
 __global__ __launch_bounds__(kThreads) void bias_act_fwd_kernel(const T* __restrict__ x, const T* __restrict__ bias,
-                                                                T* y, T* pre, uint32_t total_vec, FastDiv rowdiv,
+                                                                T* y, T* pre, uint32_t total_vec, uint32_t I, uint32_t vpr, FastDiv rowdiv,
                                                                 FastDiv cdiv, uint32_t C) {
-    // rowdiv divides a vector index by the number of vectors per row (I / VEC)
+    // rowdiv divides a vector index by vpr, the number of vectors per row
     for (uint32_t base = blockIdx.x * (kThreads * kUnroll); base < total_vec; base += gridDim.x * (kThreads * kUnroll)) {
         float v[kUnroll][VEC];
-        uint32_t idx[kUnroll];
 #pragma unroll
         for (int u = 0; u < kUnroll; ++u) {
-            idx[u] = base + u * kThreads + threadIdx.x;
-            const uint32_t li = min(idx[u], total_vec - 1);      // past the end: last vector again (ignored below)
-            if constexpr (VEC == 1) v[u][0] = ld(x + li);
-            else Vec<T>::load(x + (size_t)li * VEC, v[u]);
+            const uint32_t idx = base + u * kThreads + threadIdx.x;
+            const RowVec<VEC, RAGGED> rv(min(idx, total_vec - 1), I, vpr, rowdiv);      // past the end: last vector again (ignored below)
+            row_load<T, VEC, RAGGED>(x, rv.off, v[u]);
         }
 #pragma unroll
         for (int u = 0; u < kUnroll; ++u) {
-            if (idx[u] < total_vec) {
+            const uint32_t idx = base + u * kThreads + threadIdx.x;
+            if (idx < total_vec) {
+                const RowVec<VEC, RAGGED> rv(idx, I, vpr, rowdiv);
                 float b = 0.0f;
-                if constexpr (HAS_BIAS) {
-                    uint32_t row = rowdiv.div(idx[u]);
-                    uint32_t c = row - cdiv.div(row) * C;
-                    b = ld(bias + c);
-                }
+                if constexpr (HAS_BIAS) b = ld(bias + (rv.row - cdiv.div(rv.row) * C));
                 float p[VEC], o[VEC];
 #pragma unroll
                 for (int k = 0; k < VEC; ++k) {
                     p[k] = v[u][k] + b;
                     o[k] = Act<ACT>::f(p[k]);
                 }
-                if constexpr (VEC == 1) {
-                    if constexpr (WRITE_PRE) st(pre + idx[u], p[0]);
-                    st(y + idx[u], o[0]);
-                } else {
-                    if constexpr (WRITE_PRE) Vec<T>::store(pre + (size_t)idx[u] * VEC, p);
-                    Vec<T>::store(y + (size_t)idx[u] * VEC, o);
-                }
+                if constexpr (WRITE_PRE) row_store<T, VEC, RAGGED>(pre, rv.off, p, rv.skip);
+                row_store<T, VEC, RAGGED>(y, rv.off, o, rv.skip);
             }
         }
     }
@@ -114,14 +108,14 @@ constexpr int kChanVecs = 4;   // vectors per thread of the channel-layout pullb
 // "channel" layout: grid (S, C).  Workgroup (s, c) handles vectors [s*chunk, (s+1)*chunk) of
 // the nq = I*N/VEC vectors of channel c and publishes its partial sum; the workgroup of a
 // channel that arrives last adds the S partials in index order (same result on every run).
-template <typename T, int ACT, int VEC>
+template <typename T, int ACT, int VEC, bool RAGGED>
 __global__ __launch_bounds__(kThreads) void bias_act_bwd_channel_kernel(const T* __restrict__ delta,
                                                                         const T* __restrict__ out,
                                                                         const T* __restrict__ pre, T* dx, T* dbias,
                                                                         float* partial, uint32_t* counters,
                                                                         uint32_t cstride, uint32_t nq,
                                                                         uint32_t chunk, FastDiv rowdiv,
-                                                                        uint32_t vec_per_row, uint32_t C) {
+                                                                        uint32_t vec_per_row, uint32_t I, uint32_t C) {
     __shared__ float smem[kThreads / 64];
     __shared__ uint32_t last_flag;
     const uint32_t c = blockIdx.y, s = blockIdx.x, S = gridDim.x;
@@ -133,7 +127,20 @@ __global__ __launch_bounds__(kThreads) void bias_act_bwd_channel_kernel(const T*
     const bool single = chunk <= kThreads * kChanVecs;
     float r0[kChanVecs][VEC];
     size_t off0[kChanVecs];
+    uint32_t skip0[kChanVecs];
     bool have0[kChanVecs];
+    // vector q of the channel: its offset and the elements that the vector before it holds too
+    auto locate = [&](uint32_t q, size_t& off, uint32_t& skip) {
+        const uint32_t n = rowdiv.div(q);
+        if constexpr (RAGGED) {
+            const uint32_t start = (q - n * vec_per_row) * VEC;
+            skip = start + VEC > I ? start + VEC - I : 0u;
+            off = ((size_t)n * C + c) * I + (start - skip);
+        } else {
+            skip = 0;
+            off = ((size_t)q + (size_t)vec_per_row * ((size_t)n * (C - 1) + c)) * VEC;
+        }
+    };
     if (single) {
         // all loads of the thread are issued before the first use
 #pragma unroll
@@ -141,26 +148,28 @@ __global__ __launch_bounds__(kThreads) void bias_act_bwd_channel_kernel(const T*
             const uint32_t q = q0 + u * kThreads + threadIdx.x;
             have0[u] = q < q1;
             const uint32_t qq = have0[u] ? q : q1 - 1;            // past the end: last vector again (ignored)
-            const uint32_t n = rowdiv.div(qq);
-            off0[u] = ((size_t)qq + (size_t)vec_per_row * ((size_t)n * (C - 1) + c)) * VEC;
+            locate(qq, off0[u], skip0[u]);
         }
 #pragma unroll
-        for (int u = 0; u < kChanVecs; ++u) dx_vec<T, ACT, VEC>(delta, out, pre, off0[u], r0[u]);
+        for (int u = 0; u < kChanVecs; ++u) dx_vec<T, ACT, VEC, RAGGED>(delta, out, pre, off0[u], r0[u]);
 #pragma unroll
         for (int u = 0; u < kChanVecs; ++u)
             if (have0[u]) {
 #pragma unroll
-                for (int k = 0; k < VEC; ++k) acc += r0[u][k];
+                for (int k = 0; k < VEC; ++k)
+                    if (!RAGGED || (uint32_t)k >= skip0[u]) acc += r0[u][k];
             }
     } else {
         for (uint32_t q = q0 + threadIdx.x; q < q1; q += kThreads) {
-            const uint32_t n = rowdiv.div(q);
-            const size_t off = ((size_t)q + (size_t)vec_per_row * ((size_t)n * (C - 1) + c)) * VEC;
+            size_t off;
+            uint32_t skip;
+            locate(q, off, skip);
             float r[VEC];
-            dx_vec<T, ACT, VEC>(delta, out, pre, off, r);
-            if (dx) store_vec<T, VEC>(dx, off, r);
+            dx_vec<T, ACT, VEC, RAGGED>(delta, out, pre, off, r);
+            if (dx) row_store<T, VEC, RAGGED>(dx, off, r, skip);
 #pragma unroll
-            for (int k = 0; k < VEC; ++k) acc += r[k];
+            for (int k = 0; k < VEC; ++k)
+                if (!RAGGED || (uint32_t)k >= skip) acc += r[k];
         }
     }
     acc = block_sum(acc, smem);
@@ -172,7 +181,7 @@ __global__ __launch_bounds__(kThreads) void bias_act_bwd_channel_kernel(const T*
     if (single && dx) {
 #pragma unroll
         for (int u = 0; u < kChanVecs; ++u)
-            if (have0[u]) store_vec<T, VEC>(dx, off0[u], r0[u]);
+            if (have0[u]) row_store<T, VEC, RAGGED>(dx, off0[u], r0[u], skip0[u]);
     }
     if (!last) return;
     if (threadIdx.x < 64) {
@@ -288,49 +297,44 @@ static int bias_act_fwd_impl(hipStream_t s, int act, int64_t I, int64_t C, int64
     const int64_t total = I * C * N;
     const bool ptr_ok = aligned16(x) && aligned16(y) && (pre == nullptr || aligned16(pre));
     const FastDiv cdiv((uint32_t)C);
+    // rows: without a bias the tensor is one of them; rows below a vector go element by element
+    const int64_t len = bias ? I : total, rows = bias ? C * N : 1;
+#define LAUNCH_FWD_AS(A, VV, R)                                                                                    \
+    do {                                                                                                           \
+        const uint32_t vpr = (uint32_t)ceil_div(len, VV), tv = (uint32_t)(vpr * rows);                             \
+        const FastDiv rowdiv(vpr);                                                                                 \
+        const dim3 grid(grid_for(tv));                                                                             \
+        if (bias && pre)                                                                                           \
+            launch_exact(ps, bias_act_fwd_kernel<T, A, VV, true, true, R>, grid, dim3(kThreads), 0, s, x, bias, y, pre, tv, (uint32_t)len, vpr, rowdiv, cdiv, (uint32_t)C); \
+        else if (bias)                                                                                             \
+            launch_exact(ps, bias_act_fwd_kernel<T, A, VV, true, false, R>, grid, dim3(kThreads), 0, s, x, bias, y, pre, tv, (uint32_t)len, vpr, rowdiv, cdiv, (uint32_t)C); \
+        else if (pre)                                                                                              \
+            launch_exact(ps, bias_act_fwd_kernel<T, A, VV, false, true, R>, grid, dim3(kThreads), 0, s, x, bias, y, pre, tv, (uint32_t)len, vpr, rowdiv, cdiv, (uint32_t)C); \
+        else                                                                                                       \
+            launch_exact(ps, bias_act_fwd_kernel<T, A, VV, false, false, R>, grid, dim3(kThreads), 0, s, x, bias, y, pre, tv, (uint32_t)len, vpr, rowdiv, cdiv, (uint32_t)C); \
+    } while (0)
 #define LAUNCH_FWD(A)                                                                                              \
     do {                                                                                                           \
-        if (ptr_ok && I % V == 0) {                                                                                \
-            const uint32_t tv = (uint32_t)(total / V);                                                             \
-            const FastDiv rowdiv((uint32_t)(I / V));                                                               \
-            if (bias && pre)                                                                                       \
-                launch_exact(ps, bias_act_fwd_kernel<T, A, V, true, true>, dim3(grid_for(tv)), dim3(kThreads), 0, s, x, bias, y, pre, tv, rowdiv, cdiv, (uint32_t)C); \
-            else if (bias)                                                                                         \
-                launch_exact(ps, bias_act_fwd_kernel<T, A, V, true, false>, dim3(grid_for(tv)), dim3(kThreads), 0, s, x, bias, y, pre, tv, rowdiv, cdiv, (uint32_t)C); \
-            else if (pre)                                                                                          \
-                launch_exact(ps, bias_act_fwd_kernel<T, A, V, false, true>, dim3(grid_for(tv)), dim3(kThreads), 0, s, x, bias, y, pre, tv, rowdiv, cdiv, (uint32_t)C); \
-            else                                                                                                   \
-                launch_exact(ps, bias_act_fwd_kernel<T, A, V, false, false>, dim3(grid_for(tv)), dim3(kThreads), 0, s, x, bias, y, pre, tv, rowdiv, cdiv, (uint32_t)C); \
-        } else if (ptr_ok && bias && total % V == 0) {                                                             \
+        if (ptr_ok && len % V == 0) {                                                                              \
+            LAUNCH_FWD_AS(A, V, false);                                                                            \
+        } else if (ptr_ok && bias && I < 4 * V && total % V == 0) {                                                \
             const uint32_t tv = (uint32_t)(total / V);                                                             \
             const FastDiv idiv((uint32_t)I);                                                                       \
             if (pre)                                                                                               \
                 bias_act_fwd_smallI_kernel<T, A, V, true><<<grid_for(tv), kThreads, 0, s>>>(x, bias, y, pre, tv, idiv, cdiv, (uint32_t)C); \
             else                                                                                                   \
                 bias_act_fwd_smallI_kernel<T, A, V, false><<<grid_for(tv), kThreads, 0, s>>>(x, bias, y, pre, tv, idiv, cdiv, (uint32_t)C); \
-        } else if (ptr_ok && !bias && total % V == 0) {                                                            \
-            const uint32_t tv = (uint32_t)(total / V);                                                             \
-            if (pre)                                                                                               \
-                launch_exact(ps, bias_act_fwd_kernel<T, A, V, false, true>, dim3(grid_for(tv)), dim3(kThreads), 0, s, x, bias, y, pre, tv, cdiv, cdiv, (uint32_t)C); \
-            else                                                                                                   \
-                launch_exact(ps, bias_act_fwd_kernel<T, A, V, false, false>, dim3(grid_for(tv)), dim3(kThreads), 0, s, x, bias, y, pre, tv, cdiv, cdiv, (uint32_t)C); \
+        } else if (len >= V) {                                                                                     \
+            LAUNCH_FWD_AS(A, V, true);                                                                             \
         } else {                                                                                                   \
-            const uint32_t tv = (uint32_t)total;                                                                   \
-            const FastDiv rowdiv((uint32_t)I);                                                                     \
-            if (bias && pre)                                                                                       \
-                launch_exact(ps, bias_act_fwd_kernel<T, A, 1, true, true>, dim3(grid_for(tv)), dim3(kThreads), 0, s, x, bias, y, pre, tv, rowdiv, cdiv, (uint32_t)C); \
-            else if (bias)                                                                                         \
-                launch_exact(ps, bias_act_fwd_kernel<T, A, 1, true, false>, dim3(grid_for(tv)), dim3(kThreads), 0, s, x, bias, y, pre, tv, rowdiv, cdiv, (uint32_t)C); \
-            else if (pre)                                                                                          \
-                launch_exact(ps, bias_act_fwd_kernel<T, A, 1, false, true>, dim3(grid_for(tv)), dim3(kThreads), 0, s, x, bias, y, pre, tv, rowdiv, cdiv, (uint32_t)C); \
-            else                                                                                                   \
-                launch_exact(ps, bias_act_fwd_kernel<T, A, 1, false, false>, dim3(grid_for(tv)), dim3(kThreads), 0, s, x, bias, y, pre, tv, rowdiv, cdiv, (uint32_t)C); \
+            LAUNCH_FWD_AS(A, 1, false);                                                                            \
         }                                                                                                          \
     } while (0)
     {
         ProfScope ps("bias_act_fwd_kernel", s, true);
         LUX_DISPATCH_ACT(act, LAUNCH_FWD);
     }
+#undef LAUNCH_FWD_AS
 #undef LAUNCH_FWD
     LUX_CHECK_LAUNCH();
     return LUXHIP_OK;
@@ -388,9 +392,8 @@ static int bias_act_bwd_impl(hipStream_t s, int act, int64_t I, int64_t C, int64
 
     const bool channel_layout = I >= 64 && C <= 65535;
     if (channel_layout) {
-        const bool vec = ptr_ok && I % V == 0;
-        const int vv = vec ? V : 1;
-        const uint32_t nq = (uint32_t)(I * N / vv);
+        const bool whole = ptr_ok && I % V == 0;
+        const uint32_t vpr = (uint32_t)ceil_div(I, V), nq = (uint32_t)(vpr * N);
         int64_t S = ceil_div(nq, kThreads * kChanVecs);
         const int64_t smax = std::min<int64_t>(kThreads, std::max<int64_t>(1, 16384 / C));
         if (S > smax) S = smax;
@@ -401,14 +404,14 @@ static int bias_act_bwd_impl(hipStream_t s, int act, int64_t I, int64_t C, int64
         uint32_t* counters = nullptr;
         int rc = bwd_scratch(s, fixed, (size_t)C * S * sizeof(float), &partial, &counters);
         if (rc != LUXHIP_OK) return rc;
-        const FastDiv rowdiv((uint32_t)(I / vv));
+        const FastDiv rowdiv(vpr);
         dim3 grid((unsigned)S, (unsigned)C);
 #define LAUNCH_CH(A)                                                                                               \
     do {                                                                                                           \
-        if (vec)                                                                                                   \
-            launch_exact(ps, bias_act_bwd_channel_kernel<T, A, V>, dim3(grid), dim3(kThreads), 0, s, delta, out, pre, dx, dbias, partial, counters, counter_stride(C), nq, chunk, rowdiv, (uint32_t)(I / vv), (uint32_t)C); \
+        if (whole)                                                                                                 \
+            launch_exact(ps, bias_act_bwd_channel_kernel<T, A, V, false>, dim3(grid), dim3(kThreads), 0, s, delta, out, pre, dx, dbias, partial, counters, counter_stride(C), nq, chunk, rowdiv, vpr, (uint32_t)I, (uint32_t)C); \
         else                                                                                                       \
-            launch_exact(ps, bias_act_bwd_channel_kernel<T, A, 1>, dim3(grid), dim3(kThreads), 0, s, delta, out, pre, dx, dbias, partial, counters, counter_stride(C), nq, chunk, rowdiv, (uint32_t)(I / vv), (uint32_t)C); \
+            launch_exact(ps, bias_act_bwd_channel_kernel<T, A, V, true>, dim3(grid), dim3(kThreads), 0, s, delta, out, pre, dx, dbias, partial, counters, counter_stride(C), nq, chunk, rowdiv, vpr, (uint32_t)I, (uint32_t)C); \
     } while (0)
         {
             ProfScope ps("bias_act_bwd_channel_kernel", s, true);
