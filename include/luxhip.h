@@ -168,6 +168,14 @@ int luxhip_bias_activation_fwd(luxhip_stream_t s, int dtype, int act, int64_t I,
 int luxhip_bias_activation_bwd(luxhip_stream_t s, int dtype, int act, int64_t I, int64_t C, int64_t N,
                                const void* delta, const void* out, const void* pre, void* dx, void* dbias);
 
+/* luxhip_bias_activation_bwd with the operator's input and bias in place of the pre-activation, which
+ * it forms again with the rounding that a stored one has: the forward pass need not keep it (pre == NULL
+ * there).  Same results, bit for bit.  x is read where the activation's derivative needs the
+ * pre-activation; bias may be NULL, dbias only if bias is. */
+int luxhip_bias_activation_bwd_from_x(luxhip_stream_t s, int dtype, int act, int64_t I, int64_t C, int64_t N,
+                                      const void* delta, const void* out, const void* x, const void* bias, void* dx,
+                                      void* dbias);
+
 /* luxhip_bias_activation_bwd for callers that cannot allocate device memory (code under HIP graph
  * capture, tight serving loops, harnesses that forbid hipMalloc).  It has no counterpart in the
  * reference.  Same arguments and results; the partial sums and arrival counters of the bias

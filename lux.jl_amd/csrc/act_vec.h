@@ -6,18 +6,35 @@
 
 namespace luxhip {
 
+// How the pre-activation of an element comes from what `pre` points to
+struct Stored {                                  // it is the pre-activation
+    __device__ __forceinline__ float operator()(float p, int) const { return p; }
+};
+template <typename T, int N>
+struct PlusBias {                                // it is the operator's input: the bias of element k, rounded to what a stored pre-activation holds
+    float b[N];
+    __device__ __forceinline__ float operator()(float x, int k) const {
+        const float p = x + b[N == 1 ? 0 : k];
+        if constexpr (sizeof(T) == 2) return bf16_to_f32(f32_to_bf16(p));
+        else return p;
+    }
+};
 // RAGGED: any alignment (common.h, row_load)
-template <typename T, int ACT, int VEC, bool RAGGED = false>
-__device__ __forceinline__ void dx_vec(const T* delta, const T* out, const T* pre, size_t off, float (&dx)[VEC]) {
+template <typename T, int ACT, int VEC, bool RAGGED = false, class Pre = Stored>
+__device__ __forceinline__ void dx_vec(const T* delta, const T* out, const T* pre, size_t off, float (&dx)[VEC], const Pre& pre_of = Pre()) {
     float d[VEC], o[VEC], p[VEC];
     if constexpr (VEC == 1) {
         d[0] = ld(delta + off);
         if constexpr (ACT != LUXHIP_ACT_IDENTITY && !Act<ACT>::needs_pre) o[0] = ld(out + off);
-        if constexpr (Act<ACT>::needs_pre) p[0] = ld(pre + off);
+        if constexpr (Act<ACT>::needs_pre) p[0] = pre_of(ld(pre + off), 0);
     } else {
         row_load<T, VEC, RAGGED>(delta, off, d);
         if constexpr (ACT != LUXHIP_ACT_IDENTITY && !Act<ACT>::needs_pre) row_load<T, VEC, RAGGED>(out, off, o);
-        if constexpr (Act<ACT>::needs_pre) row_load<T, VEC, RAGGED>(pre, off, p);
+        if constexpr (Act<ACT>::needs_pre) {
+            row_load<T, VEC, RAGGED>(pre, off, p);
+#pragma unroll
+            for (int k = 0; k < VEC; ++k) p[k] = pre_of(p[k], k);
+        }
     }
 #pragma unroll
     for (int k = 0; k < VEC; ++k) {

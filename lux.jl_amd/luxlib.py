@@ -181,13 +181,12 @@ def rrule_bias_activation(act: str, x: DeviceArray, bias: Optional[DeviceArray])
     dt = _same_dtype(x, bias)
     I, Cc, N = _icn(x)
     y = DeviceArray(x.shape, dt)
-    pre = DeviceArray(x.shape, dt) if aid in _NEEDS_PRE else None
-    _lib.call("luxhip_bias_activation_fwd", current_stream(), x.code, aid, I, Cc, N, x.ptr, _p(bias), y.ptr, _p(pre))
+    _lib.call("luxhip_bias_activation_fwd", current_stream(), x.code, aid, I, Cc, N, x.ptr, _p(bias), y.ptr, None)
 
-    def back(delta: DeviceArray):
+    def back(delta: DeviceArray):     # x .+ bias is formed again where the derivative needs it
         dx = DeviceArray(x.shape, dt)
         db = None if bias is None else DeviceArray(bias.shape, dt)
-        _lib.call("luxhip_bias_activation_bwd", current_stream(), x.code, aid, I, Cc, N, delta.ptr, y.ptr, _p(pre),
+        _lib.call("luxhip_bias_activation_bwd_from_x", current_stream(), x.code, aid, I, Cc, N, delta.ptr, y.ptr, x.ptr, _p(bias),
                   dx.ptr, _p(db))
         return dx, db
 

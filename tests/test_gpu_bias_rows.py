@@ -1,4 +1,4 @@
-"""bias_activation over rows that are no multiple of a vector or not aligned to one."""
+"""bias_activation over rows that are no multiple of a vector or not aligned to one, and its pullback from the operator's input."""
 import numpy as np
 import pytest
 
@@ -34,3 +34,21 @@ def test_rows(gpu, dtype, act, I, C, N, shift):
     assert_close(y.to_numpy(), wy, dtype, "y")
     assert_close(gx.to_numpy(), wdx, dtype, "dx")
     assert_close(gb.to_numpy().reshape(-1), wdb.reshape(-1), dtype, "db", scale=np.sqrt(I * N))
+
+
+@pytest.mark.parametrize("dtype", ["f32", "bf16"])
+@pytest.mark.parametrize("act", ["swish", "gelu", "softplus", "relu"])
+@pytest.mark.parametrize("I,C,N", [(64, 3, 5), (71, 3, 5), (1, 96, 40), (4, 6, 9), (5, 7, 3)])
+def test_from_x_is_the_stored_pre_activation(gpu, dtype, act, I, C, N):
+    rng = np.random.default_rng(stable_seed("from x", dtype, act, I, C, N))
+    x, b, d = (dev(gpu, a, dtype) for a in host_inputs(dtype, rng.normal(size=(I, C, N)), rng.normal(size=C), rng.normal(size=(I, C, N))))
+    code, aid, s = x.code, gpu._lib.ACT_IDS[act], gpu.current_stream()
+    y, pre, got, want = (gpu.DeviceArray((I, C, N), dtype) for _ in range(4))
+    db, wdb = gpu.DeviceArray((C,), dtype), gpu.DeviceArray((C,), dtype)
+    gpu._lib.call("luxhip_bias_activation_fwd", s, code, aid, I, C, N, x.ptr, b.ptr, y.ptr, pre.ptr)
+    gpu._lib.call("luxhip_bias_activation_bwd", s, code, aid, I, C, N, d.ptr, y.ptr, pre.ptr, want.ptr, wdb.ptr)
+    gpu._lib.call("luxhip_bias_activation_bwd_from_x", s, code, aid, I, C, N, d.ptr, y.ptr, x.ptr, b.ptr, got.ptr, db.ptr)
+    np.testing.assert_array_equal(got.to_numpy(), want.to_numpy())
+    np.testing.assert_array_equal(db.to_numpy(), wdb.to_numpy())
+    with pytest.raises(gpu.LuxHipError, match="dbias"):
+        gpu._lib.call("luxhip_bias_activation_bwd_from_x", s, code, aid, I, C, N, d.ptr, y.ptr, x.ptr, b.ptr, got.ptr, None)
