@@ -122,6 +122,8 @@ def load():
         fn = getattr(lib, name)          # AttributeError if the symbol is not exported
         fn.argtypes = argtypes
         fn.restype = C.c_int
+        if _host is not None:
+            _host.bind(name, C.cast(fn, C.c_void_p).value)
     lib.luxhip_last_error.argtypes = []
     lib.luxhip_last_error.restype = C.c_char_p
     _lib = lib
@@ -141,6 +143,15 @@ def check(status: int):
     raise LuxHipError(status, msg)
 
 
-def call(name: str, *args):
+def _ctypes_call(name: str, *args):
     """Call an entry point and raise on a non-zero status."""
     check(getattr(load(), name)(*args))
+
+
+try:
+    from . import _host                  # csrc/python_host.cpp; arrays are made of its types
+except ImportError:                      # not built: importing still works, operators say what is missing
+    _host, call = None, _ctypes_call
+else:
+    _host.configure(load, _ctypes_call, check, C.c_void_p, C.Array, ConvDimsStruct)
+    call = _host.call

@@ -32,49 +32,22 @@ def _from_bf16_bits(b: np.ndarray) -> np.ndarray:
     return (b.astype(np.uint32) << np.uint32(16)).view(np.float32)
 
 
-class DeviceArray:
-    """A dense column-major tensor in HBM.  `shape` is the Julia-style logical shape."""
+if _lib._host is not None:
+    _Array, _Stat = _lib._host.Array, _lib._host.Stat
+else:
+    class _Array:
+        def __init__(self, *args, **kwargs):
+            raise ImportError("lux.jl_amd/_host.so is missing: build it with `make -C lux.jl_amd/csrc`")
 
-    __slots__ = ("shape", "dtype", "ptr", "_owner", "_base")
+    _Stat = _Array
 
-    def __init__(self, shape, dtype="f32", ptr=None, base=None):
-        if dtype not in DTYPES:
-            raise TypeError(f"unsupported dtype {dtype!r} (use 'f32' or 'bf16'; 'u8' for masks)")
-        self.shape = tuple(int(s) for s in shape)
-        self.dtype = dtype
-        self._base = base
-        if ptr is None:
-            p = C.c_void_p()
-            _lib.call("luxhip_malloc", C.byref(p), max(self.nbytes, 1))
-            self.ptr = p.value
-            self._owner = True
-        else:
-            self.ptr = int(ptr)
-            self._owner = False
 
-    # ------------------------------------------------------------------ properties
-    @property
-    def size(self) -> int:
-        n = 1
-        for s in self.shape:
-            n *= s
-        return n
+class DeviceArray(_Array):
+    """A dense column-major tensor in HBM: `DeviceArray(shape, dtype="f32", ptr=None, base=None)`.  `shape` is the Julia-style
+    logical shape; without `ptr` the array owns its memory, with it it borrows (and keeps `base`).  Attributes: shape, dtype, ptr,
+    size, ndim, itemsize, nbytes and code, the storage type's number in the C ABI (csrc/python_host.cpp)."""
 
-    @property
-    def ndim(self) -> int:
-        return len(self.shape)
-
-    @property
-    def itemsize(self) -> int:
-        return DTYPES[self.dtype][1]
-
-    @property
-    def nbytes(self) -> int:
-        return self.size * self.itemsize
-
-    @property
-    def code(self) -> int:
-        return DTYPES[self.dtype][0]
+    __slots__ = ()
 
     # ------------------------------------------------------------------ transfers
     @classmethod
@@ -117,39 +90,17 @@ class DeviceArray:
             raise ValueError(f"cannot reshape {self.shape} to {shape}")
         return DeviceArray(shape, self.dtype, ptr=self.ptr, base=self)
 
-    def __del__(self):
-        if getattr(self, "_owner", False) and self.ptr:
-            try:
-                _lib.load().luxhip_free(C.c_void_p(self.ptr))
-            except Exception:
-                pass
-            self.ptr = 0
-
     def __repr__(self):
         return f"DeviceArray(shape={self.shape}, dtype={self.dtype}, ptr=0x{self.ptr:x})"
 
 
-class StatArray:
+class StatArray(_Stat):
     """fp32 statistics buffer (saved mean / inverse std) of `n` entries."""
 
-    __slots__ = ("n", "ptr")
-
-    def __init__(self, n: int):
-        self.n = int(n)
-        p = C.c_void_p()
-        _lib.call("luxhip_malloc", C.byref(p), max(4 * self.n, 4))
-        self.ptr = p.value
+    __slots__ = ()
 
     def to_numpy(self):
         host = np.empty(self.n, np.float32)
         if self.n:
             _lib.call("luxhip_memcpy_d2h", host.ctypes.data, self.ptr, host.nbytes, current_stream())
         return host
-
-    def __del__(self):
-        if self.ptr:
-            try:
-                _lib.load().luxhip_free(C.c_void_p(self.ptr))
-            except Exception:
-                pass
-            self.ptr = 0

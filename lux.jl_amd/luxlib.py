@@ -1271,7 +1271,7 @@ def fused_conv_bias_activation(act: str, weight: DeviceArray, x: DeviceArray, b,
         return _from_inner_output(cdims, fused_conv_bias_activation(act, _inner_weight(cdims, weight), _depth_unfold(cdims, x), b,
                                                                     cdims.inner))
     y = DeviceArray(cdims.y_shape, dt)
-    _lib.call("luxhip_conv_fwd", current_stream(), y.code, _act_id(act), C.byref(cdims._c), x.ptr, weight.ptr, _p(b),
+    _lib.call("luxhip_conv_fwd", current_stream(), y.code, _act_id(act), cdims._c, x.ptr, weight.ptr, _p(b),
               y.ptr, None, None)
     return y
 
@@ -1342,7 +1342,7 @@ def rrule_fused_conv_bias_activation(act: str, weight, x, b, cdims: DenseConvDim
     # the channel-contiguous copy of x, kept for the filter gradient; where the kernels pad the channels of a group to whole
     # 16-byte chunks their copy is not of x's shape, and making it again costs less than a second, unpadded one
     xt = DeviceArray(x.shape, dt) if (cdims._c.Cin // cdims.groups) * x.itemsize % 16 == 0 else None
-    _lib.call("luxhip_conv_fwd", current_stream(), y.code, aid, C.byref(cdims._c), x.ptr, weight.ptr, _p(b), y.ptr, _p(pre),
+    _lib.call("luxhip_conv_fwd", current_stream(), y.code, aid, cdims._c, x.ptr, weight.ptr, _p(b), y.ptr, _p(pre),
               _p(xt))
 
     def back(delta):
@@ -1350,7 +1350,7 @@ def rrule_fused_conv_bias_activation(act: str, weight, x, b, cdims: DenseConvDim
         dx = DeviceArray(x.shape, dt)
         db = None if b is None else DeviceArray(b.shape, dt)
         dz = None if aid == 0 else DeviceArray(cdims.y_shape, dt)
-        _lib.call("luxhip_fused_conv_bwd", current_stream(), y.code, aid, C.byref(cdims._c), delta.ptr, y.ptr, _p(pre),
+        _lib.call("luxhip_fused_conv_bwd", current_stream(), y.code, aid, cdims._c, delta.ptr, y.ptr, _p(pre),
                   x.ptr, weight.ptr, _p(dz), dw.ptr, dx.ptr, _p(db), _p(xt))
         return dw, dx, db
 
@@ -1367,7 +1367,7 @@ def conv_data_grad(dy, weight, cdims):
     if cdims.inner is not None:
         return _depth_fold(cdims, conv_data_grad(_to_inner_output(cdims, dy), _inner_weight(cdims, weight), cdims.inner))
     dx = DeviceArray(cdims.x_shape, dy.dtype)
-    _lib.call("luxhip_conv_bwd_data", current_stream(), dy.code, C.byref(cdims._c), dy.ptr, weight.ptr, dx.ptr)
+    _lib.call("luxhip_conv_bwd_data", current_stream(), dy.code, cdims._c, dy.ptr, weight.ptr, dx.ptr)
     return dx
 
 
@@ -1376,7 +1376,7 @@ def conv_filter_grad(x, dy, cdims):
     if cdims.inner is not None:
         return conv_filter_grad(_depth_unfold(cdims, x), _to_inner_output(cdims, dy), cdims.inner).reshape(cdims.w_shape)
     dw = DeviceArray(cdims.w_shape, x.dtype)
-    _lib.call("luxhip_conv_bwd_filter", current_stream(), x.code, C.byref(cdims._c), x.ptr, dy.ptr, dw.ptr)
+    _lib.call("luxhip_conv_bwd_filter", current_stream(), x.code, cdims._c, x.ptr, dy.ptr, dw.ptr)
     return dw
 
 
