@@ -486,9 +486,12 @@ int luxhip_malloc(void** out, size_t bytes) {
         // give the pool back to the driver and retry once
         for (auto& kv : g_pool.free_blocks) (void)hipFree(kv.second);
         g_pool.free_blocks.clear();
+        (void)hipGetLastError();      // or the next launch reports this error as its own
         e = hipMalloc(&p, r);
-        if (e != hipSuccess)
+        if (e != hipSuccess) {
+            (void)hipGetLastError();
             return set_error(LUXHIP_HIP_ERROR, "hipMalloc(%zu) failed: %s", r, hipGetErrorString(e));
+        }
     }
     g_pool.live[p] = r;
     *out = p;
