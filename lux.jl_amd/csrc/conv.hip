@@ -303,81 +303,96 @@ static int runs_copy_pack(hipStream_t s, const ConvGeom& g, Runs r, const bf16_t
     return LUXHIP_OK;
 }
 
-// First pass of the fused pullback (bf16; P and C multiples of 8, 16-byte aligned pointers): one pass over delta
-// writes dz = delta .* act'(y, pre) as it lies (p contiguous: what the window and the direct filter-gradient kernels
-// read), its channel-contiguous copy dzT (what the input-gradient kernels read) and the bias gradient's partial sums,
-// where a pass for dz and the bias gradient followed by a transposing copy reads dz once more.  A workgroup walks
-// `chunk` tiles of 64 positions x 64 channels of one image; a tile goes through LDS as fp32 (rows of 65 words: the
-// 64 lanes of a wave hit 64 banks in both phases).  Phase 1: 16-byte vectors along p, dz stored, per-channel sums
-// kept in registers; phase 2: eight channels of one position per thread, 16 bytes of dzT.  The eight threads of a
+// First pass of the fused pullback: one pass over delta writes dz = delta .* act'(y, pre) channel-contiguous with its channels padded to Cp (dzT: what
+// the input-gradient and the general filter-gradient kernels read), as it lies (dz, may be null: what the window and the direct filter-gradient
+// kernels read) and the bias gradient's partial sums, where a pass for dz and the bias gradient followed by a transposing copy
+// reads dz once more and always writes it.  A workgroup walks `chunk` tiles of 64 positions x 64 channels of one image; a tile goes through LDS as fp32 (rows
+// of 65 words: the 64 lanes of a wave hit 64 banks in both phases).  Phase 1: 16-byte vectors along p, dz stored, per-channel sums
+// kept in registers; phase 2: a vector of channels of one position per thread, 16 bytes of dzT.  The threads of a
 // channel add their sums in a fixed order; partial[(n * gridDim.x + blockIdx.x) * C + c].  The z slices behind
-// the N images repack the filter for the input-gradient kernel (as in whcn_to_cwhn_pack_kernel).
-template <int ACT>
-__global__ __launch_bounds__(256) void conv_dz_cwhn_pack_kernel(const bf16_t* __restrict__ delta, const bf16_t* __restrict__ y,
-                                                                const bf16_t* __restrict__ pre, bf16_t* dz, bf16_t* __restrict__ dzT,
-                                                                float* __restrict__ partial, int P, int C, int N, int chunk,
-                                                                const bf16_t* __restrict__ w, bf16_t* __restrict__ wout, ConvGeom g) {
+// the N images repack the filter for the input-gradient kernel (for its first launch where that is a general one, ps.total > 0).
+// RAGGED: any P, C and alignment of delta, y, pre and dz; otherwise P and C are whole vectors, Cp is C and every pointer is 16-byte aligned.
+// Bound by HBM (5.6 TB/s at large sizes).  56 x 56 x 128 x 64 in fp32, swish: 57 + 37 us in two passes, 63 in one; 112 x 112 x 64 x 32 in bf16 (nothing reads dz as it
+// lies): 36.8 + 4.8 for the filter, 29.7 together; 14 x 14 x 16 -> 32 x 4 in fp32, whole step: 44 -> 38.3.
+template <typename T, int ACT, bool RAGGED>
+__global__ __launch_bounds__(256) void conv_dz_cwhn_pack_kernel(const T* __restrict__ delta, const T* __restrict__ y, const T* __restrict__ pre, T* dz,
+                                                                T* __restrict__ dzT, float* __restrict__ partial, int P, int C, int Cp, int N, int chunk,
+                                                                const T* __restrict__ w, T* __restrict__ wout, ConvGeom g, PackSubs ps) {
+    constexpr int V = Vec<T>::N, VR = 64 / V, PER = 64 * VR / 256, PITCH = 65;
     if ((int)blockIdx.z >= N) {
-        const int block = ((int)(blockIdx.z - N) * (int)gridDim.y + (int)blockIdx.y) * (int)gridDim.x + (int)blockIdx.x;
-        pack_filter_element<bf16_t>(w, wout, g, 1, block * 256 + (int)threadIdx.x);
+        const int64_t block = ((int64_t)(blockIdx.z - N) * gridDim.y + blockIdx.y) * gridDim.x + blockIdx.x;
+        if (ps.total > 0) pack_sub_element<T>(w, wout, g, ps, block * 256 + threadIdx.x);
+        else pack_filter_element<T>(w, wout, g, 1, (int)(block * 256 + threadIdx.x));
         return;
     }
-    constexpr int PITCH = 65;
     __shared__ float tile[64 * PITCH];
     const int n = blockIdx.z, c0 = blockIdx.y * 64;
-    const size_t image = (size_t)n * C * P;
-    float bsum[2] = {0.0f, 0.0f};
+    const size_t image = (size_t)n * C * P, imageT = (size_t)n * Cp * P;
+    float bsum[PER] = {};
     const int tiles_p = (P + 63) / 64;
     const int t_end = min(tiles_p, ((int)blockIdx.x + 1) * chunk);
     for (int tp = blockIdx.x * chunk; tp < t_end; ++tp) {
         const int p0 = tp * 64;
-        float r[2][8];
-        bool ok[2];
+        float r[PER][V];
 #pragma unroll
-        for (int it = 0; it < 2; ++it) {                 // loads first, then the stores
-            const int idx = threadIdx.x + it * 256, cl = idx >> 3, pv = idx & 7;
-            ok[it] = c0 + cl < C && p0 + pv * 8 < P;
-            if (ok[it]) {
-                dx_vec<bf16_t, ACT, 8>(delta, y, pre, image + (size_t)(c0 + cl) * P + p0 + pv * 8, r[it]);
+        for (int it = 0; it < PER; ++it) {               // loads first, then the stores
+            const int idx = threadIdx.x + it * 256, c = c0 + idx / VR, p = p0 + idx % VR * V;
+            const size_t off = image + (size_t)c * P + p;
+            if (c < C && p + V <= P) {
+                dx_vec<T, ACT, V, RAGGED>(delta, y, pre, off, r[it]);
             } else {
 #pragma unroll
-                for (int k = 0; k < 8; ++k) r[it][k] = 0.0f;
+                for (int k = 0; k < V; ++k) {
+                    float v[1] = {0.0f};
+                    if constexpr (RAGGED) {
+                        if (c < C && p + k < P) dx_vec<T, ACT, 1>(delta, y, pre, off + k, v);
+                    }
+                    r[it][k] = v[0];
+                }
             }
         }
 #pragma unroll
-        for (int it = 0; it < 2; ++it) {
-            const int idx = threadIdx.x + it * 256, cl = idx >> 3, pv = idx & 7;
-            if (ok[it] && dz != nullptr) store_vec<bf16_t, 8>(dz, image + (size_t)(c0 + cl) * P + p0 + pv * 8, r[it]);
+        for (int it = 0; it < PER; ++it) {
+            const int idx = threadIdx.x + it * 256, cl = idx / VR, pv = idx % VR, c = c0 + cl, p = p0 + pv * V;
+            if (dz != nullptr && c < C) {
+                const size_t off = image + (size_t)c * P + p;
+                if (p + V <= P) {
+                    row_store<T, V, RAGGED>(dz, off, r[it], 0);
+                } else if constexpr (RAGGED) {
+#pragma unroll
+                    for (int k = 0; k < V; ++k)
+                        if (p + k < P) st(dz + off + k, r[it][k]);
+                }
+            }
             float t = 0.0f;
 #pragma unroll
-            for (int k = 0; k < 8; ++k) {
-                tile[cl * PITCH + pv * 8 + k] = r[it][k];
+            for (int k = 0; k < V; ++k) {
+                tile[cl * PITCH + pv * V + k] = r[it][k];
                 t += r[it][k];
             }
             bsum[it] += t;
         }
         __syncthreads();
 #pragma unroll
-        for (int it = 0; it < 2; ++it) {
-            const int idx = threadIdx.x + it * 256, pl = idx >> 3, cv = idx & 7;
-            if (p0 + pl < P && c0 + cv * 8 < C) {
-                float v[8];
+        for (int it = 0; it < PER; ++it) {
+            const int idx = threadIdx.x + it * 256, pl = idx / VR, cv = idx % VR;
+            if (p0 + pl < P && c0 + cv * V < Cp) {
+                float v[V];
 #pragma unroll
-                for (int k = 0; k < 8; ++k) v[k] = tile[(cv * 8 + k) * PITCH + pl];
-                store_vec<bf16_t, 8>(dzT, image + (size_t)(p0 + pl) * C + c0 + cv * 8, v);
+                for (int k = 0; k < V; ++k) v[k] = tile[(cv * V + k) * PITCH + pl];
+                store_vec<T, V>(dzT, imageT + (size_t)(p0 + pl) * Cp + c0 + cv * V, v);
             }
         }
         __syncthreads();
     }
     if (partial != nullptr) {
 #pragma unroll
-        for (int it = 0; it < 2; ++it) {
-            const int idx = threadIdx.x + it * 256, cl = idx >> 3, pv = idx & 7;
-            // the eight threads of a channel are neighbouring lanes: (((s0 + s1) + (s2 + s3)) + ((s4 + s5) + (s6 + s7)))
+        for (int it = 0; it < PER; ++it) {
+            const int idx = threadIdx.x + it * 256, cl = idx / VR, pv = idx % VR;
+            // the threads of a channel are neighbouring lanes: (((s0 + s1) + (s2 + s3)) + ((s4 + s5) + (s6 + s7))) ...
             float t = bsum[it];
-            t += __shfl_xor(t, 1);
-            t += __shfl_xor(t, 2);
-            t += __shfl_xor(t, 4);
+#pragma unroll
+            for (int o = 1; o < VR; o *= 2) t += __shfl_xor(t, o);
             if (pv == 0 && c0 + cl < C) partial[((size_t)n * gridDim.x + blockIdx.x) * C + c0 + cl] = t;
         }
     }
@@ -389,10 +404,11 @@ __global__ __launch_bounds__(256) void conv_dz_cwhn_pack_kernel(const bf16_t* __
 // its own or extra workgroups of the launch that adds up the filter gradient's partial sums (both are a few microseconds).
 struct BiasPartials {
     const float* partial = nullptr;
-    bf16_t* dbias = nullptr;
+    void* dbias = nullptr;
     int C = 0, slices = 0;
 };
-__device__ __forceinline__ void conv_dbias_finalize_channel(const float* __restrict__ partial, bf16_t* dbias, int C, int S, int c) {
+template <typename T>
+__device__ __forceinline__ void conv_dbias_finalize_channel(const float* __restrict__ partial, T* dbias, int C, int S, int c) {
     __shared__ float sw[4];
     float t = 0.0f;
     for (int sl = threadIdx.x; sl < S; sl += 256) t += partial[(size_t)sl * C + c];
@@ -401,8 +417,9 @@ __device__ __forceinline__ void conv_dbias_finalize_channel(const float* __restr
     __syncthreads();
     if (threadIdx.x == 0) st(dbias + c, ((sw[0] + sw[1]) + sw[2]) + sw[3]);
 }
-__global__ __launch_bounds__(256) void conv_dbias_finalize_kernel(const float* __restrict__ partial, bf16_t* dbias, int C, int S) {
-    conv_dbias_finalize_channel(partial, dbias, C, S, (int)blockIdx.x);
+template <typename T>
+__global__ __launch_bounds__(256) void conv_dbias_finalize_kernel(const float* __restrict__ partial, T* dbias, int C, int S) {
+    conv_dbias_finalize_channel<T>(partial, dbias, C, S, (int)blockIdx.x);
 }
 
 // dw[a, b, ci, g*Cout_g + col] = sum over slices of partial[slice][m' = t*Cin_g + ci][col].
@@ -414,7 +431,7 @@ __global__ __launch_bounds__(256) void wgrad_reduce_kernel(const float* __restri
                                                            int grp, int slices, int parts, int reduce_blocks, int Mrows, int Cp, int run, int64_t slice_stride,
                                                            BiasPartials bp) {
     if ((int)blockIdx.x >= reduce_blocks) {       // workgroups behind the reduction: one channel of the bias gradient each
-        conv_dbias_finalize_channel(bp.partial, bp.dbias, bp.C, bp.slices, (int)blockIdx.x - reduce_blocks);
+        conv_dbias_finalize_channel<T>(bp.partial, static_cast<T*>(bp.dbias), bp.C, bp.slices, (int)blockIdx.x - reduce_blocks);
         return;
     }
     // Cp: channels per tap in the partial sums (padded); run > 0: rows are [kb][run / 4 positions][4 channels] instead
@@ -552,43 +569,6 @@ static size_t dz_cwhn_partial_bytes(int P, int C, int N) {
     const int64_t groups = ceil_div(ceil_div(P, 64), dz_cwhn_chunk(P, C, N));
     return align256((size_t)groups * N * C * sizeof(float));
 }
-static bool dz_cwhn_ok(int P, int C, int N, const void* delta, const void* y, const void* pre, const void* dz, const void* dzT) {
-    return P % 8 == 0 && C % 8 == 0 && N >= 1 && aligned16(delta) && aligned16(y) && aligned16(pre) && aligned16(dz) && aligned16(dzT) &&
-           ceil_div(C, 64) <= 65535 && N + 4096 <= 65535;
-}
-// dz (may be NULL for the identity: dz is delta), dzT, the bias gradient (if dbias != NULL) and, if wout != NULL, the filter
-// repacked for the input-gradient kernel
-static int conv_dz_cwhn_pack(hipStream_t s, int act, const ConvGeom& g, const bf16_t* delta, const bf16_t* y, const bf16_t* pre,
-                             bf16_t* dz, bf16_t* dzT, float* partial, bf16_t* dbias, const bf16_t* w, bf16_t* wout, BiasPartials* later) {
-    const int P = g.OW * g.OH, C = g.Cout, N = g.N;
-    const int chunk = dz_cwhn_chunk(P, C, N);
-    const int64_t gx = ceil_div(ceil_div(P, 64), chunk), gy = ceil_div(C, 64);
-    const int64_t pack_blocks = wout != nullptr ? ceil_div((int64_t)g.kW * g.kH * g.Cin_g * g.Cout, 256) : 0;
-    const int64_t gz = N + ceil_div(pack_blocks, gx * gy);
-    LUX_UNSUPPORTED_IF(gz > 65535, "conv: filter too large for the combined layout pass");
-    float* const part = dbias != nullptr ? partial : nullptr;
-    const dim3 grid((unsigned)gx, (unsigned)gy, (unsigned)gz);
-#define LAUNCH_DZC(A) conv_dz_cwhn_pack_kernel<A><<<grid, 256, 0, s>>>(delta, y, pre, dz, dzT, part, P, C, N, chunk, w, wout, g)
-    {
-        ProfScope ps("conv_dz_cwhn_pack_kernel", s);
-        LUX_DISPATCH_ACT(act, LAUNCH_DZC);
-    }
-#undef LAUNCH_DZC
-    LUX_CHECK_LAUNCH();
-    if (dbias != nullptr) {
-        if (later != nullptr) {           // the caller adds the channels' sums to a later launch
-            later->partial = partial; later->dbias = dbias; later->C = C; later->slices = (int)(gx * N);
-            return LUXHIP_OK;
-        }
-        ProfScope ps2("conv_dbias_finalize_kernel", s);
-        conv_dbias_finalize_kernel<<<(unsigned)C, 256, 0, s>>>(partial, dbias, C, (int)(gx * N));
-        LUX_CHECK_LAUNCH();
-    }
-    return LUXHIP_OK;
-}
-
-// ----------------------------------------------------------------------------- any channel count, any stride (conv_any.h)
-// Channels of a group padded to whole 16-byte chunks
 template <typename T>
 static int padded(int c) {
     constexpr int V = GemmTraits<T>::VEC;
@@ -753,6 +733,52 @@ struct AnyPlan {
 
 // Padded channel-contiguous copy of the first `groups` groups of `in`, which has Cin channels (if out != NULL), and the packed
 // filter of all groups of a launch (if wout != NULL), in one launch
+// The single pass pays where a tile is not mostly empty; smaller ragged planes and channel counts take the two passes
+template <typename T>
+static bool dz_cwhn_ok(int P, int C, int N) {
+    return ((P >= 32 && C >= 16) || (sizeof(T) == 2 && P % 8 == 0 && C % 8 == 0)) && ceil_div(C, 64) <= 65535 && N >= 1 && N + 4096 <= 65535;
+}
+
+// dz may be null; wout: the filter for the input gradient, packed by `ps` (general kernels) or as pack_filter does (ps null)
+template <typename T>
+static int conv_dz_cwhn_pack(hipStream_t s, int act, const ConvGeom& g, int Cp, const T* delta, const T* y, const T* pre, T* dz, T* dzT, float* partial, T* dbias,
+                             const T* w, T* wout, const PackSubs* ps, BiasPartials* later) {
+    constexpr int V = Vec<T>::N;
+    const int P = g.OW * g.OH, C = g.Cout, N = g.N;
+    const int chunk = dz_cwhn_chunk(P, C, N);
+    const int64_t gx = ceil_div(ceil_div(P, 64), chunk), gy = ceil_div(C, 64);
+    const int64_t pack_blocks = wout == nullptr ? 0 : ceil_div(ps != nullptr ? ps->total : (int64_t)g.kW * g.kH * g.Cin_g * g.Cout, 256);
+    const int64_t gz = N + ceil_div(pack_blocks, gx * gy);
+    LUX_UNSUPPORTED_IF(gz > 65535, "conv: filter too large for the combined layout pass");
+    float* const part = dbias != nullptr ? partial : nullptr;
+    PackSubs subs;
+    subs.n = 0; subs.total = 0;
+    if (wout != nullptr && ps != nullptr) subs = *ps;
+    const bool whole = P % V == 0 && C % V == 0 && Cp == C && aligned16(delta) && aligned16(y) && aligned16(pre) && aligned16(dz);
+    const dim3 grid((unsigned)gx, (unsigned)gy, (unsigned)gz);
+#define LAUNCH_DZC(A)                                                                                                                         \
+    do {                                                                                                                                      \
+        if (whole) conv_dz_cwhn_pack_kernel<T, A, false><<<grid, 256, 0, s>>>(delta, y, pre, dz, dzT, part, P, C, Cp, N, chunk, w, wout, g, subs); \
+        else conv_dz_cwhn_pack_kernel<T, A, true><<<grid, 256, 0, s>>>(delta, y, pre, dz, dzT, part, P, C, Cp, N, chunk, w, wout, g, subs);        \
+    } while (0)
+    {
+        ProfScope prof("conv_dz_cwhn_pack_kernel", s);
+        LUX_DISPATCH_ACT(act, LAUNCH_DZC);
+    }
+#undef LAUNCH_DZC
+    LUX_CHECK_LAUNCH();
+    if (dbias != nullptr) {
+        if (later != nullptr) {           // the caller adds the channels' sums to a later launch
+            later->partial = partial; later->dbias = dbias; later->C = C; later->slices = (int)(gx * N);
+            return LUXHIP_OK;
+        }
+        ProfScope ps2("conv_dbias_finalize_kernel", s);
+        conv_dbias_finalize_kernel<T><<<(unsigned)C, 256, 0, s>>>(partial, dbias, C, (int)(gx * N));
+        LUX_CHECK_LAUNCH();
+    }
+    return LUXHIP_OK;
+}
+
 template <typename T>
 static int pad_and_pack(hipStream_t s, const T* in, T* out, int P, int Cin, int Cg, int groups, int N, int zeros, const T* w, T* wout, const ConvGeom& g,
                         const PackSubs* ps) {
@@ -972,14 +998,14 @@ static size_t wgrad_partial_bytes(const ConvGeom& g) {
     return align256(bytes);
 }
 
-// runs: xT is the copy of runs_copy_pack.  dy: WHCN cotangent (used by the window and the direct bf16 kernels); dyT: its channel-contiguous copy with padded channels,
+// runs: xT is the copy of runs_copy_pack.  dy: WHCN cotangent (used by the window and the direct bf16 kernels; null: not there); dyT: its channel-contiguous copy with padded channels,
 // followed by BK positions of zeros where there are fewer than BK positions in all (used by the general kernel).  Where
 // channels are padded, xT / dyT hold the groups `gr` alone, else all of them.
 template <typename T>
 static int run_wgrad(hipStream_t s, const ConvGeom& g, Groups gr, Runs runs, const T* xT, const T* dy, const T* dyT, float* partial, T* dw,
                      const void* zeros, const BiasPartials* bias = nullptr) {
-    const bool direct = wgrad_direct_ok<T>(g, xT, dy);
-    const bool window = wgrad_window_shape<T>(g) && aligned16(xT) && aligned16(dy) && aligned16(partial);
+    const bool direct = dy != nullptr && wgrad_direct_ok<T>(g, xT, dy);
+    const bool window = dy != nullptr && wgrad_window_shape<T>(g) && aligned16(xT) && aligned16(dy) && aligned16(partial);
     WgradPlan plan;
     int rc = wgrad_plan<T>(g, !direct && !window, runs, &plan);
     if (rc != LUXHIP_OK) return rc;
@@ -1226,12 +1252,11 @@ static int fused_conv_bwd_t(hipStream_t s, int dtype, int act, const ConvGeom& g
     AnyPlan<T> plan(g, true);
     const int n = groups_at_a_time<T>(g, dw != nullptr && !kept, true);
     const size_t xb = kept ? 0 : xt_bytes<T>(g, n), yb = dyt_bytes<T>(g, n), wb = filter_bytes<T>(g, any, plan), pb = wgrad_partial_bytes<T>(g);
-    // bf16: dz, its channel-contiguous copy and the bias gradient in one pass, when both a pass over delta and a
-    // transposing copy would run
-    bool one_pass = false;
-    if constexpr (sizeof(T) == 2)
-        one_pass = (act != LUXHIP_ACT_IDENTITY || dbias != nullptr) && (dw != nullptr || dx != nullptr) && padded<T>(g.Cout_g) == g.Cout_g &&
-                   dy_zeros<T>(g) == 0 && dz_cwhn_ok(g.OW * g.OH, g.Cout, g.N, delta, y, pre, dz, nullptr);
+    // dz channel-contiguous, the bias gradient and, where the filter gradient reads it, dz as it lies in one pass, when both a pass over
+    // delta and a transposing copy would run
+    const int Cp = padded<T>(g.Cout_g);
+    const bool one_pass = (act != LUXHIP_ACT_IDENTITY || dbias != nullptr) && (dw != nullptr || dx != nullptr) &&
+                          (Cp == g.Cout_g || g.groups == 1) && dy_zeros<T>(g) == 0 && dz_cwhn_ok<T>(g.OW * g.OH, g.Cout, g.N);
     const size_t bb = one_pass && dbias != nullptr ? dz_cwhn_partial_bytes(g.OW * g.OH, g.Cout, g.N) : 0;
     // reserve everything up front: the bias-gradient pass below uses the start of the same
     // workspace, and the buffer must not be reallocated while pointers into it are live
@@ -1246,17 +1271,15 @@ static int fused_conv_bwd_t(hipStream_t s, int dtype, int act, const ConvGeom& g
     bool packed = dx != nullptr;          // the filter is in wD when the input gradient starts
     BiasPartials bias_later;              // set by the single pass when the filter gradient's reduction will finish the bias gradient
     if (one_pass) {
-        if constexpr (sizeof(T) == 2) {
-            bf16_t* dz_out = act == LUXHIP_ACT_IDENTITY ? nullptr : reinterpret_cast<bf16_t*>(dz);
-            packed = packed && !any;
-            rc = conv_dz_cwhn_pack(s, act, g, reinterpret_cast<const bf16_t*>(delta), reinterpret_cast<const bf16_t*>(y),
-                                   reinterpret_cast<const bf16_t*>(pre), dz_out, reinterpret_cast<bf16_t*>(dzT),
-                                   reinterpret_cast<float*>(ws.data + xb + yb + wb + pb), reinterpret_cast<bf16_t*>(dbias),
-                                   reinterpret_cast<const bf16_t*>(w), packed ? reinterpret_cast<bf16_t*>(wD) : nullptr,
-                                   dw != nullptr ? &bias_later : nullptr);
-            if (rc != LUXHIP_OK) return rc;
-            if (dz_out) dzp = dz;
-        }
+        const bool lies = dw != nullptr && (wgrad_direct_ok<T>(g, xT, dz) || (wgrad_window_shape<T>(g) && aligned16(xT) && aligned16(dz)));
+        T* const dz_out = act != LUXHIP_ACT_IDENTITY && lies ? dz : nullptr;
+        packed = packed && !(any && plan.launches.empty());
+        PackSubs ps;
+        if (packed && any) ps = plan.pack(g, true, 0);
+        rc = conv_dz_cwhn_pack<T>(s, act, g, g.groups == 1 ? Cp : g.Cout, delta, y, pre, dz_out, dzT, reinterpret_cast<float*>(ws.data + xb + yb + wb + pb), dbias, w,
+                                  packed ? wD : nullptr, packed && any ? &ps : nullptr, dw != nullptr ? &bias_later : nullptr);
+        if (rc != LUXHIP_OK) return rc;
+        if (act != LUXHIP_ACT_IDENTITY) dzp = dz_out;             // null: only the channel-contiguous one is there
     } else {
         if (act != LUXHIP_ACT_IDENTITY || dbias != nullptr) {
             T* dz_out = act == LUXHIP_ACT_IDENTITY ? nullptr : dz;
