@@ -155,17 +155,18 @@ static int ragged_gradients(hipStream_t s, int act, int64_t M, int64_t K, int64_
     return ragged_product(s, K, N, M, sw, Side{padded ? out : dz_dense, padded ? Mp : M, N, true, true}, nullptr, dx, K, nullptr, LUXHIP_ACT_IDENTITY, slices_x, front);
 }
 
+// Whether the two products of a pullback may run at the same time.  One after the other dW is done with x before dx is written, so a caller may let dx
+// take x's memory.
+static bool dx_apart_from_x(int dtype, int64_t K, int64_t N, const void* x, int64_t ldx, const void* dx) {
+    const size_t e = dtype == LUXHIP_F32 ? 4 : 2;
+    const uintptr_t px = reinterpret_cast<uintptr_t>(x), pd = reinterpret_cast<uintptr_t>(dx);
+    return pd + (size_t)(K * N) * e <= px || px + (size_t)((N - 1) * ldx + K) * e <= pd;
+}
+
 // dW (M x K) = dz (M x N) * x' and dx (K x N) = W' * dz in one launch; false if they are not small enough for it
 template <typename T>
 static bool gradient_pair(hipStream_t s, int64_t M, int64_t K, int64_t N, const T* dz, const T* W, int64_t ldw, const T* x, int64_t ldx,
                           T* dW, T* dx, int* rc) {
-    if (gemm_tile_override() != 0 || M < 1 || N < 1 || K < 1 || ldw < M || ldx < K) return false;
-    // one after the other dW is done with x before dx is written, so a caller may let dx take x's memory
-    auto apart = [](const T* a, int64_t na, const T* b, int64_t nb) {
-        const uintptr_t pa = reinterpret_cast<uintptr_t>(a), pb = reinterpret_cast<uintptr_t>(b);
-        return pa + (size_t)na * sizeof(T) <= pb || pb + (size_t)nb * sizeof(T) <= pa;
-    };
-    if (!apart(dx, K * N, x, (N - 1) * ldx + K)) return false;
     DenseArgs<T> a = dense_args<T>(false, false, M, K, N, dz, M, x, ldx, nullptr, dW, M, nullptr, LUXHIP_ACT_IDENTITY);
     DenseArgs<T> b = dense_args<T>(true, true, K, N, M, W, ldw, dz, M, nullptr, dx, K, nullptr, LUXHIP_ACT_IDENTITY);
     return launch_split_pair<T>(s, a, b, rc);
@@ -560,6 +561,16 @@ int luxhip_fused_dense_bwd(luxhip_stream_t s, int dtype, int act, int64_t M, int
                               (const bf16_t*)x, ldx, (bf16_t*)dz, (bf16_t*)dW, (bf16_t*)dx, (bf16_t*)dbias, &done);
         if (done) return rc;
     }
+    const bool together = dW != nullptr && dx != nullptr && W != nullptr && x != nullptr && gemm_tile_override() == 0 && M >= 1 && N >= 1 && K >= 1 &&
+                          ldw >= M && ldx >= K && dx_apart_from_x(dtype, K, N, x, ldx, dx);
+    if (together) {
+        const bool done = dtype == LUXHIP_F32
+            ? launch_small_layer_bwd<float>((hipStream_t)s, act, M, K, N, (const float*)delta, (const float*)y, (const float*)pre, (const float*)W, ldw,
+                                            (const float*)x, ldx, (float*)dW, (float*)dx, (float*)dbias, &rc)
+            : launch_small_layer_bwd<bf16_t>((hipStream_t)s, act, M, K, N, (const bf16_t*)delta, (const bf16_t*)y, (const bf16_t*)pre, (const bf16_t*)W, ldw,
+                                             (const bf16_t*)x, ldx, (bf16_t*)dW, (bf16_t*)dx, (bf16_t*)dbias, &rc);
+        if (done) return rc;
+    }
     if (act != LUXHIP_ACT_IDENTITY || dbias != nullptr) {
         // dz = delta .* act'(y, pre) and dbias = sum over the batch, one pass (dense layout: I = 1)
         void* dz_out = act == LUXHIP_ACT_IDENTITY ? nullptr : dz;
@@ -567,7 +578,7 @@ int luxhip_fused_dense_bwd(luxhip_stream_t s, int dtype, int act, int64_t M, int
         if (rc != LUXHIP_OK) return rc;
         if (dz_out) dzp = dz_out;
     }
-    if (dW != nullptr && dx != nullptr && W != nullptr && x != nullptr) {
+    if (together) {
         const bool done = dtype == LUXHIP_F32
             ? gradient_pair<float>((hipStream_t)s, M, K, N, (const float*)dzp, (const float*)W, ldw, (const float*)x, ldx, (float*)dW, (float*)dx, &rc)
             : gradient_pair<bf16_t>((hipStream_t)s, M, K, N, (const bf16_t*)dzp, (const bf16_t*)W, ldw, (const bf16_t*)x, ldx, (bf16_t*)dW, (bf16_t*)dx, &rc);

@@ -52,6 +52,14 @@ bool launch_split(hipStream_t s, DenseArgs<T>& a, bool a_kmajor, bool b_kmajor, 
 template <typename T>
 bool launch_split_pair(hipStream_t s, DenseArgs<T>& a, DenseArgs<T>& b, int* rc);
 
+// gemm_small.hip: fp32 products that are faster in tiles of 32; false if the problem is another one
+bool launch_small(hipStream_t s, DenseArgs<float>& a, bool a_kmajor, bool b_kmajor, int* rc);
+// the pullback of a small dense layer in one launch: dz = delta .* act'(y, pre), dW = dz x', dx = W' dz, dbias (may be null) = sum over n of dz;
+// delta, y, pre: M x N without gaps.  false if the layer is another one
+template <typename T>
+bool launch_small_layer_bwd(hipStream_t s, int act, int64_t M, int64_t K, int64_t N, const T* delta, const T* y, const T* pre, const T* W, int64_t ldw,
+                            const T* x, int64_t ldx, T* dW, T* dx, T* dbias, int* rc);
+
 // gemm_split_batched_f32.hip: batched fp32 products that are faster there; false if the problem is another one
 bool launch_split_batched(hipStream_t s, DenseArgs<float>& a, bool a_kmajor, bool b_kmajor, int* rc);
 

@@ -120,14 +120,16 @@ bool split_takes(const DenseArgs<T>& a) {
 template <typename T>
 bool launch_split(hipStream_t s, DenseArgs<T>& a, bool ak, bool bk, int* rc) {
     if (!split_takes(a)) return false;
+    if constexpr (sizeof(T) == 4) {
+        if (launch_small(s, a, ak, bk, rc)) return true;
+    }
     const split::Choice c = split::choose<T>(a.M, a.N, a.K);
     *rc = c.w == 2 ? split::launch_layouts<T, 2>(s, a, ak, bk, c.slices) : split::launch_layouts<T, 1>(s, a, ak, bk, c.slices);
     return true;
 }
 
 // One launch for two products that do not depend on each other (dW: both operands contiguous along m / n; dx: both along
-// k), where both are small: a launch of its own costs 2 to 4 us, as much as such a product (256 x 128 x 64 in fp32: 4.3 +
-// 6.9 us apart).
+// k), where both are small, but too large for gemm_small.hip: a launch of its own costs 2 to 4 us.
 template <typename T>
 bool launch_split_pair(hipStream_t s, DenseArgs<T>& a, DenseArgs<T>& b, int* rc) {
     using namespace split;
