@@ -430,31 +430,34 @@ __global__ __launch_bounds__(64) void ln_param_grad_kernel(const T* __restrict__
         if (!RAGGED || (uint32_t)e >= ln_skip<VEC, RAGGED>(q, L)) { pg[o + e] = ag[e]; pb[o + e] = ab[e]; }
 }
 
-// dgamma[l] = sum_s pg[s][l], dbeta likewise.  Workgroup of LW positions x (1024 / LW) slice groups:
-// group g adds slices g, g + G, ... and the G group sums are added in group order.  LW = 32 gives
-// L / 32 workgroups (128-byte row segments): enough of them to fill the device for L of a few thousand.
+// dgamma[l] = sum_s pg[s][l], dbeta likewise.  Workgroup of LW positions x (1024 / LW) slice groups: group g adds slices g, g + G, ...,
+// U of each sum in flight whether or not there are as many, and the G group sums are added in group order.  Bound by the latency of the trips:
+// the last few slices of a thread took one each (249 slices of 1862 positions: pass 20.2 -> 19.2 us).  16 positions a workgroup or eight loads in
+// flight gain nothing with 768 slices and lose with 4096 positions (69.1 -> 72.1 and 69.5).  LW = 32: 128-byte row segments, and
+// L / 32 workgroups fill the device for L of a few thousand.
 constexpr int kLnFinalizeWidth = 32;
 template <typename T>
 __global__ __launch_bounds__(1024) void ln_param_finalize_kernel(const float* __restrict__ pg, const float* __restrict__ pb,
                                                                  T* dgamma, T* dbeta, uint32_t L, uint32_t S) {
-    constexpr int LW = kLnFinalizeWidth, G = 1024 / LW;
+    constexpr int LW = kLnFinalizeWidth, G = 1024 / LW, U = 4;
     __shared__ float sg[G][LW], sb[G][LW];
     const uint32_t lx = threadIdx.x % LW, grp = threadIdx.x / LW;
-    const uint32_t l = blockIdx.x * LW + lx;
+    const uint32_t l = blockIdx.x * LW + lx, lc = min(l, L - 1);
     float tg = 0.0f, tb = 0.0f;
-    if (l < L) {
-        uint32_t s = grp;
-        for (; s + 3 * G < S; s += 4 * G) {          // four independent loads in flight
-            const float g0 = pg[(size_t)s * L + l], g1 = pg[(size_t)(s + G) * L + l];
-            const float g2 = pg[(size_t)(s + 2 * G) * L + l], g3 = pg[(size_t)(s + 3 * G) * L + l];
-            const float b0 = pb[(size_t)s * L + l], b1 = pb[(size_t)(s + G) * L + l];
-            const float b2 = pb[(size_t)(s + 2 * G) * L + l], b3 = pb[(size_t)(s + 3 * G) * L + l];
-            tg = (((tg + g0) + g1) + g2) + g3;
-            tb = (((tb + b0) + b1) + b2) + b3;
+    for (uint32_t s = grp; s < S; s += U * G) {
+        float vg[U], vb[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {                // past the end: the last slice again, not added
+            const size_t at = (size_t)min(s + u * G, S - 1) * L + lc;
+            vg[u] = pg[at];
+            vb[u] = pb[at];
         }
-        for (; s < S; s += G) {
-            tg += pg[(size_t)s * L + l];
-            tb += pb[(size_t)s * L + l];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            if (s + u * G < S) {
+                tg += vg[u];
+                tb += vb[u];
+            }
         }
     }
     sg[grp][lx] = tg;
