@@ -135,13 +135,22 @@ __global__ __launch_bounds__(THREADS) void skinny_gemm_kernel(Args<T> a) {
         publish_done();
         if (!arrive_last(a.counters + block, (uint32_t)a.slices, &flag)) return;
         const float* all = a.partial + (size_t)block * a.slices * (NMAX * MT);
+        // the values of a thread (as many as any has, in the workgroup) and four slices on their way together, without conditions between
+        auto add = [&](auto COUNT) {
+            constexpr int count = decltype(COUNT)::value;
 #pragma unroll
-        for (int u = 0; u < 4; ++u) {
-            const int e = threadIdx.x + u * THREADS;
-            v[u] = 0.0f;
-            if (e < total)
+            for (int u = 0; u < count; ++u) v[u] = 0.0f;
 #pragma unroll 4
-                for (int q = 0; q < a.slices; ++q) v[u] += fetch(all + (size_t)q * (NMAX * MT) + e);
+            for (int q = 0; q < a.slices; ++q)
+#pragma unroll
+                for (int u = 0; u < count; ++u)
+                    v[u] += fetch(all + (size_t)q * (NMAX * MT) + min((int)threadIdx.x + u * THREADS, total - 1));
+        };
+        switch ((total - 1) / THREADS) {
+            case 0: add(std::integral_constant<int, 1>{}); break;
+            case 1: add(std::integral_constant<int, 2>{}); break;
+            case 2: add(std::integral_constant<int, 3>{}); break;
+            default: add(std::integral_constant<int, 4>{}); break;
         }
     }
 #pragma unroll
@@ -166,9 +175,18 @@ int launch(hipStream_t s, const DenseArgs<T>& d) {
     a.ldw = d.A.sk; a.ldx = d.B.sr; a.ldy = d.ldc;
     a.M = d.M; a.N = d.N; a.K = d.K; a.act = d.act;
     const int64_t cus = num_cus() > 0 ? num_cus() : 256, blocks = ceil_div(d.M, MT);
-    // at most one workgroup (eight waves with sixteen loads in flight each) per compute unit: a second one gains nothing
-    // (11008 x 4096: 18.6 us against 20.4 with two in bf16, 29.7 against 38.2 in fp32); at least two steps of k per wave
-    int64_t slices = std::max<int64_t>(1, std::min<int64_t>(cus / blocks, d.K / (2 * KSTEP * WAVES)));
+    // At most one workgroup (eight waves with sixteen loads in flight each) per compute unit: a second one gains nothing
+    // (11008 x 4096: 18.6 us against 20.4 with two in bf16, 29.7 against 38.2 in fp32).  Below that a workgroup's step of k costs what its 64 (32)
+    // KiB take at the 35 bytes per ns that a compute unit loads, the hand-off 3.2 us and 0.2 for each slice's partial sums, apart from their bytes
+    // (us, at least two steps a wave before / now: bf16 1355 -> 3753, 2 columns 8.5 / 6.9, 4096 -> 4096, 16 columns 13.7 / 12.1, 12000 -> 704, 6 columns 9.5 / 8.6;
+    // fp32 700 -> 2000, 16 columns 7.6 / 6.8; 4096 -> 11008, 3 columns 18.1 / 18.1; 598 -> 1028, 15 columns stays whole: 6.8, in three slices 7.3).
+    const double step_us = sizeof(T) == 2 ? 1.9 : 0.95, slice_us = 0.2 + (double)d.N * MT * 4.0 / 35e3;
+    int64_t slices = 1;
+    double t_best = 1e30;
+    for (int64_t sl = 1; sl <= std::max<int64_t>(1, cus / blocks) && sl <= ceil_div(d.K, KSTEP * WAVES); ++sl) {
+        const double t = (double)ceil_div(d.K, sl * KSTEP * WAVES) * step_us + (sl > 1 ? 3.2 + (double)sl * slice_us : 0.0);
+        if (t < t_best) { t_best = t; slices = sl; }
+    }
     if (blocks > (int64_t)kWorkspaceCounters) slices = 1;
     if (slices > 1 && !workspace_holds(s, (size_t)blocks * slices * NMAX * MT * sizeof(float))) slices = 1;
     a.kwave = (int)(ceil_div(ceil_div(d.K, slices * WAVES), KSTEP) * KSTEP);

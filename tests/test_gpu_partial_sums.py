@@ -38,3 +38,16 @@ def test_dense_bias_gradient(gpu, dtype, M, N):
     gW, gx, gb = back(dev(gpu, d, dtype))
     assert_close(gb.to_numpy().reshape(-1), f64(d).sum(1), dtype, "db")
     assert_close(gW.to_numpy(), f64(d) @ f64(x).T, dtype, "dW")
+
+
+@pytest.mark.parametrize("dtype,K", [("bf16", 1440), ("f32", 1203)])
+@pytest.mark.parametrize("N", [1, 4, 5, 8, 9, 12, 13, 16])
+def test_slices_of_a_few_columns(gpu, dtype, K, N):
+    """Serving a few columns, the contraction in several slices: one to four values a thread.  Values are -1, 0 or 1, so every partial sum and
+    (below 2^8 in bf16: 1440 terms of variance 4/9 stay within 6.5 x 25) the result are exact."""
+    rng = np.random.default_rng(stable_seed("few columns", dtype, N))
+    W, x = rng.integers(-1, 2, size=(700, K)).astype(np.float32), rng.integers(-1, 2, size=(K, N)).astype(np.float32)
+    got = gpu.matmul(dev(gpu, W, dtype), dev(gpu, x, dtype), None, False, False).to_numpy()
+    want = W @ x
+    assert np.abs(want).max() < 256
+    np.testing.assert_array_equal(got, want)
