@@ -33,10 +33,10 @@ struct ConvGeom {
 // Epilogue of fprop / dgrad: element (m = (p, q, n), col) -> out[(m - n*PQ) + PQ*(col_off + col +
 // Ctot_out*n)], with bias per output channel and the activation.  The image index of a row is
 // decoded once per row, the channel terms once per column.  CHECK (tiles that stick out of the
-// matrix), the activation mode and HAS_PRE are resolved once per tile.
-template <class ML, typename T, int WM, int WN, bool CHECK, int ACT_MODE, bool HAS_PRE>
+// matrix), the activation are resolved once per tile.
+template <class ML, typename T, int WM, int WN, bool CHECK, int ACT>
 __device__ __forceinline__ void conv_epilogue_as(const f32x16_v (&acc)[WM][WN], int m0, int n0, int M, int PQ, FastDiv divPQ,
-                                                 int Ncols, int col_off, int Ctot_out, const T* bias, T* out, T* pre, int act) {
+                                                 int Ncols, int col_off, int Ctot_out, const T* bias, T* out, T* pre) {
     const int mb = ML::lane_m(m0), nb = ML::lane_n(n0);
     int64_t rowoff[WM];
     bool mok[WM];
@@ -57,13 +57,12 @@ __device__ __forceinline__ void conv_epilogue_as(const f32x16_v (&acc)[WM][WN], 
                 float v[WM];
 #pragma unroll
                 for (int i = 0; i < WM; ++i) v[i] = acc[i][j][r] + b;
-                if constexpr (HAS_PRE) {
+                if (pre != nullptr) {
 #pragma unroll
                     for (int i = 0; i < WM; ++i)
                         if (!CHECK || mok[i]) st(pre + coloff + rowoff[i], v[i]);
                 }
-                if constexpr (ACT_MODE == 1) act_vec_as<LUXHIP_ACT_RELU>(v);
-                else if constexpr (ACT_MODE == 2) act_vec(act, v);
+                act_vec_as<ACT>(v);
 #pragma unroll
                 for (int i = 0; i < WM; ++i)
                     if (!CHECK || mok[i]) st(out + coloff + rowoff[i], v[i]);
@@ -75,21 +74,15 @@ template <class ML, typename T, int WM, int WN>
 __device__ __forceinline__ void conv_epilogue(const f32x16_v (&acc)[WM][WN], int m0, int n0, int M, int PQ, FastDiv divPQ,
                                               int Ncols, int col_off, int Ctot_out, const T* bias, T* out, T* pre, int act) {
     const bool check = m0 + ML::TILE_M > M || n0 + ML::TILE_N > Ncols;
-    const bool has_pre = pre != nullptr;
-    // activation: 0 none, 1 relu (inline), 2 any (dispatched per column of the accumulator tile)
-#define LUX_CONV_EPI(C, A, P) conv_epilogue_as<ML, T, WM, WN, C, A, P>(acc, m0, n0, M, PQ, divPQ, Ncols, col_off, Ctot_out, bias, out, pre, act)
-    if (check) {                                 // rare: general variants
-        if (has_pre) LUX_CONV_EPI(true, 2, true);
-        else LUX_CONV_EPI(true, 2, false);
-    } else if (has_pre) {
-        LUX_CONV_EPI(false, 2, true);
-    } else if (act == LUXHIP_ACT_IDENTITY) {
-        LUX_CONV_EPI(false, 0, false);
-    } else if (act == LUXHIP_ACT_RELU) {
-        LUX_CONV_EPI(false, 1, false);
-    } else {
-        LUX_CONV_EPI(false, 2, false);
-    }
+    // one activation's code for all columns in one piece, see dense_epilogue
+#define LUX_CONV_EPI_AS(C, A) conv_epilogue_as<ML, T, WM, WN, C, A>(acc, m0, n0, M, PQ, divPQ, Ncols, col_off, Ctot_out, bias, out, pre)
+#define LUX_CONV_EPI(A)                           \
+    do {                                          \
+        if (check) LUX_CONV_EPI_AS(true, A);      \
+        else LUX_CONV_EPI_AS(false, A);           \
+    } while (0)
+    LUX_DISPATCH_ACT(act, LUX_CONV_EPI);
+#undef LUX_CONV_EPI_AS
 #undef LUX_CONV_EPI
 }
 

@@ -153,18 +153,21 @@ __global__ __launch_bounds__(THREADS) void skinny_gemm_kernel(Args<T> a) {
             default: add(std::integral_constant<int, 4>{}); break;
         }
     }
+    // the bias of all values together, and one activation's code for them in one piece
+    auto each = [&](auto&& f) {
 #pragma unroll
-    for (int u = 0; u < 4; ++u) {
-        const int e = threadIdx.x + u * THREADS;
-        if (e < total) {
-            const int n = e / MT, m = m0 + e % MT;
-            const int64_t off = (int64_t)n * a.ldy + m;
-            float o[1] = {v[u] + (a.bias ? ld(a.bias + m) : 0.0f)};
-            if (a.pre) st(a.pre + off, o[0]);
-            act_vec(a.act, o);
-            st(a.y + off, o[0]);
+        for (int u = 0; u < 4; ++u) {
+            const int e = threadIdx.x + u * THREADS, n = e / MT, m = m0 + e % MT;
+            if (e < total) f(u, (int64_t)n * a.ldy + m);
         }
+    };
+    if (a.bias) {
+#pragma unroll
+        for (int u = 0; u < 4; ++u) v[u] += ld(a.bias + m0 + (threadIdx.x + u * THREADS) % MT);
     }
+    if (a.pre) each([&](int u, int64_t off) { st(a.pre + off, v[u]); });
+    act_vec(a.act, v);
+    each([&](int u, int64_t off) { st(a.y + off, v[u]); });
 }
 
 template <typename T>
