@@ -136,17 +136,17 @@ __global__ __launch_bounds__(THREADS) void skinny_gemm_kernel(Args<T> a) {
         if (!arrive_last(a.counters + block, (uint32_t)a.slices, &flag)) return;
         const float* all = a.partial + (size_t)block * a.slices * (NMAX * MT);
         // the values of a thread (as many as any has, in the workgroup) and four slices on their way together, without conditions between
+#pragma unroll
+        for (int u = 0; u < 4; ++u) v[u] = 0.0f;
         auto add = [&](auto COUNT) {
             constexpr int count = decltype(COUNT)::value;
-#pragma unroll
-            for (int u = 0; u < count; ++u) v[u] = 0.0f;
 #pragma unroll 4
             for (int q = 0; q < a.slices; ++q)
 #pragma unroll
                 for (int u = 0; u < count; ++u)
                     v[u] += fetch(all + (size_t)q * (NMAX * MT) + min((int)threadIdx.x + u * THREADS, total - 1));
         };
-        switch ((total - 1) / THREADS) {
+        if (w * 64 < total) switch ((total - 1) / THREADS) {        // waves without a value have none to ask for
             case 0: add(std::integral_constant<int, 1>{}); break;
             case 1: add(std::integral_constant<int, 2>{}); break;
             case 2: add(std::integral_constant<int, 3>{}); break;
