@@ -33,7 +33,7 @@ struct ConvGeom {
 // Epilogue of fprop / dgrad: element (m = (p, q, n), col) -> out[(m - n*PQ) + PQ*(col_off + col +
 // Ctot_out*n)], with bias per output channel and the activation.  The image index of a row is
 // decoded once per row, the channel terms once per column.  CHECK (tiles that stick out of the
-// matrix), the activation are resolved once per tile.
+// matrix) and the activation are resolved once per tile.
 template <class ML, typename T, int WM, int WN, bool CHECK, int ACT>
 __device__ __forceinline__ void conv_epilogue_as(const f32x16_v (&acc)[WM][WN], int m0, int n0, int M, int PQ, FastDiv divPQ,
                                                  int Ncols, int col_off, int Ctot_out, const T* bias, T* out, T* pre) {

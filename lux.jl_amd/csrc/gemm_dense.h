@@ -12,8 +12,8 @@
 
 namespace luxhip {
 
-// Epilogue of one tile: C = act(acc + bias), optional pre-activation copy.  CHECK: bounds tests;
-// the activation are resolved once per tile, so the common cases have no branch per element.
+// Epilogue of one tile: C = act(acc + bias), optional pre-activation copy.  CHECK (bounds tests)
+// and the activation are resolved once per tile, so there is no choice between them per element.
 // WM consecutive values of one column -> memory; one store when the lane's rows are consecutive
 // (ML::M_STEP == 1), the storage type is bf16 and the destination allows it
 template <class ML, typename T, int WM, bool CHECK>
