@@ -53,14 +53,15 @@ static DenseArgs<T> dense_args(bool a_kmajor, bool b_kmajor, int64_t M, int64_t 
 }
 
 // ------------------------------------------------------------------------------- ragged products on the 256 x 256 kernel
-// An operand of a large bf16 product as the caller has it, or (`ready`) as the kernel reads it: k contiguous, rows of whole steps.
+// An operand of a large bf16 product as the caller has it, or (`ready`) as the kernel reads it: k contiguous, rows of whole steps, no further apart
+// than it can address (rows of a taller matrix are copied).
 struct Side {
     const bf16_t* p;
     int64_t ld, rows;
     bool kmajor, ready;
 };
 static Side side(const bf16_t* p, int64_t ld, int64_t rows, bool kmajor, int64_t K) {
-    return Side{p, ld, rows, kmajor, kmajor && K % 64 == 0 && ld % 8 == 0 && aligned16(p)};
+    return Side{p, ld, rows, kmajor, kmajor && K % 64 == 0 && ld % 8 == 0 && kk256_row_distance_ok(ld) && aligned16(p)};
 }
 static int64_t whole_steps(int64_t K) { return ceil_div(K, 64) * 64; }
 static size_t copy_bytes(const Side& a, int64_t K) { return a.ready ? 0 : align256((size_t)a.rows * whole_steps(K) * sizeof(bf16_t)); }
@@ -86,7 +87,7 @@ static double big_time(int64_t M, int64_t N, int64_t K, const Side& A, const Sid
 static int ragged_slices(hipStream_t s, int64_t M, int64_t N, int64_t K, const Side& A, const Side& B, size_t front) {
     if (option_gemm_pretranspose() == 0 || gemm_tile_override() != 0 || M < 256 || N < 256 || K < 128) return 0;
     const int64_t Kp = whole_steps(K), tiles = ceil_div(M, 256) * ceil_div(N, 256), chunk_limit = (int64_t(1) << 31) - 2048;
-    if (256 * Kp * 2 >= (int64_t(1) << 31) || tiles >= (int64_t(1) << 27) || M * (Kp / 8) >= chunk_limit || N * (Kp / 8) >= chunk_limit ||
+    if (!kk256_row_distance_ok(Kp) || tiles >= (int64_t(1) << 27) || M * (Kp / 8) >= chunk_limit || N * (Kp / 8) >= chunk_limit ||
         (M + 8) * N >= (int64_t(1) << 33) || ceil_div(K, 64) > 65535) return 0;
     const bool whole = M % 256 == 0 && N % 256 == 0 && K % 32 == 0 && aligned16(A.p) && A.ld % 8 == 0 && aligned16(B.p) && B.ld % 8 == 0;
     if (whole && tiles >= 128) return 0;

@@ -36,6 +36,9 @@ struct DenseArgs {
     int structure = 0;
 };
 
+// The 256 x 256 bf16 kernel (gemm_kk256.h) addresses the 256 rows of a tile, ld elements apart, in 31 bits of bytes
+constexpr bool kk256_row_distance_ok(int64_t ld) { return 256 * ld * 2 < (int64_t(1) << 31); }
+
 template <typename T, bool A_KMAJOR, bool B_KMAJOR>
 int launch_layout(hipStream_t s, DenseArgs<T>& a);
 

@@ -330,7 +330,7 @@ __global__ __launch_bounds__(THREADS) void dense_gemm_kk256_kernel(Args a) {
 // computed twice, with the same result.  The results and the bias need no more alignment than their elements.
 inline bool applicable(const DenseArgs<bf16_t>& a) {
     return a.M >= TILE && a.N >= TILE && a.K % BK == 0 && a.K >= 2 * BK && a.A.sk == 1 && a.B.sk == 1 && a.A.vec_ok && a.B.vec_ok &&
-           256 * a.A.sr * 2 < (int64_t(1) << 31) && 256 * a.B.sr * 2 < (int64_t(1) << 31) && ceil_div(a.M, TILE) * ceil_div(a.N, TILE) < (int64_t(1) << 31);
+           kk256_row_distance_ok(a.A.sr) && kk256_row_distance_ok(a.B.sr) && ceil_div(a.M, TILE) * ceil_div(a.N, TILE) < (int64_t(1) << 31);
 }
 
 // C = act(sum over slices of the partial sums + bias), eight m of a column per thread, slices in order.

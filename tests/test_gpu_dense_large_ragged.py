@@ -63,3 +63,37 @@ def test_layer(gpu, act, M, K, N):
     dz = np.asarray(stored(dz), np.float32)
     assert_close(gW.to_numpy(), dz @ f32(x).T, "bf16", f"{act} dW")
     assert_close(gx.to_numpy(), f32(W).T @ dz, "bf16", f"{act} dx")
+
+
+class TallView:
+    """The first `rows` rows of a bf16 matrix of 2^22 + 8 rows and 256 columns: 256 of its columns are 2^31 bytes apart and more, which the
+    256 x 256 kernel does not address."""
+    ld = (1 << 22) + 8
+
+    def __init__(self, gpu, values):                        # values: rows x 256
+        self.memory = gpu.DeviceArray((self.ld, values.shape[1]), "bf16")
+        self.ptr = self.memory.ptr
+        packed = dev(gpu, values, "bf16")
+        for j in range(values.shape[1]):
+            gpu._lib.call("luxhip_memcpy_d2d", self.ptr + 2 * j * self.ld, packed.ptr + 2 * j * values.shape[0], 2 * values.shape[0], gpu.current_stream())
+        gpu._lib.call("luxhip_stream_synchronize", gpu.current_stream())       # before `packed` is given back
+
+
+def test_rows_of_a_tall_matrix(gpu):
+    """An operand whose leading dimension the 256 x 256 kernel does not take: copied for the product and for the layer's input gradient."""
+    rng = np.random.default_rng(stable_seed("tall"))
+    K, M, N, columns = 4096, 256, 5001, 8001
+    W, x, B, delta = host_inputs("bf16", rng.standard_normal((K, M), np.float32), rng.standard_normal((M, columns), np.float32),
+                                 rng.standard_normal((K, N), np.float32), rng.standard_normal((K, columns), np.float32))
+    tall, dB, got = TallView(gpu, W), dev(gpu, B, "bf16"), gpu.DeviceArray((M, N), "bf16")
+    product = lambda: gpu._lib.call("luxhip_matmul", gpu.current_stream(), dB.code, 1, 0, M, N, K, tall.ptr, tall.ld, dB.ptr, K, None, got.ptr, M)
+    assert {"kmajor_rows_kernel", "dense_gemm_kernel<bf16>"} <= set(kernels_of(gpu, product))
+    assert_close(got.to_numpy(), W.T @ B, "bf16", "W' B")
+    dx, dd = dev(gpu, x, "bf16"), dev(gpu, delta, "bf16")
+    gW, gx, gb = (gpu.DeviceArray(s, "bf16") for s in ((K, M), (M, columns), (K,)))
+    layer = lambda: gpu._lib.call("luxhip_fused_dense_bwd", gpu.current_stream(), dd.code, 0, K, M, columns, dd.ptr, None, None, tall.ptr, tall.ld, dx.ptr, M,
+                                  None, gW.ptr, gx.ptr, gb.ptr)
+    assert {"kmajor_rows_kernel", "dense_gemm_kernel<bf16>"} <= set(kernels_of(gpu, layer))
+    assert_close(gW.to_numpy(), delta @ x.T, "bf16", "dW")
+    assert_close(gx.to_numpy(), W.T @ delta, "bf16", "dx")
+    assert_close(gb.to_numpy(), f64(delta).sum(1), "bf16", "db")
