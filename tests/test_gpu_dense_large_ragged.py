@@ -82,7 +82,7 @@ class TallView:
 def test_rows_of_a_tall_matrix(gpu):
     """An operand whose leading dimension the 256 x 256 kernel does not take: copied for the product and for the layer's input gradient."""
     rng = np.random.default_rng(stable_seed("tall"))
-    K, M, N, columns = 4096, 256, 5001, 8001
+    K, M, N, columns = 4096, 256, 5001, 12001
     W, x, B, delta = host_inputs("bf16", rng.standard_normal((K, M), np.float32), rng.standard_normal((M, columns), np.float32),
                                  rng.standard_normal((K, N), np.float32), rng.standard_normal((K, columns), np.float32))
     tall, dB, got = TallView(gpu, W), dev(gpu, B, "bf16"), gpu.DeviceArray((M, N), "bf16")
