@@ -733,6 +733,34 @@ struct AnyPlan {
 
 // Padded channel-contiguous copy of the first `groups` groups of `in`, which has Cin channels (if out != NULL), and the packed
 // filter of all groups of a launch (if wout != NULL), in one launch
+template <typename T>
+static int pad_and_pack(hipStream_t s, const T* in, T* out, int P, int Cin, int Cg, int groups, int N, int zeros, const T* w, T* wout, const ConvGeom& g,
+                        const PackSubs* ps) {
+    constexpr int V = GemmTraits<T>::VEC;
+    const int Cp = padded<T>(Cg), Ct = groups * Cp;
+    PackSubs none;
+    none.n = 0; none.total = 0;
+    int64_t blocks = 0;
+    const int tiles_p = (int)ceil_div(std::max(P, zeros), 64), tiles_c = (int)ceil_div(Ct, 64);
+    if (out != nullptr) blocks = Ct == V ? ceil_div((int64_t)P * N + zeros, 256) : (int64_t)tiles_p * tiles_c * (N + (zeros > 0));
+    const int64_t pack = wout != nullptr ? ceil_div(ps->total, 256) : 0;
+    LUX_UNSUPPORTED_IF((blocks + pack) * 256 >= kMostThreads, "conv: tensor too large for the layout transform");
+    if (blocks + pack == 0) return LUXHIP_OK;
+    ProfScope prof("whcn_to_cwhn_kernel", s);
+    pad_to_cwhn_pack_kernel<T><<<(unsigned)(blocks + pack), 256, 0, s>>>(in, out, P, Cin, Cg, Cp, groups, N, zeros, tiles_p, tiles_c, (int)blocks, w, wout,
+                                                                         g, wout != nullptr ? *ps : none);
+    LUX_CHECK_LAUNCH();
+    return LUXHIP_OK;
+}
+
+// Channel-contiguous copy of a tensor in the padded layout (the plain layout where no padding is needed)
+template <typename T>
+static int to_cwhn_padded(hipStream_t s, const T* in, T* out, int P, int Cin, int Cg, int groups, int N, int zeros, const ConvGeom& g) {
+    if (padded<T>(Cg) == Cg && Cin == Cg * groups && zeros == 0 && P % GemmTraits<T>::VEC == 0 && aligned16(in))
+        return transpose_to_cwhn<T>(s, in, out, P, Cin, N);
+    return pad_and_pack<T>(s, in, out, P, Cin, Cg, groups, N, zeros, nullptr, nullptr, g, nullptr);
+}
+
 // The single pass pays where a tile is not mostly empty; smaller ragged planes and channel counts take the two passes
 template <typename T>
 static bool dz_cwhn_ok(int P, int C, int N) {
@@ -747,9 +775,15 @@ static int conv_dz_cwhn_pack(hipStream_t s, int act, const ConvGeom& g, int Cp, 
     const int P = g.OW * g.OH, C = g.Cout, N = g.N;
     const int chunk = dz_cwhn_chunk(P, C, N);
     const int64_t gx = ceil_div(ceil_div(P, 64), chunk), gy = ceil_div(C, 64);
+    // a filter that is large beside the cotangent does not fit the z slices: it has a launch of its own then, as in the two passes
     const int64_t pack_blocks = wout == nullptr ? 0 : ceil_div(ps != nullptr ? ps->total : (int64_t)g.kW * g.kH * g.Cin_g * g.Cout, 256);
-    const int64_t gz = N + ceil_div(pack_blocks, gx * gy);
-    LUX_UNSUPPORTED_IF(gz > 65535, "conv: filter too large for the combined layout pass");
+    const int64_t pack_z = ceil_div(pack_blocks, gx * gy);
+    const bool fits = N + pack_z <= 65535 && (ps != nullptr || pack_z * gx * gy * 256 < (int64_t(1) << 31));
+    if (!fits) {
+        const int rc = ps != nullptr ? pad_and_pack<T>(s, nullptr, nullptr, 0, 1, 1, 1, 0, 0, w, wout, g, ps) : pack_filter<T>(s, w, wout, g, 1);
+        if (rc != LUXHIP_OK) return rc;
+    }
+    const int64_t gz = N + (fits ? pack_z : 0);
     float* const part = dbias != nullptr ? partial : nullptr;
     PackSubs subs;
     subs.n = 0; subs.total = 0;
@@ -777,34 +811,6 @@ static int conv_dz_cwhn_pack(hipStream_t s, int act, const ConvGeom& g, int Cp, 
         LUX_CHECK_LAUNCH();
     }
     return LUXHIP_OK;
-}
-
-template <typename T>
-static int pad_and_pack(hipStream_t s, const T* in, T* out, int P, int Cin, int Cg, int groups, int N, int zeros, const T* w, T* wout, const ConvGeom& g,
-                        const PackSubs* ps) {
-    constexpr int V = GemmTraits<T>::VEC;
-    const int Cp = padded<T>(Cg), Ct = groups * Cp;
-    PackSubs none;
-    none.n = 0; none.total = 0;
-    int64_t blocks = 0;
-    const int tiles_p = (int)ceil_div(std::max(P, zeros), 64), tiles_c = (int)ceil_div(Ct, 64);
-    if (out != nullptr) blocks = Ct == V ? ceil_div((int64_t)P * N + zeros, 256) : (int64_t)tiles_p * tiles_c * (N + (zeros > 0));
-    const int64_t pack = wout != nullptr ? ceil_div(ps->total, 256) : 0;
-    LUX_UNSUPPORTED_IF((blocks + pack) * 256 >= kMostThreads, "conv: tensor too large for the layout transform");
-    if (blocks + pack == 0) return LUXHIP_OK;
-    ProfScope prof("whcn_to_cwhn_kernel", s);
-    pad_to_cwhn_pack_kernel<T><<<(unsigned)(blocks + pack), 256, 0, s>>>(in, out, P, Cin, Cg, Cp, groups, N, zeros, tiles_p, tiles_c, (int)blocks, w, wout,
-                                                                         g, wout != nullptr ? *ps : none);
-    LUX_CHECK_LAUNCH();
-    return LUXHIP_OK;
-}
-
-// Channel-contiguous copy of a tensor in the padded layout (the plain layout where no padding is needed)
-template <typename T>
-static int to_cwhn_padded(hipStream_t s, const T* in, T* out, int P, int Cin, int Cg, int groups, int N, int zeros, const ConvGeom& g) {
-    if (padded<T>(Cg) == Cg && Cin == Cg * groups && zeros == 0 && P % GemmTraits<T>::VEC == 0 && aligned16(in))
-        return transpose_to_cwhn<T>(s, in, out, P, Cin, N);
-    return pad_and_pack<T>(s, in, out, P, Cin, Cg, groups, N, zeros, nullptr, nullptr, g, nullptr);
 }
 
 // Groups [first, first + n) of a convolution.  Where channels are padded, the copies hold as many groups at a time as take no

@@ -40,3 +40,27 @@ def test_pullback(gpu, dtype, act, plane, cin, cout, n, groups, single):
     assert_close(gw.to_numpy(), wdw, dtype, "dw", scale=per * rms(x) * 0.5)
     assert_close(gx.to_numpy(), wdx, dtype, "dx", scale=np.sqrt(k * k * cout / groups) * rms(delta) * rms(w) * 0.5)
     assert_close(gb.to_numpy(), wdb, dtype, "db", scale=per * 0.5)
+
+
+@pytest.mark.parametrize("dtype", ["f32", "bf16"])
+@pytest.mark.parametrize("tap", [0, 42])
+def test_filter_that_is_large_beside_the_cotangent(gpu, dtype, tap):
+    """One tile of the cotangent and 16.9 million filter elements, more than its launch's z slices hold: they are packed in a launch of their own, for
+    the general kernels and for the whole-tap ones."""
+    xs, ws = (8, 8, 5376, 1), (7, 7, 5376, 64)
+    rng = np.random.default_rng(stable_seed("large filter", dtype))
+    x, w, b, delta = host_inputs(dtype, rng.standard_normal(xs, np.float32), rng.standard_normal(ws, np.float32), rng.standard_normal(64, np.float32),
+                                 rng.standard_normal((8, 8, 64, 1), np.float32))
+    gd, od = gpu.DenseConvDims(xs, ws, padding=3), O.ConvDims(xs, ws, padding=3)
+    gpu.set_option("conv_tile", tap)
+    try:
+        _, back = gpu.pullback(gpu.fused_conv_bias_activation, "identity", dev(gpu, w, dtype), dev(gpu, x, dtype), dev(gpu, b, dtype), gd)
+        grads, dd = [], dev(gpu, delta, dtype)
+        kernels = kernels_of(gpu, lambda: grads.extend(back(dd)))
+    finally:
+        gpu.set_option("conv_tile", 0)
+    assert {"conv_dz_cwhn_pack_kernel", "pack_filter_kernel" if tap else "whcn_to_cwhn_kernel"} <= set(kernels)
+    per = rms(delta) * 8                                    # sums of up to 64 positions, and of 7 x 7 x 64 cotangents
+    assert_close(grads[0].to_numpy(), O.conv_filter_grad(f64(x), f64(delta), od), dtype, "dw", scale=per * rms(x) * 0.5)
+    assert_close(grads[1].to_numpy(), O.conv_data_grad(f64(delta), f64(w), od), dtype, "dx", scale=per * 7 * rms(w) * 0.5)
+    assert_close(grads[2].to_numpy(), f64(delta).sum((0, 1, 3)), dtype, "db", scale=per * 0.5)
