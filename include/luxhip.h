@@ -170,8 +170,10 @@ int luxhip_bias_activation_bwd(luxhip_stream_t s, int dtype, int act, int64_t I,
 
 /* luxhip_bias_activation_bwd with the operator's input and bias in place of the pre-activation, which
  * it forms again with the rounding that a stored one has: the forward pass need not keep it (pre == NULL
- * there).  Same results, bit for bit.  x is read where the activation's derivative needs the
- * pre-activation; bias may be NULL, dbias only if bias is. */
+ * there).  Same results, bit for bit, as long as x and bias hold what the forward pass read: a caller
+ * that may change either before this call has run (an update in place, a buffer used again) keeps the
+ * pre-activation and calls luxhip_bias_activation_bwd.  x is read where the activation's derivative
+ * needs the pre-activation; bias may be NULL, dbias only if bias is. */
 int luxhip_bias_activation_bwd_from_x(luxhip_stream_t s, int dtype, int act, int64_t I, int64_t C, int64_t N,
                                       const void* delta, const void* out, const void* x, const void* bias, void* dx,
                                       void* dbias);

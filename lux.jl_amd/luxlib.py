@@ -171,7 +171,8 @@ def bias_activation_inplace(act: str, x: DeviceArray, bias: Optional[DeviceArray
 
 
 def rrule_bias_activation(act: str, x: DeviceArray, bias: Optional[DeviceArray]):
-    """CRC.rrule(bias_activation) (impl/bias_activation.jl:64-104): (y, Δ -> (∂x, ∂b))."""
+    """CRC.rrule(bias_activation) (impl/bias_activation.jl:64-104): (y, Δ -> (∂x, ∂b)).  The reference keeps x .+ bias; here Δ's
+    pullback forms it again from x and bias, which must keep their values until then (see `pullback`)."""
     _check_bias(x, bias)
     if _is_closure(act):
         z, back_z = rrule_bias_activation("identity", x, bias)
@@ -183,7 +184,7 @@ def rrule_bias_activation(act: str, x: DeviceArray, bias: Optional[DeviceArray])
     y = DeviceArray(x.shape, dt)
     _lib.call("luxhip_bias_activation_fwd", current_stream(), x.code, aid, I, Cc, N, x.ptr, _p(bias), y.ptr, None)
 
-    def back(delta: DeviceArray):     # x .+ bias is formed again where the derivative needs it
+    def back(delta: DeviceArray):
         dx = DeviceArray(x.shape, dt)
         db = None if bias is None else DeviceArray(bias.shape, dt)
         _lib.call("luxhip_bias_activation_bwd_from_x", current_stream(), x.code, aid, I, Cc, N, delta.ptr, y.ptr, x.ptr, _p(bias),
@@ -1399,7 +1400,11 @@ _RRULES = {
 
 def pullback(f, *args, **kwargs):
     """`y, back = pullback(f, args...)`; `back(Δ)` returns the tangents of the array
-    arguments in the order the rrule lists them."""
+    arguments in the order the rrule lists them.
+
+    `back` may read the arrays that `f` was called with (inputs, weights, biases, scales) and its result y again: the rules keep
+    the arrays, not copies of their values, so all of them must hold what `f` saw until `back` has run.  One that is updated in
+    place before that (a bias by an optimiser, an input's buffer by the next batch) changes the tangents without an error."""
     try:
         rule = _RRULES[f]
     except KeyError:
