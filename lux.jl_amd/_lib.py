@@ -3,7 +3,9 @@
 from __future__ import annotations
 
 import ctypes as C
+import importlib
 import os
+import warnings
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "libluxhip.so")
@@ -149,8 +151,11 @@ def _ctypes_call(name: str, *args):
 
 
 try:
-    from . import _host                  # csrc/python_host.cpp; arrays are made of its types
-except ImportError:                      # not built: importing still works, operators say what is missing
+    _host = importlib.import_module(__package__ + "._host")      # csrc/python_host.cpp; arrays are made of its types
+except ModuleNotFoundError:                  # not built for this interpreter: array.py's own classes, and every call through ctypes
+    _host, call = None, _ctypes_call
+except ImportError as reason:
+    warnings.warn(f"the native part of the host side does not load, calls go through ctypes: {reason}", RuntimeWarning)
     _host, call = None, _ctypes_call
 else:
     _host.configure(load, _ctypes_call, check, C.c_void_p, C.Array, ConvDimsStruct)

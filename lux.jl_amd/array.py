@@ -35,11 +35,58 @@ def _from_bf16_bits(b: np.ndarray) -> np.ndarray:
 if _lib._host is not None:
     _Array, _Stat = _lib._host.Array, _lib._host.Stat
 else:
-    class _Array:
-        def __init__(self, *args, **kwargs):
-            raise ImportError("lux.jl_amd/_host.so is missing: build it with `make -C lux.jl_amd/csrc`")
+    # What csrc/python_host.cpp has in native code, for interpreters that it was not built for
+    def _malloc(nbytes: int) -> int:
+        p = C.c_void_p()
+        _lib.call("luxhip_malloc", C.byref(p), nbytes)
+        return p.value
 
-    _Stat = _Array
+    def _free(ptr):
+        try:
+            _lib.load().luxhip_free(C.c_void_p(ptr))
+        except Exception:
+            pass
+
+    class _Array:
+        __slots__ = ("shape", "dtype", "ptr", "_owner", "_base")
+
+        def __init__(self, shape, dtype="f32", ptr=None, base=None):
+            if dtype not in DTYPES:
+                raise TypeError(f"unsupported dtype {dtype!r} (use 'f32' or 'bf16'; 'u8' for masks)")
+            self.shape = tuple(int(s) for s in shape)
+            self.dtype = dtype
+            self._base = base
+            self.ptr = _malloc(max(self.nbytes, 1)) if ptr is None else int(ptr)
+            self._owner = ptr is None
+
+        @property
+        def size(self) -> int:
+            n = 1
+            for s in self.shape:
+                n *= s
+            return n
+
+        ndim = property(lambda self: len(self.shape))
+        itemsize = property(lambda self: DTYPES[self.dtype][1])
+        nbytes = property(lambda self: self.size * self.itemsize)
+        code = property(lambda self: DTYPES[self.dtype][0])
+
+        def __del__(self):
+            if getattr(self, "_owner", False) and self.ptr:
+                _free(self.ptr)
+                self.ptr = 0
+
+    class _Stat:
+        __slots__ = ("n", "ptr")
+
+        def __init__(self, n):
+            self.n = int(n)
+            self.ptr = _malloc(max(4 * self.n, 4))
+
+        def __del__(self):
+            if getattr(self, "ptr", 0):
+                _free(self.ptr)
+                self.ptr = 0
 
 
 class DeviceArray(_Array):

@@ -2,10 +2,42 @@
 and report as the ctypes calls that stand behind them do."""
 import ctypes as C
 import gc
+import importlib.abc
+import importlib.util
+import os
+import sys
+import warnings
 import weakref
 
 import numpy as np
 import pytest
+
+
+def _package(name, refusal):
+    """A copy of the package under `name`, in an interpreter whose import of the native part raises `refusal`."""
+    class Refuse(importlib.abc.MetaPathFinder):
+        def find_spec(self, fullname, path=None, target=None):
+            if fullname == name + "._host":
+                raise refusal
+
+    here = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "lux.jl_amd")
+    spec = importlib.util.spec_from_file_location(name, os.path.join(here, "__init__.py"), submodule_search_locations=[here])
+    module, refuse = importlib.util.module_from_spec(spec), Refuse()
+    sys.modules[name] = module
+    sys.meta_path.insert(0, refuse)
+    try:
+        spec.loader.exec_module(module)
+    finally:
+        sys.meta_path.remove(refuse)
+    return module
+
+
+@pytest.fixture(scope="module")
+def plain():
+    """The package where its native part was not built: arrays and calls in Python and ctypes."""
+    with warnings.catch_warnings():
+        warnings.simplefilter("error")
+        return _package("lux_plain", ModuleNotFoundError("No module named 'lux_plain._host'", name="lux_plain._host"))
 
 
 def _borrowed(lux, shape, dtype="f32", ptr=1 << 40, base=None):
@@ -86,3 +118,33 @@ def test_calls_report_the_librarys_status(gpu):
     x, m = gpu.DeviceArray.from_numpy(np.arange(5)), gpu.DeviceArray.from_numpy(np.full(5, 2.0))
     gpu._lib.call("luxhip_dropout_mul", gpu.current_stream(), 0, 1, dims, dims, x.ptr, m.ptr, a.ptr)
     np.testing.assert_array_equal(a.to_numpy(), 2.0 * np.arange(5))
+
+
+def test_without_the_native_part(plain):
+    assert plain._lib._host is None and plain._lib.call is plain._lib._ctypes_call
+    test_array_attributes(plain)
+    test_a_view_keeps_its_base(plain)
+    test_calls_refuse_what_ctypes_refuses(plain)
+
+
+def test_a_native_part_that_does_not_load_says_why():
+    with pytest.warns(RuntimeWarning, match="undefined symbol: PyThing"):
+        broken = _package("lux_broken", ImportError("_host.so: undefined symbol: PyThing"))
+    assert broken.DeviceArray((2, 3), ptr=1 << 40).nbytes == 24
+
+
+@pytest.mark.gpu
+def test_operators_without_the_native_part(gpu, plain):
+    plain.init(0)
+    rng = np.random.default_rng(3)
+    W, x, b, d = (rng.normal(size=s).astype(np.float32) for s in ((24, 16), (16, 9), (24,), (24, 9)))
+    results = []
+    for lux in (gpu, plain):
+        y, back = lux.pullback(lux.fused_dense_bias_activation, "gelu", *(lux.DeviceArray.from_numpy(a) for a in (W, x, b)))
+        g = lux.DeviceArray.from_numpy(np.ones((24, 1)))
+        z, back2 = lux.pullback(lux.layernorm, y, g, g, "identity", (1,), 1e-5)              # its statistics are StatArrays
+        results.append([a.to_numpy() for a in (y, z, *back(lux.DeviceArray.from_numpy(d)), *back2(lux.DeviceArray.from_numpy(d)))])
+    for native, ctypes_only in zip(*results):
+        np.testing.assert_array_equal(native, ctypes_only)
+    with pytest.raises(plain.LuxHipError, match="failed"):
+        plain.DeviceArray((1 << 30, 1 << 30))
