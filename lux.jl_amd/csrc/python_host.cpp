@@ -214,6 +214,35 @@ bool shape_size(PyObject* shape, int64_t* out) {
     return true;
 }
 
+// A new reference to the shape as a tuple of ints
+PyObject* shape_tuple(PyObject* shape) {
+    bool plain = PyTuple_CheckExact(shape);
+    for (Py_ssize_t i = 0; plain && i < PyTuple_GET_SIZE(shape); ++i) plain = PyLong_CheckExact(PyTuple_GET_ITEM(shape, i));
+    if (plain) {
+        Py_INCREF(shape);
+        return shape;
+    }
+    PyObject* all = PySequence_Tuple(shape);
+    if (all == nullptr) return nullptr;
+    PyObject* out = PyTuple_New(PyTuple_GET_SIZE(all));
+    for (Py_ssize_t i = 0; out != nullptr && i < PyTuple_GET_SIZE(all); ++i) {
+        PyObject* v = PyObject_CallOneArg((PyObject*)&PyLong_Type, PyTuple_GET_ITEM(all, i));
+        if (v == nullptr) Py_CLEAR(out);
+        else PyTuple_SET_ITEM(out, i, v);
+    }
+    Py_DECREF(all);
+    return out;
+}
+
+// The storage type of a name: its own (borrowed) string, or NULL with an error
+PyObject* storage_type(PyObject* dtype, int* item, int* code) {
+    auto is = [&](PyObject* name) { return dtype == name || (PyUnicode_Check(dtype) && PyUnicode_Compare(dtype, name) == 0); };
+    if (is(g_f32)) { *item = 4; *code = LUXHIP_F32; return g_f32; }
+    if (is(g_bf16)) { *item = 2; *code = LUXHIP_BF16; return g_bf16; }
+    if (is(g_u8)) { *item = 1; *code = -1; return g_u8; }
+    return PyErr_Format(PyExc_TypeError, "unsupported dtype %R (use 'f32' or 'bf16'; 'u8' for masks)", dtype);
+}
+
 int array_init(Array* self, PyObject* args, PyObject* kw) {
     static const char* names[] = {"shape", "dtype", "ptr", "base", nullptr};
     PyObject *shape = nullptr, *dtype = g_f32, *ptr = Py_None, *base = Py_None;
@@ -224,29 +253,10 @@ int array_init(Array* self, PyObject* args, PyObject* kw) {
         return -1;
     }
     int item = 0, code = 0;
-    if (dtype == g_f32 || (PyUnicode_Check(dtype) && PyUnicode_Compare(dtype, g_f32) == 0)) { item = 4; code = LUXHIP_F32; dtype = g_f32; }
-    else if (dtype == g_bf16 || (PyUnicode_Check(dtype) && PyUnicode_Compare(dtype, g_bf16) == 0)) { item = 2; code = LUXHIP_BF16; dtype = g_bf16; }
-    else if (PyUnicode_Check(dtype) && PyUnicode_Compare(dtype, g_u8) == 0) { item = 1; code = -1; dtype = g_u8; }
-    else {
-        PyErr_Format(PyExc_TypeError, "unsupported dtype %R (use 'f32' or 'bf16'; 'u8' for masks)", dtype);
-        return -1;
-    }
-    bool plain = PyTuple_CheckExact(shape);
-    for (Py_ssize_t i = 0; plain && i < PyTuple_GET_SIZE(shape); ++i) plain = PyLong_CheckExact(PyTuple_GET_ITEM(shape, i));
-    if (plain) {
-        Py_INCREF(shape);
-    } else {
-        PyObject* all = PySequence_Tuple(shape);
-        if (all == nullptr) return -1;
-        shape = PyTuple_New(PyTuple_GET_SIZE(all));
-        for (Py_ssize_t i = 0; shape != nullptr && i < PyTuple_GET_SIZE(all); ++i) {
-            PyObject* v = PyObject_CallOneArg((PyObject*)&PyLong_Type, PyTuple_GET_ITEM(all, i));
-            if (v == nullptr) Py_CLEAR(shape);
-            else PyTuple_SET_ITEM(shape, i, v);
-        }
-        Py_DECREF(all);
-        if (shape == nullptr) return -1;
-    }
+    dtype = storage_type(dtype, &item, &code);
+    if (dtype == nullptr) return -1;
+    shape = shape_tuple(shape);
+    if (shape == nullptr) return -1;
     int64_t size;
     if (!shape_size(shape, &size)) {
         Py_DECREF(shape);
@@ -299,9 +309,38 @@ PyObject* array_size(Array* self, void*) { return PyLong_FromLongLong(self->size
 PyObject* array_ndim(Array* self, void*) { return PyLong_FromSsize_t(self->shape != nullptr ? PyTuple_GET_SIZE(self->shape) : 0); }
 PyObject* array_nbytes(Array* self, void*) { return PyLong_FromLongLong(self->size * self->item); }
 
+PyObject* attribute(PyObject* value, const char* name) {
+    if (value == nullptr) PyErr_SetString(PyExc_AttributeError, name);       // __init__ has not run
+    Py_XINCREF(value);
+    return value;
+}
+PyObject* array_shape(Array* self, void*) { return attribute(self->shape, "shape"); }
+PyObject* array_dtype(Array* self, void*) { return attribute(self->dtype, "dtype"); }
+// The caller's to answer for, as with the attributes of a Python object: the memory stays as it is
+int array_set_shape(Array* self, PyObject* value, void*) {
+    int64_t size;
+    PyObject* shape = value != nullptr ? shape_tuple(value) : PyErr_Format(PyExc_AttributeError, "shape cannot be deleted");
+    if (shape == nullptr) return -1;
+    if (!shape_size(shape, &size)) {
+        Py_DECREF(shape);
+        return -1;
+    }
+    Py_XSETREF(self->shape, shape);
+    self->size = size;
+    return 0;
+}
+int array_set_dtype(Array* self, PyObject* value, void*) {
+    int item, code;
+    PyObject* dtype = value != nullptr ? storage_type(value, &item, &code) : PyErr_Format(PyExc_AttributeError, "dtype cannot be deleted");
+    if (dtype == nullptr) return -1;
+    Py_INCREF(dtype);
+    Py_XSETREF(self->dtype, dtype);
+    self->item = item;
+    self->code = code;
+    return 0;
+}
+
 PyMemberDef array_members[] = {
-    {"shape", T_OBJECT_EX, offsetof(Array, shape), READONLY, nullptr},
-    {"dtype", T_OBJECT_EX, offsetof(Array, dtype), READONLY, nullptr},
     {"ptr", T_ULONGLONG, offsetof(Array, ptr), 0, nullptr},
     {"itemsize", T_INT, offsetof(Array, item), READONLY, nullptr},
     {"code", T_INT, offsetof(Array, code), READONLY, nullptr},
@@ -310,6 +349,8 @@ PyMemberDef array_members[] = {
     {nullptr, 0, 0, 0, nullptr},
 };
 PyGetSetDef array_getset[] = {
+    {"shape", (getter)array_shape, (setter)array_set_shape, nullptr, nullptr},
+    {"dtype", (getter)array_dtype, (setter)array_set_dtype, nullptr, nullptr},
     {"size", (getter)array_size, nullptr, nullptr, nullptr},
     {"ndim", (getter)array_ndim, nullptr, nullptr, nullptr},
     {"nbytes", (getter)array_nbytes, nullptr, nullptr, nullptr},
@@ -344,8 +385,8 @@ void stat_dealloc(Stat* self) {
     Py_TYPE(self)->tp_free((PyObject*)self);
 }
 PyMemberDef stat_members[] = {
-    {"n", T_LONGLONG, offsetof(Stat, n), READONLY, nullptr},
-    {"ptr", T_ULONGLONG, offsetof(Stat, ptr), READONLY, nullptr},
+    {"n", T_LONGLONG, offsetof(Stat, n), 0, nullptr},
+    {"ptr", T_ULONGLONG, offsetof(Stat, ptr), 0, nullptr},
     {nullptr, 0, 0, 0, nullptr},
 };
 PyTypeObject StatType = {PyVarObject_HEAD_INIT(nullptr, 0)};

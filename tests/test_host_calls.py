@@ -59,6 +59,14 @@ def test_array_attributes(lux):
         _borrowed(lux, ("x",))
 
 
+def test_shape_and_dtype_can_be_set(lux, plain):
+    for a in (_borrowed(lux, (6, 4)), _borrowed(plain, (6, 4))):
+        a.shape = (3, 8)
+        assert (a.shape, a.size, a.ndim, a.nbytes) == ((3, 8), 24, 2, 96)
+        a.shape, a.dtype = (24,), "bf16"
+        assert (a.ndim, a.dtype, a.itemsize, a.nbytes, a.code) == (1, "bf16", 2, 48, lux._lib.BF16)
+
+
 def test_a_view_keeps_its_base(lux):
     class Owner:
         pass
