@@ -67,7 +67,9 @@ Conv convert(PyObject* o, T* out) {
     } else if constexpr (std::is_same_v<T, const int64_t*> || std::is_same_v<T, const luxhip_conv_dims_t*>) {
         constexpr bool dims = std::is_same_v<T, const luxhip_conv_dims_t*>;
         void* where;
-        if (dims ? (PyObject*)Py_TYPE(o) != g_conv_dims : PyObject_IsInstance(o, g_ctypes_array) != 1) return Conv::SLOW;
+        const int is = dims ? (PyObject*)Py_TYPE(o) == g_conv_dims : PyObject_IsInstance(o, g_ctypes_array);
+        if (is < 0) PyErr_Clear();                               // an error of the argument's own: ctypes says what it makes of it
+        if (is != 1) return Conv::SLOW;
         if (!ctypes_memory(o, dims ? (Py_ssize_t)sizeof(luxhip_conv_dims_t) : 8, !dims, &where)) return Conv::SLOW;
         *out = (T)where;
         return Conv::DONE;

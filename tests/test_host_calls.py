@@ -112,6 +112,17 @@ def test_calls_refuse_what_ctypes_refuses(lux):
             lux._lib.call("luxhip_dropout_mul", None, 0, 2, wrong, wrong, 1 << 40, 1 << 40, 1 << 40)
 
 
+def test_an_argument_whose_class_raises(lux):
+    class Odd:
+        @property
+        def __class__(self):
+            raise RuntimeError("no class")
+
+    for call in (lux._lib._ctypes_call, lux._lib.call):
+        with pytest.raises(C.ArgumentError):
+            call("luxhip_dropout_mul", None, 0, 2, Odd(), Odd(), 1 << 40, 1 << 40, 1 << 40)
+
+
 @pytest.mark.gpu
 def test_calls_report_the_librarys_status(gpu):
     with pytest.raises(gpu.LuxHipError) as want:
