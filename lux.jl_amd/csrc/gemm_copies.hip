@@ -134,7 +134,7 @@ int dense_dz_kmajor(hipStream_t s, int act, int64_t M, int64_t N, const bf16_t* 
         else dense_dz_kmajor_kernel<A, true><<<grid, 256, 0, s>>>(delta, out, pre, M, dz, ldz, dzT, ldt, part, (uint32_t)M, (uint32_t)N);        \
     } while (0)
     {
-        ProfScope ps("dense_dz_transposed_kernel", s);
+        ProfScope ps("dense_dz_kmajor_kernel", s);
         LUX_DISPATCH_ACT(act, LAUNCH_DZK);
     }
 #undef LAUNCH_DZK

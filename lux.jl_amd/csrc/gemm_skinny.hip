@@ -202,7 +202,8 @@ int launch(hipStream_t s, const DenseArgs<T>& d) {
         a.partial = reinterpret_cast<float*>(ws.data);
         a.counters = ws.counters;
     }
-    ProfScope ps(sizeof(T) == 2 ? "skinny_gemm_kernel<bf16>" : "skinny_gemm_kernel<f32>", s);
+    ProfScope ps(sizeof(T) == 2 ? (a.slices > 1 ? "skinny_gemm_kernel<bf16>+slices" : "skinny_gemm_kernel<bf16>")
+                                : (a.slices > 1 ? "skinny_gemm_kernel<f32>+slices" : "skinny_gemm_kernel<f32>"), s);
     skinny_gemm_kernel<T><<<dim3((unsigned)(blocks * a.slices)), dim3(THREADS), 0, s>>>(a);
     LUX_CHECK_LAUNCH();
     return LUXHIP_OK;

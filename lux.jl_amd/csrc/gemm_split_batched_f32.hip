@@ -21,7 +21,7 @@ static int batched_slices(int64_t tiles, int64_t K, int structure) {
 template <bool AK, bool BKM, bool EP>
 static int launch_batched_as(hipStream_t s, DenseArgs<float>& a, int64_t units, const Plan& p) {
     using B = Body<float, 1, AK, BKM>;
-    ProfScope ps(EP ? "batched_gemm_kernel+softmax_rule" : "batched_gemm_kernel<f32>", s);
+    ProfScope ps(EP ? "split_batched_kernel+softmax_rule" : p.slices > 1 ? "split_batched_kernel+slices" : "split_batched_kernel", s);
     split_batched_kernel<float, AK, BKM, EP><<<dim3((unsigned)units), dim3(THREADS), B::LDS_BYTES, s>>>(a, p);
     LUX_CHECK_LAUNCH();
     return LUXHIP_OK;

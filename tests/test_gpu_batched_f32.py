@@ -4,7 +4,7 @@ import numpy as np
 import pytest
 
 from oracle import luxlib_oracle as O
-from tests.util import assert_close, dev, f64, stable_seed
+from tests.util import assert_close, dev, f64, kernels_of, stable_seed
 
 pytestmark = pytest.mark.gpu
 
@@ -18,7 +18,10 @@ def test_products(gpu, lhs, rhs, M, N, K):
     rng = np.random.default_rng(stable_seed("batched f32", lhs, rhs, M, N, K))
     a = rng.normal(size=(M, K, 3) if lhs == 2 else (K, M, 3)).astype(np.float32)
     b = rng.normal(size=(K, N, 3) if rhs == 1 else (N, K, 3)).astype(np.float32)
-    got = gpu.batched_matmul(dev(gpu, a, "f32"), dev(gpu, b, "f32"), lhs, rhs).to_numpy()
+    da, db, out = dev(gpu, a, "f32"), dev(gpu, b, "f32"), []
+    kernels = kernels_of(gpu, lambda: out.append(gpu.batched_matmul(da, db, lhs, rhs)))
+    assert set(kernels) == {"split_batched_kernel+slices" if K > 500 else "split_batched_kernel"}
+    got = out[0].to_numpy()
     assert_close(got, O.batched_matmul(f64(a), f64(b), lhs, rhs), "f32", f"{M} x {N} x {K} {lhs} {rhs}")
     np.testing.assert_array_equal(got, gpu.batched_matmul(dev(gpu, a, "f32"), dev(gpu, b, "f32"), lhs, rhs).to_numpy())
 
@@ -29,8 +32,16 @@ def test_products(gpu, lhs, rhs, M, N, K):
 def test_attention(gpu, causal, E, H, L):
     rng = np.random.default_rng(stable_seed("attention f32", E, H, L))
     q, k, v, d = (rng.normal(size=(E, H, L, 2)).astype(np.float32) for _ in range(4))
-    (y, w), back = gpu.pullback(gpu.scaled_dot_product_attention, *(dev(gpu, t, "f32") for t in (q, k, v)), 1, 3, None, None, True if causal else None)
-    grads = [g.to_numpy() for g in back(dev(gpu, d, "f32"))]
+    dq, dk, dv, dd = (dev(gpu, t, "f32") for t in (q, k, v, d))
+    out, grads = [], []
+    kernels = kernels_of(gpu, lambda: out.extend(gpu.pullback(gpu.scaled_dot_product_attention, dq, dk, dv, 1, 3, None, None, True if causal else None)))
+    (y, w), back = out
+    kernels_back = kernels_of(gpu, lambda: grads.extend(g.to_numpy() for g in back(dd)))
+    # 8 features are less than a stage: the products that contract over them stay on the general tiles
+    assert "batched_gemm_kernel<f32>" not in kernels_back and ("batched_gemm_kernel<f32>" in kernels) == (E < 16)
+    assert ("split_batched_kernel+softmax_rule" if E >= 16 else "batched_gemm_kernel+softmax_rule") in kernels_back
+    for products in (kernels, kernels_back):
+        assert ("split_batched_kernel+slices" in products) == (L > 200)
     Q, K, V, D = (np.moveaxis(f64(t), (3, 1, 2, 0), (0, 1, 2, 3)) for t in (q, k, v, d))       # (B, H, L, E)
     z = Q @ np.swapaxes(K, 2, 3) / np.sqrt(E)
     if causal:

@@ -26,8 +26,7 @@ def test_pullback(gpu, dtype, act, plane, cin, cout, n, groups, single):
     gd, od = gpu.DenseConvDims(xs, ws, padding=k // 2, groups=groups), O.ConvDims(xs, ws, padding=k // 2, groups=groups)
     y, back = gpu.pullback(gpu.fused_conv_bias_activation, act, dev(gpu, w, dtype), dev(gpu, x, dtype), dev(gpu, b, dtype), gd)
     dd = dev(gpu, delta, dtype)
-    if single:
-        assert "conv_dz_cwhn_pack_kernel" in kernels_of(gpu, lambda: back(dd))
+    assert ("conv_dz_cwhn_pack_kernel" in kernels_of(gpu, lambda: back(dd))) == single
     gw, gx, gb = back(dd)
     wy, wdw, wdx, wdb = O.fused_conv_pullback(act, f64(w), f64(x), f64(b), od, f64(delta))
     if dtype == "bf16":                                     # y, the pre-activation and dz are stored in bf16 in between

@@ -8,10 +8,10 @@ from tests.util import assert_close, dev, f64, host_inputs, kernels_of, stable_s
 
 pytestmark = pytest.mark.gpu
 
-# one more and one less than a whole tile, whole tiles whose K is no whole step, short and long K (1537 x 3841 x 5001: two slices; 1793 x 3071 x
-# 8200: three or more), every layout
+# one more and one less than a whole tile, whole tiles whose K is no whole step, short and long K (1537 x 3841 x 5001 and 1793 x 3071 x 8200: two
+# slices, 1281 x 2049 x 12001: four), every layout
 SHAPES = [(3841, 4095, 1001, "tt"), (3584, 4096, 1001, "nn"), (2047, 6401, 1090, "tn"), (7681, 7937, 450, "nt"), (1537, 3841, 5001, "nt"),
-          (1793, 3071, 8200, "tn")]
+          (1793, 3071, 8200, "tn"), (1281, 2049, 12001, "tt")]
 
 
 @pytest.mark.parametrize("M,N,K,layout", SHAPES)
@@ -22,7 +22,8 @@ def test_products(gpu, M, N, K, layout):
                              rng.standard_normal(M, np.float32))
     dA, dB, db = (dev(gpu, a, "bf16") for a in (A, B, bias))
     got = gpu.matmul(dA, dB, db, tA, tB).to_numpy()
-    assert "dense_gemm_kernel<bf16>" in kernels_of(gpu, lambda: gpu.matmul(dA, dB, db, tA, tB))
+    kernels = kernels_of(gpu, lambda: gpu.matmul(dA, dB, db, tA, tB))
+    assert "dense_gemm_kernel<bf16>" in kernels and ("slices_reduce_kernel" in kernels) == (K > 5000)
     f32 = lambda a: np.asarray(f64(a), np.float32)          # products of bf16 are exact, sums over K in fp32: 1e-6 of a result
     want = (f32(A).T if tA else f32(A)) @ (f32(B).T if tB else f32(B)) + f32(bias)[:, None]
     assert_close(got, want, "bf16", f"{M} x {N} x {K} {layout}")
@@ -51,7 +52,7 @@ def test_layer(gpu, act, M, K, N):
                                  0.1 * rng.standard_normal(M, np.float32), rng.standard_normal((M, N), np.float32))
     y, back = gpu.pullback(gpu.fused_dense_bias_activation, act, *(dev(gpu, a, "bf16") for a in (W, x, b)))
     ddelta = dev(gpu, delta, "bf16")
-    assert "dense_dz_transposed_kernel" in kernels_of(gpu, lambda: back(ddelta))
+    assert "dense_dz_kmajor_kernel" in kernels_of(gpu, lambda: back(ddelta))
     gW, gx, gb = back(ddelta)
     f32 = lambda a: np.asarray(f64(a), np.float32)
     z = f32(W) @ f32(x) + f32(b)[:, None]

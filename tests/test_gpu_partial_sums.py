@@ -3,7 +3,7 @@ import numpy as np
 import pytest
 
 from oracle import luxlib_oracle as O
-from tests.util import assert_close, dev, f64, host_inputs, stable_seed
+from tests.util import assert_close, dev, f64, host_inputs, kernels_of, stable_seed
 
 pytestmark = pytest.mark.gpu
 
@@ -47,7 +47,9 @@ def test_slices_of_a_few_columns(gpu, dtype, K, N):
     (below 2^8 in bf16: 1440 terms of variance 4/9 stay within 6.5 x 25) the result are exact."""
     rng = np.random.default_rng(stable_seed("few columns", dtype, N))
     W, x = rng.integers(-1, 2, size=(700, K)).astype(np.float32), rng.integers(-1, 2, size=(K, N)).astype(np.float32)
-    got = gpu.matmul(dev(gpu, W, dtype), dev(gpu, x, dtype), None, False, False).to_numpy()
+    dW, dx, out = dev(gpu, W, dtype), dev(gpu, x, dtype), []
+    assert set(kernels_of(gpu, lambda: out.append(gpu.matmul(dW, dx, None, False, False)))) == {f"skinny_gemm_kernel<{dtype}>+slices"}
+    got = out[0].to_numpy()
     want = W @ x
     assert np.abs(want).max() < 256
     np.testing.assert_array_equal(got, want)
