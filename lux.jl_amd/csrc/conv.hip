@@ -569,6 +569,9 @@ static size_t dz_cwhn_partial_bytes(int P, int C, int N) {
     const int64_t groups = ceil_div(ceil_div(P, 64), dz_cwhn_chunk(P, C, N));
     return align256((size_t)groups * N * C * sizeof(float));
 }
+
+// ----------------------------------------------------------------------------- any channel count, any stride (conv_any.h)
+// Channels of a group padded to whole 16-byte chunks
 template <typename T>
 static int padded(int c) {
     constexpr int V = GemmTraits<T>::VEC;

@@ -130,7 +130,9 @@ static int ragged_product(hipStream_t s, int64_t M, int64_t N, int64_t K, Side A
 }
 
 // The pullback of a dense layer whose two gradient products both go to the 256 x 256 kernel: the pass over delta writes dz as both
-// of them read it, with the bias gradient's partial sums.  *done: false if it is a problem of other kernels (nothing was launched).
+// of them read it, with the bias gradient's partial sums.  *done: false if it is a problem of other kernels (nothing was launched).  Where only one
+// of the two goes there (1049 of 8000 layers of feed-forward blocks, 512 to 4096 wide on 256 to 16384 columns; both in 3546) dz is written
+// once by the general pass and that product copies it again.
 static int ragged_gradients(hipStream_t s, int act, int64_t M, int64_t K, int64_t N, const bf16_t* delta, const bf16_t* y, const bf16_t* pre,
                             const bf16_t* W, int64_t ldw, const bf16_t* x, int64_t ldx, bf16_t* dz, bf16_t* dW, bf16_t* dx, bf16_t* dbias, bool* done) {
     *done = false;

@@ -12,8 +12,6 @@
 
 namespace luxhip {
 
-// Epilogue of one tile: C = act(acc + bias), optional pre-activation copy.  CHECK (bounds tests)
-// and the activation are resolved once per tile, so there is no choice between them per element.
 // WM consecutive values of one column -> memory; one store when the lane's rows are consecutive
 // (ML::M_STEP == 1), the storage type is bf16 and the destination allows it
 template <class ML, typename T, int WM, bool CHECK>
@@ -36,6 +34,8 @@ __device__ __forceinline__ void store_column(T* col, const float (&v)[WM], int m
         if (!CHECK || mb + i * ML::M_STEP < M) st(col + i * ML::M_STEP, v[i]);
 }
 
+// Epilogue of one tile: C = act(acc + bias), optional pre-activation copy.  CHECK (bounds tests)
+// and the activation are resolved once per tile, so there is no choice between them per element.
 template <class ML, typename T, int WM, int WN, bool CHECK, int ACT, bool PRE>
 __device__ __forceinline__ void dense_epilogue_as(const f32x16_v (&acc)[WM][WN], const DenseArgs<T>& a, int m0, int n0) {
     const int mb = ML::lane_m(m0), nb = ML::lane_n(n0);

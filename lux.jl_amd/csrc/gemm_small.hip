@@ -255,8 +255,9 @@ static bool product_pays(const DenseArgs<float>& a, bool ak) {
     return 2.1 + (double)ceil_div(tiles, cus) * tile_time(a.K, ak ? 8.0 : 7.2) < split::estimate<float>(c.w, c.slices, a.M, a.N, a.K) + 2.3;
 }
 
-// Whether the whole pullback is: the longer of the two contractions starts first, and where the tiles are more than the compute units its last
-// ones end half a tile late.  Fitted to 60 layers of 16 to 2048 in every dimension with tanh and gelu (within 11 % rms).  Of those none below the limit was
+// Whether the whole pullback is one launch: up to a constant of its own estimated time, not by an estimate of the other way (past the constants some
+// layers that would gain stay with the passes: 1023 -> 517 with 301 columns and gelu is 20.6 by this estimate, 25 in three launches).  The longer of
+// the two contractions starts first, and where the tiles are more than the compute units its last ones end half a tile late.  Fitted to 60 layers of 16 to 2048 in every dimension with tanh and gelu (within 11 % rms).  Of those none below the limit was
 // slower than the passes over delta and the pair of products in graphs, where the host does not count (us, there / here: fp32, gelu
 // 301 x 77 x 560 14.0 / 6.6, 641 x 496 x 240 20.7 / 15.6, 1339 x 56 x 53 16.4 / 17.3; bf16 288 x 176 x 634 12.1 / 9.2, 567 x 67 x 178 12.9 / 13.2).
 template <typename T>
