@@ -196,8 +196,6 @@ struct Array {
     PyObject_HEAD
     PyObject *shape, *dtype, *base;
     unsigned long long ptr;
-    int64_t size;
-    int item, code;
     char owner;
 };
 
@@ -272,9 +270,6 @@ int array_init(Array* self, PyObject* args, PyObject* kw) {
     Py_XSETREF(self->dtype, dtype);
     Py_INCREF(base);
     Py_XSETREF(self->base, base);
-    self->size = size;
-    self->item = item;
-    self->code = code;
     if (ptr == Py_None) {
         uintptr_t p;
         const int64_t bytes = size > INT64_MAX / 8 ? INT64_MAX : size * item;
@@ -292,6 +287,7 @@ int array_init(Array* self, PyObject* args, PyObject* kw) {
 }
 int array_traverse(Array* self, visitproc visit, void* arg) {
     Py_VISIT(self->shape);
+    Py_VISIT(self->dtype);
     Py_VISIT(self->base);
     return 0;
 }
@@ -307,52 +303,56 @@ void array_dealloc(Array* self) {
     Py_XDECREF(self->base);
     Py_TYPE(self)->tp_free((PyObject*)self);
 }
-PyObject* array_size(Array* self, void*) { return PyLong_FromLongLong(self->size); }
-PyObject* array_ndim(Array* self, void*) { return PyLong_FromSsize_t(self->shape != nullptr ? PyTuple_GET_SIZE(self->shape) : 0); }
-PyObject* array_nbytes(Array* self, void*) { return PyLong_FromLongLong(self->size * self->item); }
-
-PyObject* attribute(PyObject* value, const char* name) {
-    if (value == nullptr) PyErr_SetString(PyExc_AttributeError, name);       // __init__ has not run
-    Py_XINCREF(value);
-    return value;
-}
-PyObject* array_shape(Array* self, void*) { return attribute(self->shape, "shape"); }
-PyObject* array_dtype(Array* self, void*) { return attribute(self->dtype, "dtype"); }
-// The caller's to answer for, as with the attributes of a Python object: the memory stays as it is
-int array_set_shape(Array* self, PyObject* value, void*) {
-    int64_t size;
-    PyObject* shape = value != nullptr ? shape_tuple(value) : PyErr_Format(PyExc_AttributeError, "shape cannot be deleted");
-    if (shape == nullptr) return -1;
-    if (!shape_size(shape, &size)) {
-        Py_DECREF(shape);
-        return -1;
+// shape and dtype may be set, as attributes of any Python object: what follows from them is worked out when it is asked for
+bool size_now(Array* self, int64_t* size) {
+    PyObject* shape = self->shape != nullptr ? shape_tuple(self->shape) : nullptr;
+    if (shape == nullptr) {
+        if (self->shape == nullptr) PyErr_SetString(PyExc_AttributeError, "shape");      // __init__ has not run
+        return false;
     }
-    Py_XSETREF(self->shape, shape);
-    self->size = size;
-    return 0;
+    const bool ok = shape_size(shape, size);
+    Py_DECREF(shape);
+    return ok;
 }
-int array_set_dtype(Array* self, PyObject* value, void*) {
+bool type_now(Array* self, int* item, int* code) {
+    if (self->dtype != nullptr) return storage_type(self->dtype, item, code) != nullptr;
+    PyErr_SetString(PyExc_AttributeError, "dtype");
+    return false;
+}
+PyObject* array_size(Array* self, void*) {
+    int64_t size;
+    return size_now(self, &size) ? PyLong_FromLongLong(size) : nullptr;
+}
+PyObject* array_ndim(Array* self, void*) {
+    if (self->shape == nullptr) return PyErr_Format(PyExc_AttributeError, "shape");
+    const Py_ssize_t n = PyObject_Length(self->shape);
+    return n < 0 ? nullptr : PyLong_FromSsize_t(n);
+}
+PyObject* array_nbytes(Array* self, void*) {
+    int64_t size;
     int item, code;
-    PyObject* dtype = value != nullptr ? storage_type(value, &item, &code) : PyErr_Format(PyExc_AttributeError, "dtype cannot be deleted");
-    if (dtype == nullptr) return -1;
-    Py_INCREF(dtype);
-    Py_XSETREF(self->dtype, dtype);
-    self->item = item;
-    self->code = code;
-    return 0;
+    return size_now(self, &size) && type_now(self, &item, &code) ? PyLong_FromLongLong(size * item) : nullptr;
+}
+PyObject* array_itemsize(Array* self, void*) {
+    int item, code;
+    return type_now(self, &item, &code) ? PyLong_FromLong(item) : nullptr;
+}
+PyObject* array_code(Array* self, void*) {
+    int item, code;
+    return type_now(self, &item, &code) ? PyLong_FromLong(code) : nullptr;
 }
 
 PyMemberDef array_members[] = {
+    {"shape", T_OBJECT_EX, offsetof(Array, shape), 0, nullptr},
+    {"dtype", T_OBJECT_EX, offsetof(Array, dtype), 0, nullptr},
     {"ptr", T_ULONGLONG, offsetof(Array, ptr), 0, nullptr},
-    {"itemsize", T_INT, offsetof(Array, item), READONLY, nullptr},
-    {"code", T_INT, offsetof(Array, code), READONLY, nullptr},
     {"_base", T_OBJECT, offsetof(Array, base), 0, nullptr},
     {"_owner", T_BOOL, offsetof(Array, owner), 0, nullptr},
     {nullptr, 0, 0, 0, nullptr},
 };
 PyGetSetDef array_getset[] = {
-    {"shape", (getter)array_shape, (setter)array_set_shape, nullptr, nullptr},
-    {"dtype", (getter)array_dtype, (setter)array_set_dtype, nullptr, nullptr},
+    {"itemsize", (getter)array_itemsize, nullptr, nullptr, nullptr},
+    {"code", (getter)array_code, nullptr, nullptr, nullptr},
     {"size", (getter)array_size, nullptr, nullptr, nullptr},
     {"ndim", (getter)array_ndim, nullptr, nullptr, nullptr},
     {"nbytes", (getter)array_nbytes, nullptr, nullptr, nullptr},
